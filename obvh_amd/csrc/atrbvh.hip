@@ -8,21 +8,20 @@
 //  (sort)         stable radix sort of (code, face) over 63 bits (rocPRIM),
 //                 the equivalent of cub::DeviceRadixSort (CubWrapper.cu:8-46)
 //  atr_tree       Karras radix tree, duplicates split by 64 + clz(i ^ j)
-//                 (LBVH.cu:156-302), written in kr_bvh_node layout
-//  atr_boxes      bottom-up working boxes and areas (LBVH.cu:414-446,551-665)
+//                 (LBVH.cu:156-302), and the leaves, as 64-byte working records
 //  atr_treelets   one optimiser pass: bottom-up over the current tree; a node
 //                 holding at least gamma triangles is optimised as a treelet
 //                 root right after its subtree (AgglomerativeTreelet.cu:
-//                 405-561, Treelet.cuh:55-127).  A half-wave (32 lanes) of
-//                 the wave whose lane completes the node forms the treelet
-//                 (largest-area expansion), builds the distance matrix
+//                 405-561, Treelet.cuh:55-127).  A half-wave (32 lanes) forms
+//                 the treelet (largest-area expansion), takes the distances
 //                 (union box areas), merges the closest pair ts-1 times and
-//                 writes the new topology when its SAH is lower; the two
-//                 halves take two treelets at once.  Each half runs the
-//                 reference's 32-lane __shfl_down tournaments exactly, so
-//                 ties resolve as in the warp code.
-//  (final)        leaf bounds from the working boxes, then bounds / counts /
-//                 costs bottom-up with kr_aabb_expand (atrbvh.cu:95-179).
+//                 writes the new topology when its SAH is lower, choosing as
+//                 the reference's 32-lane __shfl_down tournaments do, ties
+//                 included; then it goes on with the parent.  The first pass
+//                 also makes the working boxes and areas (LBVH.cu:551-665).
+//  atr_export     nodes, parents and leaf bounds from the records
+//  (final)        bounds / counts / costs bottom-up with kr_aabb_expand
+//                 (atrbvh.cu:95-179).
 // Every bottom-up pass uses the phased arrival protocol of phased.hpp.
 // Working-box min/max order -0 below +0 (as fminf/fmaxf on the reference
 // GPU); the final bounds use kr_min/kr_max like kr_aabb_expand.
@@ -53,12 +52,6 @@ __device__ __forceinline__ float box_area3(float x, float y, float z) { return 2
 __device__ __forceinline__ float box_area(float4 mn, float4 mx) {
     return box_area3(mx.x - mn.x, mx.y - mn.y, mx.z - mn.z);
 }
-// calculateBoundingBoxAndSurfaceArea (Commons.cuh:173-181)
-__device__ __forceinline__ float union_area(float4 amn, float4 amx, float4 bmn, float4 bmx) {
-    return box_area3(zmax(amx.x, bmx.x) - zmin(amn.x, bmn.x), zmax(amx.y, bmx.y) - zmin(amn.y, bmn.y),
-                     zmax(amx.z, bmx.z) - zmin(amn.z, bmn.z));
-}
-
 // calculateLeafBoundingBox (LBVH.cu:414-430)
 __device__ __forceinline__ void tri_box(const kr_vec3* V, const kr_uvec4 f, float4& mn, float4& mx) {
     const f3 a = ldv3a(V, f.x), b = ldv3a(V, f.y), c = ldv3a(V, f.z);
@@ -158,20 +151,46 @@ __device__ __forceinline__ int lcp64(const uint64_t* k, int n, int i, int j, uin
     return __clzll((long long)(ki ^ kj));
 }
 
-__global__ void atr_tree(uint32_t nf, AtrWs ws, kr_bvh_node* nodes, uint32_t* parents) {
+// Working record of a node, four float4 (64 B, half a cache line, so that one
+// trip to memory brings everything a treelet reads of a node):
+//   [0] box min, surface area        [1] box max, SAH cost of the subtree
+//   [2] left, right, parent, 0       (a leaf: face id, 0, parent, 0)
+//   [3] first and last leaf position, triangles below, 0
+// The box has fminf/fmaxf semantics with -0 below +0.  `nodes` and `parents`
+// are written from the records once, after the optimiser (atr_export).
+struct AtrRec {
+    float4* r;
+    __device__ __forceinline__ explicit AtrRec(const AtrWs& ws, uint32_t node) : r(ws.rec + 4 * (size_t)node) {}
+    __device__ __forceinline__ uint4 topo() const { return *reinterpret_cast<const uint4*>(r + 2); }
+    __device__ __forceinline__ uint4 span() const { return *reinterpret_cast<const uint4*>(r + 3); }
+    __device__ __forceinline__ void set_sah(float v) const { reinterpret_cast<float*>(r + 1)[3] = v; }
+    __device__ __forceinline__ void set_kids(uint32_t l, uint32_t rr) const {
+        *reinterpret_cast<uint2*>(r + 2) = make_uint2(l, rr);
+    }
+    __device__ __forceinline__ void set_parent(uint32_t p) const { reinterpret_cast<uint32_t*>(r + 2)[2] = p; }
+    __device__ __forceinline__ void set_span(uint32_t lo, uint32_t hi, uint32_t tri) const {
+        *reinterpret_cast<uint4*>(r + 3) = make_uint4(lo, hi, tri, 0u);
+    }
+};
+
+__global__ __launch_bounds__(256) void atr_tree(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, float ct, AtrWs ws) {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int n = (int)nf;
     const uint32_t I = nf - 1;
-    if (nf == 1) {
-        if (i == 0) {
-            kr_bvh_node L = {};
-            L.u.primitivesOffset = ws.vals_out[0];
-            L.nPrimitives = 1;
-            nodes[0] = L;
-            parents[0] = kNoNode;
-        }
-        return;
+    if (i >= n) return;
+    {  // leaf i in code order
+        const uint32_t face = ws.vals_out[i];
+        const AtrRec L(ws, I + (uint32_t)i);
+        float4 mn, mx;
+        tri_box(V, F[face], mn, mx);
+        mn.w = box_area(mn, mx);
+        mx.w = ct * mn.w;
+        L.r[0] = mn;
+        L.r[1] = mx;
+        L.set_kids(face, 0u);
+        L.set_span((uint32_t)i, (uint32_t)i, 1u);
     }
+    if (i == 0) AtrRec(ws, 0u).set_parent(kNoNode);  // the root (or the only leaf)
     if (i >= n - 1) return;
     const uint64_t* k = ws.keys_out;
     const uint64_t ki = k[i];
@@ -193,69 +212,50 @@ __global__ void atr_tree(uint32_t nf, AtrWs ws, kr_bvh_node* nodes, uint32_t* pa
         divisor <<= 1;
     }
     const int split = i + s * dir + min(dir, 0);
-    uint32_t li = (uint32_t)split, ri = (uint32_t)split + 1;
-    if (min(i, j) == split) {
-        li = (uint32_t)split + I;
-        kr_bvh_node L = {};
-        L.u.primitivesOffset = ws.vals_out[split];
-        L.nPrimitives = 1;
-        nodes[li] = L;
-    }
-    if (max(i, j) == split + 1) {
-        ri = (uint32_t)split + 1 + I;
-        kr_bvh_node R = {};
-        R.u.primitivesOffset = ws.vals_out[split + 1];
-        R.nPrimitives = 1;
-        nodes[ri] = R;
-    }
-    kr_bvh_node N = {};
-    N.u.children.left = li;
-    N.u.children.right = ri;
-    nodes[i] = N;
-    parents[li] = (uint32_t)i;
-    parents[ri] = (uint32_t)i;
-    if (i == 0) parents[0] = kNoNode;
-}
-
-struct AtrBoxUp {
-    const kr_vec3* V;
-    const kr_uvec4* F;
-    const kr_bvh_node* nodes;
-    AtrWs ws;
-    __device__ void leaf(uint32_t cur) {
-        float4 mn, mx;
-        tri_box(V, F[nodes[cur].u.primitivesOffset], mn, mx);
-        ws.bmin[cur] = mn;
-        ws.bmax[cur] = mx;
-        ws.area[cur] = box_area(mn, mx);
-    }
-    __device__ void merge(uint32_t p, uint32_t l, uint32_t r) {
-        const float4 amn = ws.bmin[l], amx = ws.bmax[l], bmn = ws.bmin[r], bmx = ws.bmax[r];
-        const float4 mn = make_float4(zmin(amn.x, bmn.x), zmin(amn.y, bmn.y), zmin(amn.z, bmn.z), 0.0f);
-        const float4 mx = make_float4(zmax(amx.x, bmx.x), zmax(amx.y, bmx.y), zmax(amx.z, bmx.z), 0.0f);
-        ws.bmin[p] = mn;
-        ws.bmax[p] = mx;
-        ws.area[p] = box_area(mn, mx);
-    }
-};
-
-__global__ __launch_bounds__(1024) void atr_boxes(const kr_vec3* V, const kr_uvec4* F, const kr_bvh_node* nodes,
-                                                  const uint32_t* parents, uint32_t nf, AtrWs ws, uint32_t phase,
-                                                  uint32_t chunk) {
-    AtrBoxUp op{V, F, nodes, ws};
-    phased_up(nodes, parents, nf, ws.ph, phase, chunk, op);
+    const uint32_t li = (uint32_t)split + (min(i, j) == split ? I : 0u);
+    const uint32_t ri = (uint32_t)split + 1 + (max(i, j) == split + 1 ? I : 0u);
+    AtrRec(ws, (uint32_t)i).set_kids(li, ri);
+    AtrRec(ws, li).set_parent((uint32_t)i);
+    AtrRec(ws, ri).set_parent((uint32_t)i);
 }
 
 __global__ void atr_clear(AtrWs ws, uint32_t nf) { phase_clear(ws.ph, nf); }
 
 // ------------------------------------------------------- optimiser --
+//
+// A treelet is a chain of dependent steps (find the largest leaf, read its
+// children, again; find the closest pair, merge, again), so a pass is bound
+// by latency: tree levels x time per treelet (a 200 K-triangle hairball has
+// 24 levels of treelet roots; the phases' longest paths add up to 47).  Hence
+//  - one half-wave (32 lanes, as the reference's warps) per treelet and per
+//    path to the root: the lanes climb alone below the first treelet roots,
+//    which go to a ready list; the half-waves of the workgroup then take
+//    roots from it and each follows its path upwards.  (Running the treelets
+//    on the wave whose lane completed the node put a phase's few roots,
+//    neighbours in the deferred list, on one wave, two at a time.  A whole
+//    wave per treelet makes one 10 % faster but halves their number in
+//    flight: 1.75 against 1.65 ms for the build and transform below);
+//  - one 64-byte record per node and the top four levels of a treelet's
+//    subtree read level by level: four trips to memory instead of two per
+//    expansion;
+//  - tournaments as integer DPP minima and a ballot instead of shuffle
+//    rounds, boxes in LDS, distances in registers.
+// 200 K-triangle hairball, treelet size 9, 2 passes: 5529 -> 930 us; a treelet
+// takes about 20 K cycles (5 K reading, 4 K forming, 10 K merging).
+
+constexpr int kDistStride = kMaxTreelet + 1;  // odd: the lanes of a row update touch different banks
 
 struct TreeletLds {
-    uint32_t tin[kMaxTreelet];
-    uint32_t tl[kMaxTreelet];
-    float ta[kMaxTreelet];  // leaf areas, then the SAH of the merged nodes
-    float dist[kMaxTreelet * (kMaxTreelet - 1) / 2];
+    float4 box[kMaxTreelet][2];  // treelet leaf: min, SAH; max, node id
+    uint2 kids[kMaxTreelet];     // its children; after its merge step, those of the node the step made
+    float area[kMaxTreelet];
+    float dist[kMaxTreelet * kDistStride];  // union areas, [row][column], row > column
 };
+
+constexpr int kHalf = 32;
+constexpr int kHeapLevels = 4;  // levels below a treelet root loaded at once
+constexpr int kHeapNodes = (2 << kHeapLevels) - 2;
+constexpr int kPairSteps = (kMaxTreelet * (kMaxTreelet - 1) / 2 + kHalf - 1) / kHalf;  // distance entries per lane
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -266,272 +266,488 @@ __device__ __forceinline__ void wave_sync() {
 __device__ __forceinline__ int trm_row(int index) { return (int)((-1 + sqrtf(8.0f * index + 1)) / 2) + 1; }
 __device__ __forceinline__ int trm_index(int row, int col) { return ((row - 1) * row) / 2 + col; }
 
-__device__ __forceinline__ float4 shfl4(float4 v, int src) {
-    return make_float4(__shfl(v.x, src), __shfl(v.y, src), __shfl(v.z, src), 0.0f);
+// Lane a of the lower half's value in the lower half, lane b of the upper
+// half's in the upper half (a, b uniform, within the half).
+__device__ __forceinline__ uint32_t half_pick(uint32_t v, int a, int b, bool upper) {
+    const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)v, a);
+    const uint32_t y = (uint32_t)__builtin_amdgcn_readlane((int)v, kHalf + b);
+    return upper ? y : x;
+}
+__device__ __forceinline__ float half_pickf(float v, int a, int b, bool upper) {
+    return __uint_as_float(half_pick(__float_as_uint(v), a, b, upper));
+}
+// Integer min / max over each half (every lane active).
+template <bool MIN>
+__device__ __forceinline__ int32_t half_reduce(int32_t v, bool upper) {
+    auto f = [](int32_t a, int32_t b) { return MIN ? min(a, b) : max(a, b); };
+    v = f(v, dpp_mov<0xB1>(v));
+    v = f(v, dpp_mov<0x4E>(v));
+    v = f(v, dpp_mov<0x141>(v));
+    v = f(v, dpp_mov<0x140>(v));
+    const int32_t a = f(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16));
+    const int32_t b = f(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48));
+    return upper ? b : a;
+}
+// The other lane of a pair (lane ^ 1).
+__device__ __forceinline__ float dpp_xor1(float v) {
+    const int i = __float_as_int(v);
+    return __int_as_float(dpp_mov<0xB1>(i));
+}
+__device__ __forceinline__ uint32_t dpp_xor1(uint32_t v) {
+    return (uint32_t)dpp_mov<0xB1>((int)v);
 }
 
-// Optimise the treelet rooted at `root` with one half of the wave: lanes
-// 0-31 and 32-63 each take a treelet (`valid` false: that half idles), as
-// the reference's 32-lane warps do; every tournament is a width-32
-// shuffle-down within the half, so ties break as in the warp code.  All 64
-// lanes execute (the loops depend only on ts).  Two treelets found in the
-// same round of the climb have disjoint subtrees, so running them together
-// equals running them one after the other.
-__device__ void treelet_half(uint32_t root, bool valid, kr_bvh_node* nodes, uint32_t* parents, const AtrWs& ws,
-                             uint32_t N, int ts, float ci, TreeletLds& S) {
-    const int hl = lane_id() & 31;  // lane within the half
-    const int hb = lane_id() & 32;  // first lane of the half
-    const uint32_t I = N - 1;
-    // formTreelet: expand the treelet leaf with the largest area ts-2 times
-    if (valid && hl == 0) {
-        const uint32_t L = nodes[root].u.children.left, R = nodes[root].u.children.right;
-        S.tin[0] = root;
-        S.tl[0] = L;
-        S.tl[1] = R;
-        S.ta[0] = ws.area[L];
-        S.ta[1] = ws.area[R];
-    }
-    wave_sync();
-    for (int it = 0; it < ts - 2; ++it) {
-        int idx = -1;
-        float a = -FLT_MAX;
-        if (valid && hl < 2 + it) {
-            idx = hl;
-            a = S.tl[hl] >= I ? -FLT_MAX : S.ta[hl];
-        }
-        for (int n = 2 + it, amount = n / 2; n > 1; n = (n + 1) / 2, amount = n / 2) {
-            const int oi = __shfl_down(idx, amount, 32);
-            const float oa = __shfl_down(a, amount, 32);
-            if (oa > a) { a = oa; idx = oi; }
-        }
-        if (valid && hl == 0) {
-            const uint32_t rep = S.tl[idx];
-            const uint32_t l2 = nodes[rep].u.children.left, r2 = nodes[rep].u.children.right;
-            S.tin[it + 1] = rep;
-            S.tl[idx] = l2;
-            S.tl[it + 2] = r2;
-            S.ta[idx] = ws.area[l2];
-            S.ta[it + 2] = ws.area[r2];
-        }
-        wave_sync();
-    }
-    // lane state: node, subtree SAH, box of treelet leaf `hl`
-    uint32_t tnode = 0;
-    float tsah = 0.0f;
-    float4 bmn = make_float4(0, 0, 0, 0), bmx = bmn;
-    if (valid && hl < ts) {
-        tnode = S.tl[hl];
-        tsah = ws.sah[tnode];
-        bmn = ws.bmin[tnode];
-        bmx = ws.bmax[tnode];
-    }
-    // distance matrix: union areas of every pair (row > col)
+// Box min / max.  v_min_f32 and v_max_f32 order -0 below +0 and so equal zmin
+// and zmax on values that are not NaN; kSane says that they are not.
+template <bool kSane>
+__device__ __forceinline__ float bmin(float a, float b) {
+    if (!kSane) return zmin(a, b);
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+template <bool kSane>
+__device__ __forceinline__ float bmax(float a, float b) {
+    if (!kSane) return zmax(a, b);
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// calculateBoundingBoxAndSurfaceArea (Commons.cuh:173-181)
+template <bool kSane>
+__device__ __forceinline__ float join_area(float4 amn, float4 amx, float4 bmn, float4 bmx) {
+    return box_area3(bmax<kSane>(amx.x, bmx.x) - bmin<kSane>(amn.x, bmn.x),
+                     bmax<kSane>(amx.y, bmx.y) - bmin<kSane>(amn.y, bmn.y),
+                     bmax<kSane>(amx.z, bmx.z) - bmin<kSane>(amn.z, bmn.z));
+}
+
+// The ts - 1 merges of the closest pair (AgglomerativeTreelet.cu:80-222) over
+// the treelet leaves in S, one treelet per half of the wave.  The step at
+// `last` leaves in slot `last` the node it makes: box, SAH and children (its
+// id is tin[last - 1]).  Returns the SAH of the whole treelet.
+//
+// The closest-pair search of a half is the reference's 32-lane strided scan
+// and __shfl_down tournament: among equal distances the lane (entry mod 32)
+// whose bit-reversed number is lowest wins, and within a lane the lowest
+// entry.  Lane hl plays the reference's lane rev(hl) (`logical`), so the winner
+// is the lowest set bit of a ballot.
+//
+// kSane: every box coordinate is below 2^61 in magnitude, so distances are
+// finite and not negative (their bits order as integers) and the union is
+// symmetric: each lane keeps its entries' distances in registers and makes
+// those that a merge touches again from the boxes.  A wave alone on its SIMD
+// issues this chain at about 5 cycles an instruction, so its length is its
+// time (1400 cycles per merge while the matrix was moved through LDS, as the
+// general form still does).
+template <bool kSane>
+__device__ __forceinline__ float treelet_merge(TreeletLds& S, int ts, float ci, int hl, int logical, bool upper,
+                                               uint32_t tin, const uint32_t (&pair_rc)[kPairSteps]) {
     const int npairs = ts * (ts - 1) / 2;
-    for (int base = 0; base < npairs; base += 32) {
-        const int e = base + hl;
-        int r = 0, c = 0;
-        if (e < npairs) {
-            r = trm_row(e);
-            c = e - trm_index(r, 0);
-        }
-        const float4 amn = shfl4(bmn, hb + r), amx = shfl4(bmx, hb + r), cmn = shfl4(bmn, hb + c),
-                     cmx = shfl4(bmx, hb + c);
-        if (e < npairs) S.dist[e] = union_area(amn, amx, cmn, cmx);
+    float dist[kPairSteps];
+    auto entry = [&](int k) { return (int)(pair_rc[k] >> 8) * kDistStride + (int)(pair_rc[k] & 255u); };
+    auto measure = [&](int k) {
+        const int r = (int)(pair_rc[k] >> 8), c = (int)(pair_rc[k] & 255u);
+        return join_area<kSane>(S.box[r][0], S.box[r][1], S.box[c][0], S.box[c][1]);
+    };
+#pragma unroll
+    for (int k = 0; k < kPairSteps; ++k) {
+        if (kHalf * k >= npairs) break;
+        dist[k] = measure(k);
+        if (!kSane && logical + kHalf * k < npairs) S.dist[entry(k)] = dist[k];
     }
     wave_sync();
+    float total = 0.0f;
     for (int last = ts - 1; last > 0; --last) {
-        // findMinimumDistance: 32 lanes, strided, then the shfl_down tournament
         const int size = last * (1 + last) / 2;
-        float md = FLT_MAX;
-        int mi = 0;
-        for (int j = hl; j < size; j += 32) {
-            const float d = S.dist[j];
-            if (d < md) { md = d; mi = j; }
+        // findMinimumDistance
+        float moved = 0.0f;
+        if (!kSane) moved = S.dist[last * kDistStride + min(hl, kMaxTreelet)];
+        int32_t key = 0x7F7FFFFF;  // FLT_MAX
+        uint32_t rc = 1u << 8;     // entry 0
+#pragma unroll
+        for (int k = 0; k < kPairSteps; ++k) {
+            if (kHalf * k >= size) break;
+            const float d = kSane ? dist[k] : S.dist[entry(k)];
+            const int32_t kk = kSane ? __float_as_int(d) : f2ord(d + 0.0f);
+            if (logical + kHalf * k < size && (kSane || d < FLT_MAX) && kk < key) { key = kk; rc = pair_rc[k]; }
         }
-        for (int n = 32, amount = 16; n > 1; n = (n + 1) / 2, amount = n / 2) {
-            const int oi = __shfl_down(mi, amount, 32);
-            const float od = __shfl_down(md, amount, 32);
-            if (od < md) { md = od; mi = oi; }
-        }
-        const int min_index = __shfl(mi, hb);
-        const int row = trm_row(min_index), col = min_index - trm_index(row, 0);
+        const int32_t best = half_reduce<true>(key, upper);
+        const uint64_t eq = __ballot(key == best);
+        rc = half_pick(rc, __builtin_ctz((uint32_t)eq), __builtin_ctz((uint32_t)(eq >> 32)), upper);
+        const int row = (int)(rc >> 8), col = (int)(rc & 255u);
         // updateState
-        const float s = __shfl(tsah, hb + row) + __shfl(tsah, hb + col);
-        const uint32_t li = (uint32_t)__shfl((int)tnode, hb + row), ri = (uint32_t)__shfl((int)tnode, hb + col);
-        float4 amn = shfl4(bmn, hb + row), amx = shfl4(bmx, hb + row);
-        const float4 cmn = shfl4(bmn, hb + col), cmx = shfl4(bmx, hb + col);
-        amn = make_float4(zmin(cmn.x, amn.x), zmin(cmn.y, amn.y), zmin(cmn.z, amn.z), 0.0f);
-        amx = make_float4(zmax(cmx.x, amx.x), zmax(cmx.y, amx.y), zmax(cmx.z, amx.z), 0.0f);
-        if (hl == col) {
-            tnode = S.tin[last - 1];
-            bmn = amn;
-            bmx = amx;
-            S.ta[last] = s + ci * box_area(amn, amx);
-            tsah = S.ta[last];
+        const float4 r0 = S.box[row][0], r1 = S.box[row][1], c0 = S.box[col][0], c1 = S.box[col][1];
+        const float4 l0 = S.box[last][0], l1 = S.box[last][1];
+        const float4 nmn = make_float4(bmin<kSane>(c0.x, r0.x), bmin<kSane>(c0.y, r0.y), bmin<kSane>(c0.z, r0.z), 0.0f);
+        const float4 nmx = make_float4(bmax<kSane>(c1.x, r1.x), bmax<kSane>(c1.y, r1.y), bmax<kSane>(c1.z, r1.z), 0.0f);
+        total = (r0.w + c0.w) + ci * box_area(nmn, nmx);
+        const uint32_t made = half_pick(tin, last - 1, last - 1, upper);
+        wave_sync();
+        if (hl == row) {  // the last slot moves to the pair's free slot
+            S.box[row][0] = l0;
+            S.box[row][1] = l1;
         }
-        const uint32_t last_node = (uint32_t)__shfl((int)tnode, hb + last);
-        const float last_sah = __shfl(tsah, hb + last);
-        const float4 lmn = shfl4(bmn, hb + last), lmx = shfl4(bmx, hb + last);
-        if (hl == row) {
-            tnode = last_node;
-            tsah = last_sah;
-            bmn = lmn;
-            bmx = lmx;
+        if (hl == col || hl == last) {
+            S.box[hl][0] = make_float4(nmn.x, nmn.y, nmn.z, total);
+            S.box[hl][1] = make_float4(nmx.x, nmx.y, nmx.z, __uint_as_float(made));
         }
-        if (hl == last) {
-            tnode = li;
-            S.tl[last] = ri;
-            bmn = amn;
-            bmx = amx;
-        }
+        if (hl == last) S.kids[last] = make_uint2(__float_as_uint(r1.w), __float_as_uint(c1.w));
         wave_sync();
         // updateDistancesMatrix
-        if (last > 1) {
-            if (hl < last && hl != row) {
-                const float v = S.dist[trm_index(last, hl)];
-                S.dist[trm_index(max(row, hl), min(row, hl))] = v;
+        if (kSane) {
+#pragma unroll
+            for (int k = 0; k < kPairSteps; ++k) {
+                if (kHalf * k >= size - last) break;  // the entries of the next step
+                const int r = (int)(pair_rc[k] >> 8), c = (int)(pair_rc[k] & 255u);
+                const float d = measure(k);
+                if (r == row || r == col || c == row || c == col) dist[k] = d;
             }
+        } else if (hl < last) {
+            if (hl != row) S.dist[max(row, hl) * kDistStride + min(row, hl)] = moved;
             wave_sync();
-            int dr = hl, dc = hl;
-            if (hl < last && hl != col) {
-                dr = max(col, hl);
-                dc = min(col, hl);
-            }
-            const float4 xmn = shfl4(bmn, hb + (dr & 31)), xmx = shfl4(bmx, hb + (dr & 31));
-            const float4 ymn = shfl4(bmn, hb + (dc & 31)), ymx = shfl4(bmx, hb + (dc & 31));
-            if (hl < last && hl != col) S.dist[trm_index(dr, dc)] = union_area(xmn, xmx, ymn, ymx);
+            const int a = max(col, hl), b = min(col, hl);
+            if (hl != col)
+                S.dist[a * kDistStride + b] = join_area<false>(S.box[a][0], S.box[a][1], S.box[b][0], S.box[b][1]);
         }
         wave_sync();
     }
-    // updateTreelet: keep the new topology when its SAH is lower
-    if (valid && S.ta[1] < ws.sah[S.tin[0]]) {
-        if (hl >= 1 && hl < ts) {
-            const uint32_t v = S.tin[hl - 1];
-            const uint32_t right = S.tl[hl];
-            nodes[v].u.children.left = tnode;
-            nodes[v].u.children.right = right;
-            parents[tnode] = v;
-            parents[right] = v;
-            ws.sah[v] = S.ta[hl];
-            ws.bmin[v] = bmn;
-            ws.bmax[v] = bmx;
-            ws.area[v] = box_area(bmn, bmx);
-        }
-    }
-    wave_sync();
+    return total;
 }
 
-// One optimiser pass, one phase of the bottom-up protocol (phased.hpp), with
-// a wave-uniform climb so that whole waves can stop to optimise treelets.
-__global__ __launch_bounds__(1024) void atr_treelets(kr_bvh_node* nodes, uint32_t* parents, AtrWs ws, uint32_t nf,
-                                                     int ts, int gamma, float ci, float ct, uint32_t phase,
-                                                     uint32_t chunk) {
-    __shared__ TreeletLds lds[2 * 1024 / kWave];
-    TreeletLds& S = lds[2 * wave_id() + (lane_id() >> 5)];
+// One optimiser pass, one phase of the bottom-up protocol (phased.hpp).
+// kFirst: the pass also makes the internal nodes' working boxes.
+template <bool kFirst, int kThreads>
+__global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, int ts, int gamma, float ci,
+                                                     uint32_t phase, uint32_t chunk) {
+    __shared__ TreeletLds lds[kThreads / kHalf];
+    __shared__ uint32_t nready, nextready;
     const uint32_t I = nf - 1;
     const uint32_t tag = (phase << 24) | (blockIdx.x + 1u);
     const uint64_t lo = (uint64_t)blockIdx.x * chunk, hi = lo + chunk;
     const uint32_t nin = phase == 0 ? 0 : min(ws.ph.nlist[phase - 1], I);
     const uint2* in = phase == 0 ? nullptr : ws.ph.list + (size_t)(phase - 1) * (I + 1);
     uint2* out = ws.ph.list + (size_t)phase * (I + 1);
+    // The roots this workgroup takes have disjoint leaf spans inside its
+    // chunk, so there are at most `chunk` of them.
+    uint32_t* ready = ws.ready + lo;
+    if (threadIdx.x == 0) nready = nextready = 0;
+    __syncthreads();
+    auto defer = [&](uint32_t node, uint32_t key) {
+        const uint32_t slot = atomicAdd(&ws.ph.nlist[phase], 1u);
+        if (slot < I) out[slot] = make_uint2(node, key);
+    };
+
+    // Below the treelet roots: one lane per leaf (or deferred node).
     const uint32_t nstart = phase == 0 ? chunk : nin;
-    for (uint32_t base = 0; base < nstart; base += blockDim.x) {  // uniform over the workgroup
-        const uint32_t r0 = base + threadIdx.x;
-        bool active = false, at_node = false;
-        uint32_t cur = 0, p = kNoNode, steps = 0;
-        uint2 span = make_uint2(0, 0);
-        if (r0 < nstart) {
-            if (phase == 0) {
-                const uint64_t pos = lo + r0;
-                if (pos < nf) {
-                    cur = I + (uint32_t)pos;
-                    ws.tri[cur] = 1;
-                    ws.sah[cur] = ct * ws.area[cur];
-                    span = make_uint2((uint32_t)pos, (uint32_t)pos);
-                    ws.ph.span[cur] = span;
-                    p = parents[cur];
-                    active = true;
+    for (uint32_t r0 = threadIdx.x; r0 < nstart; r0 += blockDim.x) {
+        uint32_t p;          // the node to complete next
+        bool both = false;   // its children are known to be complete
+        uint32_t key;        // a leaf position below it
+        if (phase == 0) {
+            const uint64_t pos = lo + r0;
+            if (pos >= nf) break;
+            key = (uint32_t)pos;
+            p = AtrRec(ws, I + key).topo().z;
+        } else {
+            // Ownership comes from the listed key only: once its owner has
+            // completed the node and an ancestor, a treelet there may rewire
+            // the node's children while other workgroups still scan this
+            // list.
+            const uint2 e = in[r0];
+            p = e.x;
+            key = e.y;
+            if (p >= I || key < lo || key >= hi) continue;
+            const uint4 t = AtrRec(ws, p).topo();
+            const uint4 sl = AtrRec(ws, t.x).span(), sr = AtrRec(ws, t.y).span();
+            if (min(sl.x, sr.x) < lo || max(sl.y, sr.y) >= hi) {  // wider than this workgroup: next phase
+                defer(p, min(sl.x, sr.x));
+                continue;
+            }
+            both = true;
+        }
+        for (uint32_t step = 0; p < I && step < nf; ++step) {
+            const AtrRec P(ws, p);
+            const uint4 t = P.topo();
+            if (!both) {
+                const uint64_t old = __hip_atomic_fetch_add(&ws.ph.visit[p], ((uint64_t)tag << 32) | 1ull,
+                                                            __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+                const uint32_t t1 = (uint32_t)(old >> 32);
+                if ((uint32_t)old == 0) break;  // first arrival: the sibling continues
+                if (t1 != tag && (t1 >> 24) >= phase) {
+                    defer(p, key);
+                    break;
                 }
+            }
+            both = false;
+            const AtrRec L(ws, t.x), R(ws, t.y);
+            const uint4 sl = L.span(), sr = R.span();
+            const uint32_t tri = sl.z + sr.z;
+            if ((int32_t)tri >= gamma) {
+                const uint32_t slot = atomicAdd(&nready, 1u);
+                if (slot < chunk && lo + slot < nf) ready[slot] = p;  // always (the roots' spans are disjoint)
+                break;
+            }
+            const float4 lb = L.r[1], rb = R.r[1];
+            float area;
+            if (kFirst) {
+                const float4 la = L.r[0], ra = R.r[0];
+                float4 mn = make_float4(zmin(la.x, ra.x), zmin(la.y, ra.y), zmin(la.z, ra.z), 0.0f);
+                float4 mx = make_float4(zmax(lb.x, rb.x), zmax(lb.y, rb.y), zmax(lb.z, rb.z), 0.0f);
+                area = box_area(mn, mx);
+                mn.w = area;
+                mx.w = ci * area + lb.w + rb.w;
+                P.r[0] = mn;
+                P.r[1] = mx;
             } else {
-                // Ownership comes from the listed key only: once its owner has
-                // completed the node and an ancestor, a treelet there may
-                // rewire the node's children while other workgroups still
-                // scan this list.
-                const uint2 e = in[r0];
-                cur = e.x;
-                if (cur < I && e.y >= lo && e.y < hi) {
-                    const uint32_t l = nodes[cur].u.children.left, r = nodes[cur].u.children.right;
-                    const uint2 sa = ws.ph.span[l], sb = ws.ph.span[r];
-                    span = make_uint2(min(sa.x, sb.x), max(sa.y, sb.y));
-                    if (span.x < lo || span.y >= hi) {
-                        const uint32_t slot = atomicAdd(&ws.ph.nlist[phase], 1u);
-                        if (slot < I) out[slot] = make_uint2(cur, span.x);
-                    } else {
-                        active = true;
-                        at_node = true;  // both children are complete
-                    }
+                area = P.r[0].w;
+                P.set_sah(ci * area + lb.w + rb.w);
+            }
+            P.set_span(min(sl.x, sr.x), max(sl.y, sr.y), tri);
+            p = t.z;
+        }
+    }
+    __syncthreads();
+
+    // The treelets: each half-wave takes a ready root and follows its path
+    // up to the first arrival at a node, a deferred node or the tree's root.
+    const bool upper = lane_id() >= kHalf;
+    const int hl = lane_id() & (kHalf - 1);
+    TreeletLds& S = lds[2 * wave_id() + (upper ? 1 : 0)];
+    const int logical = (int)(__brev((uint32_t)hl) >> 27);
+    uint32_t pair_rc[kPairSteps];  // row << 8 | column of distance entry logical + 32 k
+#pragma unroll
+    for (int k = 0; k < kPairSteps; ++k) {
+        const int e = min(logical + kHalf * k, kMaxTreelet * (kMaxTreelet - 1) / 2 - 1), r = trm_row(e);
+        pair_rc[k] = (uint32_t)(r << 8 | (e - trm_index(r, 0)));
+    }
+    const uint32_t nroots = (uint32_t)min((uint64_t)min(nready, chunk), (uint64_t)nf - lo);
+    bool have = false;
+    uint32_t root = 0, steps = 0;
+    uint4 rt = make_uint4(0u, 0u, kNoNode, 0u);  // the root's left, right, parent
+    for (;;) {
+        {  // idle halves take the next ready root
+            const uint64_t idle = __ballot(!have && hl == 0);
+            if (idle) {
+                uint32_t slot = 0;
+                if (!have && hl == 0) slot = atomicAdd(&nextready, 1u);
+                slot = half_pick(slot, 0, 0, upper);
+                if (!have && slot < nroots) {
+                    have = true;
+                    root = ready[slot];
+                    rt = AtrRec(ws, root).topo();
+                    steps = 0;
                 }
             }
+            if (__ballot(have) == 0) break;
         }
-        while (__ballot(active) != 0) {  // wave-uniform climb
-            bool treelet = false;
-            uint32_t node = cur;
-            if (active && !at_node) {
-                if (p == kNoNode || p >= I || ++steps > nf) {
-                    active = false;
-                } else {
-                    const uint64_t old = __hip_atomic_fetch_add(&ws.ph.visit[p], ((uint64_t)tag << 32) | 1ull,
-                                                                __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    const uint32_t t1 = (uint32_t)(old >> 32);
-                    if ((uint32_t)old == 0) {
-                        active = false;  // first arrival: the sibling continues
-                    } else if (t1 != tag && (t1 >> 24) >= phase) {
-                        const uint32_t slot = atomicAdd(&ws.ph.nlist[phase], 1u);
-                        if (slot < I) out[slot] = make_uint2(p, span.x);
-                        active = false;
-                    } else {
-                        const uint32_t l = nodes[p].u.children.left, r = nodes[p].u.children.right;
-                        span = make_uint2(min(span.x, ws.ph.span[l == cur ? r : l].x),
-                                          max(span.y, ws.ph.span[l == cur ? r : l].y));
-                        node = p;
-                        at_node = true;
-                    }
+        const AtrRec X(ws, root);
+        const uint32_t parent = rt.z;
+        uint4 pt = make_uint4(0u, 0u, kNoNode, 0u);  // the parent's topology, needed after the treelet
+        if (have && parent < I) pt = AtrRec(ws, parent).topo();
+
+        // The top four levels of the subtree, one node per lane (the children
+        // of lane x's node on lanes 2x + 2 and 2x + 3): four trips to memory
+        // instead of one per expansion.
+        uint32_t id = hl == 0 ? rt.x : rt.y, lkid = 0, rkid = 0, tin = root;
+        float4 mn = make_float4(0, 0, 0, 0), mx = mn;
+        uint4 sp = make_uint4(0u, 0u, 0u, 0u);
+        float4 xmn = mn, xmx = mn;
+        bool loaded = have && hl < 2;
+        if (loaded) {
+            const AtrRec C(ws, id);
+            mn = C.r[0];
+            mx = C.r[1];
+            const uint4 t = C.topo();
+            lkid = t.x;
+            rkid = t.y;
+            sp = C.span();
+            if (!kFirst && hl == 0) {
+                xmn = X.r[0];
+                xmx = X.r[1];
+            }
+        }
+#pragma unroll
+        for (int level = 1; level < kHeapLevels; ++level) {
+            const int first = (2 << level) - 2;  // lanes [first, 2 first + 2)
+            const int up = (hl - 2) >> 1;
+            const uint32_t pid = (uint32_t)__shfl((int)id, up, kHalf);
+            const uint32_t pl = (uint32_t)__shfl((int)lkid, up, kHalf), pr = (uint32_t)__shfl((int)rkid, up, kHalf);
+            const bool pok = __shfl((int)loaded, up, kHalf) != 0;
+            if (hl >= first && hl < 2 * first + 2 && pok && pid < I) {
+                id = (hl & 1) ? pr : pl;
+                loaded = true;
+                const AtrRec C(ws, id);
+                mn = C.r[0];
+                mx = C.r[1];
+                const uint4 t = C.topo();
+                lkid = t.x;
+                rkid = t.y;
+            }
+        }
+        // the root's own box, SAH, triangles and span (lane 0 of the half)
+        const uint32_t tri = sp.z + dpp_xor1(sp.z);
+        const uint32_t slo = min(sp.x, dpp_xor1(sp.x)), shi = max(sp.y, dpp_xor1(sp.y));
+        if (kFirst) {
+            xmn = make_float4(zmin(mn.x, dpp_xor1(mn.x)), zmin(mn.y, dpp_xor1(mn.y)), zmin(mn.z, dpp_xor1(mn.z)), 0.0f);
+            xmx = make_float4(zmax(mx.x, dpp_xor1(mx.x)), zmax(mx.y, dpp_xor1(mx.y)), zmax(mx.z, dpp_xor1(mx.z)), 0.0f);
+            xmn.w = box_area(xmn, xmx);
+        }
+        xmx.w = ci * xmn.w + mx.w + dpp_xor1(mx.w);
+
+        // formTreelet (Treelet.cuh:55-127): expand the treelet leaf with the
+        // largest area ts - 2 times.  A single largest area among values that
+        // compare is the reference's winner whatever its tournament order.
+        // The loop stops early (for both halves) at a tie, an area that does
+        // not compare, or a node whose children are below the loaded levels.
+        int slot = hl < 2 ? hl : -1;  // treelet leaf index of this lane's node
+        int it = 0;
+        for (; it < ts - 2; ++it) {
+            const bool inner = have && slot >= 0 && id < I;
+            const int32_t key = inner && mn.w >= 0.0f ? __float_as_int(mn.w + 0.0f) + 1 : 0;
+            const int32_t best = half_reduce<false>(key, upper);
+            const uint64_t eq = __ballot(key == best && have);
+            const uint32_t ea = (uint32_t)eq, eb = (uint32_t)(eq >> 32);
+            constexpr uint32_t kTop = (1u << (kHeapNodes / 2 - 1)) - 1;  // lanes whose children are loaded
+            if ((ea & (ea - 1)) != 0 || (eb & (eb - 1)) != 0 || ((ea | eb) & ~kTop) != 0 ||
+                __ballot(inner && !(mn.w >= 0.0f)) != 0)
+                break;  // wave-uniform
+            const int ia = ea ? __builtin_ctz(ea) : 0, ib = eb ? __builtin_ctz(eb) : 0;
+            const uint32_t rep = half_pick(id, ia, ib, upper);
+            const int from = (int)half_pick((uint32_t)slot, ia, ib, upper);
+            const int idx = upper ? ib : ia;
+            if (hl == it + 1) tin = rep;
+            if (hl == idx) slot = -1;
+            if (hl == 2 * idx + 2) slot = from;
+            if (hl == 2 * idx + 3) slot = it + 2;
+        }
+        // to leaf order: lane hl takes treelet leaf hl
+        if (have && slot >= 0) {
+            S.box[slot][0] = make_float4(mn.x, mn.y, mn.z, mx.w);
+            S.box[slot][1] = make_float4(mx.x, mx.y, mx.z, __uint_as_float(id));
+            S.kids[slot] = make_uint2(lkid, rkid);
+            S.area[slot] = mn.w;
+        }
+        wave_sync();
+        const int sl = min(hl, kMaxTreelet - 1);
+        {
+            const float4 b0 = S.box[sl][0], b1 = S.box[sl][1];
+            mn = make_float4(b0.x, b0.y, b0.z, S.area[sl]);
+            mx = make_float4(b1.x, b1.y, b1.z, b0.w);
+            id = __float_as_uint(b1.w);
+        }
+        // the remaining expansions, by the reference's tournament where the
+        // largest area is tied or does not compare
+        if (it < ts - 2) {
+            const uint2 kk = S.kids[sl];
+            lkid = kk.x;
+            rkid = kk.y;
+            for (; it < ts - 2; ++it) {
+                int idx = -1;
+                float w = -FLT_MAX;
+                if (have && hl < 2 + it) {
+                    idx = hl;
+                    w = id >= I ? -FLT_MAX : mn.w;
+                }
+                for (int n = 2 + it, amount = n / 2; n > 1; n = (n + 1) / 2, amount = n / 2) {
+                    const int oi = __shfl_down(idx, amount, kHalf);
+                    const float ow = __shfl_down(w, amount, kHalf);
+                    if (ow > w) { w = ow; idx = oi; }
+                }
+                const int ia = __builtin_amdgcn_readlane(idx, 0) & (kHalf - 1);
+                const int ib = __builtin_amdgcn_readlane(idx, kHalf) & (kHalf - 1);
+                const uint32_t rep = half_pick(id, ia, ib, upper);
+                const uint32_t l2 = half_pick(lkid, ia, ib, upper), r2 = half_pick(rkid, ia, ib, upper);
+                idx = upper ? ib : ia;
+                if (hl == it + 1) tin = rep;
+                if (have && (hl == idx || hl == it + 2)) {
+                    id = hl == idx ? l2 : r2;
+                    const AtrRec C(ws, id);
+                    mn = C.r[0];
+                    mx = C.r[1];
+                    const uint4 t = C.topo();
+                    lkid = t.x;
+                    rkid = t.y;
                 }
             }
-            if (active && at_node) {
-                const uint32_t l = nodes[node].u.children.left, r = nodes[node].u.children.right;
-                const int32_t tri = ws.tri[l] + ws.tri[r];
-                ws.tri[node] = tri;
-                ws.sah[node] = ci * ws.area[node] + ws.sah[l] + ws.sah[r];
-                ws.ph.span[node] = span;
-                treelet = tri >= gamma;
+            wave_sync();
+            if (hl < ts) {
+                S.box[hl][0] = make_float4(mn.x, mn.y, mn.z, mx.w);
+                S.box[hl][1] = make_float4(mx.x, mx.y, mx.z, __uint_as_float(id));
             }
-            uint64_t vote = __ballot(treelet);
-            while (vote) {  // two treelets at a time, one per half-wave
-                const int k1 = __builtin_ctzll(vote);
-                vote &= vote - 1;
-                const int k2 = vote ? __builtin_ctzll(vote) : k1;
-                if (vote) vote &= vote - 1;
-                const uint32_t n1 = (uint32_t)__shfl((int)node, k1), n2 = (uint32_t)__shfl((int)node, k2);
-                const bool upper = lane_id() >= 32;
-                treelet_half(upper ? n2 : n1, !upper || k2 != k1, nodes, parents, ws, nf, ts, ci, S);
-            }
-            if (active && at_node) {
-                cur = node;
-                p = parents[cur];
-                at_node = false;
+            wave_sync();
+        }
+
+        const float big = fmaxf(fmaxf(fmaxf(fabsf(mn.x), fabsf(mn.y)), fmaxf(fabsf(mn.z), fabsf(mx.x))),
+                                fmaxf(fabsf(mx.y), fabsf(mx.z)));
+        const bool sane = big < 0x1p61f && mn.x == mn.x && mn.y == mn.y && mn.z == mn.z && mx.x == mx.x &&
+                          mx.y == mx.y && mx.z == mx.z;
+        float total;
+        if (__ballot(have && hl < ts && !sane) == 0)
+            total = treelet_merge<true>(S, ts, ci, hl, logical, upper, tin, pair_rc);
+        else
+            total = treelet_merge<false>(S, ts, ci, hl, logical, upper, tin, pair_rc);
+
+        // updateTreelet: keep the new topology when its SAH is lower
+        const uint64_t better = __ballot(have && hl == 0 && total < xmx.w);
+        const bool keep = ((better >> (upper ? kHalf : 0)) & 1ull) != 0;
+        const uint32_t v = (uint32_t)__shfl_up((int)tin, 1, kHalf);  // tin[hl - 1]
+        if (have && hl == 0) {
+            X.set_span(slo, shi, tri);
+            if (!keep) {
+                if (kFirst) X.r[0] = xmn;
+                if (kFirst) X.r[1] = xmx;
+                else X.set_sah(xmx.w);
             }
         }
+        if (keep && hl >= 1 && hl < ts) {
+            const float4 b0 = S.box[hl][0], b1 = S.box[hl][1];
+            const uint2 kk = S.kids[hl];
+            float4 nmn = make_float4(b0.x, b0.y, b0.z, 0.0f), nmx = make_float4(b1.x, b1.y, b1.z, b0.w);
+            nmn.w = box_area(nmn, nmx);
+            const AtrRec N(ws, v);
+            N.r[0] = nmn;
+            N.r[1] = nmx;
+            N.set_kids(kk.x, kk.y);
+            AtrRec(ws, kk.x).set_parent(v);
+            AtrRec(ws, kk.y).set_parent(v);
+        }
+
+        // up to the parent
+        bool arrive = have && parent < I && ++steps <= nf;
+        uint64_t old = 0;
+        if (arrive && hl == 0)
+            old = __hip_atomic_fetch_add(&ws.ph.visit[parent], ((uint64_t)tag << 32) | 1ull, __ATOMIC_ACQ_REL,
+                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t count = half_pick((uint32_t)old, 0, 0, upper);
+        const uint32_t t1 = half_pick((uint32_t)(old >> 32), 0, 0, upper);
+        have = arrive && count != 0;  // else the sibling continues
+        if (have && t1 != tag && (t1 >> 24) >= phase) {
+            if (hl == 0) defer(parent, slo);
+            have = false;
+        }
+        root = parent;
+        rt = pt;
     }
 }
 
-__global__ void atr_leaf_bounds(kr_bvh_node* nodes, AtrWs ws, uint32_t nf) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nf) return;
-    const uint32_t v = nf - 1 + i;
-    const float4 mn = ws.bmin[v], mx = ws.bmax[v];
-    nodes[v].bounds.min = kr_vec3{mn.x, mn.y, mn.z};
-    nodes[v].bounds.max = kr_vec3{mx.x, mx.y, mx.z};
+// The tree from the records: topology, leaf bounds and faces (internal bounds
+// follow bottom-up).
+__global__ __launch_bounds__(256) void atr_export(AtrWs ws, uint32_t nf, kr_bvh_node* nodes, uint32_t* parents) {
+    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= 2 * nf - 1) return;
+    const AtrRec R(ws, v);
+    const uint4 t = R.topo();
+    kr_bvh_node n = {};
+    n.u.children.left = t.x;  // a leaf: the face id (primitivesOffset)
+    n.u.children.right = t.y;
+    if (v >= nf - 1) {
+        const float4 mn = R.r[0], mx = R.r[1];
+        n.bounds.min = kr_vec3{mn.x, mn.y, mn.z};
+        n.bounds.max = kr_vec3{mx.x, mx.y, mx.z};
+        n.nPrimitives = 1;
+    }
+    nodes[v] = n;
+    parents[v] = t.z;
 }
 
 // Bounds / counts / costs of the final tree (atrbvh.cu:124-179: ct = 1.0,
@@ -593,11 +809,8 @@ size_t atr_carve(AtrWs* ws, void* base, size_t cap, uint32_t nf) {
     ws->keys_out = c.take<uint64_t>(nf);
     ws->vals_in = c.take<uint32_t>(nf);
     ws->vals_out = c.take<uint32_t>(nf);
-    ws->bmin = c.take<float4>(total);
-    ws->bmax = c.take<float4>(total);
-    ws->area = c.take<float>(total);
-    ws->tri = c.take<int32_t>(total);
-    ws->sah = c.take<float>(total);
+    ws->rec = c.take<float4>(4 * total);
+    ws->ready = c.take<uint32_t>(nf);
     ws->sort_bytes = atr_sort_bytes(nf);
     ws->sort_tmp = c.take<char>(ws->sort_bytes);
     return c.used;
@@ -621,18 +834,32 @@ kr_error atr_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, int treele
     size_t sb = ws.sort_bytes;
     OBVH_HIP_TRY(rocprim::radix_sort_pairs(ws.sort_tmp, sb, ws.keys_in, ws.keys_out, ws.vals_in, ws.vals_out, nf, 0,
                                            63, stream));
-    hipLaunchKernelGGL(atr_tree, blocks(nf, 256), dim3(256), 0, stream, nf, ws, nodes, parents);
-    phased_launch(atr_boxes, nf, stream, (const kr_vec3*)V, (const kr_uvec4*)F, (const kr_bvh_node*)nodes,
-                  (const uint32_t*)parents, nf, ws);
-    if (nf > 1) {
-        int gamma = treelet_size;
-        for (int it = 0; it < iterations; ++it) {
-            hipLaunchKernelGGL(atr_clear, dim3(gb), dim3(256), 0, stream, ws, nf);
-            phased_launch(atr_treelets, nf, stream, nodes, parents, ws, nf, treelet_size, gamma, ci, ct);
-            gamma *= 2;
+    hipLaunchKernelGGL(atr_tree, blocks(nf, 256), dim3(256), 0, stream, V, F, nf, ct, ws);
+    int gamma = treelet_size;
+    for (int it = 0; it < iterations && nf > 1; ++it) {
+        if (it > 0) hipLaunchKernelGGL(atr_clear, dim3(gb), dim3(256), 0, stream, ws, nf);
+        // Phases of 512, 8192, 131072 (large meshes) and all leaves.  A phase
+        // costs its own path of treelets, the last one runs on one CU.
+        // Measured with treelet size 7, 2 passes: 200 K triangles 1.04 ms with
+        // 16384, 1.01 with 8192, 1.14 with 4096, 1.16 with 8192 and 131072;
+        // 2 M triangles 4.09, 5.00, 6.78 and 3.46 ms.
+        uint32_t phase = 0;
+        for (uint32_t chunk : {512u, 8192u, nf > (1u << 19) ? 131072u : nf, nf}) {
+            const uint32_t c = min(chunk, nf);
+            const dim3 grid((nf + c - 1) / c);
+            if (phase == 0) {
+                auto k = it == 0 ? atr_treelets<true, 512> : atr_treelets<false, 512>;
+                hipLaunchKernelGGL(k, grid, dim3(512), 0, stream, ws, nf, treelet_size, gamma, ci, phase, c);
+            } else {
+                auto k = it == 0 ? atr_treelets<true, 1024> : atr_treelets<false, 1024>;
+                hipLaunchKernelGGL(k, grid, dim3(1024), 0, stream, ws, nf, treelet_size, gamma, ci, phase, c);
+            }
+            ++phase;
+            if (c == nf) break;
         }
+        gamma *= 2;
     }
-    hipLaunchKernelGGL(atr_leaf_bounds, blocks(nf, 256), dim3(256), 0, stream, nodes, ws, nf);
+    hipLaunchKernelGGL(atr_export, blocks(2 * nf - 1, 256), dim3(256), 0, stream, ws, nf, nodes, parents);
     hipLaunchKernelGGL(atr_clear, dim3(gb), dim3(256), 0, stream, ws, nf);
     phased_launch(atr_final, nf, stream, nodes, (const uint32_t*)parents, counts, costs, nf, ws);
     OBVH_HIP_TRY(hipGetLastError());

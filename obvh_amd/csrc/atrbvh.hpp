@@ -16,11 +16,8 @@ struct AtrWs {
     uint64_t* keys_out;  // sorted codes
     uint32_t* vals_in;   // face ids
     uint32_t* vals_out;  // face ids in code order
-    float4* bmin;        // per node: working box (fminf/fmaxf semantics, -0 below +0)
-    float4* bmax;
-    float* area;         // per node: surface area of the working box
-    int32_t* tri;        // per node: triangles below (optimiser pass)
-    float* sah;          // per node: SAH cost of the subtree (optimiser pass)
+    float4* rec;         // per node: 64-byte working record, see AtrRec in atrbvh.hip
+    uint32_t* ready;     // treelet roots ready to run, one segment per workgroup's chunk
     char* sort_tmp;
     size_t sort_bytes;
 };

@@ -47,20 +47,26 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 // DPP steps leave each 16-lane row's result in all of its lanes (xor 1, xor 2,
 // half-row mirror, row mirror); the four rows are combined on the scalar
 // unit.  Every lane of the wave must be active.
+// (mov_dpp with every lane enabled: the compiler folds it into the min / max,
+// where update_dpp with an old value cost a move and two wait states more)
+template <int kCtrl>
+__device__ __forceinline__ int32_t dpp_mov(int32_t v) {
+    return __builtin_amdgcn_mov_dpp(v, kCtrl, 0xF, 0xF, true);
+}
 __device__ __forceinline__ int32_t wave_min_i32(int32_t v) {
-    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
-    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
-    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));  // row_half_mirror
-    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));  // row_mirror
+    v = min(v, dpp_mov<0xB1>(v));   // quad_perm [1,0,3,2]
+    v = min(v, dpp_mov<0x4E>(v));   // quad_perm [2,3,0,1]
+    v = min(v, dpp_mov<0x141>(v));  // row_half_mirror
+    v = min(v, dpp_mov<0x140>(v));  // row_mirror
     const int32_t a = __builtin_amdgcn_readlane(v, 0), b = __builtin_amdgcn_readlane(v, 16);
     const int32_t c = __builtin_amdgcn_readlane(v, 32), d = __builtin_amdgcn_readlane(v, 48);
     return min(min(a, b), min(c, d));
 }
 __device__ __forceinline__ int32_t wave_max_i32(int32_t v) {
-    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
-    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
+    v = max(v, dpp_mov<0xB1>(v));
+    v = max(v, dpp_mov<0x4E>(v));
+    v = max(v, dpp_mov<0x141>(v));
+    v = max(v, dpp_mov<0x140>(v));
     const int32_t a = __builtin_amdgcn_readlane(v, 0), b = __builtin_amdgcn_readlane(v, 16);
     const int32_t c = __builtin_amdgcn_readlane(v, 32), d = __builtin_amdgcn_readlane(v, 48);
     return max(max(a, b), max(c, d));

@@ -85,3 +85,38 @@ def test_atrbvh_then_transform_and_collapse(torch, oracle_lib, kind):
     assert np.array_equal(obbs.cpu().numpy(), eo) and np.array_equal(mats.cpu().numpy(), em)
     e = oracle_lib.collapse(nh, ph, t["counts"].cpu().numpy().view(np.uint32), CI, CT)
     assert np.array_equal(col["collapsed"].cpu().numpy(), e["collapsed"].view(np.uint8))
+
+
+def edge_mesh(nf, kind):
+    """nf triangles: small random ones, some stored several times (ties); `huge` scales them past 2^61
+    (distances overflow), `flat` puts them in a plane with an integer grid (zero extents, equal areas)."""
+    rng = np.random.default_rng(nf)
+    c = rng.uniform(-1.0, 1.0, (nf, 1, 3))
+    V = c + rng.uniform(-0.02, 0.02, (nf, 3, 3))
+    if kind == "flat":
+        V = np.round(V * 64.0)
+        V[:, :, 2] = -0.0
+    V[nf // 3:nf // 3 + nf // 8] = V[0]
+    if kind == "huge":
+        V = V * 2.0 ** 62
+    F = np.zeros((nf, 4), dtype=np.uint32)
+    F[:, :3] = np.arange(3 * nf).reshape(nf, 3)
+    return V.reshape(-1, 3).astype(np.float32), F
+
+
+# edges of the phases (512 and 8192 leaves; one workgroup up to 512), the smallest and largest treelets, distances
+# past one entry per lane (treelet size 9 and up), boxes that take the general merge
+@pytest.mark.parametrize("nf,ts,its,kind", [(1, 3, 1, "plain"), (2, 3, 1, "plain"), (3, 3, 2, "plain"),
+                                            (20, 20, 1, "plain"), (512, 8, 2, "plain"), (513, 9, 2, "plain"),
+                                            (1500, 20, 2, "plain"), (8193, 12, 3, "plain"), (3000, 3, 3, "flat"),
+                                            (3000, 16, 2, "flat"), (2500, 9, 2, "huge"), (2500, 20, 2, "huge")])
+def test_atrbvh_edges(torch, oracle_lib, nf, ts, its, kind):
+    say(f"[atrbvh] {nf} triangles treelet={ts} passes={its} {kind}")
+    V, F = edge_mesh(nf, kind)
+    t = ops.atrbvh_build(torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda(), ts, its, CI, CT)
+    torch.cuda.synchronize()
+    en, ep, ec, eco = oracle_lib.atrbvh_build(V, F, ts, its, CI, CT)
+    assert np.array_equal(t["parents"].cpu().numpy().view(np.uint32), ep), "parents differ"
+    assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), en.view(np.uint8)), "nodes differ"
+    assert np.array_equal(t["counts"].cpu().numpy().view(np.uint32), ec)
+    assert np.array_equal(t["costs"].cpu().numpy(), eco, equal_nan=True)
