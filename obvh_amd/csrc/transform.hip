@@ -1192,13 +1192,16 @@ __device__ __forceinline__ void cand_search(const Pts<NP, kRef>& L, f3 p0, f3 p1
         hi = ch ? pn[i] : hi;
         q0 = pick(ch, P[i], q0);
     }
-    // apex a = 0: q0 (candidates 3..11), a = 1: q1 (12..20); on apex q the
-    // faces j = 0, 1, 2 have edges (e_j, f_{j+1}, f_j) with f_i = q - p_i
-    // normalised and normal cross(f_{j+1}, e_j) normalised (transforms.cu:641-700)
+    // the node's first valid apex (q0, candidates 3..11, or else q1), then q1
+    // (12..20) if both are; on apex q the faces j = 0, 1, 2 have edges
+    // (e_j, f_{j+1}, f_j) with f_i = q - p_i normalised and normal
+    // cross(f_{j+1}, e_j) normalised (transforms.cu:641-700).  A node of four
+    // distinct points has one apex: its wave runs the loop once, whichever
+    // side each lane's apex is on.
 #pragma unroll 1
     for (int a = 0; a < 2; ++a) {
-        if (!(a == 0 ? q0v : q1v)) continue;
-        const f3 q = pick(a == 0, q0, q1);
+        if (a == 1 && !(q0v && q1v)) continue;
+        const f3 q = pick(a == 0 && q0v, q0, q1);
         const f3 f0 = vm::normalize(sub3(q, p0));
         const f3 f1 = vm::normalize(sub3(q, p1));
         const f3 f2 = vm::normalize(sub3(q, p2));
