@@ -148,11 +148,12 @@ kr_error obvh_dito_soa(const float* x, const float* y, const float* z, kr_size c
     if (count > 0 && (!x || !y || !z)) return fail("obvh_dito_soa: NULL point array");
     if (count > 0xFFFFFFF0ull) return fail("obvh_dito_soa: more than 2^32 - 16 points");
     if (count == 0) {  // the empty set's box, written by the set-up kernel
-        TRY(obvh::dito_launch(x, y, z, nullptr, nullptr, count, 1, count, out_obb, trace, 0, 0, workspace,
+        TRY(obvh::dito_launch(x, y, z, nullptr, count, 1, count, out_obb, trace, 0, 0, workspace,
                               workspace_bytes, (hipStream_t)stream));
         return nullptr;
     }
-    TRY(obvh::dito_one_launch(x, y, z, nullptr, count, out_obb, trace, workspace, workspace_bytes, true,
+    bool clear = true;
+    TRY(obvh::dito_one_launch(x, y, z, nullptr, count, out_obb, trace, workspace, workspace_bytes, clear,
                               (hipStream_t)stream));
     return nullptr;
 }
@@ -173,15 +174,17 @@ kr_error obvh_dito_soa_noalloc(const float* x, const float* y, const float* z, k
     bool first = false;
     TRY(noalloc_scratch(&ws, &first));
     if (count == 0) {
-        TRY(obvh::dito_launch(x, y, z, nullptr, nullptr, count, 1, count, out_obb, trace, 0, 0, ws,
+        TRY(obvh::dito_launch(x, y, z, nullptr, count, 1, count, out_obb, trace, 0, 0, ws,
                               kNoAllocScratchBytes, (hipStream_t)stream));
         return nullptr;
     }
     // the completion counters keep a fixed place in the array; the launches
-    // leave them zero, so only the first call on a device clears them
-    TRY(obvh::dito_one_launch(x, y, z, nullptr, count, out_obb, trace, ws, kNoAllocScratchBytes, first,
+    // leave them zero, so only the first call on a device that uses them
+    // clears them
+    bool clear = first;
+    TRY(obvh::dito_one_launch(x, y, z, nullptr, count, out_obb, trace, ws, kNoAllocScratchBytes, clear,
                               (hipStream_t)stream));
-    if (first) noalloc_scratch_used();
+    if (first && !clear) noalloc_scratch_used();
     return nullptr;
 }
 
@@ -197,7 +200,7 @@ kr_error obvh_dito_batch(const float* x, const float* y, const float* z, const k
     if (nsets == 0) return nullptr;
     if (!offsets || !out_obbs) return fail("obvh_dito_batch: NULL offsets or output");
     if (total_points > 0 && (!x || !y || !z)) return fail("obvh_dito_batch: NULL point array");
-    TRY(obvh::dito_launch(x, y, z, nullptr, (const uint64_t*)offsets, 0, nsets, total_points, out_obbs, traces,
+    TRY(obvh::dito_launch(x, y, z, (const uint64_t*)offsets, 0, nsets, total_points, out_obbs, traces,
                           tile_points, workers, workspace, workspace_bytes, (hipStream_t)stream));
     return nullptr;
 }
@@ -288,13 +291,12 @@ kr_obb3 kr_cuda_points_obb(const kr_vec3* points, kr_size count, kr_scalar* elap
         return nan_box;
     }
     hipEventRecord(c->ev[0], nullptr);
-    // two launches; a fresh workspace first gets its completion counters zeroed
+    // a fresh workspace first gets its completion counters zeroed
     kr_error r = obvh::dito_one_launch(nullptr, nullptr, nullptr, (const float*)c->pts, count, (kr_obb3*)c->out,
                                        nullptr, c->dws, c->dws_bytes, c->dws_clear, nullptr);
     hipEventRecord(c->ev[1], nullptr);
     kr_obb3 o = nan_box;
     if (!r) {
-        c->dws_clear = false;
         if ((e = hipMemcpy(&o, c->out, sizeof(kr_obb3), hipMemcpyDeviceToHost)) != hipSuccess) {
             obvh_hip_error(e, "kr_cuda_points_obb: hipMemcpy D2H");
             o = nan_box;

@@ -81,16 +81,6 @@ __device__ __forceinline__ bool pair_better(float v, uint32_t k, float ov, uint3
     if (MIN) return (ov < v) || (ov == v && ok < k);
     return (ov > v) || (ov == v && ok < k);
 }
-template <bool MIN>
-__device__ __forceinline__ void wave_pair(float& v, uint32_t& k) {
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) {
-        float ov = __shfl_xor(v, m, kWave);
-        uint32_t ok = (uint32_t)__shfl_xor((int)k, m, kWave);
-        if (pair_better<MIN>(v, k, ov, ok)) { v = ov; k = ok; }
-    }
-}
-
 // Bump allocator over a caller-provided workspace (256 B aligned pieces).
 struct Carver {
     char* base;

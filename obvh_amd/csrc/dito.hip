@@ -10,17 +10,10 @@
 //            cut into tiles of `tile` points) and writes the result of empty
 //            sets; a grid kernel fills tile -> set.
 //  pass 1    workgroups (4 x wave64) take tiles in grid-stride order (one
-//            tile per workgroup by default).  Lane l of a
-//            wave reads points chunk + j*64 + l, j < 8 (coalesced SoA or AoS),
-//            forms the 7 slab projections, and keeps per slab side the running
-//            extreme with the index where it was first reached: one strict
-//            compare and two selects per point and side (a group-extreme
-//            scheme that searched the group on improvement ran nearly every
-//            search, since some lane of a wave improves on most groups, and
-//            issued 3.5x the VALU work of pass 2).  (value, index) pairs reduce
-//            lexicographically (ties keep the lower index): order free, and
-//            equal to the reference's sequential strict-compare scan.
-//            Output: 14 pairs per tile.
+//            tile per workgroup by default), form the 7 slab projections of
+//            every point and keep per slab side the extreme and the point that
+//            reached it first; equal to the reference's sequential
+//            strict-compare scan.  Output: 14 (value, index) pairs per tile.
 //  cand      one wave per set reduces its tile partials, then runs the
 //            candidate search (base triangle + ditetrahedron, up to 21 axis
 //            triples) over a 14-entry point array held in registers: every
@@ -31,8 +24,15 @@
 //  final     one wave per set reduces and finalises the box.
 //
 // No atomics or cross-workgroup fences: kernel boundaries order the phases.
-// Each pass reads 12 B per point, 24 B per point per fit.
+// Each pass reads 12 B per point, 24 B per point per fit, at 6.0-6.2 TB/s of the
+// 6.3-6.5 that plain streaming reads reach here, from HBM or from the Infinity
+// Cache alike: an axis pass arranged to follow its slab pass through that cache
+// (one launch, tiles in an order with a lag) was no faster than two passes.
+// A single set takes one launch (see "one-launch fits" below).
 #include <float.h>
+#include <stddef.h>
+
+#include <atomic>
 
 #include "common.hpp"
 #include "dito.hpp"
@@ -41,8 +41,8 @@ namespace obvh {
 
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
-constexpr int kG = 8;               // points per lane per chunk
-constexpr int kChunk = kWave * kG;  // points per wave per chunk
+constexpr int kRows = 8;     // points per lane in one unrolled step
+constexpr int kChunk = 512;  // tiles are multiples of it
 constexpr uint32_t kNoIdx = 0xFFFFFFFFu;
 
 struct PtsSoA {
@@ -69,13 +69,31 @@ __device__ __forceinline__ uint64_t set_off(const uint64_t* offs, uint64_t singl
 // outside the point arrays or the carved tile arrays (`cap_tiles` entries).
 __device__ __forceinline__ bool set_valid(uint64_t b, uint64_t e, uint64_t total) { return b <= e && e <= total; }
 
+__device__ __forceinline__ kr_obb3 nan_box() {
+    const float nan = __builtin_nanf("");
+    kr_obb3 o;
+    o.mid = o.v0 = o.v1 = o.v2 = o.ext = kr_vec3{nan, nan, nan};
+    return o;
+}
+__device__ __forceinline__ obvh_dito_trace plain_trace(int degenerate) {
+    obvh_dito_trace t = {};
+    t.pair_k = t.p2_sel = t.q0_sel = t.q1_sel = -1;
+    t.best = -1;
+    t.degenerate = degenerate;
+    t.result_aabb = degenerate == 3;
+    return t;
+}
+
 __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_t single_count,
                                                    uint32_t nsets, uint32_t tile, uint64_t total,
                                                    uint32_t cap_tiles, DitoWs ws,
                                                    kr_obb3* out, obvh_dito_trace* trace) {
-    __shared__ uint32_t carry;
+    __shared__ uint32_t carry, limit;
     __shared__ uint32_t wsum[1024 / kWave];
-    if (threadIdx.x == 0) carry = 0;
+    if (threadIdx.x == 0) {
+        carry = 0;
+        limit = 0xFFFFFFFFu;
+    }
     if (threadIdx.x == 0 && offs == nullptr) {
         ws.offsets_single[0] = 0;
         ws.offsets_single[1] = single_count;
@@ -88,15 +106,8 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
             const uint64_t b = set_off(offs, single_count, s), e = set_off(offs, single_count, s + 1);
             const uint64_t n = e - b;
             if (!set_valid(b, e, total)) {
-                const float nan = __builtin_nanf("");
-                kr_obb3 o;
-                o.mid = o.v0 = o.v1 = o.v2 = o.ext = kr_vec3{nan, nan, nan};
-                out[s] = o;
-                obvh_dito_trace t = {};
-                t.pair_k = t.p2_sel = t.q0_sel = t.q1_sel = -1;
-                t.best = -1;
-                t.degenerate = 4;
-                trace[s] = t;
+                out[s] = nan_box();
+                if (trace) trace[s] = plain_trace(4);
             } else if (n != 0) {
                 nt = (uint32_t)((n + tile - 1) / tile);
             } else {
@@ -108,12 +119,7 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
                 o.v2 = kr_vec3{0, 0, 1};
                 o.ext = kr_vec3{0.001f, 0.001f, 0.001f};
                 out[s] = o;
-                obvh_dito_trace t = {};
-                t.pair_k = t.p2_sel = t.q0_sel = t.q1_sel = -1;
-                t.best = -1;
-                t.degenerate = 3;
-                t.result_aabb = 1;
-                trace[s] = t;
+                if (trace) trace[s] = plain_trace(3);
             }
         }
         uint32_t v = nt;
@@ -128,14 +134,20 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
         uint32_t wpre = 0;
         for (int w = 0; w < wave_id(); ++w) wpre += wsum[w];
         const uint32_t incl = carry + wpre + v;
-        if (s < nsets) ws.first_tile[s] = incl - nt;
+        // Offsets that never decrease need at most cap_tiles - 1 tiles.  Where
+        // others (sets that overlap) need more, the sets from the first that
+        // does not fit on are invalid: no tiles, a NaN box.
+        if (nt != 0 && incl >= cap_tiles) {
+            atomicMin(&limit, incl - nt);
+            out[s] = nan_box();
+            if (trace) trace[s] = plain_trace(4);
+        }
         __syncthreads();
+        if (s < nsets) ws.first_tile[s] = min(incl - nt, limit);
         if (threadIdx.x == blockDim.x - 1) carry = incl;
         __syncthreads();
     }
-    // valid offsets need at most cap_tiles - 1 tiles; the clamp only guards
-    // the carved arrays
-    if (threadIdx.x == 0) ws.first_tile[nsets] = carry < cap_tiles ? carry : cap_tiles;
+    if (threadIdx.x == 0) ws.first_tile[nsets] = min(carry, limit);
 }
 
 __global__ __launch_bounds__(256) void dito_tile_table(uint32_t nsets, DitoWs ws) {
@@ -152,99 +164,241 @@ __global__ __launch_bounds__(256) void dito_tile_table(uint32_t nsets, DitoWs ws
 
 // --------------------------------------------------------------- pass 1 --
 
-// Slab extremes of points [base, end) of the set starting at sbeg: 14
-// (value, index within the set) pairs written to v_out / i_out by threads
-// 0..13 of the workgroup.
-template <class P>
-__device__ __forceinline__ void tile_pass1(P pts, uint64_t sbeg, uint64_t base, uint64_t end,
-                                           float (&sh_v)[kWaves][14], uint32_t (&sh_i)[kWaves][14],
-                                           float* v_out, uint32_t* i_out) {
-    const int lane = lane_id(), wave = wave_id();
-    const float NaN = __builtin_nanf("");
-    const uint32_t nchunks = (uint32_t)((end - base + kChunk - 1) / kChunk);
-    // per lane and slab side: running extreme and the index where it was
-    // first reached (points of one lane are visited in increasing index)
-    float rmn[7], rmx[7];
-    uint32_t imn[7], imx[7];
+// The lower half of the wave keeps a over its own and the upper half's lane,
+// the upper half b.
+__device__ __forceinline__ float min_swap32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return fminf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// The same between the even and odd rows of 16 lanes.
+__device__ __forceinline__ float min_swap16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return fminf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <int kCtrl>
+__device__ __forceinline__ float dpp_movf(float v) {
+    return __int_as_float(dpp_mov<kCtrl>(__float_as_int(v)));
+}
+// Minima of 14 values over the wave by recursive halving (each step halves the
+// values a lane carries: 16 minima instead of 84): lanes 4q .. 4q + 3 get that
+// of value 7 (q / 8) + q % 8 (q % 8 < 7).
+__device__ __forceinline__ float wave_min14(const float (&v)[14]) {
+    const float INF = FLT_MAX * 2.0f;
+    float w[8], u[4];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) w[k] = min_swap32(v[k], v[7 + k]);
+    w[7] = INF;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = min_swap16(w[k], w[k + 4]);
+    const bool b3 = (lane_id() & 8) != 0, b2 = (lane_id() & 4) != 0;
+    const float x0 = fminf(b3 ? u[2] : u[0], dpp_movf<0x128>(b3 ? u[0] : u[2]));  // row_ror:8
+    const float x1 = fminf(b3 ? u[3] : u[1], dpp_movf<0x128>(b3 ? u[1] : u[3]));
+    float y = fminf(b2 ? x1 : x0, dpp_movf<0x141>(b2 ? x0 : x1));  // row_half_mirror
+    y = fminf(y, dpp_movf<0x4E>(y));
+    return fminf(y, dpp_movf<0xB1>(y));
+}
+// Minima of 6 values: lanes 8q .. 8q + 7 get that of value 3 (q / 4) + q % 4
+// (q % 4 < 3).
+__device__ __forceinline__ float wave_min6(const float (&v)[6]) {
+    const float INF = FLT_MAX * 2.0f;
+    float w[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w[k] = min_swap32(v[k], v[3 + k]);
+    const float u0 = min_swap16(w[0], w[2]), u1 = min_swap16(w[1], INF);
+    const bool b3 = (lane_id() & 8) != 0;
+    float y = fminf(b3 ? u1 : u0, dpp_movf<0x128>(b3 ? u0 : u1));
+    y = fminf(y, dpp_movf<0x141>(y));
+    y = fminf(y, dpp_movf<0x4E>(y));
+    return fminf(y, dpp_movf<0xB1>(y));
+}
+
+template <int kThreads>
+struct FitLds {
+    float wext[kThreads / kWave][16];  // per wave: slab minima (slots 0..6) and negated maxima (8..14)
+    float ext[16];                     // of the tile
+    uint32_t idx[16];                  // where they are first reached (point or chunk), within the tile
+    float wrng[kThreads / kWave][8];   // per wave: minima (0..2) and negated maxima (4..6) on the axes
+    float rng[8];
+    SetState st;
+    uint32_t last, fail;
+};
+__device__ __forceinline__ int side_slot(int side) { return side < 7 ? side : side + 1; }
+
+// Ranges of two more points on the three axes.
+__device__ __forceinline__ void axes_step(f3 p, f3 q, const f3 (&b)[3], float (&r)[6]) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float d = dot3(p, b[k]), e = dot3(q, b[k]);
+        r[k] = fminf(fminf(r[k], d), e);
+        r[3 + k] = fmaxf(fmaxf(r[3 + k], d), e);
+    }
+}
+// Slab extremes of two more points (a three-operand min / max each).
+__device__ __forceinline__ void slabs_step(f3 p, f3 q, float (&e)[14]) {
+    float u[7], v[7];
+    slab7(p, u);
+    slab7(q, v);
 #pragma unroll
     for (int k = 0; k < 7; ++k) {
-        rmn[k] = NaN;  // NaN never compares: the first real value wins
-        rmx[k] = NaN;
-        imn[k] = imx[k] = kNoIdx;
+        e[k] = fminf(fminf(e[k], u[k]), v[k]);
+        e[7 + k] = fmaxf(fmaxf(e[7 + k], u[k]), v[k]);
     }
-    for (uint32_t c = wave; c < nchunks; c += kWaves) {
-        const uint64_t cb = base + (uint64_t)c * kChunk + lane;
-        const bool full = base + (uint64_t)(c + 1) * kChunk <= end;
-        f3 p[kG];
+}
+__device__ __forceinline__ void state_axes(const SetState& st, f3 (&b)[3]) {  // uniform
+    float ax[9];
 #pragma unroll
-        for (int j = 0; j < kG; ++j) {
-            const uint64_t idx = cb + (uint64_t)j * kWave;
-            p[j] = (full || idx < end) ? pts.load(idx) : f3{NaN, NaN, NaN};
-        }
-        // Per point and slab side a strict compare against the running
-        // extreme keeps the first point that reaches it, as the sequential
-        // scan does; !(v >= cur) also takes the first value, while cur is
-        // NaN.  NaN values (the short last chunk's missing points, or
-        // non-finite input) are skipped here; the candidate step applies the
-        // reference scan's rule for a NaN at point 0.
-        const uint32_t i0 = (uint32_t)(cb - sbeg);
+    for (int k = 0; k < 9; ++k)
+        ax[k] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(st.ax[k])));
 #pragma unroll
-        for (int j = 0; j < kG; ++j) {
-            float pr[7];
-            slab7(p[j], pr);
-            const uint32_t idx = i0 + (uint32_t)j * kWave;
-#pragma unroll
-            for (int k = 0; k < 7; ++k) {
-                if (!(pr[k] >= rmn[k]) && pr[k] == pr[k]) { rmn[k] = pr[k]; imn[k] = idx; }
-                if (!(pr[k] <= rmx[k]) && pr[k] == pr[k]) { rmx[k] = pr[k]; imx[k] = idx; }
-            }
-        }
-    }
-    // wave: (value, index) lexicographic, then the workgroup over waves
-#pragma unroll
-    for (int side = 0; side < 14; ++side) {
-        const int k = side < 7 ? side : side - 7;
-        float v = side < 7 ? rmn[k] : rmx[k];
-        uint32_t i = side < 7 ? imn[k] : imx[k];
-        if (i == kNoIdx) v = side < 7 ? FLT_MAX * 2.0f : -FLT_MAX * 2.0f;
-        if (side < 7) wave_pair<true>(v, i); else wave_pair<false>(v, i);
-        if (lane == 0) {
-            sh_v[wave][side] = v;
-            sh_i[wave][side] = i;
-        }
-    }
+    for (int k = 0; k < 3; ++k) b[k] = f3{ax[3 * k], ax[3 * k + 1], ax[3 * k + 2]};
+}
+
+// The tile's slab extremes into L.ext (maxima negated), L.idx cleared; e: each
+// lane's, maxima negated.
+template <int kThreads>
+__device__ __forceinline__ void tile_extremes(const float (&e)[14], FitLds<kThreads>& L) {
+    const float y = wave_min14(e);
+    if ((lane_id() & 3) == 0) L.wext[wave_id()][lane_id() >> 2] = y;
     __syncthreads();
-    if (threadIdx.x < 14) {
-        const int side = threadIdx.x;
-        float v = sh_v[0][side];
-        uint32_t i = sh_i[0][side];
-        for (int w = 1; w < kWaves; ++w) {
-            const float ov = sh_v[w][side];
-            const uint32_t oi = sh_i[w][side];
-            if (oi == kNoIdx) continue;
-            const bool better = (i == kNoIdx) ||
-                                (side < 7 ? pair_better<true>(v, i, ov, oi) : pair_better<false>(v, i, ov, oi));
-            if (better) { v = ov; i = oi; }
-        }
-        v_out[side] = v;
-        i_out[side] = i;
+    if (threadIdx.x < 16) {
+        float a = L.wext[0][threadIdx.x];
+        for (int w = 1; w < kThreads / kWave; ++w) a = fminf(a, L.wext[w][threadIdx.x]);
+        L.ext[threadIdx.x] = a;
+        L.idx[threadIdx.x] = kNoIdx;
     }
     __syncthreads();
 }
 
-template <class P>
-__global__ __launch_bounds__(kBlock) void dito_pass1(P pts, const uint64_t* offs, uint32_t nsets,
-                                                     uint32_t tile, DitoWs ws) {
-    __shared__ float sh_v[kWaves][14];
-    __shared__ uint32_t sh_i[kWaves][14];
+
+// A tile's points: uniform pointers and 32-bit byte offsets, so that a load is
+// one instruction (a 64-bit address per lane costs two more).  load4: four
+// consecutive points, at any alignment of the arrays.
+__device__ __forceinline__ float load_at(const float* p, uint32_t byte) {
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + byte);
+}
+__device__ __forceinline__ float4 load4_at(const float* p, uint32_t byte) {
+    float4 v;
+    __builtin_memcpy(&v, reinterpret_cast<const char*>(p) + byte, sizeof(v));
+    return v;
+}
+struct TileSoA {
+    const float *x, *y, *z;
+    __device__ __forceinline__ TileSoA(const PtsSoA& p, uint64_t base) : x(p.x + base), y(p.y + base), z(p.z + base) {}
+    __device__ __forceinline__ f3 load(uint32_t i) const {
+        return f3{load_at(x, 4 * i), load_at(y, 4 * i), load_at(z, 4 * i)};
+    }
+    __device__ __forceinline__ void load4(uint32_t i, f3* p) const {
+        const float4 a = load4_at(x, 4 * i), b = load4_at(y, 4 * i), c = load4_at(z, 4 * i);
+        p[0] = f3{a.x, b.x, c.x};
+        p[1] = f3{a.y, b.y, c.y};
+        p[2] = f3{a.z, b.z, c.z};
+        p[3] = f3{a.w, b.w, c.w};
+    }
+};
+struct TileAoS {
+    const float* xyz;
+    __device__ __forceinline__ TileAoS(const PtsAoS& p, uint64_t base) : xyz(p.xyz + 3 * base) {}
+    __device__ __forceinline__ f3 load(uint32_t i) const {
+        return f3{load_at(xyz, 12 * i), load_at(xyz, 12 * i + 4), load_at(xyz, 12 * i + 8)};
+    }
+    __device__ __forceinline__ void load4(uint32_t i, f3* p) const {
+        const float4 a = load4_at(xyz, 12 * i), b = load4_at(xyz, 12 * i + 16), c = load4_at(xyz, 12 * i + 32);
+        p[0] = f3{a.x, a.y, a.z};
+        p[1] = f3{a.w, b.x, b.y};
+        p[2] = f3{b.z, b.w, c.x};
+        p[3] = f3{c.y, c.z, c.w};
+    }
+};
+__device__ __forceinline__ TileSoA tile_of(const PtsSoA& p, uint64_t base) { return TileSoA(p, base); }
+__device__ __forceinline__ TileAoS tile_of(const PtsAoS& p, uint64_t base) { return TileAoS(p, base); }
+
+// A tile is read in steps of 2048 points, 512 consecutive ones per wave: lane l
+// takes points 4 l .. 4 l + 3 of each half.  Row r = 8 c + j of a lane (step c)
+// is point tile_point(r) of the tile; a lane's rows ascend.
+constexpr uint32_t kStepPts = kBlock * kRows;
+static_assert(kRows == 8, "two halves of four points");
+__device__ __forceinline__ uint32_t tile_point(uint32_t r) {
+    return (r >> 3) * kStepPts + (threadIdx.x >> 6) * (kStepPts / kWaves) + ((r >> 2) & 1u) * (4 * kWave) +
+           (threadIdx.x & (kWave - 1)) * 4 + (r & 3u);
+}
+
+// f(c, points) for every step c of a tile's cnt points.  Past the end a lane
+// gets copies of the last point, which no strict rule takes.
+template <class T, class F>
+__device__ __forceinline__ void stream_tile(const T& pts, uint32_t cnt, F f) {
+    uint32_t c = 0;
+    for (; (c + 1) * kStepPts <= cnt; ++c) {
+        f3 p[kRows];
+        pts.load4(tile_point(8 * c), p);
+        pts.load4(tile_point(8 * c + 4), p + 4);
+        f(c, p);
+    }
+    if (c * kStepPts + (threadIdx.x >> 6) * (kStepPts / kWaves) < cnt) {  // wave-uniform
+        f3 p[kRows];
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) p[j] = pts.load(min(tile_point(8 * c + j), cnt - 1));
+        f(c, p);
+    }
+}
+
+// Slab pass over a tile of cnt points: its 14 extremes (L.ext, maxima negated)
+// and the points where they are first reached (L.idx; kNoIdx: nowhere, all NaN
+// or beyond infinity).  Streaming, bound by memory (6.0 TB/s): per point and
+// side one strict compare and two selects keep the first point that reaches
+// the extreme, as the sequential scan does; NaN values are never taken.  What
+// a small tile cost was the reduction: shuffling 14 (value, index) pairs
+// through the wave was 700 instructions; now the values halve (45) and only
+// the lanes that hold an extreme look at indices.  Ends with a barrier.
+template <class T>
+__device__ __forceinline__ void tile_pass1(const T& pts, uint32_t cnt, FitLds<kBlock>& L) {
+    const float INF = FLT_MAX * 2.0f;
+    float run[14];     // extremes, maxima negated
+    uint32_t row[14];  // where they were first reached
+#pragma unroll
+    for (int k = 0; k < 14; ++k) { run[k] = INF; row[k] = 0xFFFFFFFFu; }
+    stream_tile(pts, cnt, [&](uint32_t c, const f3 (&p)[kRows]) {
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) {
+            float pr[7];
+            slab7(p[j], pr);
+#pragma unroll
+            for (int k = 0; k < 14; ++k) {
+                const float v = k < 7 ? pr[k] : -pr[k - 7];
+                if (v < run[k]) { run[k] = v; row[k] = 8 * c + j; }
+            }
+        }
+    });
+    tile_extremes(run, L);
+#pragma unroll
+    for (int k = 0; k < 14; ++k) {
+        const bool hit = run[k] == L.ext[side_slot(k)] && row[k] != 0xFFFFFFFFu;
+        if (__ballot(hit) == 0) continue;  // (one atomic per wave: of equal points every lane is here)
+        const int32_t first = wave_min_i32(hit ? (int32_t)tile_point(row[k]) : 0x7FFFFFFF);
+        if (lane_id() == 0) atomicMin(&L.idx[side_slot(k)], (uint32_t)first);
+    }
+    __syncthreads();
+}
+
+// The tile's pairs (value, index within the set; `first`: of the tile's first
+// point) by threads 0..13.
+__device__ __forceinline__ void store_pairs(const FitLds<kBlock>& L, uint32_t first, float* v_out, uint32_t* i_out) {
+    if (threadIdx.x >= 14) return;
+    const int side = threadIdx.x, slot = side_slot(side);
+    const uint32_t i = L.idx[slot];
+    v_out[side] = side < 7 ? L.ext[slot] : -L.ext[slot];
+    i_out[side] = i == kNoIdx ? kNoIdx : first + i;
+}
+
+__global__ __launch_bounds__(kBlock) void dito_pass1(PtsSoA pts, const uint64_t* offs, uint32_t nsets, uint32_t tile,
+                                                     DitoWs ws) {
+    __shared__ FitLds<kBlock> L;
     const uint32_t T = ws.first_tile[nsets];
     for (uint32_t t = blockIdx.x; t < T; t += gridDim.x) {
         const uint32_t s = ws.tile_set[t];
         const uint64_t sbeg = offs[s], send = offs[s + 1];
-        const uint32_t ft = ws.first_tile[s];
-        const uint64_t base = sbeg + (uint64_t)(t - ft) * tile;
-        const uint64_t end = base + tile < send ? base + tile : send;
-        tile_pass1(pts, sbeg, base, end, sh_v, sh_i, &ws.part1_v[(size_t)t * 14], &ws.part1_i[(size_t)t * 14]);
+        const uint64_t first = (uint64_t)(t - ws.first_tile[s]) * tile;
+        tile_pass1(tile_of(pts, sbeg + first), (uint32_t)min((uint64_t)tile, send - sbeg - first), L);
+        store_pairs(L, (uint32_t)first, &ws.part1_v[(size_t)t * 14], &ws.part1_i[(size_t)t * 14]);
     }
 }
 
@@ -422,92 +576,109 @@ __device__ void dito_candidate_search(const float mn[7], const float mx[7], cons
     tr.best = best_id;
 }
 
-// One wave: reduce the nt tile partials of a set (points [sbeg, send),
-// first tile ft), then search; state and trace written by lane 0.
-template <class P>
-__device__ __forceinline__ void set_cand(P pts, uint64_t sbeg, uint64_t send, uint32_t ft, uint32_t nt,
-                                         const float* part1_v, const uint32_t* part1_i, SetState* state,
-                                         obvh_dito_trace* trace) {
+// Agent-scope relaxed accesses: they go past the XCDs' L2 caches, so what one
+// workgroup stores (and waits for, `drain`) before it counts itself done is
+// what a workgroup that saw the count loads, without writing back or
+// invalidating an L2.
+template <class T>
+__device__ __forceinline__ T ld_agent(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void st_agent(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// One wave: the set's slab extremes (indices within the set, 14 sides) from
+// the partials of its nt tiles (first tile ft).  kAgent: the partials were
+// written by other workgroups of this launch.
+template <bool kAgent>
+__device__ __forceinline__ void reduce_partials(uint32_t ft, uint32_t nt, const float* part1_v,
+                                                const uint32_t* part1_i, uint32_t (&ix)[14]) {
     const int lane = lane_id();
     // Lane l reduces side l % 16 (sides 0..13) over the tiles j = l / 16
     // (mod 4); two shuffle steps join the four groups.  (value, index) pairs
     // order lexicographically (no NaN values: pass 1 never takes one), so
     // the order of the reduction does not matter.
-    float v[14];
-    uint32_t ix[14];
-    const f3 pt0 = pts.load(sbeg);  // for the NaN rule below, read beside the partials
-    {
-        const int side = lane & 15;
-        const bool mn = side < 7;
-        float a = mn ? FLT_MAX * 2.0f : -FLT_MAX * 2.0f;
-        uint32_t ai = kNoIdx;
-        if (side < 14) {
-            // sixteen tiles' pairs are read before any is compared: one
-            // memory round trip per 64 tiles instead of one per 4
-            constexpr int kB = 16;
-            for (uint32_t j0 = (uint32_t)(lane >> 4); j0 < nt; j0 += 4 * kB) {
-                float ov[kB];
-                uint32_t oi[kB];
+    const int side = lane & 15;
+    const bool mn = side < 7;
+    float a = mn ? FLT_MAX * 2.0f : -FLT_MAX * 2.0f;
+    uint32_t ai = kNoIdx;
+    if (side < 14) {
+        // sixteen tiles' pairs are read before any is compared: one
+        // memory round trip per 64 tiles instead of one per 4
+        constexpr int kB = 16;
+        for (uint32_t j0 = (uint32_t)(lane >> 4); j0 < nt; j0 += 4 * kB) {
+            float ov[kB];
+            uint32_t oi[kB];
 #pragma unroll
-                for (int u = 0; u < kB; ++u) {
-                    const uint32_t j = j0 + 4u * u;
-                    ov[u] = j < nt ? part1_v[(size_t)(ft + j) * 14 + side] : 0.0f;
-                    oi[u] = j < nt ? part1_i[(size_t)(ft + j) * 14 + side] : kNoIdx;
-                }
+            for (int u = 0; u < kB; ++u) {
+                const uint32_t j = j0 + 4u * u;
+                const size_t at = (size_t)(ft + j) * 14 + side;
+                ov[u] = j < nt ? (kAgent ? ld_agent(&part1_v[at]) : part1_v[at]) : 0.0f;
+                oi[u] = j < nt ? (kAgent ? ld_agent(&part1_i[at]) : part1_i[at]) : kNoIdx;
+            }
 #pragma unroll
-                for (int u = 0; u < kB; ++u) {
-                    if (j0 + 4u * u >= nt) continue;
-                    const bool better = (ai == kNoIdx) || (mn ? pair_better<true>(a, ai, ov[u], oi[u])
-                                                              : pair_better<false>(a, ai, ov[u], oi[u]));
-                    if (better) { a = ov[u]; ai = oi[u]; }
-                }
+            for (int u = 0; u < kB; ++u) {
+                if (j0 + 4u * u >= nt) continue;
+                const bool better = (ai == kNoIdx) || (mn ? pair_better<true>(a, ai, ov[u], oi[u])
+                                                          : pair_better<false>(a, ai, ov[u], oi[u]));
+                if (better) { a = ov[u]; ai = oi[u]; }
             }
         }
-#pragma unroll
-        for (int m = 16; m < kWave; m <<= 1) {
-            const float ov = __shfl_xor(a, m, kWave);
-            const uint32_t oi = (uint32_t)__shfl_xor((int)ai, m, kWave);
-            if (mn ? pair_better<true>(a, ai, ov, oi) : pair_better<false>(a, ai, ov, oi)) { a = ov; ai = oi; }
-        }
-#pragma unroll
-        for (int k = 0; k < 14; ++k) {
-            v[k] = __shfl(a, k, kWave);
-            ix[k] = (uint32_t)__shfl((int)ai, k, kWave);
-        }
     }
-    const uint64_t n = send - sbeg;
+#pragma unroll
+    for (int m = 16; m < kWave; m <<= 1) {
+        const float ov = __shfl_xor(a, m, kWave);
+        const uint32_t oi = (uint32_t)__shfl_xor((int)ai, m, kWave);
+        if (mn ? pair_better<true>(a, ai, ov, oi) : pair_better<false>(a, ai, ov, oi)) { a = ov; ai = oi; }
+    }
+#pragma unroll
+    for (int k = 0; k < 14; ++k) ix[k] = (uint32_t)__builtin_amdgcn_readlane((int)ai, k);
+}
+
+// One wave: the candidate search of a set (n points from sbeg) from its slab
+// extremes' indices; st and tr in every lane.
+template <class P>
+__device__ __forceinline__ void set_search(P pts, uint64_t sbeg, uint64_t n, uint32_t (&ix)[14], SetState& st,
+                                           obvh_dito_trace& tr) {
     // The reference scan starts from point 0 and compares strictly
     // (dito.cpp:116-173): a slab whose value at point 0 is NaN stays (NaN, 0),
     // since no later compare against NaN succeeds; otherwise NaN values are
     // never taken and the result is the (value, first index) minimum over
-    // the other points, which is what the reductions above computed.
+    // the other points, which is what the reductions above computed.  A side
+    // without an index has no value beyond infinity: point 0 holds it.
     {
+        const f3 pt0 = pts.load(sbeg);
         float pr0[7];
         slab7(pt0, pr0);
 #pragma unroll
-        for (int k = 0; k < 7; ++k) {
-            if (pr0[k] != pr0[k]) {
-                v[k] = v[7 + k] = pr0[k];
-                ix[k] = ix[7 + k] = 0;
-            }
-        }
+        for (int k = 0; k < 7; ++k)
+            if (pr0[k] != pr0[k]) ix[k] = ix[7 + k] = 0;
     }
 #pragma unroll
     for (int side = 0; side < 14; ++side)
-        if ((uint64_t)ix[side] >= n) ix[side] = 0;  // not reachable (a slab that is NaN everywhere is NaN at point 0)
-    obvh_dito_trace tr = {};
+        if ((uint64_t)ix[side] >= n) ix[side] = 0;
+    tr = {};
     tr.pair_k = tr.p2_sel = tr.q0_sel = tr.q1_sel = -1;
     tr.best = -1;
     float mn[7], mx[7];
     f3 minv[7], maxv[7];
 #pragma unroll
     for (int k = 0; k < 7; ++k) {
-        mn[k] = v[k];
-        mx[k] = v[7 + k];
         tr.slab_min_idx[k] = ix[k];
         tr.slab_max_idx[k] = ix[7 + k];
         minv[k] = pts.load(sbeg + ix[k]);
         maxv[k] = pts.load(sbeg + ix[7 + k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+        float pr[7];
+        slab7(minv[k], pr);
+        mn[k] = pr[k];
+        slab7(maxv[k], pr);
+        mx[k] = pr[k];
     }
     f3 sel[14];
     if (n > 14) {
@@ -518,110 +689,89 @@ __device__ __forceinline__ void set_cand(P pts, uint64_t sbeg, uint64_t send, ui
 #pragma unroll
         for (int i = 1; i < 14; ++i) sel[i] = (uint64_t)i < n ? pts.load(sbeg + i) : sel[0];
     }
-    SetState st = {};
+    st = {};
     dito_candidate_search(mn, mx, minv, maxv, sel, st, tr);
-    if (lane == 0) {
+}
+
+// One wave: reduce the nt tile partials of a set (points [sbeg, send),
+// first tile ft), then search; state and trace written by lane 0.
+template <class P>
+__device__ __forceinline__ void set_cand(P pts, uint64_t sbeg, uint64_t send, uint32_t ft, uint32_t nt,
+                                         const float* part1_v, const uint32_t* part1_i, SetState* state,
+                                         obvh_dito_trace* trace) {
+    uint32_t ix[14];
+    reduce_partials<false>(ft, nt, part1_v, part1_i, ix);
+    SetState st;
+    obvh_dito_trace tr;
+    set_search(pts, sbeg, send - sbeg, ix, st, tr);
+    if (lane_id() == 0) {
         *state = st;
         *trace = tr;
     }
 }
 
 // One wave per set: reduce the tile partials, then the wave searches.
-template <class P>
-__global__ __launch_bounds__(kBlock) void dito_cand(P pts, const uint64_t* offs, uint32_t nsets, uint64_t total,
+__global__ __launch_bounds__(kBlock) void dito_cand(PtsSoA pts, const uint64_t* offs, uint32_t nsets, uint64_t total,
                                                     DitoWs ws, obvh_dito_trace* trace) {
     const uint32_t s = blockIdx.x * kWaves + wave_id();
     if (s >= nsets) return;
     const uint64_t sbeg = offs[s], send = offs[s + 1];
     if (send == sbeg || !set_valid(sbeg, send, total)) return;
     const uint32_t ft = ws.first_tile[s], nt = ws.first_tile[s + 1] - ft;
+    if (nt == 0) return;
     set_cand(pts, sbeg, send, ft, nt, ws.part1_v, ws.part1_i, &ws.state[s], &trace[s]);
 }
 
 // --------------------------------------------------------------- pass 2 --
 
-// Ranges of the points [base, end) on the set's three axes: 6 floats (min
-// b0..b2, max b0..b2) written to out6 by threads 0..5.
-template <class P>
-__device__ __forceinline__ void tile_pass2(P pts, uint64_t base, uint64_t end, const SetState* st,
-                                           float (&sh)[kWaves][6], float* out6) {
-    const int lane = lane_id(), wave = wave_id();
-    const float INF = FLT_MAX * 2.0f, NaN = __builtin_nanf("");
+// Ranges of a tile's cnt points on the set's three axes: 6 floats (min b0..b2,
+// max b0..b2) written to out6 by threads 0..7.  Ends with a barrier.
+template <class T>
+__device__ __forceinline__ void tile_pass2(const T& pts, uint32_t cnt, const SetState* st, FitLds<kBlock>& L,
+                                           float* out6) {
+    const float INF = FLT_MAX * 2.0f;
     float r[6] = {INF, INF, INF, -INF, -INF, -INF};
     if (st->mode != 1) {
-        const f3 b0 = f3{st->ax[0], st->ax[1], st->ax[2]};
-        const f3 b1 = f3{st->ax[3], st->ax[4], st->ax[5]};
-        const f3 b2 = f3{st->ax[6], st->ax[7], st->ax[8]};
-        const uint32_t nchunks = (uint32_t)((end - base + kChunk - 1) / kChunk);
-        for (uint32_t c = wave; c < nchunks; c += kWaves) {
-            const uint64_t cb = base + (uint64_t)c * kChunk + lane;
-            const bool full = base + (uint64_t)(c + 1) * kChunk <= end;
-            f3 p[kG];
+        f3 b[3];
+        state_axes(*st, b);
+        stream_tile(pts, cnt, [&](uint32_t, const f3 (&p)[kRows]) {
 #pragma unroll
-            for (int j = 0; j < kG; ++j) {
-                const uint64_t idx = cb + (uint64_t)j * kWave;
-                p[j] = (full || idx < end) ? pts.load(idx) : f3{NaN, NaN, NaN};
-            }
-#pragma unroll
-            for (int j = 0; j < kG; ++j) {
-                const float d0 = dot3(p[j], b0), d1 = dot3(p[j], b1), d2 = dot3(p[j], b2);
-                r[0] = fminf(r[0], d0); r[3] = fmaxf(r[3], d0);
-                r[1] = fminf(r[1], d1); r[4] = fmaxf(r[4], d1);
-                r[2] = fminf(r[2], d2); r[5] = fmaxf(r[5], d2);
-            }
-        }
+            for (int j = 0; j < kRows; j += 2) axes_step(p[j], p[j + 1], b, r);
+        });
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { r[k] = wave_min(r[k]); r[3 + k] = wave_max(r[3 + k]); }
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) sh[wave][k] = r[k];
-    }
+    for (int k = 3; k < 6; ++k) r[k] = -r[k];
+    const float y = wave_min6(r);
+    if ((lane_id() & 7) == 0) L.wrng[wave_id()][lane_id() >> 3] = y;
     __syncthreads();
-    if (threadIdx.x < 6) {
-        const int k = threadIdx.x;
-        float a = sh[0][k];
-        for (int w = 1; w < kWaves; ++w) a = k < 3 ? fminf(a, sh[w][k]) : fmaxf(a, sh[w][k]);
-        out6[k] = a;
+    const int q = threadIdx.x;
+    if (q < 8 && (q & 3) < 3) {
+        float a = L.wrng[0][q];
+        for (int w = 1; w < kWaves; ++w) a = fminf(a, L.wrng[w][q]);
+        out6[q < 4 ? q : q - 1] = q < 4 ? a : -a;
     }
     __syncthreads();
 }
 
-template <class P>
-__global__ __launch_bounds__(kBlock) void dito_pass2(P pts, const uint64_t* offs, uint32_t nsets,
-                                                     uint32_t tile, DitoWs ws) {
-    __shared__ float sh[kWaves][6];
+__global__ __launch_bounds__(kBlock) void dito_pass2(PtsSoA pts, const uint64_t* offs, uint32_t nsets, uint32_t tile,
+                                                     DitoWs ws) {
+    __shared__ FitLds<kBlock> L;
     const uint32_t T = ws.first_tile[nsets];
     for (uint32_t t = blockIdx.x; t < T; t += gridDim.x) {
         const uint32_t s = ws.tile_set[t];
         const uint64_t sbeg = offs[s], send = offs[s + 1];
-        const uint32_t ft = ws.first_tile[s];
-        const uint64_t base = sbeg + (uint64_t)(t - ft) * tile;
-        const uint64_t end = base + tile < send ? base + tile : send;
-        tile_pass2(pts, base, end, &ws.state[s], sh, &ws.part2[(size_t)t * 6]);
+        const uint64_t first = (uint64_t)(t - ws.first_tile[s]) * tile;
+        tile_pass2(tile_of(pts, sbeg + first), (uint32_t)min((uint64_t)tile, send - sbeg - first), &ws.state[s], L,
+                   &ws.part2[(size_t)t * 6]);
     }
 }
 
 // ---------------------------------------------------------------- final --
 
-// One wave: reduce the nt tile ranges of a set (first tile ft) and write
-// its box (lane 0).
+// The box of a set from its ranges on the axes (min b0..b2, max b0..b2); one
+// lane.  Returns whether it is the AABB.
 template <class P>
-__device__ __forceinline__ void set_final(P pts, uint64_t sbeg, uint32_t ft, uint32_t nt, const float* part2,
-                                          const SetState* state, kr_obb3* out, obvh_dito_trace* trace) {
-    const float INF = FLT_MAX * 2.0f;
-    float a[6] = {INF, INF, INF, -INF, -INF, -INF};
-    for (uint32_t j = lane_id(); j < nt; j += kWave) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            const float o = part2[(size_t)(ft + j) * 6 + k];
-            a[k] = k < 3 ? fminf(a[k], o) : fmaxf(a[k], o);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) { a[k] = wave_min(a[k]); a[3 + k] = wave_max(a[3 + k]); }
-    if (lane_id() != 0) return;
-    const SetState st = *state;
+__device__ __forceinline__ int set_box(P pts, uint64_t sbeg, float (&a)[6], const SetState& st, kr_obb3* out) {
     const f3 b0 = f3{st.ax[0], st.ax[1], st.ax[2]};
     const f3 b1 = f3{st.ax[3], st.ax[4], st.ax[5]};
     const f3 b2 = f3{st.ax[6], st.ax[7], st.ax[8]};
@@ -666,17 +816,36 @@ __device__ __forceinline__ void set_final(P pts, uint64_t sbeg, uint32_t ft, uin
     o.ext.y = kmax(o.ext.y, 0.001f);
     o.ext.z = kmax(o.ext.z, 0.001f);
     *out = o;
-    trace->result_aabb = result_aabb;
+    return result_aabb;
 }
 
+// One wave: reduce the nt tile ranges of a set (first tile ft) and write
+// its box (lane 0).
 template <class P>
-__global__ __launch_bounds__(kBlock) void dito_final(P pts, const uint64_t* offs, uint32_t nsets, uint64_t total,
+__device__ __forceinline__ void set_final(P pts, uint64_t sbeg, uint32_t ft, uint32_t nt, const float* part2,
+                                          const SetState* state, kr_obb3* out, obvh_dito_trace* trace) {
+    const float INF = FLT_MAX * 2.0f;
+    float a[6] = {INF, INF, INF, -INF, -INF, -INF};
+    for (uint32_t j = lane_id(); j < nt; j += kWave) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const float o = part2[(size_t)(ft + j) * 6 + k];
+            a[k] = k < 3 ? fminf(a[k], o) : fmaxf(a[k], o);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { a[k] = wave_min(a[k]); a[3 + k] = wave_max(a[3 + k]); }
+    if (lane_id() == 0) trace->result_aabb = set_box(pts, sbeg, a, *state, out);
+}
+
+__global__ __launch_bounds__(kBlock) void dito_final(PtsSoA pts, const uint64_t* offs, uint32_t nsets, uint64_t total,
                                                      DitoWs ws, kr_obb3* out, obvh_dito_trace* trace) {
     const uint32_t s = blockIdx.x * kWaves + wave_id();
     if (s >= nsets) return;
     const uint64_t sbeg = offs[s], send = offs[s + 1];
     if (send == sbeg || !set_valid(sbeg, send, total)) return;
     const uint32_t ft = ws.first_tile[s], nt = ws.first_tile[s + 1] - ft;
+    if (nt == 0) return;
     set_final(pts, sbeg, ft, nt, ws.part2, &ws.state[s], &out[s], &trace[s]);
 }
 
@@ -693,24 +862,23 @@ __global__ __launch_bounds__(kBlock) void dito_final(P pts, const uint64_t* offs
 // each last workgroup resets its counter, so later calls need no clear.
 
 __global__ void dito_one_clear(DitoWs ws) {
-    if (threadIdx.x < 2) ws.done[threadIdx.x] = 0;
+    if (threadIdx.x < 4) ws.done[threadIdx.x] = 0;
 }
 
 template <class P>
 __global__ __launch_bounds__(kBlock) void dito_one_a(P pts, uint64_t n, uint32_t tile, DitoWs ws,
                                                      obvh_dito_trace* trace) {
-    __shared__ float sh_v[kWaves][14];
-    __shared__ uint32_t sh_i[kWaves][14];
-    __shared__ uint32_t last;
+    __shared__ FitLds<kBlock> L;
     const uint32_t t = blockIdx.x, T = gridDim.x;
-    const uint64_t base = (uint64_t)t * tile, end = base + tile < n ? base + tile : n;
+    const uint64_t base = (uint64_t)t * tile;
+    tile_pass1(tile_of(pts, base), (uint32_t)min((uint64_t)tile, n - base), L);
     // threads 0..13 (wave 0) write the tile's pairs; thread 0's release
     // orders them before its count
-    tile_pass1(pts, 0, base, end, sh_v, sh_i, &ws.part1_v[(size_t)t * 14], &ws.part1_i[(size_t)t * 14]);
+    store_pairs(L, (uint32_t)base, &ws.part1_v[(size_t)t * 14], &ws.part1_i[(size_t)t * 14]);
     if (threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(&ws.done[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
+        L.last = __hip_atomic_fetch_add(&ws.done[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
     __syncthreads();
-    if (!last || wave_id() != 0) return;
+    if (!L.last || wave_id() != 0) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     set_cand(pts, 0, n, 0, T, ws.part1_v, ws.part1_i, ws.state, trace);
     if (lane_id() == 0) __hip_atomic_store(&ws.done[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -719,18 +887,280 @@ __global__ __launch_bounds__(kBlock) void dito_one_a(P pts, uint64_t n, uint32_t
 template <class P>
 __global__ __launch_bounds__(kBlock) void dito_one_b(P pts, uint64_t n, uint32_t tile, DitoWs ws, kr_obb3* out,
                                                      obvh_dito_trace* trace) {
-    __shared__ float sh[kWaves][6];
-    __shared__ uint32_t last;
+    __shared__ FitLds<kBlock> L;
     const uint32_t t = blockIdx.x, T = gridDim.x;
-    const uint64_t base = (uint64_t)t * tile, end = base + tile < n ? base + tile : n;
-    tile_pass2(pts, base, end, ws.state, sh, &ws.part2[(size_t)t * 6]);  // threads 0..5 write
+    const uint64_t base = (uint64_t)t * tile;
+    tile_pass2(tile_of(pts, base), (uint32_t)min((uint64_t)tile, n - base), ws.state, L,
+               &ws.part2[(size_t)t * 6]);  // threads 0..7 write
     if (threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(&ws.done[1], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
+        L.last = __hip_atomic_fetch_add(&ws.done[1], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
     __syncthreads();
-    if (!last || wave_id() != 0) return;
+    if (!L.last || wave_id() != 0) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     set_final(pts, 0, 0, T, ws.part2, ws.state, out, trace);
     if (lane_id() == 0) __hip_atomic_store(&ws.done[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ------------------------------------------------------- one-launch fits --
+//
+// A single set in one launch: its tiles hand their partial results over inside
+// the launch with the agent-scope accesses above.
+//
+// Waiting ends: the tiles wait for each other, and there are at most `cap` of
+// them, an eighth of the workgroups the device holds (so up to eight such
+// launches may share it; larger sets take two launches).  The polls are
+// bounded all the same; a fit that exceeds the bound gets a NaN box.
+
+constexpr uint32_t kPollLimit = 1u << 22;
+
+constexpr int kStateWords = sizeof(SetState) / 4;
+constexpr int kTraceWords = sizeof(obvh_dito_trace) / 4;
+constexpr int kTraceResult = offsetof(obvh_dito_trace, result_aabb) / 4;
+static_assert(kStateWords <= kWave && kTraceWords <= kWave, "copied by one wave");
+
+// Points [first, first + cnt) of tile rows j (index j * kThreads + thread);
+// past the end a copy of the last one, which no strict rule takes.
+template <class P, int J, int kThreads>
+__device__ __forceinline__ void load_tile(P pts, uint64_t first, uint32_t cnt, f3 (&p)[J]) {
+    const uint32_t t = threadIdx.x;
+    if (cnt == (uint32_t)(J * kThreads)) {  // uniform
+#pragma unroll
+        for (int j = 0; j < J; ++j) p[j] = pts.load(first + (uint32_t)j * kThreads + t);
+        return;
+    }
+#pragma unroll
+    for (int c = 0; c < J; c += kRows) {
+        if ((uint32_t)(c * kThreads) < cnt) {
+#pragma unroll
+            for (int j = c; j < c + kRows; ++j) p[j] = pts.load(first + min((uint32_t)j * kThreads + t, cnt - 1));
+        } else {
+#pragma unroll
+            for (int j = c; j < c + kRows; ++j) p[j] = p[0];
+        }
+    }
+}
+
+template <int kSide>
+__device__ __forceinline__ float slab_side(f3 p) {  // the side's projection, negated for a maximum
+    float pr[7];
+    slab7(p, pr);
+    return kSide < 7 ? pr[kSide % 7] : -pr[kSide % 7];
+}
+
+// Where the tile reaches its extreme on one side: the lanes whose own extreme
+// equals it (usually one lane of one wave) look for the first of their points.
+template <int kSide, int J, int kThreads>
+__device__ __forceinline__ void find_side(const f3 (&p)[J], uint32_t cnt, float own, FitLds<kThreads>& L) {
+    const float target = L.ext[side_slot(kSide)];
+    if (__ballot(own == target) == 0) return;
+    uint32_t at = kNoIdx;
+#pragma unroll
+    for (int c = J - kRows; c >= 0; c -= kRows) {
+        if ((uint32_t)(c * kThreads) >= cnt) continue;
+#pragma unroll
+        for (int j = c + kRows - 1; j >= c; --j)
+            if (slab_side<kSide>(p[j]) == target) at = (uint32_t)j;
+    }
+    // (one atomic per wave: in a set of equal points every lane is here)
+    const int32_t first = wave_min_i32(at == kNoIdx ? 0x7FFFFFFF : (int32_t)(at * kThreads + threadIdx.x));
+    if (lane_id() == 0 && first != 0x7FFFFFFF) atomicMin(&L.idx[side_slot(kSide)], (uint32_t)first);
+}
+
+// Wave 0: the set's state for the axis pass, from the flag's set-up.
+// False when the poll limit is exceeded.
+__device__ __forceinline__ bool wait_state(const FitSync* sync, const SetState* state, SetState* lds) {
+    uint32_t up = 0;
+    for (uint32_t i = 0; i < kPollLimit && up == 0; ++i) {
+        if (i > 0) __builtin_amdgcn_s_sleep(8);
+        up = __builtin_amdgcn_readfirstlane((int)ld_agent(&sync->flag));
+    }
+    asm volatile("" ::: "memory");
+    if (lane_id() < kStateWords)
+        reinterpret_cast<uint32_t*>(lds)[lane_id()] = ld_agent(reinterpret_cast<const uint32_t*>(state) + lane_id());
+    return up != 0;
+}
+
+__device__ __forceinline__ void fit_fail(kr_obb3* out, obvh_dito_trace* trace) {
+    *out = nan_box();
+    if (trace) trace->degenerate = 4;
+}
+
+// After the slab pass of tile `part` of nt (partials from tile ft), L.ext and
+// L.idx (indices from the tile's first point, `first` of the set): publish
+// them; the last tile searches.  Returns whether this workgroup did (L.st then
+// holds the state).  Ends with a barrier.
+template <class P, int kThreads>
+__device__ __forceinline__ bool tile_search(P pts, uint64_t sbeg, uint64_t n, uint32_t first, uint32_t part,
+                                            uint32_t ft, uint32_t nt, const DitoWs& ws, SetState* state,
+                                            FitSync* sync, obvh_dito_trace* trace, FitLds<kThreads>& L) {
+    const int lane = lane_id(), wave = wave_id();
+    if (nt > 1) {
+        if (wave == 0) {
+            if (lane < 14) {
+                const size_t at = (size_t)(ft + part) * 14 + lane;
+                const int slot = side_slot(lane);
+                const uint32_t i = L.idx[slot];
+                st_agent(&ws.part1_v[at], lane < 7 ? L.ext[slot] : -L.ext[slot]);
+                st_agent(&ws.part1_i[at], i == kNoIdx ? kNoIdx : first + i);
+            }
+            drain();
+            if (lane == 0)
+                L.last = __hip_atomic_fetch_add(&sync->done1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nt - 1;
+        }
+        __syncthreads();
+        if (L.last == 0) return false;
+    }
+    if (wave == 0) {
+        uint32_t ix[14];
+        if (nt == 1) {
+#pragma unroll
+            for (int k = 0; k < 14; ++k) ix[k] = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.idx[side_slot(k)]);
+        } else {
+            asm volatile("" ::: "memory");
+            reduce_partials<true>(ft, nt, ws.part1_v, ws.part1_i, ix);
+        }
+        SetState st;
+        obvh_dito_trace tr;
+        set_search(pts, sbeg, n, ix, st, tr);
+        if (lane == 0) L.st = st;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (nt > 1) {
+            if (lane < kStateWords)
+                st_agent(reinterpret_cast<uint32_t*>(state) + lane, reinterpret_cast<const uint32_t*>(&L.st)[lane]);
+            drain();
+            if (lane == 0) st_agent(&sync->flag, 1u);
+        }
+        if (trace && lane == 0) {  // the box's workgroup writes result_aabb
+#pragma unroll
+            for (int k = 0; k < kTraceWords; ++k)
+                if (k != kTraceResult) reinterpret_cast<uint32_t*>(trace)[k] = reinterpret_cast<const uint32_t*>(&tr)[k];
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
+// After the axis pass: r, each lane's ranges (maxima not negated).  The last
+// tile of the set writes the box.
+template <class P, int kThreads>
+__device__ __forceinline__ void tile_box(P pts, uint64_t sbeg, float (&r)[6], uint32_t part, uint32_t ft, uint32_t nt,
+                                         const DitoWs& ws, FitSync* sync, kr_obb3* out, obvh_dito_trace* trace,
+                                         FitLds<kThreads>& L) {
+    const float INF = FLT_MAX * 2.0f;
+    const int lane = lane_id(), wave = wave_id();
+#pragma unroll
+    for (int k = 3; k < 6; ++k) r[k] = -r[k];
+    const float y = wave_min6(r);
+    if ((lane & 7) == 0) L.wrng[wave][lane >> 3] = y;
+    __syncthreads();
+    if (wave != 0) return;
+    if (lane < 8) {
+        float a = L.wrng[0][lane];
+        for (int w = 1; w < kThreads / kWave; ++w) a = fminf(a, L.wrng[w][lane]);
+        L.rng[lane] = a;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float a[6];
+    if (nt == 1) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            a[k] = L.rng[k];
+            a[3 + k] = -L.rng[4 + k];
+        }
+    } else {
+        if (lane < 6) st_agent(&ws.part2[(size_t)(ft + part) * 6 + lane], lane < 3 ? L.rng[lane] : -L.rng[lane + 1]);
+        drain();
+        uint32_t old = 0;
+        if (lane == 0) old = __hip_atomic_fetch_add(&sync->done2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)old) != nt - 1) return;
+        asm volatile("" ::: "memory");
+        float q[6] = {INF, INF, INF, -INF, -INF, -INF};
+        for (uint32_t j = lane; j < nt; j += kWave) {
+            float o[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) o[k] = ld_agent(&ws.part2[(size_t)(ft + j) * 6 + k]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) { q[k] = fminf(q[k], o[k]); q[3 + k] = fmaxf(q[3 + k], o[3 + k]); }
+        }
+#pragma unroll
+        for (int k = 3; k < 6; ++k) q[k] = -q[k];
+        const float z = wave_min6(q);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            a[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(z), 8 * k));
+            a[3 + k] = -__int_as_float(__builtin_amdgcn_readlane(__float_as_int(z), 32 + 8 * k));
+        }
+        if (lane == 0) {  // nobody reads them any more: zero for the next call on this workspace
+            st_agent(&sync->done1, 0u);
+            st_agent(&sync->done2, 0u);
+            st_agent(&sync->flag, 0u);
+        }
+    }
+    if (lane == 0) {
+        const int aabb = set_box(pts, sbeg, a, L.st, out);
+        if (trace) st_agent(&trace->result_aabb, aabb);
+    }
+}
+
+// A workgroup keeps its tile's points in registers between the passes; the
+// last tile to finish the slab pass searches, the others wait for its state.
+// Up to 8192 points one workgroup does it all (no hand-over: 23 -> 12.4 us);
+// 131 072 points take 64 tiles (26.7 -> 20.9 us).  Batches read their points
+// again instead: tiles that wait in registers for their set's search held
+// 75 MB for 68 us each, three times the time of two readings.
+template <class P, int J, int kThreads>
+__device__ __forceinline__ void one_tile(P pts, uint64_t n, uint32_t part, uint32_t nt, const DitoWs& ws, kr_obb3* out,
+                                         obvh_dito_trace* trace, FitLds<kThreads>& L) {
+    constexpr uint32_t kTilePts = J * kThreads;
+    const float INF = FLT_MAX * 2.0f;
+    FitSync* sync = reinterpret_cast<FitSync*>(ws.done);
+    const uint64_t first = (uint64_t)part * kTilePts;
+    const uint32_t cnt = (uint32_t)min((uint64_t)kTilePts, n - first);
+    f3 p[J];
+    load_tile<P, J, kThreads>(pts, first, cnt, p);
+    float e[14];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) { e[k] = INF; e[7 + k] = -INF; }
+#pragma unroll
+    for (int j = 0; j < J; j += 2) slabs_step(p[j], p[j + 1], e);
+#pragma unroll
+    for (int k = 7; k < 14; ++k) e[k] = -e[k];
+    tile_extremes(e, L);
+    find_side<0>(p, cnt, e[0], L); find_side<1>(p, cnt, e[1], L); find_side<2>(p, cnt, e[2], L);
+    find_side<3>(p, cnt, e[3], L); find_side<4>(p, cnt, e[4], L); find_side<5>(p, cnt, e[5], L);
+    find_side<6>(p, cnt, e[6], L); find_side<7>(p, cnt, e[7], L); find_side<8>(p, cnt, e[8], L);
+    find_side<9>(p, cnt, e[9], L); find_side<10>(p, cnt, e[10], L); find_side<11>(p, cnt, e[11], L);
+    find_side<12>(p, cnt, e[12], L); find_side<13>(p, cnt, e[13], L);
+    __syncthreads();
+    if (tile_search(pts, 0, n, (uint32_t)first, part, 0, nt, ws, ws.state, sync, trace, L)) {
+        load_tile<P, J, kThreads>(pts, first, cnt, p);  // the search used the registers
+    } else {
+        if (wave_id() == 0) {
+            const bool ok = wait_state(sync, ws.state, &L.st);
+            if (lane_id() == 0) L.fail = ok ? 0u : 1u;
+        }
+        __syncthreads();
+        if (L.fail != 0) {
+            if (threadIdx.x == 0) fit_fail(out, trace);
+            return;
+        }
+    }
+    f3 b[3];
+    state_axes(L.st, b);
+    float r[6] = {INF, INF, INF, -INF, -INF, -INF};
+#pragma unroll
+    for (int j = 0; j < J; j += 2) axes_step(p[j], p[j + 1], b, r);
+    tile_box(pts, 0, r, part, 0, nt, ws, sync, out, trace, L);
+}
+
+// A set of n > 0 points, gridDim.x tiles.
+template <class P, int J, int kThreads>
+__global__ __launch_bounds__(kThreads) void dito_one(P pts, uint64_t n, DitoWs ws, kr_obb3* out,
+                                                     obvh_dito_trace* trace) {
+    __shared__ FitLds<kThreads> L;
+    one_tile<P, J, kThreads>(pts, n, blockIdx.x, gridDim.x, ws, out, trace, L);
 }
 
 // ----------------------------------------------------------------- host --
@@ -740,10 +1170,11 @@ size_t dito_max_tiles(uint32_t nsets, uint64_t total, uint32_t tile) {
 }
 
 size_t dito_carve(DitoWs* ws, void* base, size_t cap, uint32_t nsets, uint64_t total, uint32_t tile) {
+    tile = min(tile, kDitoMaxTile);
     Carver c{(char*)base, 0, cap};
     const size_t T = dito_max_tiles(nsets, total, tile);
     ws->offsets_single = c.take<uint64_t>(2);
-    ws->done = c.take<uint32_t>(2);
+    ws->done = c.take<uint32_t>(4);
     ws->first_tile = c.take<uint32_t>(nsets + 1);
     ws->tile_set = c.take<uint32_t>(T);
     ws->part1_v = c.take<float>(T * 14);
@@ -755,30 +1186,63 @@ size_t dito_carve(DitoWs* ws, void* base, size_t cap, uint32_t nsets, uint64_t t
 }
 
 uint32_t dito_auto_tile(uint32_t nsets, uint64_t total) {
-    // about 4096 tiles for the whole job, between 512 and 65536 points each
+    // about 4096 tiles for the whole job, between 512 and 32768 points each
+    // (8192 sets, 897 M points: 3.52 ms with 32768, 3.54 with 16384, 3.59 with
+    // 65536)
     (void)nsets;
     uint64_t want = total / 4096;
     uint64_t t = (want + kChunk - 1) / kChunk * kChunk;
     if (t < (uint64_t)kChunk) t = kChunk;
-    if (t > 65536) t = 65536;
+    if (t > 32768) t = 32768;
     return (uint32_t)t;
 }
 
+// Tiles of one set that may wait for each other: an eighth of the workgroups
+// the device holds at four per CU.
+static kr_error one_cap(uint32_t* cap) {
+    static std::atomic<uint32_t> cached[64];
+    int dev = 0;
+    OBVH_HIP_TRY(hipGetDevice(&dev));
+    uint32_t v = dev >= 0 && dev < 64 ? cached[dev].load(std::memory_order_relaxed) : 0;
+    if (v == 0) {
+        int cus = 0;
+        OBVH_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        v = (uint32_t)max(cus / 2, 1);
+        if (dev >= 0 && dev < 64) cached[dev].store(v, std::memory_order_relaxed);
+    }
+    *cap = v;
+    return nullptr;
+}
+
+constexpr int kOneRows = 8;  // points per lane of the single fit's workgroups
+
 template <class P>
-static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, DitoWs ws, kr_obb3* out, obvh_dito_trace* tr,
-                       bool clear, hipStream_t stream) {
+static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, uint32_t cap, DitoWs ws, kr_obb3* out,
+                       obvh_dito_trace* trace, bool& clear, hipStream_t stream) {
+    if (n <= 1024 * kOneRows) {
+        hipLaunchKernelGGL((dito_one<P, kOneRows, 1024>), dim3(1), dim3(1024), 0, stream, p, n, ws, out, trace);
+        return;
+    }
     if (clear) hipLaunchKernelGGL(dito_one_clear, dim3(1), dim3(64), 0, stream, ws);
+    clear = false;
+    constexpr uint32_t kOneTile = kBlock * kOneRows;
+    const uint64_t F = (n + kOneTile - 1) / kOneTile;
+    if (F <= cap) {
+        hipLaunchKernelGGL((dito_one<P, kOneRows, kBlock>), dim3((uint32_t)F), dim3(kBlock), 0, stream, p, n, ws, out,
+                           trace);
+        return;
+    }
+    obvh_dito_trace* tr = trace ? trace : ws.trace_tmp;
     hipLaunchKernelGGL(dito_one_a<P>, dim3(T), dim3(kBlock), 0, stream, p, n, tile, ws, tr);
     hipLaunchKernelGGL(dito_one_b<P>, dim3(T), dim3(kBlock), 0, stream, p, n, tile, ws, out, tr);
 }
 
 kr_error dito_one_launch(const float* x, const float* y, const float* z, const float* xyz, uint64_t n,
-                         kr_obb3* out, obvh_dito_trace* trace, void* workspace, size_t ws_bytes, bool clear,
+                         kr_obb3* out, obvh_dito_trace* trace, void* workspace, size_t ws_bytes, bool& clear,
                          hipStream_t stream) {
-    if (n == 0) return "obvh_dito: the two-launch fit needs at least one point";
-    // Tiles of 2048 points (one chunk per wave) up to 1024 tiles, larger
-    // beyond: each workgroup pays one agent-scope release and the last one
-    // reduces every tile, so a small set wants few tiles.  At least the
+    if (n == 0) return "obvh_dito: the single-set fit needs at least one point";
+    // The two-launch form's tiles: at most 1024, since each workgroup pays one
+    // agent-scope release and the last one reduces every tile.  At least the
     // batched path's tile, so the workspace size of obvh_dito_workspace_size
     // always suffices.
     uint64_t tl = (n + 1023) / 1024;
@@ -789,30 +1253,23 @@ kr_error dito_one_launch(const float* x, const float* y, const float* z, const f
     if (workspace == nullptr || ws_bytes < need) return "obvh_dito: workspace too small";
     const uint64_t T = (n + tile - 1) / tile;
     if (T > dito_max_tiles(1, n, tile)) return "obvh_dito: tile count";
-    obvh_dito_trace* tr = trace ? trace : ws.trace_tmp;
-    if (xyz) launch_one(PtsAoS{xyz}, n, tile, (uint32_t)T, ws, out, tr, clear, stream);
-    else launch_one(PtsSoA{x, y, z}, n, tile, (uint32_t)T, ws, out, tr, clear, stream);
+    uint32_t cap = 0;
+    if (kr_error e = one_cap(&cap)) return e;
+    cap = (uint32_t)min((uint64_t)cap, (uint64_t)dito_max_tiles(1, n, tile));
+    if (xyz) launch_one(PtsAoS{xyz}, n, tile, (uint32_t)T, cap, ws, out, trace, clear, stream);
+    else launch_one(PtsSoA{x, y, z}, n, tile, (uint32_t)T, cap, ws, out, trace, clear, stream);
     OBVH_HIP_TRY(hipGetLastError());
     return nullptr;
 }
 
-template <class P>
-static void launch_passes(P p, const uint64_t* offs, uint32_t nsets, uint64_t total, uint32_t tile, uint32_t workers,
-                          DitoWs ws, kr_obb3* out, obvh_dito_trace* tr, hipStream_t stream) {
-    const dim3 set_grid((nsets + kWaves - 1) / kWaves);
-    hipLaunchKernelGGL(dito_pass1<P>, dim3(workers), dim3(kBlock), 0, stream, p, offs, nsets, tile, ws);
-    hipLaunchKernelGGL(dito_cand<P>, set_grid, dim3(kBlock), 0, stream, p, offs, nsets, total, ws, tr);
-    hipLaunchKernelGGL(dito_pass2<P>, dim3(workers), dim3(kBlock), 0, stream, p, offs, nsets, tile, ws);
-    hipLaunchKernelGGL(dito_final<P>, set_grid, dim3(kBlock), 0, stream, p, offs, nsets, total, ws, out, tr);
-}
-
-kr_error dito_launch(const float* x, const float* y, const float* z, const float* xyz,
+kr_error dito_launch(const float* x, const float* y, const float* z,
                      const uint64_t* offsets, uint64_t single_count, uint32_t nsets, uint64_t total,
                      kr_obb3* out, obvh_dito_trace* trace, uint32_t tile, uint32_t workers,
                      void* workspace, size_t ws_bytes, hipStream_t stream) {
     if (nsets == 0) return nullptr;
     if (tile == 0) tile = dito_auto_tile(nsets, total);
     if (tile % kChunk != 0) return "obvh_dito: tile_points must be a multiple of 512";
+    tile = min(tile, kDitoMaxTile);
     DitoWs ws;
     const size_t need = dito_carve(&ws, workspace, ws_bytes, nsets, total, tile);
     if (workspace == nullptr || ws_bytes < need) return "obvh_dito: workspace too small";
@@ -829,8 +1286,12 @@ kr_error dito_launch(const float* x, const float* y, const float* z, const float
     uint32_t tb = (uint32_t)((T + 255) / 256);
     if (tb > 4096) tb = 4096;
     hipLaunchKernelGGL(dito_tile_table, dim3(tb), dim3(256), 0, stream, nsets, ws);
-    if (xyz) launch_passes(PtsAoS{xyz}, offs, nsets, total, tile, workers, ws, out, tr, stream);
-    else launch_passes(PtsSoA{x, y, z}, offs, nsets, total, tile, workers, ws, out, tr, stream);
+    const PtsSoA p{x, y, z};
+    const dim3 set_grid((nsets + kWaves - 1) / kWaves);
+    hipLaunchKernelGGL(dito_pass1, dim3(workers), dim3(kBlock), 0, stream, p, offs, nsets, tile, ws);
+    hipLaunchKernelGGL(dito_cand, set_grid, dim3(kBlock), 0, stream, p, offs, nsets, total, ws, tr);
+    hipLaunchKernelGGL(dito_pass2, dim3(workers), dim3(kBlock), 0, stream, p, offs, nsets, tile, ws);
+    hipLaunchKernelGGL(dito_final, set_grid, dim3(kBlock), 0, stream, p, offs, nsets, total, ws, out, tr);
     OBVH_HIP_TRY(hipGetLastError());
     return nullptr;
 }

@@ -348,3 +348,71 @@ def test_obb_tree_renumbering_canary(torch, oracle_lib, mesh, builder):
     assert np.array_equal(m1[old2new], m0)
     eo, em = oracle_lib.obb_tree(nodes, parents, V, F)
     assert np.array_equal(o0, eo) and np.array_equal(m0, em)
+
+
+def tied_points(n, seed):
+    """n points whose extremes are reached several times: small integers, with the last point a copy of an
+    extreme one, and a run of equal points."""
+    rng = np.random.default_rng(seed)
+    p = rng.integers(-40, 41, (n, 3)).astype(np.float32)
+    p[n // 2:n // 2 + n // 5] = p[0]
+    p[-1] = p[int(np.argmax(p[:, 0]))]
+    return p
+
+
+# edges of the single fit's forms: one workgroup (8192 points), tiles of 2048 that wait for each other (up to 128),
+# two launches above; of a tile's rows and steps
+@pytest.mark.parametrize("n", [1, 255, 1024, 1025, 2049, 8191, 8192, 8193, 10240, 10241, 262144, 262145, 300001])
+@pytest.mark.parametrize("kind", ["gaussian", "tied", "nan"])
+def test_dito_single_forms(torch, oracle_lib, n, kind):
+    say(f"[dito_soa] n={n} {kind}")
+    p = tied_points(n, n) if kind == "tied" else synth.gaussian_points(n, seed=n)
+    if kind == "nan":
+        p[n // 2::7] = np.nan
+        p[n // 3, 1] = np.inf
+    exp, etr = oracle_lib.points_obb(p, trace=True)
+    x, y, z = soa(torch, p)
+    ws = torch.full((int(ops.lib().obvh_dito_workspace_size(n)),), 0x5A, dtype=torch.uint8, device="cuda")
+    for _ in range(2):  # the second call on what the first left in the workspace
+        out, tr = ops.dito(x, y, z, trace=True, workspace=ws)
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), exp, equal_nan=True), (out.cpu().numpy(), exp)
+        assert_trace_equal(ops.trace_to_numpy(tr)[0], etr)
+    if n <= 262145:
+        assert np.array_equal(ops.points_obb(p), oracle_lib.points_obb(p), equal_nan=True)
+
+
+# tiles of one step and more, remainders of a wave's 512 points, every alignment of a set's first point
+@pytest.mark.parametrize("tile", [0, 512, 2048, 32768])
+def test_dito_batch_tile_edges(torch, oracle_lib, tile):
+    say(f"[dito_batch] tile edges, tile={tile}")
+    sizes = np.array([1, 3, 511, 512, 513, 1, 2047, 2048, 2049, 4097, 2, 6145, 32767, 32769, 70001], dtype=np.int64)
+    pts = np.concatenate([tied_points(int(n), 5 + k) if k % 2 else synth.gaussian_points(int(n), seed=k)
+                          for k, n in enumerate(sizes)])
+    pts[600:5000:97, 2] = np.nan
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    exp, etr = oracle_lib.points_obb_batch(pts, off.astype(np.uint64))
+    x, y, z = soa(torch, pts)
+    out, tr = ops.dito_batch(x, y, z, torch.from_numpy(off).cuda(), tile_points=tile, trace=True)
+    torch.cuda.synchronize()
+    gtr = ops.trace_to_numpy(tr)
+    for s in range(len(sizes)):
+        assert np.array_equal(out[s].cpu().numpy(), exp[s], equal_nan=True), (s, sizes[s])
+        assert_trace_equal(gtr[s], etr[s])
+
+
+def test_dito_batch_overlapping_sets(torch, oracle_lib):
+    """Offsets that go back make sets overlap: the sets that fit the tile table keep their boxes, those beyond it and
+    the decreasing ones are invalid (NaN, degenerate 4)."""
+    say("[dito_batch] overlapping sets")
+    n = 5 * 512
+    p = synth.gaussian_points(n, seed=3)
+    x, y, z = soa(torch, p)
+    off = torch.tensor([0, n, 0, n, 0, n, 0, n], dtype=torch.int64).cuda()  # 20 tiles, the table has 13
+    out, tr = ops.dito_batch(x, y, z, off, tile_points=512, trace=True)
+    torch.cuda.synchronize()
+    got, g = out.cpu().numpy(), ops.trace_to_numpy(tr)
+    exp = oracle_lib.points_obb(p)
+    assert np.array_equal(got[0], exp) and np.array_equal(got[2], exp)
+    for s in (1, 3, 4, 5, 6):
+        assert np.isnan(got[s]).all() and g[s]["degenerate"] == 4, s
