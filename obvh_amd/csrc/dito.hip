@@ -1188,12 +1188,13 @@ size_t dito_carve(DitoWs* ws, void* base, size_t cap, uint32_t nsets, uint64_t t
 uint32_t dito_auto_tile(uint32_t nsets, uint64_t total) {
     // about 4096 tiles for the whole job, between 512 and 32768 points each
     // (8192 sets, 897 M points: 3.52 ms with 32768, 3.54 with 16384, 3.59 with
-    // 65536)
-    (void)nsets;
+    // 65536); up to 65536 for a single set, whose workspace for 2^28 points
+    // must fit the static array of the no-allocation entry
     uint64_t want = total / 4096;
     uint64_t t = (want + kChunk - 1) / kChunk * kChunk;
     if (t < (uint64_t)kChunk) t = kChunk;
-    if (t > 32768) t = 32768;
+    const uint64_t most = nsets == 1 ? 65536 : 32768;
+    if (t > most) t = most;
     return (uint32_t)t;
 }
 
