@@ -22,7 +22,8 @@
 //  atr_export     nodes, parents and leaf bounds from the records
 //  (final)        bounds / counts / costs bottom-up with kr_aabb_expand
 //                 (atrbvh.cu:95-179).
-// Every bottom-up pass uses the phased arrival protocol of phased.hpp.
+// The optimiser passes use the phased arrival protocol of phased.hpp, the last
+// pass that of bottomup.hpp.
 // Working-box min/max order -0 below +0 (as fminf/fmaxf on the reference
 // GPU); the final bounds use kr_min/kr_max like kr_aabb_expand.
 #include <float.h>
@@ -30,6 +31,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "atrbvh.hpp"
+#include "bottomup.hpp"
 #include "common.hpp"
 
 namespace obvh {
@@ -752,43 +754,9 @@ __global__ __launch_bounds__(256) void atr_export(AtrWs ws, uint32_t nf, kr_bvh_
 
 // Bounds / counts / costs of the final tree (atrbvh.cu:124-179: ct = 1.0,
 // ci = 1.2, kr_aabb_expand), the same pass as the LBVH builder's.
-__device__ __forceinline__ f3 kmin3(f3 a, f3 b) { return f3{kmin(a.x, b.x), kmin(a.y, b.y), kmin(a.z, b.z)}; }
-__device__ __forceinline__ f3 kmax3(f3 a, f3 b) { return f3{kmax(a.x, b.x), kmax(a.y, b.y), kmax(a.z, b.z)}; }
-__device__ __forceinline__ float kr_area(f3 mn, f3 mx) {
-    const f3 d = sub3(mx, mn);
-    return 2.0f * (d.x * d.y + d.x * d.z + d.y * d.z);
-}
-struct AtrFinalUp {
-    kr_bvh_node* nodes;
-    uint32_t* counts;
-    float* costs;
-    __device__ void leaf(uint32_t cur) {
-        const kr_bvh_node L = nodes[cur];
-        costs[cur] = 1.0f * kr_area(f3{L.bounds.min.x, L.bounds.min.y, L.bounds.min.z},
-                                    f3{L.bounds.max.x, L.bounds.max.y, L.bounds.max.z});
-        counts[cur] = 1;
-    }
-    __device__ void merge(uint32_t p, uint32_t l, uint32_t r) {
-        const kr_bvh_node A = nodes[l], B = nodes[r];
-        f3 mn{A.bounds.min.x, A.bounds.min.y, A.bounds.min.z}, mx{A.bounds.max.x, A.bounds.max.y, A.bounds.max.z};
-        const f3 bmn{B.bounds.min.x, B.bounds.min.y, B.bounds.min.z}, bmx{B.bounds.max.x, B.bounds.max.y,
-                                                                          B.bounds.max.z};
-        mn = kmin3(mn, bmn);
-        mx = kmax3(mx, bmn);
-        mn = kmin3(mn, bmx);
-        mx = kmax3(mx, bmx);
-        counts[p] = counts[l] + counts[r];
-        costs[p] = (float)1.2 * kr_area(mn, mx) + costs[r] + costs[l];
-        nodes[p].bounds.min = kr_vec3{mn.x, mn.y, mn.z};
-        nodes[p].bounds.max = kr_vec3{mx.x, mx.y, mx.z};
-    }
-};
-
-__global__ __launch_bounds__(1024) void atr_final(kr_bvh_node* nodes, const uint32_t* parents, uint32_t* counts,
-                                                  float* costs, uint32_t nf, AtrWs ws, uint32_t phase,
-                                                  uint32_t chunk) {
-    AtrFinalUp op{nodes, counts, costs};
-    phased_up(nodes, parents, nf, ws.ph, phase, chunk, op);
+__global__ __launch_bounds__(kUpTile) void atr_final(BoundsUp op, uint32_t nf, uint32_t* visit) {
+    __shared__ UpTile<BoundsPay> L;
+    bottom_up(nf, visit, L, op);
 }
 
 // ------------------------------------------------------------- host --
@@ -861,7 +829,8 @@ kr_error atr_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, int treele
     }
     hipLaunchKernelGGL(atr_export, blocks(2 * nf - 1, 256), dim3(256), 0, stream, ws, nf, nodes, parents);
     hipLaunchKernelGGL(atr_clear, dim3(gb), dim3(256), 0, stream, ws, nf);
-    phased_launch(atr_final, nf, stream, nodes, (const uint32_t*)parents, counts, costs, nf, ws);
+    hipLaunchKernelGGL(atr_final, up_grid(nf), dim3(kUpTile), 0, stream, BoundsUp{nodes, parents, counts, costs}, nf,
+                       reinterpret_cast<uint32_t*>(ws.ph.visit));
     OBVH_HIP_TRY(hipGetLastError());
     return nullptr;
 }

@@ -1,7 +1,7 @@
 // collapse.hip -- BVH collapse on gfx950 (kr_cuda_bvh_collapse,
 // src/ads/common/cuda/transforms.cu:18-211,1061-1125).
 //
-//  collapse_mark    bottom-up (phased arrival protocol, phased.hpp): leaf
+//  collapse_mark    bottom-up in one launch (bottomup.hpp): leaf
 //                   cost ct * area; an internal node with count = counts of
 //                   its children, node_cost = ci*area + cost(left) +
 //                   cost(right), leaf_cost = ct*area*count is collapsed when
@@ -22,6 +22,7 @@
 
 #include <rocprim/device/device_scan.hpp>
 
+#include "bottomup.hpp"
 #include "collapse.hpp"
 #include "common.hpp"
 
@@ -37,46 +38,64 @@ __device__ __forceinline__ float aabb_area(const kr_aabb3& b) {
 }
 
 __global__ void collapse_clear(CollapseWs ws, uint32_t nf) {
-    phase_clear(ws.ph, nf);
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) ws.visit[i] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) *ws.error = 0;
     const uint32_t total = 2 * nf - 1;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x)
         ws.flag[i] = 0;
 }
 
+struct CollapsePay {
+    uint32_t count;
+    float cost;
+};
 struct CollapseUp {
     const kr_bvh_node* nodes;
+    const uint32_t* parents;
     kr_bvh_node* out;
     uint32_t* counts;
     float* costs;
     uint8_t* flag;
     float ci, ct;
-    __device__ void leaf(uint32_t cur) { costs[cur] = ct * aabb_area(nodes[cur].bounds); }
-    __device__ void merge(uint32_t p, uint32_t l, uint32_t r) {
-        const uint32_t count = counts[l] + counts[r];
-        counts[p] = count;
+    __device__ __forceinline__ uint2 kids(uint32_t p) const {
+        return make_uint2(nodes[p].u.children.left, nodes[p].u.children.right);
+    }
+    __device__ __forceinline__ uint32_t parent(uint32_t n) const { return parents[n]; }
+    __device__ __forceinline__ CollapsePay leaf(uint32_t n) const {
+        const float cost = ct * aabb_area(nodes[n].bounds);
+        costs[n] = cost;
+        return CollapsePay{counts[n], cost};
+    }
+    __device__ __forceinline__ CollapsePay merge(uint32_t p, uint32_t l, uint32_t r, const CollapsePay& a,
+                                                 const CollapsePay& b) const {
+        const uint32_t count = a.count + b.count;
         const float area = aabb_area(nodes[p].bounds);
-        const float node_cost = ci * area + costs[l] + costs[r];
+        const float node_cost = ci * area + a.cost + b.cost;
         const float leaf_cost = ct * area * (float)count;
-        if (leaf_cost < node_cost && count <= kMaxLeafSize) {
-            costs[p] = leaf_cost;
-            flag[p] = 1;
-            flag[l] = 1;
-            flag[r] = 1;
-            out[l].nPrimitives = kCollapsed;
-            out[r].nPrimitives = kCollapsed;
-        } else {
-            costs[p] = node_cost;
-        }
+        if (!(leaf_cost < node_cost && count <= kMaxLeafSize)) return CollapsePay{count, node_cost};
+        flag[p] = 1;
+        flag[l] = 1;
+        flag[r] = 1;
+        out[l].nPrimitives = kCollapsed;
+        out[r].nPrimitives = kCollapsed;
+        return CollapsePay{count, leaf_cost};
+    }
+    __device__ __forceinline__ void store(uint32_t n, const CollapsePay& r) const {
+        counts[n] = r.count;
+        costs[n] = r.cost;
+    }
+    __device__ __forceinline__ void publish(uint32_t n, const CollapsePay& r) const {
+        st_agent(&counts[n], r.count);
+        st_agent(&costs[n], r.cost);
+    }
+    __device__ __forceinline__ CollapsePay fetch(uint32_t n) const {
+        return CollapsePay{ld_agent(&counts[n]), ld_agent(&costs[n])};
     }
 };
 
-__global__ __launch_bounds__(1024) void collapse_mark(const kr_bvh_node* nodes, const uint32_t* parents,
-                                                      kr_bvh_node* out, uint32_t* counts, float* costs, float ci,
-                                                      float ct, uint32_t nf, CollapseWs ws, uint32_t phase,
-                                                      uint32_t chunk) {
-    CollapseUp op{nodes, out, counts, costs, ws.flag, ci, ct};
-    phased_up(nodes, parents, nf, ws.ph, phase, chunk, op);
+__global__ __launch_bounds__(kUpTile) void collapse_mark(CollapseUp op, uint32_t nf, uint32_t* visit) {
+    __shared__ UpTile<CollapsePay> L;
+    bottom_up(nf, visit, L, op);
 }
 
 __global__ void collapse_roots(const uint32_t* parents, const uint32_t* counts, CollapseWs ws, uint32_t total) {
@@ -137,7 +156,7 @@ static size_t collapse_scan_bytes(uint32_t total) {
 size_t collapse_carve(CollapseWs* ws, void* base, size_t cap, uint32_t nf) {
     Carver c{(char*)base, 0, cap};
     const size_t total = nf ? 2 * (size_t)nf - 1 : 0;
-    phase_carve(&ws->ph, c, nf);
+    ws->visit = c.take<uint32_t>(nf);
     ws->flag = c.take<uint8_t>(total);
     ws->rootcnt = c.take<uint32_t>(total);
     ws->offset = c.take<uint32_t>(total);
@@ -160,7 +179,8 @@ kr_error collapse_launch(const kr_bvh_node* nodes, const uint32_t* parents, kr_b
     uint32_t gb = (total + 255) / 256;
     if (gb > 2048) gb = 2048;
     hipLaunchKernelGGL(collapse_clear, dim3(gb), dim3(256), 0, stream, ws, nf);
-    phased_launch(collapse_mark, nf, stream, nodes, parents, out, counts, costs, ci, ct, nf, ws);
+    hipLaunchKernelGGL(collapse_mark, up_grid(nf), dim3(kUpTile), 0, stream,
+                       CollapseUp{nodes, parents, out, counts, costs, ws.flag, ci, ct}, nf, ws.visit);
     if (mark_done) OBVH_HIP_TRY(hipEventRecord(mark_done, stream));
     hipLaunchKernelGGL(collapse_roots, blocks(total, 256), dim3(256), 0, stream, parents, (const uint32_t*)counts, ws,
                        total);

@@ -3,12 +3,11 @@
 #include <hip/hip_runtime.h>
 
 #include "obvh/obvh.h"
-#include "phased.hpp"
 
 namespace obvh {
 
 struct CollapseWs {
-    PhaseWs ph;           // bottom-up pass state
+    uint32_t* visit;      // per internal node: children done (bottom-up pass)
     uint8_t* flag;        // per node: collapsed (the node or an ancestor's leaf holds it)
     uint32_t* rootcnt;    // per node: primitives if it becomes a leaf of the collapsed tree, else 0
     uint32_t* offset;     // exclusive scan of rootcnt

@@ -11,14 +11,20 @@ namespace obvh {
 
 constexpr int kWave = 64;
 
-// Agent (device) scope release/acquire.  On gfx950 these lower to an L2
-// write-back / invalidate, which makes data written by one XCD visible to
-// another; used only at set/tile completion points, never per element.
-__device__ __forceinline__ void fence_release_agent() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
-__device__ __forceinline__ void fence_acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
-__device__ __forceinline__ uint32_t atomic_add_acqrel(uint32_t* p, uint32_t v) {
-    return __hip_atomic_fetch_add(p, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+// Agent-scope relaxed accesses: they go past the XCDs' L2 caches, so what one
+// workgroup stores (and waits for, `drain`) before it counts itself done is
+// what a workgroup that saw the count loads, without writing back or
+// invalidating an L2.
+template <class T>
+__device__ __forceinline__ T ld_agent(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+template <class T>
+__device__ __forceinline__ void st_agent(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits for this wave's stores.
+__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }
 __device__ __forceinline__ int wave_id() { return (int)(threadIdx.x / kWave); }

@@ -576,20 +576,6 @@ __device__ void dito_candidate_search(const float mn[7], const float mx[7], cons
     tr.best = best_id;
 }
 
-// Agent-scope relaxed accesses: they go past the XCDs' L2 caches, so what one
-// workgroup stores (and waits for, `drain`) before it counts itself done is
-// what a workgroup that saw the count loads, without writing back or
-// invalidating an L2.
-template <class T>
-__device__ __forceinline__ T ld_agent(const T* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T>
-__device__ __forceinline__ void st_agent(T* p, T v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // One wave: the set's slab extremes (indices within the set, 14 sides) from
 // the partials of its nt tiles (first tile ft).  kAgent: the partials were
 // written by other workgroups of this launch.

@@ -16,12 +16,12 @@
 //  4. Karras radix tree, duplicate codes split by 32 + clz(i ^ j)
 //     (lbvh.cu:284-396); leaves written in sorted order.
 //  5. bottom-up bounds, primitive counts, SAH costs (ct = 1.0, ci = 1.2),
-//     lbvh.cu:399-457, with the phased workgroup-local arrival protocol
-//     described at lbvh_aabbs.
+//     lbvh.cu:399-457, in one launch (bottomup.hpp).
 #include <float.h>
 
 #include <rocprim/device/device_radix_sort.hpp>
 
+#include "bottomup.hpp"
 #include "common.hpp"
 #include "lbvh.hpp"
 
@@ -48,11 +48,6 @@ __device__ __forceinline__ Box tri_box(const kr_vec3* V, kr_uvec4 f) {
 __device__ __forceinline__ f3 box_center(Box b) {
     return f3{(b.mn.x + b.mx.x) * 0.5f, (b.mn.y + b.mx.y) * 0.5f, (b.mn.z + b.mx.z) * 0.5f};
 }
-__device__ __forceinline__ float box_area(f3 mn, f3 mx) {
-    f3 d = sub3(mx, mn);
-    return 2.0f * (d.x * d.y + d.x * d.z + d.y * d.z);
-}
-
 __global__ void lbvh_init(const kr_vec3* V, uint32_t nf, LbvhWs ws) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
@@ -64,7 +59,7 @@ __global__ void lbvh_init(const kr_vec3* V, uint32_t nf, LbvhWs ws) {
             for (int k = 0; k < 3; ++k) { ws.cbox[k] = 0x7FFFFFFF; ws.cbox[3 + k] = (int32_t)0x80000000; }
         }
     }
-    phase_clear(ws.ph, nf);
+    for (uint32_t i = t; i < nf; i += gridDim.x * blockDim.x) ws.visit[i] = 0;
 }
 
 __global__ __launch_bounds__(256) void lbvh_centroid_box(const kr_vec3* V, const kr_uvec4* F, uint32_t nf,
@@ -192,37 +187,9 @@ __global__ __launch_bounds__(256) void lbvh_tree(const kr_vec3* V, const kr_uvec
     if (t == 0) parents[0] = kInv;
 }
 
-// Bottom-up bounds / counts / costs (lbvh.cu:399-457) with the phased
-// arrival protocol of phased.hpp.
-struct LbvhUp {
-    kr_bvh_node* nodes;
-    uint32_t* counts;
-    float* costs;
-    __device__ void leaf(uint32_t cur) {
-        const kr_bvh_node L = nodes[cur];
-        costs[cur] = 1.0f * box_area(f3{L.bounds.min.x, L.bounds.min.y, L.bounds.min.z},
-                                     f3{L.bounds.max.x, L.bounds.max.y, L.bounds.max.z});
-        counts[cur] = 1;
-    }
-    __device__ void merge(uint32_t p, uint32_t l, uint32_t r) {
-        const float ci = (float)1.2;
-        const kr_bvh_node A = nodes[l], B = nodes[r];
-        Box bn{f3{A.bounds.min.x, A.bounds.min.y, A.bounds.min.z},
-               f3{A.bounds.max.x, A.bounds.max.y, A.bounds.max.z}};
-        bn = expand3(bn, f3{B.bounds.min.x, B.bounds.min.y, B.bounds.min.z});  // kr_aabb_expand
-        bn = expand3(bn, f3{B.bounds.max.x, B.bounds.max.y, B.bounds.max.z});
-        counts[p] = counts[l] + counts[r];
-        costs[p] = ci * box_area(bn.mn, bn.mx) + costs[r] + costs[l];
-        nodes[p].bounds.min = kr_vec3{bn.mn.x, bn.mn.y, bn.mn.z};
-        nodes[p].bounds.max = kr_vec3{bn.mx.x, bn.mx.y, bn.mx.z};
-    }
-};
-
-__global__ __launch_bounds__(1024) void lbvh_aabbs(kr_bvh_node* nodes, const uint32_t* parents, uint32_t* counts,
-                                                   float* costs, uint32_t nf, LbvhWs ws, uint32_t phase,
-                                                   uint32_t chunk) {
-    LbvhUp op{nodes, counts, costs};
-    phased_up(nodes, parents, nf, ws.ph, phase, chunk, op);
+__global__ __launch_bounds__(kUpTile) void lbvh_aabbs(BoundsUp op, uint32_t nf, uint32_t* visit) {
+    __shared__ UpTile<BoundsPay> L;
+    bottom_up(nf, visit, L, op);
 }
 
 size_t lbvh_sort_bytes(uint32_t nf) {
@@ -235,7 +202,7 @@ size_t lbvh_sort_bytes(uint32_t nf) {
 size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf) {
     Carver c{(char*)base, 0, cap};
     ws->cbox = c.take<int32_t>(8);
-    phase_carve(&ws->ph, c, nf);
+    ws->visit = c.take<uint32_t>(nf);
     ws->keys_in = c.take<uint32_t>(nf);
     ws->keys_out = c.take<uint32_t>(nf);
     ws->vals_in = c.take<uint32_t>(nf);
@@ -262,7 +229,8 @@ kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_no
     OBVH_HIP_TRY(rocprim::radix_sort_pairs(ws.sort_tmp, sb, ws.keys_in, ws.keys_out, ws.vals_in, ws.vals_out, nf,
                                            0, 30, stream));
     hipLaunchKernelGGL(lbvh_tree, blocks(nf, 256), dim3(256), 0, stream, V, F, nf, ws, nodes, parents, mortons);
-    phased_launch(lbvh_aabbs, nf, stream, nodes, (const uint32_t*)parents, counts, costs, nf, ws);
+    hipLaunchKernelGGL(lbvh_aabbs, up_grid(nf), dim3(kUpTile), 0, stream, BoundsUp{nodes, parents, counts, costs}, nf,
+                       ws.visit);
     OBVH_HIP_TRY(hipGetLastError());
     return nullptr;
 }

@@ -3,13 +3,12 @@
 #include <hip/hip_runtime.h>
 
 #include "obvh/obvh.h"
-#include "phased.hpp"
 
 namespace obvh {
 
 struct LbvhWs {
     int32_t* cbox;       // centroid box as order-preserving keys (min xyz, max xyz)
-    PhaseWs ph;          // bottom-up pass state
+    uint32_t* visit;     // per internal node: children done (bottom-up pass)
     uint32_t* keys_in;   // Morton codes by face
     uint32_t* keys_out;  // sorted codes
     uint32_t* vals_in;   // face ids

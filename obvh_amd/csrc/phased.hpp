@@ -1,10 +1,8 @@
-// phased.hpp -- bottom-up tree passes with the phased arrival protocol.
+// phased.hpp -- state of the phased bottom-up protocol (the ATRBVH optimiser).
 //
-// A pass visits every internal node after both of its children, computing
-// the node from its children (bounds, counts, costs, collapse flags ...).
-// Phase k runs workgroups that own leaf positions [w*chunk_k, (w+1)*chunk_k)
-// (chunks 512, 16384, then one workgroup for everything).  Phase 0 starts
-// one lane per leaf; later phases start from the nodes the previous phase
+// A pass visits every internal node after both of its children.  Phase k runs
+// workgroups that own leaf positions [w*chunk_k, (w+1)*chunk_k), the last
+// phase one workgroup for everything.  Phase 0 starts one lane per leaf; later phases start from the nodes the previous phase
 // deferred.  Each deferred node is listed with a key, a leaf position of its
 // subtree known to the lane that deferred it, and is taken by the workgroup
 // whose chunk holds the key; that workgroup runs it when the node's whole
@@ -27,20 +25,18 @@
 
 namespace obvh {
 
-constexpr int kPhases = 3;  // chunk 512, chunk 16384, everything
+constexpr int kPhases = 3;  // phases that defer, at most
 
 struct PhaseWs {
     uint64_t* visit;   // per internal node: arrivals (low word) + sum of tags (high word)
     uint32_t* nlist;   // per phase: number of deferred nodes
     uint2* list;       // per phase: deferred nodes and their keys (I + 1 entries each)
-    uint2* span;       // per node: first and last leaf position below it
 };
 
 inline void phase_carve(PhaseWs* ws, Carver& c, uint32_t nf) {
     ws->visit = c.take<uint64_t>((size_t)nf + 1);
     ws->nlist = c.take<uint32_t>(4);
     ws->list = c.take<uint2>((size_t)kPhases * ((size_t)nf + 1));
-    ws->span = c.take<uint2>(2 * (size_t)nf);
 }
 
 // Zero the arrival words and the deferred-list counters (grid-stride).
@@ -49,86 +45,6 @@ __device__ __forceinline__ void phase_clear(const PhaseWs& ws, uint32_t nf) {
     if (t == 0)
         for (int k = 0; k < 4; ++k) ws.nlist[k] = 0;
     for (uint32_t i = t; i < nf; i += gridDim.x * blockDim.x) ws.visit[i] = 0;
-}
-
-// Body of one phase.  Op provides
-//   void leaf(uint32_t node)                       a leaf (phase 0 only)
-//   void merge(uint32_t p, uint32_t l, uint32_t r) an internal node from its children
-template <class Op>
-__device__ __forceinline__ void phased_up(const kr_bvh_node* nodes, const uint32_t* parents, uint32_t nf,
-                                          const PhaseWs& ws, uint32_t phase, uint32_t chunk, Op& op) {
-    constexpr uint32_t kNone = 0xFFFFFFFFu;
-    const uint32_t I = nf - 1;
-    const uint32_t tag = (phase << 24) | (blockIdx.x + 1u);
-    const uint64_t lo = (uint64_t)blockIdx.x * chunk, hi = lo + chunk;
-    const uint32_t nin = phase == 0 ? 0 : min(ws.nlist[phase - 1], I);
-    const uint2* in = phase == 0 ? nullptr : ws.list + (size_t)(phase - 1) * (I + 1);
-    uint2* out = ws.list + (size_t)phase * (I + 1);
-    const uint32_t nstart = phase == 0 ? chunk : nin;
-    for (uint32_t r0 = threadIdx.x; r0 < nstart; r0 += blockDim.x) {
-        uint32_t cur;
-        uint2 span;
-        if (phase == 0) {
-            const uint64_t pos = lo + r0;
-            if (pos >= nf) break;
-            cur = I + (uint32_t)pos;
-            op.leaf(cur);
-            span = make_uint2((uint32_t)pos, (uint32_t)pos);
-        } else {
-            const uint2 e = in[r0];
-            cur = e.x;
-            if (cur >= I || e.y < lo || e.y >= hi) continue;  // another workgroup owns it
-            const uint32_t l = nodes[cur].u.children.left, r = nodes[cur].u.children.right;
-            const uint2 sa = ws.span[l], sb = ws.span[r];
-            span = make_uint2(min(sa.x, sb.x), max(sa.y, sb.y));
-            if (span.x < lo || span.y >= hi) {  // wider than this workgroup: next phase
-                const uint32_t slot = atomicAdd(&ws.nlist[phase], 1u);
-                if (slot < I) out[slot] = make_uint2(cur, span.x);
-                continue;
-            }
-            op.merge(cur, l, r);
-        }
-        ws.span[cur] = span;
-        uint32_t p = parents[cur];
-        for (uint32_t step = 0; p != kNone && p < I && step < nf; ++step) {
-            const uint32_t l = nodes[p].u.children.left, r = nodes[p].u.children.right;
-            const uint32_t pp = parents[p];
-            const uint64_t old = __hip_atomic_fetch_add(&ws.visit[p], ((uint64_t)tag << 32) | 1ull,
-                                                        __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if ((uint32_t)old == 0) break;  // first arrival: the sibling continues
-            const uint32_t t1 = (uint32_t)(old >> 32);
-            if (t1 != tag && (t1 >> 24) >= phase) {  // sibling done by another workgroup of this phase
-                const uint32_t slot = atomicAdd(&ws.nlist[phase], 1u);
-                if (slot < I) out[slot] = make_uint2(p, span.x);
-                break;
-            }
-            const uint32_t sib = (l == cur) ? r : l;
-            op.merge(p, l, r);
-            const uint2 so = ws.span[sib];
-            span = make_uint2(min(span.x, so.x), max(span.y, so.y));
-            ws.span[p] = span;
-            cur = p;
-            p = pp;
-        }
-    }
-}
-
-// Launch the phases of a pass: kernel(args..., phase, chunk), one lane per
-// leaf in phase 0 (512 threads), 1024 threads in the later phases and in a
-// single-phase pass (whole waves always, as the treelet tournaments read all
-// 64 lanes).  512-leaf chunks build the 2M-triangle ATRBVH in 14.5 ms against
-// 15.5 ms with 1024-leaf chunks; LBVH and collapse time is the same.
-template <class K, class... A>
-inline void phased_launch(K kernel, uint32_t nf, hipStream_t stream, A... args) {
-    uint32_t phase = 0;
-    for (uint32_t chunk : {512u, 16384u, 0u}) {
-        const bool last = (chunk == 0) || chunk >= nf;
-        const uint32_t c = last ? nf : chunk;
-        const uint32_t threads = last ? 1024u : (chunk < 1024u ? chunk : 1024u);
-        hipLaunchKernelGGL(kernel, dim3((nf + c - 1) / c), dim3(threads), 0, stream, args..., phase, c);
-        ++phase;
-        if (last) break;
-    }
 }
 
 }  // namespace obvh

@@ -80,3 +80,38 @@ def test_legacy_collapse_equals_async(torch):
     assert m["collapse_mark_time"] > 0 and m["collapse_time"] > 0
     assert torch.equal(out, r["collapsed"]) and torch.equal(cnt, r["counts"])
     assert torch.equal(costs, r["costs"]) and torch.equal(prims, r["primitives"])
+
+
+# edges of the bottom-up pass's tiles (512 leaves), of one tile and several; `random`: node indices in any order, so
+# that nearly every arrival goes through global memory
+@pytest.mark.parametrize("nf,kind", [(1, "soup"), (2, "soup"), (511, "soup"), (512, "soup"), (513, "soup"),
+                                     (1025, "soup"), (4096, "same"), (7001, "soup"), (513, "random"),
+                                     (3000, "random")])
+def test_bottom_up_edges(torch, oracle_lib, nf, kind):
+    say(f"[bottom-up] {nf} triangles {kind}")
+    rng = np.random.default_rng(nf)
+    c = np.zeros((nf, 1, 3)) if kind == "same" else rng.uniform(-1, 1, (nf, 1, 3))
+    V = (c + rng.uniform(-0.05, 0.05, (nf, 3, 3))).reshape(-1, 3).astype(np.float32)
+    F = np.zeros((nf, 4), dtype=np.uint32)
+    F[:, :3] = np.arange(3 * nf).reshape(nf, 3)
+    if kind == "random":
+        nodes, parents = random_tree(nf, seed=nf)
+        nodes = fill_bounds(nodes, V, F)
+        counts = np.zeros(2 * nf - 1, dtype=np.uint32)
+        counts[nf - 1:] = 1
+    else:
+        t = ops.lbvh_build(torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda())
+        torch.cuda.synchronize()
+        nodes, parents, counts, costs, _ = oracle_lib.lbvh_build(V, F)
+        assert np.array_equal(t["parents"].cpu().numpy().view(np.uint32), parents)
+        assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), nodes.view(np.uint8))
+        assert np.array_equal(t["counts"].cpu().numpy().view(np.uint32), counts)
+        assert np.array_equal(t["costs"].cpu().numpy(), costs)
+    r = ops.collapse(torch.from_numpy(nodes.view(np.uint8)).cuda().reshape(-1),
+                     torch.from_numpy(parents.view(np.int32)).cuda(), torch.from_numpy(counts.view(np.int32)).cuda(),
+                     CI, CT)
+    torch.cuda.synchronize()
+    e = oracle_lib.collapse(nodes, parents, counts, CI, CT)
+    assert np.array_equal(r["collapsed"].cpu().numpy(), e["collapsed"].view(np.uint8).reshape(-1))
+    assert np.array_equal(r["counts"].cpu().numpy().view(np.uint32), e["counts"])
+    assert np.array_equal(r["costs"].cpu().numpy(), e["costs"])
