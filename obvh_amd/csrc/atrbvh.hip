@@ -82,7 +82,9 @@ __global__ void atr_init(AtrWs ws, uint32_t nf) {
     if (blockIdx.x == 0 && threadIdx.x < 6) ws.sbox[threadIdx.x] = threadIdx.x < 3 ? 0x7FFFFFFF : (int32_t)0x80000000;
 }
 
-__global__ __launch_bounds__(256) void atr_scene(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, AtrWs ws) {
+constexpr int kBoxThreads = 1024;
+
+__global__ __launch_bounds__(kBoxThreads) void atr_scene(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, AtrWs ws) {
     int32_t mn[3] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF}, mx[3] = {(int32_t)0x80000000, (int32_t)0x80000000,
                                                                    (int32_t)0x80000000};
     for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(256) void atr_scene(const kr_vec3* V, const kr_uvec
     }
     // wave, then workgroup reduction; one filtered atomic per key and
     // workgroup (a few thousand same-address atomics would serialise)
-    __shared__ int32_t part[256 / kWave][6];
+    __shared__ int32_t part[kBoxThreads / kWave][6];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         mn[a] = wave_min_i32(mn[a]);
@@ -118,7 +120,7 @@ __global__ __launch_bounds__(256) void atr_scene(const kr_vec3* V, const kr_uvec
     if (threadIdx.x < 6) {
         const int a = threadIdx.x;
         int32_t v = part[0][a];
-        for (int w = 1; w < 256 / kWave; ++w) v = a < 3 ? min(v, part[w][a]) : max(v, part[w][a]);
+        for (int w = 1; w < kBoxThreads / kWave; ++w) v = a < 3 ? min(v, part[w][a]) : max(v, part[w][a]);
         const int32_t cur = __hip_atomic_load(&ws.sbox[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a < 3 ? v < cur : v > cur) {
             if (a < 3) atomicMin(&ws.sbox[a], v);
@@ -145,13 +147,25 @@ __global__ void atr_codes(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, AtrW
     ws.vals_in[f] = f;
 }
 
-// longestCommonPrefix (LBVH.cu:173-187)
-__device__ __forceinline__ int lcp64(const uint64_t* k, int n, int i, int j, uint64_t ki) {
-    if (j < 0 || j >= n) return -1;
-    const uint64_t kj = k[j];
-    if (ki == kj) return 64 + __clz(i ^ j);
-    return __clzll((long long)(ki ^ kj));
-}
+// longestCommonPrefix (LBVH.cu:173-187), the sorted codes around a
+// workgroup's nodes in LDS (most nodes span a few leaves).
+constexpr int kTreeThreads = 256;
+constexpr int kWindow = 3 * kTreeThreads;  // from kTreeThreads before the first node on
+struct Codes64 {
+    const uint64_t* k;
+    const uint64_t* window;
+    int first, n;  // first: index of window[0]
+    __device__ __forceinline__ uint64_t at(int j) const {
+        const uint32_t w = (uint32_t)(j - first);
+        return w < (uint32_t)kWindow ? window[w] : k[j];
+    }
+    __device__ __forceinline__ int lcp(int i, int j, uint64_t ki) const {
+        if (j < 0 || j >= n) return -1;
+        const uint64_t kj = at(j);
+        if (ki == kj) return 64 + __clz(i ^ j);
+        return __clzll((long long)(ki ^ kj));
+    }
+};
 
 // Working record of a node, four float4 (64 B, half a cache line, so that one
 // trip to memory brings everything a treelet reads of a node):
@@ -175,10 +189,18 @@ struct AtrRec {
     }
 };
 
-__global__ __launch_bounds__(256) void atr_tree(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, float ct, AtrWs ws) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(kTreeThreads) void atr_tree(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, float ct,
+                                                         AtrWs ws) {
+    __shared__ uint64_t window[kWindow];
+    const int i = (int)(blockIdx.x * kTreeThreads + threadIdx.x);
     const int n = (int)nf;
     const uint32_t I = nf - 1;
+    const int first = (int)(blockIdx.x * kTreeThreads) - kTreeThreads;
+    for (int w = (int)threadIdx.x; w < kWindow; w += kTreeThreads) {
+        const int j = first + w;
+        window[w] = j >= 0 && j < n ? ws.keys_out[j] : 0ull;
+    }
+    __syncthreads();
     if (i >= n) return;
     {  // leaf i in code order
         const uint32_t face = ws.vals_out[i];
@@ -194,23 +216,23 @@ __global__ __launch_bounds__(256) void atr_tree(const kr_vec3* V, const kr_uvec4
     }
     if (i == 0) AtrRec(ws, 0u).set_parent(kNoNode);  // the root (or the only leaf)
     if (i >= n - 1) return;
-    const uint64_t* k = ws.keys_out;
-    const uint64_t ki = k[i];
-    const int l1 = lcp64(k, n, i, i + 1, ki), l2 = lcp64(k, n, i, i - 1, ki);
+    const Codes64 k{ws.keys_out, window, first, n};
+    const uint64_t ki = window[kTreeThreads + threadIdx.x];
+    const int l1 = k.lcp(i, i + 1, ki), l2 = k.lcp(i, i - 1, ki);
     const int dir = (0 < l1 - l2) - (l1 - l2 < 0);
-    const int min_lcp = lcp64(k, n, i, i - dir, ki);
+    const int min_lcp = k.lcp(i, i - dir, ki);
     int lmax = 2;
-    while (lcp64(k, n, i, i + lmax * dir, ki) > min_lcp) lmax <<= 1;
+    while (k.lcp(i, i + lmax * dir, ki) > min_lcp) lmax <<= 1;
     int l = 0;
     for (int t = lmax >> 1; t >= 1; t >>= 1)
-        if (lcp64(k, n, i, i + (l + t) * dir, ki) > min_lcp) l += t;
+        if (k.lcp(i, i + (l + t) * dir, ki) > min_lcp) l += t;
     const int j = i + l * dir;
-    const int node_lcp = lcp64(k, n, i, j, ki);
+    const int node_lcp = k.lcp(i, j, ki);
     int s = 0, divisor = 2;
     const int max_div = 1 << (32 - __clz(l));
     while (divisor <= max_div) {
         const int t = (l + divisor - 1) / divisor;
-        if (lcp64(k, n, i, i + (s + t) * dir, ki) > node_lcp) s += t;
+        if (k.lcp(i, i + (s + t) * dir, ki) > node_lcp) s += t;
         divisor <<= 1;
     }
     const int split = i + s * dir + min(dir, 0);
@@ -797,12 +819,13 @@ kr_error atr_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, int treele
     uint32_t gb = (nf + 255) / 256;
     if (gb > 2048) gb = 2048;
     hipLaunchKernelGGL(atr_init, dim3(gb), dim3(256), 0, stream, ws, nf);
-    hipLaunchKernelGGL(atr_scene, dim3(gb), dim3(256), 0, stream, V, F, nf, ws);
+    hipLaunchKernelGGL(atr_scene, dim3(min((nf + kBoxThreads - 1) / kBoxThreads, 256u)), dim3(kBoxThreads), 0, stream, V, F,
+                       nf, ws);
     hipLaunchKernelGGL(atr_codes, blocks(nf, 256), dim3(256), 0, stream, V, F, nf, ws);
     size_t sb = ws.sort_bytes;
     OBVH_HIP_TRY(rocprim::radix_sort_pairs(ws.sort_tmp, sb, ws.keys_in, ws.keys_out, ws.vals_in, ws.vals_out, nf, 0,
                                            63, stream));
-    hipLaunchKernelGGL(atr_tree, blocks(nf, 256), dim3(256), 0, stream, V, F, nf, ct, ws);
+    hipLaunchKernelGGL(atr_tree, blocks(nf, kTreeThreads), dim3(kTreeThreads), 0, stream, V, F, nf, ct, ws);
     int gamma = treelet_size;
     for (int it = 0; it < iterations && nf > 1; ++it) {
         if (it > 0) hipLaunchKernelGGL(atr_clear, dim3(gb), dim3(256), 0, stream, ws, nf);

@@ -11,7 +11,7 @@
 //     order-preserving float keys.
 //  2. 30-bit Morton code of the offset triangle-box centre, safe divide by
 //     the centroid extent (lbvh.cu:252-282, vecmath.h:698-716,760).
-//  3. stable LSD radix sort of (code, face) pairs over 30 bits (rocPRIM),
+//  3. stable LSD radix sort of (code, face) pairs over 30 bits (radix.hpp),
 //     the equivalent of thrust::stable_sort_by_key (lbvh.cu:1670).
 //  4. Karras radix tree, duplicate codes split by 32 + clz(i ^ j)
 //     (lbvh.cu:284-396); leaves written in sorted order.
@@ -60,11 +60,14 @@ __global__ void lbvh_init(const kr_vec3* V, uint32_t nf, LbvhWs ws) {
         }
     }
     for (uint32_t i = t; i < nf; i += gridDim.x * blockDim.x) ws.visit[i] = 0;
+    for (uint32_t i = t; i < ws.radix.words; i += gridDim.x * blockDim.x) ws.radix.hist[i] = 0;
 }
 
-__global__ __launch_bounds__(256) void lbvh_centroid_box(const kr_vec3* V, const kr_uvec4* F, uint32_t nf,
+constexpr int kBoxThreads = 1024;
+
+__global__ __launch_bounds__(kBoxThreads) void lbvh_centroid_box(const kr_vec3* V, const kr_uvec4* F, uint32_t nf,
                                                          LbvhWs ws) {
-    __shared__ float sh[6][4];
+    __shared__ float sh[6][kBoxThreads / kWave];
     const float INF = FLT_MAX * 2.0f;
     float mn[3] = {INF, INF, INF}, mx[3] = {-INF, -INF, -INF};
     for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
@@ -79,10 +82,11 @@ __global__ __launch_bounds__(256) void lbvh_centroid_box(const kr_vec3* V, const
     if (threadIdx.x < 6) {
         const int k = threadIdx.x;
         float a = sh[k][0];
-        for (int w = 1; w < 4; ++w) a = k < 3 ? fminf(a, sh[k][w]) : fmaxf(a, sh[k][w]);
+        for (int w = 1; w < kBoxThreads / kWave; ++w) a = k < 3 ? fminf(a, sh[k][w]) : fmaxf(a, sh[k][w]);
         if (a == a && a != INF && a != -INF) {
             // filtered: only a workgroup that improves the current bound
-            // issues the atomic (thousands of same-address atomics serialise)
+            // issues the atomic (thousands of same-address atomics serialise:
+            // 2048 workgroups took 27 us, 256 take 10)
             const int32_t key = f2ord(a);
             const int32_t cur = __hip_atomic_load(&ws.cbox[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (k < 3 ? key < cur : key > cur) {
@@ -104,42 +108,118 @@ __device__ __forceinline__ uint32_t stretch3(uint32_t x) {
 __device__ __forceinline__ uint32_t quant10(float v) { return (uint32_t)kmin(kmax(v * 1024.0f, 0.0f), 1023.0f); }
 __device__ __forceinline__ float safe_div(float a, float b) { return (b != 0.0f) ? a / b : 0.0f; }
 
-__global__ __launch_bounds__(256) void lbvh_codes(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, LbvhWs ws) {
-    const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nf) return;
+constexpr int kPasses = 4;  // 8-bit digits of a 30-bit code
+
+// Morton codes, and how often each digit value occurs for the sort (one set
+// of global atomics per workgroup, hence at most 256 of them).
+__global__ __launch_bounds__(1024) void lbvh_codes(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, LbvhWs ws) {
+    __shared__ uint32_t h[kPasses * kRadixBins];
+    for (uint32_t i = threadIdx.x; i < kPasses * kRadixBins; i += blockDim.x) h[i] = 0;
+    __syncthreads();
     const f3 cmn = f3{ord2f(ws.cbox[0]), ord2f(ws.cbox[1]), ord2f(ws.cbox[2])};
     const f3 cmx = f3{ord2f(ws.cbox[3]), ord2f(ws.cbox[4]), ord2f(ws.cbox[5])};
-    Box b = tri_box(V, F[f]);
     const f3 neg = f3{-cmn.x, -cmn.y, -cmn.z};
-    Box o{add3(b.mn, neg), add3(b.mx, neg)};  // kr_aabb_offset3(bbox, -cell.min)
-    f3 c = box_center(o);
     const f3 ext = sub3(cmx, cmn);
-    c = f3{safe_div(c.x, ext.x), safe_div(c.y, ext.y), safe_div(c.z, ext.z)};
-    ws.keys_in[f] = stretch3(quant10(c.x)) << 2 | stretch3(quant10(c.y)) << 1 | stretch3(quant10(c.z));
-    ws.vals_in[f] = f;
+    for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
+        Box b = tri_box(V, F[f]);
+        Box o{add3(b.mn, neg), add3(b.mx, neg)};  // kr_aabb_offset3(bbox, -cell.min)
+        f3 c = box_center(o);
+        c = f3{safe_div(c.x, ext.x), safe_div(c.y, ext.y), safe_div(c.z, ext.z)};
+        const uint32_t key = stretch3(quant10(c.x)) << 2 | stretch3(quant10(c.y)) << 1 | stretch3(quant10(c.z));
+        ws.keys[f] = key;
+        radix_count<kPasses>(key, h);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kPasses * kRadixBins; i += blockDim.x)
+        if (h[i]) atomicAdd(&ws.radix.hist[i], h[i]);
 }
 
-__device__ __forceinline__ int delta(const uint32_t* c, int i, int j, int n) {
-    if (j > n - 1 || j < 0) return -1;
-    uint32_t a = c[i], b = c[j];
-    if (a == b) return 32 + __clz((uint32_t)i ^ (uint32_t)j);
-    return __clz(a ^ b);
+__global__ __launch_bounds__(256) void lbvh_iota(uint32_t* vals, uint32_t nf) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) vals[i] = i;
 }
+
+// The sorted codes around a workgroup's nodes in LDS (most nodes span a few
+// leaves, so nearly every probe of their searches lands there).
+constexpr int kTreeThreads = 256;
+constexpr int kWindow = 3 * kTreeThreads;  // from kTreeThreads before the first node on
+struct Codes {
+    const uint32_t* c;
+    const uint32_t* window;
+    int first, n;  // first: index of window[0]
+    __device__ __forceinline__ uint32_t at(int j) const {
+        const uint32_t w = (uint32_t)(j - first);
+        return w < (uint32_t)kWindow ? window[w] : c[j];
+    }
+    __device__ __forceinline__ int delta(int i, int j) const {
+        if (j > n - 1 || j < 0) return -1;
+        const uint32_t a = at(i), b = at(j);
+        if (a == b) return 32 + __clz((uint32_t)i ^ (uint32_t)j);
+        return __clz(a ^ b);
+    }
+};
 __device__ __forceinline__ int lid(int num) {
     if (num == 1) return 0;
     if (num % 2 == 1) return num / 2 + 1;
     return num / 2;
 }
 
-__global__ __launch_bounds__(256) void lbvh_tree(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, LbvhWs ws,
-                                                 kr_bvh_node* nodes, uint32_t* parents, uint32_t* mortons) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+// Children and parents of the radix tree (Karras).  The nodes' bounds and the
+// leaves follow in lbvh_aabbs.
+__global__ __launch_bounds__(kTreeThreads) void lbvh_tree(uint32_t nf, LbvhWs ws, kr_bvh_node* nodes,
+                                                          uint32_t* parents, uint32_t* mortons) {
+    __shared__ uint32_t window[kWindow];
+    const uint32_t t = blockIdx.x * kTreeThreads + threadIdx.x;
+    const int n = (int)nf, i = (int)t;
+    const int first = (int)(blockIdx.x * kTreeThreads) - kTreeThreads;
+    for (int w = (int)threadIdx.x; w < kWindow; w += kTreeThreads) {
+        const int j = first + w;
+        window[w] = j >= 0 && j < n ? ws.keys[j] : 0u;
+    }
+    __syncthreads();
     if (t >= nf) return;
     const uint32_t I = nf - 1;
-    // leaf t (sorted order)
-    {
-        const uint32_t prim = ws.vals_out[t];
-        Box b = tri_box(V, F[prim]);
+    if (mortons) mortons[t] = window[kTreeThreads + threadIdx.x];
+    if (t == 0) parents[0] = kInv;
+    if (t >= I) return;
+    const Codes c{ws.keys, window, first, n};
+    const int da = c.delta(i, i + 1), db = c.delta(i, i - 1);
+    const int d = (da - db > 0) - (da - db < 0);
+    const int dmin = c.delta(i, i - d);
+    int lmax = 2;
+    while (c.delta(i, i + lmax * d) > dmin) lmax *= 2;
+    int l = 0;
+    for (int s = lmax / 2; s >= 1; s /= 2)
+        if (c.delta(i, i + (l + s) * d) > dmin) l += s;
+    const int j = i + l * d;
+    const int dnode = c.delta(i, j);
+    int s = 0;
+    for (int q = lid(l); q >= 1; q = lid(q))
+        if (c.delta(i, i + (s + q) * d) > dnode) s += q;
+    const int split = i + s * d + (d < 0 ? d : 0);
+    const bool lleaf = ((i < j ? i : j) == split);
+    const bool rleaf = ((i > j ? i : j) == split + 1);
+    const uint32_t li = (uint32_t)split + (lleaf ? I : 0);
+    const uint32_t ri = (uint32_t)split + 1 + (rleaf ? I : 0);
+    parents[li] = t;
+    parents[ri] = t;
+    kr_bvh_node& N = nodes[t];
+    N.u.children.left = li;
+    N.u.children.right = ri;
+    N.nPrimitives = 0;
+    N.axis = 0;
+    N.pad_ = 0;
+}
+
+// The bottom-up pass over the bounds; a leaf's come from its triangle, and its
+// node is written here.
+struct LbvhUp : BoundsUp {
+    const kr_vec3* V;
+    const kr_uvec4* F;
+    const uint32_t* vals;
+    uint32_t I;
+    __device__ __forceinline__ BoundsPay leaf(uint32_t n) const {
+        const uint32_t prim = vals[n - I];
+        const Box b = tri_box(V, F[prim]);
         kr_bvh_node L;
         L.bounds.min = kr_vec3{b.mn.x, b.mn.y, b.mn.z};
         L.bounds.max = kr_vec3{b.mx.x, b.mx.y, b.mx.z};
@@ -148,46 +228,16 @@ __global__ __launch_bounds__(256) void lbvh_tree(const kr_vec3* V, const kr_uvec
         L.nPrimitives = 1;
         L.axis = 0;
         L.pad_ = 0;
-        nodes[I + t] = L;
-        if (mortons) mortons[t] = ws.keys_out[t];
+        nodes[n] = L;
+        BoundsPay r{b.mn, b.mx, 1u, 0.0f};
+        r.cost = 1.0f * area(r.mn, r.mx);
+        counts[n] = 1u;
+        costs[n] = r.cost;
+        return r;
     }
-    if (nf == 1) { parents[0] = kInv; return; }
-    if (t >= I) return;
-    const uint32_t* c = ws.keys_out;
-    const int n = (int)nf, i = (int)t;
-    const int da = delta(c, i, i + 1, n), db = delta(c, i, i - 1, n);
-    const int d = (da - db > 0) - (da - db < 0);
-    const int dmin = delta(c, i, i - d, n);
-    int lmax = 2;
-    while (delta(c, i, i + lmax * d, n) > dmin) lmax *= 2;
-    int l = 0;
-    for (int s = lmax / 2; s >= 1; s /= 2)
-        if (delta(c, i, i + (l + s) * d, n) > dmin) l += s;
-    const int j = i + l * d;
-    const int dnode = delta(c, i, j, n);
-    int s = 0;
-    for (int q = lid(l); q >= 1; q = lid(q))
-        if (delta(c, i, i + (s + q) * d, n) > dnode) s += q;
-    const int split = i + s * d + (d < 0 ? d : 0);
-    const bool lleaf = ((i < j ? i : j) == split);
-    const bool rleaf = ((i > j ? i : j) == split + 1);
-    const uint32_t li = (uint32_t)split + (lleaf ? I : 0);
-    const uint32_t ri = (uint32_t)split + 1 + (rleaf ? I : 0);
-    parents[li] = t;
-    parents[ri] = t;
-    kr_bvh_node N;
-    N.bounds.min = kr_vec3{FLT_MAX, FLT_MAX, FLT_MAX};
-    N.bounds.max = kr_vec3{-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    N.u.children.left = li;
-    N.u.children.right = ri;
-    N.nPrimitives = 0;
-    N.axis = 0;
-    N.pad_ = 0;
-    nodes[t] = N;
-    if (t == 0) parents[0] = kInv;
-}
+};
 
-__global__ __launch_bounds__(kUpTile) void lbvh_aabbs(BoundsUp op, uint32_t nf, uint32_t* visit) {
+__global__ __launch_bounds__(kUpTile) void lbvh_aabbs(LbvhUp op, uint32_t nf, uint32_t* visit) {
     __shared__ UpTile<BoundsPay> L;
     bottom_up(nf, visit, L, op);
 }
@@ -203,12 +253,21 @@ size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf) {
     Carver c{(char*)base, 0, cap};
     ws->cbox = c.take<int32_t>(8);
     ws->visit = c.take<uint32_t>(nf);
-    ws->keys_in = c.take<uint32_t>(nf);
-    ws->keys_out = c.take<uint32_t>(nf);
-    ws->vals_in = c.take<uint32_t>(nf);
-    ws->vals_out = c.take<uint32_t>(nf);
-    ws->sort_bytes = lbvh_sort_bytes(nf);
-    ws->sort_tmp = c.take<char>(ws->sort_bytes);
+    ws->keys = c.take<uint32_t>(nf);
+    ws->vals = c.take<uint32_t>(nf);
+    ws->keys_tmp = c.take<uint32_t>(nf);
+    ws->vals_tmp = c.take<uint32_t>(nf);
+    ws->radix = RadixWs{};
+    ws->sort_bytes = 0;
+    ws->sort_tmp = nullptr;
+    if (nf <= kRadixMax) {
+        radix_carve(&ws->radix, c, nf, kPasses);
+    } else {
+        ws->sort_bytes = lbvh_sort_bytes(nf);
+        ws->sort_tmp = c.take<char>(ws->sort_bytes);
+        ws->radix.hist = c.take<uint32_t>(kPasses * kRadixBins);
+        ws->radix.words = kPasses * kRadixBins;
+    }
     return c.used;
 }
 
@@ -223,14 +282,22 @@ kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_no
     uint32_t gb = (nf + 255) / 256;
     if (gb > 2048) gb = 2048;
     hipLaunchKernelGGL(lbvh_init, dim3(gb), dim3(256), 0, stream, V, nf, ws);
-    hipLaunchKernelGGL(lbvh_centroid_box, dim3(gb), dim3(256), 0, stream, V, F, nf, ws);
-    hipLaunchKernelGGL(lbvh_codes, blocks(nf, 256), dim3(256), 0, stream, V, F, nf, ws);
-    size_t sb = ws.sort_bytes;
-    OBVH_HIP_TRY(rocprim::radix_sort_pairs(ws.sort_tmp, sb, ws.keys_in, ws.keys_out, ws.vals_in, ws.vals_out, nf,
-                                           0, 30, stream));
-    hipLaunchKernelGGL(lbvh_tree, blocks(nf, 256), dim3(256), 0, stream, V, F, nf, ws, nodes, parents, mortons);
-    hipLaunchKernelGGL(lbvh_aabbs, up_grid(nf), dim3(kUpTile), 0, stream, BoundsUp{nodes, parents, counts, costs}, nf,
-                       ws.visit);
+    hipLaunchKernelGGL(lbvh_centroid_box, dim3(min((nf + kBoxThreads - 1) / kBoxThreads, 256u)), dim3(kBoxThreads), 0,
+                       stream, V, F, nf, ws);
+    hipLaunchKernelGGL(lbvh_codes, dim3(min((nf + 1023) / 1024, 256u)), dim3(1024), 0, stream, V, F, nf, ws);
+    if (nf <= kRadixMax) {
+        radix_sort<kPasses>(ws.keys, ws.vals, ws.keys_tmp, ws.vals_tmp, nf, ws.radix, stream);
+    } else {  // rocPRIM; its buffers swap roles
+        hipLaunchKernelGGL(lbvh_iota, dim3(gb), dim3(256), 0, stream, ws.vals_tmp, nf);
+        OBVH_HIP_TRY(hipMemcpyAsync(ws.keys_tmp, ws.keys, sizeof(uint32_t) * nf, hipMemcpyDeviceToDevice, stream));
+        size_t sb = ws.sort_bytes;
+        OBVH_HIP_TRY(rocprim::radix_sort_pairs(ws.sort_tmp, sb, ws.keys_tmp, ws.keys, ws.vals_tmp, ws.vals, nf, 0, 30,
+                                               stream));
+    }
+    hipLaunchKernelGGL(lbvh_tree, blocks(nf, kTreeThreads), dim3(kTreeThreads), 0, stream, nf, ws, nodes, parents,
+                       mortons);
+    hipLaunchKernelGGL(lbvh_aabbs, up_grid(nf), dim3(kUpTile), 0, stream,
+                       LbvhUp{{nodes, parents, counts, costs}, V, F, ws.vals, nf - 1}, nf, ws.visit);
     OBVH_HIP_TRY(hipGetLastError());
     return nullptr;
 }

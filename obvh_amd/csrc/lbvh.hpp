@@ -3,17 +3,19 @@
 #include <hip/hip_runtime.h>
 
 #include "obvh/obvh.h"
+#include "radix.hpp"
 
 namespace obvh {
 
 struct LbvhWs {
     int32_t* cbox;       // centroid box as order-preserving keys (min xyz, max xyz)
     uint32_t* visit;     // per internal node: children done (bottom-up pass)
-    uint32_t* keys_in;   // Morton codes by face
-    uint32_t* keys_out;  // sorted codes
-    uint32_t* vals_in;   // face ids
-    uint32_t* vals_out;  // face ids in sorted order
-    char* sort_tmp;      // radix-sort scratch
+    uint32_t* keys;      // Morton codes by face, then sorted
+    uint32_t* vals;      // face ids in sorted order
+    uint32_t* keys_tmp;  // the sort's other buffers
+    uint32_t* vals_tmp;
+    RadixWs radix;
+    char* sort_tmp;      // rocPRIM's scratch (more than 2^30 faces)
     size_t sort_bytes;
 };
 

@@ -416,3 +416,23 @@ def test_dito_batch_overlapping_sets(torch, oracle_lib):
     assert np.array_equal(got[0], exp) and np.array_equal(got[2], exp)
     for s in (1, 3, 4, 5, 6):
         assert np.isnan(got[s]).all() and g[s]["degenerate"] == 4, s
+
+
+# the sort's forms and tiles (one workgroup up to 4096 faces; 1, 2 and 4 faces per thread), few distinct codes
+@pytest.mark.parametrize("nf", [1023, 1024, 1025, 2049, 4096, 4097, 32768, 32769, 70000, 131073])
+@pytest.mark.parametrize("cells", [3, 1000])
+def test_lbvh_sort_edges(torch, oracle_lib, nf, cells):
+    say(f"[lbvh] sort: {nf} faces over {cells} positions per axis")
+    rng = np.random.default_rng(nf)
+    c = np.floor(rng.uniform(0, 1, (nf, 1, 3)) * cells) / cells
+    V = (c + rng.uniform(0, 1e-4, (nf, 3, 3))).reshape(-1, 3).astype(np.float32)
+    F = np.zeros((nf, 4), dtype=np.uint32)
+    F[:, :3] = np.arange(3 * nf).reshape(nf, 3)
+    t = ops.lbvh_build(torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda())
+    torch.cuda.synchronize()
+    nodes, parents, counts, costs, mortons = oracle_lib.lbvh_build(V, F)
+    assert np.array_equal(t["mortons"].cpu().numpy().view(np.uint32), mortons)
+    assert np.array_equal(t["parents"].cpu().numpy().view(np.uint32), parents)
+    assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), nodes.view(np.uint8))
+    assert np.array_equal(t["counts"].cpu().numpy().view(np.uint32), counts)
+    assert np.array_equal(t["costs"].cpu().numpy(), costs)
