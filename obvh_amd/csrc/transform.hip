@@ -11,20 +11,19 @@
 //                word tagged with the workgroup, and parents whose children
 //                finished in different workgroups are deferred.  Then the
 //                leaf OBBs and matrices (transforms.cu:803-834).
-//  climb_phase   the deferred parents, in 32768-leaf workgroups whose last
-//                one to finish then climbs the rest of the tree; arrivals
-//                within a workgroup are counted, and k-DOPs handed over, in
-//                LDS.  The merge takes the right child's extreme only if
-//                strictly better, so ties go to the left child and the
-//                selected vertex ids do not depend on scheduling.  k-DOPs
-//                carry vertex ids, not positions (7 x {min, id, max, id} =
-//                112 B per node); spans carry an exact gap flag from leaf
-//                counts.
+//  climb_upper   the deferred parents and everything above them, eight lanes a
+//                path, k-DOPs handed over past the L2 caches.  The merge
+//                takes the right child's extreme only if strictly better, so
+//                ties go to the left child and the selected vertex ids do
+//                not depend on scheduling.  k-DOPs carry vertex ids, not
+//                positions (7 x {min, id, max, id} = 112 B per node); spans
+//                carry an exact gap flag from leaf counts.
 //  candidates    one lane per internal node: gather the 14 extremal vertices
 //                and run the base-triangle + ditetrahedron search in
-//                registers (transforms.cu:413-756); the nodes the tile climb
-//                completed on a second stream beside climb_phase, the rest
-//                after it, together with each refit tile's ancestor chain.
+//                registers (transforms.cu:413-756), together with each refit
+//                tile's ancestor chain.  Large trees search the nodes the tile
+//                climb completed on a second stream beside climb_upper and
+//                the others after it.
 //  cand_redo     the search in reference mode for nodes with non-finite or
 //                huge extremal points.
 //  refit         exact projection range of every subtree vertex on each
@@ -49,8 +48,6 @@
 namespace obvh {
 
 constexpr uint32_t kInvalid = 0xFFFFFFFFu;
-constexpr uint32_t kChunk0 = 512;     // leaves per workgroup, first climb phase
-constexpr uint32_t kChunk1 = 32768;   // second phase
 
 struct Mat4 {
     float v[16];
@@ -322,15 +319,15 @@ __global__ void tree_clear(uint64_t* visit, uint32_t n, TreeWs ws) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
         *ws.error = 0;
-        for (int k = 0; k < kMaxPhases; ++k) ws.nlist[k] = 0;
-        *ws.phase_done = 0;
+        for (int k = 0; k < kNodeLists; ++k) ws.nlist[k] = 0;
     }
     for (uint32_t i = t; i < n; i += gridDim.x * blockDim.x) visit[i] = 0;
 }
 
 // Arrival word of an internal node: low 32 bits count the children that
 // finished, high 32 bits sum their tags.  tag = (phase << 24) | (owner + 1)
-// identifies the kernel phase and the workgroup that completed the child.
+// identifies the kernel (0 climb_leaves, 1 climb_upper) and the workgroup that
+// completed the child.
 __device__ __forceinline__ bool complete(uint64_t v) { return (uint32_t)v == 2u; }
 __device__ __forceinline__ uint32_t make_tag(uint32_t phase, uint32_t owner) { return (phase << 24) | (owner + 1u); }
 
@@ -395,21 +392,22 @@ __device__ __forceinline__ void span_store(TreeWs& ws, uint32_t c, uint2 s, uint
     if (span_gap(s)) ws.count[c] = cnt;
 }
 
-// Node lists (ws.list, counts in ws.nlist): 0 and 1 hold the nodes a climb
-// phase defers to the next, kUpperList the nodes completed after the tile
-// climb, kRedoList the nodes the candidate search hands to reference mode.
-constexpr int kUpperList = 2;
-constexpr int kRedoList = 3;
-static_assert(kRedoList < kMaxPhases, "one list per slot");
+// Node lists (ws.list, counts in ws.nlist): the nodes the tile climb defers, the
+// nodes completed after it, and those the candidate search hands to reference
+// mode.
+constexpr int kDeferList = 0;
+constexpr int kUpperList = 1;
+constexpr int kRedoList = 2;
+static_assert(kRedoList < kNodeLists, "one list per slot");
 
 // A deferred node is marked in bit 63 of its arrival word: its count already
-// reads 2 (both children arrived), but its k-DOP is made by the next phase,
-// so the candidate launch that runs beside the later phases must skip it.
+// reads 2 (both children arrived), but its k-DOP is made by climb_upper, so
+// the candidate launch that runs beside it must skip it.
 constexpr uint64_t kDeferred = 1ull << 63;
-__device__ __forceinline__ void defer(TreeWs& ws, uint32_t phase, uint32_t node, uint32_t I) {
+__device__ __forceinline__ void defer(TreeWs& ws, uint32_t node, uint32_t I) {
     atomicOr(reinterpret_cast<unsigned long long*>(&ws.visit[node]), (unsigned long long)kDeferred);
-    const uint32_t slot = atomicAdd(&ws.nlist[phase], 1u);
-    if (slot < I) ws.list[(size_t)phase * (I + 1) + slot] = node;
+    const uint32_t slot = atomicAdd(&ws.nlist[kDeferList], 1u);
+    if (slot < I) ws.list[(size_t)kDeferList * (I + 1) + slot] = node;
 }
 
 // k-DOP of leaf node `leaf` from the mesh.
@@ -423,7 +421,7 @@ __device__ __forceinline__ bool leaf_kdop_global(const kr_bvh_node* nodes, const
     return true;
 }
 
-// Phase 0 of the bottom-up k-DOP pass.  Workgroup w owns leaf positions
+// The tiles' part of the bottom-up k-DOP pass.  Workgroup w owns leaf positions
 // [w*kTile, (w+1)*kTile) and the internal nodes with the same indices (for a
 // Karras-ordered tree these are the internal nodes whose leaves lie in the
 // range).  The workgroup first loads the tile's topology into LDS (children
@@ -436,14 +434,14 @@ __device__ __forceinline__ bool leaf_kdop_global(const kr_bvh_node* nodes, const
 // loading it (node completed outside the tile's index range).  At the
 // first level two leaf siblings in one wave merge without an arrival count:
 // the left one takes the right one's k-DOP by lane shuffles.  Parents outside the tile use the global arrival word with
-// the workgroup's tag; such a parent is deferred to the next phase when its
+// the workgroup's tag; such a parent is deferred to climb_upper when its
 // children finished in different workgroups.  Finally tile nodes reached by
 // one child only are folded into the global arrival words, and the k-DOPs,
 // spans and arrival words of tile nodes completed here are written back
 // contiguously.  The merge keeps the left child's extreme on ties.  Last,
 // the tile's leaf boxes (transforms.cu:803-834) from the triangles each lane
 // loaded, staged in the same LDS and written back contiguously.
-constexpr uint32_t kTile = kChunk0;
+constexpr uint32_t kTile = 512;  // leaves per workgroup
 
 struct ClimbTile {
     float4 kd[kTile][7];        // k-DOP of internal node lo + s, once completed here
@@ -599,7 +597,7 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
                 const uint32_t cnt = (uint32_t)old;
                 if (cnt == 0) break;
                 if (cnt != 1) { atomicOr(ws.error, 2u); break; }
-                if ((uint32_t)(old >> 32) != tag) { defer(ws, 0, p, I); break; }  // other workgroup
+                if ((uint32_t)(old >> 32) != tag) { defer(ws, p, I); break; }  // other workgroup
                 am_left = l == cur;
                 if (!am_left && rr != cur) { atomicOr(ws.error, 2u); break; }
                 sib = am_left ? rr : l;
@@ -677,7 +675,7 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
         }
         const uint64_t old = __hip_atomic_fetch_add(&ws.visit[pos], ((uint64_t)tag << 32) | 1ull,
                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if ((uint32_t)old == 1u) defer(ws, 0, pos, I);
+        if ((uint32_t)old == 1u) defer(ws, pos, I);
         else if ((uint32_t)old != 0u) atomicOr(ws.error, 2u);
     }
     // write back the tile nodes completed here
@@ -701,57 +699,33 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
     stage_flush(U.st, obbs, mats, (size_t)I + lo, min(kTile, N - lo), bm);
 }
 
-// Phase >= 1 of the bottom-up k-DOP pass.  Workgroup w takes the nodes the
-// previous phase deferred whose index lies in [w*chunk, (w+1)*chunk) (both
-// children complete, k-DOPs in global memory), merges them and climbs.  At
-// a parent p:
-//   - one child of p completed in an earlier kernel (its arrival is in p's
-//     arrival word, read a level ahead): the sibling's k-DOP is loaded and
-//     the climb goes on;
-//   - otherwise the arrival is counted in an LDS hash keyed by p.  Each
-//     child first writes its k-DOP and span to its side of p's slot; the
-//     first arrival stops, the second reads the other side and goes on.
-//     Slots still holding one arrival at the end are pairs split between
-//     workgroups: they are folded into the global arrival words, and the
-//     second fold defers p to the next phase;
-//   - when p finds no slot (LDS full), the global arrival word with the
-//     workgroup's tag is used, as at the tile boundaries of phase 0.
-// Every completed node's k-DOP and span go to global memory as they are
-// made (the candidate search and the next phase read them).  The last phase
-// is one workgroup and defers nothing.  Arrivals within the workgroup need
-// workgroup-scope ordering only, on LDS.
-constexpr int kPSlots = 600;   // LDS hash slots (both children's k-DOPs each)
-constexpr int kPProbe = 64;
-constexpr int kPQueue = 1024;  // entries taken from the previous phase's list
-constexpr int kPhaseThreads = 512;  // workgroup size of climb_phase (the pipeline needs ~150 VGPRs)
-
-struct PhaseTile {
-    float4 kd[kPSlots][2][7];  // side 0: left child, side 1: right child
-    uint2 span[kPSlots][2];
-    uint32_t cnt[kPSlots][2];
-    uint32_t key[kPSlots];
-    uint32_t arrive[kPSlots];
-    uint32_t queue[kPQueue];
-    uint32_t done[kPQueue];    // nodes completed here, for the second candidate launch
-    uint32_t nq, ndone, dbase;
-};
-
-// Slot of node p, inserted if absent; kInvalid when the probe window is full
-// (keys are never removed, so both children of p get the same answer).
-__device__ __forceinline__ uint32_t phase_slot(PhaseTile& P, uint32_t p) {
-    uint32_t h = __umulhi(p * 2654435761u, (uint32_t)kPSlots);
-    for (int probe = 0; probe < kPProbe; ++probe) {
-        uint32_t key = __hip_atomic_load(&P.key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (key == kInvalid) key = atomicCAS(&P.key[h], kInvalid, p);
-        if (key == kInvalid || key == p) return h;
-        h = (h + 1 == (uint32_t)kPSlots) ? 0u : h + 1;
-    }
-    return kInvalid;
-}
-
-// Children, parent and arrival word of node p (zero / kInvalid past the
-// internal nodes).
-struct Topo {
+// The rest of the bottom-up k-DOP pass: the nodes the tile climb deferred (both
+// children complete) and everything above them, in one launch.  Eight lanes
+// take a deferred node and follow its path to the root: lanes 0..6 hold a slab
+// each of the k-DOP, lane 7 the span and leaf count, so a level's loads and
+// stores are one or two instructions over a few cache lines.  Children,
+// parents and arrival words are loaded two levels ahead (arrival words past the
+// L2 caches).  At a parent p
+//   - whose other child was seen to have arrived (in the tile climb or here):
+//     its data was loaded one level ahead; the path goes on at once;
+//   - otherwise the node is stored with agent-scope accesses (past the L2
+//     caches), then its arrival counted; the first path to arrive ends, the
+//     second loads the sibling past the caches and goes on.
+// Nobody waits, and a node is stored before its arrival is counted, so no order
+// of the workgroups matters.  Completed nodes are collected in LDS (one
+// counter for all of them would take an atomic of the chip per node) and
+// appended to a list for the candidate search.
+//
+// Bound by latency: a level takes 1.5 us on an idle chip (5120 triangles: 15
+// levels, 23 us) and 3 us beside the candidate search (1M triangles: 26 levels,
+// 77 us, 2M 117 us), which hides it.  Without the loads ahead 114 and 334 us;
+// with eight paths in a wave from the start 107, 226, and 31 us for 5120
+// triangles (a wave is as slow as its slowest path).  Before, 32768-leaf
+// workgroups with hand-overs in LDS and one last workgroup took 106, 190 and
+// 30 us.  Random topology (nearly every node is up here), whole transform:
+// 100000 leaves 14.1 ms then, 8.6 now.  The waves run at raised priority: they
+// are few, and issue little between their waits.
+struct Topo {  // children, parent and arrival word of a node (zero / kInvalid past the internal nodes)
     uint32_t l, r, parent;
     uint64_t v;
 };
@@ -762,163 +736,135 @@ __device__ __forceinline__ Topo topo_load(const kr_bvh_node* __restrict__ nodes,
         T.l = nodes[p].u.children.left;
         T.r = nodes[p].u.children.right;
         T.parent = parents[p];
-        T.v = ws.visit[p];
+        T.v = ld_agent(&ws.visit[p]);
     }
     return T;
 }
-// The k-DOP, span and leaf count of the other child of the node whose
-// topology is T, read only when T's arrival word says that child finished
-// in an earlier kernel (visible since the launch).
-struct Sib {
-    Kdop k;
-    uint2 s;
-    uint32_t c;
-};
-__device__ __forceinline__ void sib_load(const TreeWs& ws, const Topo& T, uint32_t child, uint32_t phase,
-                                         uint32_t I, uint32_t total, Sib& S) {
-    const uint32_t c0 = (uint32_t)T.v, t0 = (uint32_t)(T.v >> 32);
-    const uint32_t sib = T.l == child ? T.r : T.l;
-    if (c0 == 1u && (t0 >> 24) < phase && sib < total) {
-        kdop_load(ws.kdop, sib, S.k);
-        S.s = span_load(ws, sib, I, S.c);
+
+constexpr int kPathLanes = 8;
+constexpr uint32_t kUpperThreads = kWave;  // one wave per workgroup: paths spread over the chip
+constexpr uint32_t kUpperDone = 512;       // completed nodes a workgroup collects before it appends them
+
+// Lane q of a path's share of a node: slab q (lanes 0..6), or the span and
+// leaf count (lane 7).
+template <bool kAgent>
+__device__ __forceinline__ uint4 path_load(const TreeWs& ws, uint32_t node, uint32_t I, int q) {
+    auto ld64 = [](const void* p) {
+        const uint64_t* w = static_cast<const uint64_t*>(p);
+        const uint64_t v = kAgent ? ld_agent(w) : *w;
+        return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+    };
+    if (q < 7) {
+        const float4* k = &ws.kdop[(size_t)node * 7 + q];
+        const uint2 a = ld64(k), b = ld64(reinterpret_cast<const uint2*>(k) + 1);
+        return make_uint4(a.x, a.y, b.x, b.y);
     }
+    if (node >= I) {
+        const uint2 sp = leaf_span(node - I);
+        return make_uint4(sp.x, sp.y, 1u, 0u);
+    }
+    const uint2 sp = ld64(&ws.span[node]);
+    const uint32_t kept = kAgent ? ld_agent(&ws.count[node]) : ws.count[node];
+    return make_uint4(sp.x, sp.y, span_count(sp, kept), 0u);
+}
+template <bool kAgent>
+__device__ __forceinline__ void path_store(const TreeWs& ws, uint32_t node, int q, uint4 k) {
+    auto st64 = [](void* p, uint32_t x, uint32_t y) {
+        uint64_t* w = static_cast<uint64_t*>(p);
+        const uint64_t v = (uint64_t)y << 32 | x;
+        if (kAgent) st_agent(w, v);
+        else *w = v;
+    };
+    if (q < 7) {
+        float4* d = &ws.kdop[(size_t)node * 7 + q];
+        st64(d, k.x, k.y);
+        st64(reinterpret_cast<uint2*>(d) + 1, k.z, k.w);
+        return;
+    }
+    st64(&ws.span[node], k.x, k.y);
+    if (kAgent) st_agent(&ws.count[node], k.z);
+    else ws.count[node] = k.z;
+}
+__device__ __forceinline__ uint4 path_merge(uint4 l, uint4 r, int q) {
+    if (q < 7) {  // merge_left_first of one slab
+        if (__uint_as_float(r.x) < __uint_as_float(l.x)) { l.x = r.x; l.y = r.y; }
+        if (__uint_as_float(r.z) > __uint_as_float(l.z)) { l.z = r.z; l.w = r.w; }
+        return l;
+    }
+    uint32_t c;
+    const uint2 sp = span_join(make_uint2(l.x, l.y), l.z, make_uint2(r.x, r.y), r.z, c);
+    return make_uint4(sp.x, sp.y, c, 0u);
 }
 
-// One phase as workgroup `wg` of `nwg`.
-__device__ __forceinline__ void phase_pass(PhaseTile& P, const kr_bvh_node* __restrict__ nodes,
-                                           const uint32_t* __restrict__ parents, TreeWs& ws, uint32_t N,
-                                           uint32_t phase, uint32_t chunk, uint32_t wg, uint32_t nwg) {
-    const uint32_t I = N - 1, total = 2 * N - 1, t = threadIdx.x;
-    const uint32_t tag = make_tag(phase, wg);
-    const uint64_t lo = (uint64_t)wg * chunk, hi = lo + chunk;  // owned node indices
-    const uint32_t nin = min(ws.nlist[phase - 1], I);
-    const uint32_t* in = ws.list + (size_t)(phase - 1) * (I + 1);
-    for (uint32_t h = t; h < (uint32_t)kPSlots; h += blockDim.x) {
-        P.key[h] = kInvalid;
-        P.arrive[h] = 0;
-    }
-    if (t == 0) {
-        P.nq = 0;
-        P.ndone = 0;
-    }
-    const bool last = nwg == 1;
-    auto completed = [&](uint32_t node) {
-        const uint32_t d = atomicAdd(&P.ndone, 1u);
-        if (d < (uint32_t)kPQueue) {
-            P.done[d] = node;
-        } else {
-            const uint32_t slot = atomicAdd(&ws.nlist[kUpperList], 1u);
-            if (slot < I) ws.list[(size_t)kUpperList * (I + 1) + slot] = node;
-        }
+__global__ __launch_bounds__(kUpperThreads) void climb_upper(const kr_bvh_node* __restrict__ nodes,
+                                                             const uint32_t* __restrict__ parents, TreeWs ws,
+                                                             uint32_t N) {
+    __builtin_amdgcn_s_setprio(3);  // wave priority
+    const uint32_t I = N - 1, total = 2 * N - 1;
+    const int q = (int)(threadIdx.x % kPathLanes), lead = lane_id() - q;
+    const uint32_t nin = min(ws.nlist[kDeferList], I);
+    const uint32_t* in = ws.list + (size_t)kDeferList * (I + 1);
+    const uint64_t mine = (uint64_t)make_tag(1, 0) << 32 | 1ull;
+    __shared__ uint32_t done[kUpperDone], ndone;
+    if (threadIdx.x == 0) ndone = 0;
+    __syncthreads();
+    auto append = [&](uint32_t slot, uint32_t node) {
+        if (slot < I) ws.list[(size_t)kUpperList * (I + 1) + slot] = node;
     };
-    __syncthreads();
-    // the owned entries, four independent reads per lane and round
-    for (uint32_t r0 = t; r0 < nin; r0 += 4 * blockDim.x) {
-        uint32_t e[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t r = r0 + j * blockDim.x;
-            e[j] = r < nin ? in[r] : kInvalid;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (e[j] == kInvalid || e[j] < lo || e[j] >= hi) continue;
-            const uint32_t q = atomicAdd(&P.nq, 1u);
-            if (q < (uint32_t)kPQueue) P.queue[q] = e[j];
-        }
-    }
-    __syncthreads();
-    const uint32_t nq = P.nq;
-    const bool queued = nq <= (uint32_t)kPQueue;
-    // more entries than the queue holds: every lane scans the list again
-    for (uint32_t r = t; r < (queued ? nq : nin); r += blockDim.x) {
-        uint32_t cur = queued ? P.queue[r] : in[r];
-        if (!queued && (cur < lo || cur >= hi)) continue;
+    auto completed = [&](uint32_t node) {
+        if (q != 0) return;
+        const uint32_t s = __hip_atomic_fetch_add(&ndone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (s < kUpperDone) done[s] = node;
+        else append(atomicAdd(&ws.nlist[kUpperList], 1u), node);
+    };
+    // one path per wave as far as the waves go, then a second, ...
+    for (uint32_t r = blockIdx.x + threadIdx.x / kPathLanes * gridDim.x; r < nin;
+         r += gridDim.x * (kUpperThreads / kPathLanes)) {
+        uint32_t cur = in[r];
         if (cur >= I) { atomicOr(ws.error, 1u); continue; }
-        const uint32_t l0 = nodes[cur].u.children.left, r0 = nodes[cur].u.children.right;
-        if (l0 >= total || r0 >= total) { atomicOr(ws.error, 2u); continue; }
-        Kdop k;
-        uint32_t count, c0l, c0r;
-        const uint2 s0l = span_load(ws, l0, I, c0l), s0r = span_load(ws, r0, I, c0r);
-        uint2 span = span_join(s0l, c0l, s0r, c0r, count);
-        {
-            Kdop a, b;
-            kdop_load(ws.kdop, l0, a);
-            kdop_load(ws.kdop, r0, b);
-            merge_left_first(a, b, k);
-        }
-        kdop_store(ws.kdop, cur, k);
-        span_store(ws, cur, span, count);
-        completed(cur);
-        // Pipeline: the topology and arrival word of a node are read two
-        // levels ahead (A: the parent p, B: its parent), and where the
-        // sibling at the next level finished in an earlier kernel its k-DOP,
-        // span and count are read as soon as this level's merge is done
-        // (SA), so that a level costs about one memory round trip.
         uint32_t p = parents[cur];
         Topo A = topo_load(nodes, parents, ws, p, I);
-        Sib SA;
-        sib_load(ws, A, cur, phase, I, total, SA);
+        const uint32_t l0 = nodes[cur].u.children.left, r0 = nodes[cur].u.children.right;
+        if (l0 >= total || r0 >= total) { atomicOr(ws.error, 2u); continue; }
+        uint4 k = path_merge(path_load<false>(ws, l0, I, q), path_load<false>(ws, r0, I, q), q);
         Topo B = topo_load(nodes, parents, ws, A.parent, I);
-        for (uint32_t step = 0; p != kInvalid; ++step) {
-            if (p >= I || step >= N) { atomicOr(ws.error, 1u); break; }
-            const bool am_left = (A.l == cur);
+        completed(cur);
+        uint4 o = make_uint4(0, 0, 0, 0);  // the sibling, if its arrival was seen
+        bool have = false;
+        auto fetch = [&](const Topo& T, uint32_t child) {
+            const uint32_t sib = T.l == child ? T.r : T.l;
+            have = (uint32_t)T.v == 1u && sib < total;
+            asm volatile("" ::: "memory");
+            if (have) o = path_load<true>(ws, sib, I, q);
+        };
+        fetch(A, cur);
+        for (uint32_t step = 0;; ++step) {  // the same for the eight lanes
+            const bool am_left = A.l == cur;
             const uint32_t sib = am_left ? A.r : A.l;
-            if (sib >= total || (!am_left && A.r != cur)) { atomicOr(ws.error, 2u); break; }
-            const Topo C = topo_load(nodes, parents, ws, B.parent, I);
-            const uint32_t c0 = (uint32_t)A.v, t0 = (uint32_t)(A.v >> 32);
-            Kdop o;
-            uint2 so;
-            uint32_t co;
-            if (c0 == 1u && (t0 >> 24) < phase) {  // the sibling finished in an earlier kernel
-                o = SA.k;
-                so = SA.s;
-                co = SA.c;
-                ws.visit[p] = A.v + (((uint64_t)tag << 32) | 1ull);
-            } else if (c0 > 1u) {
-                atomicOr(ws.error, 2u);
+            if (p >= I || step >= N || sib >= total || (!am_left && A.r != cur)) {
+                path_store<false>(ws, cur, q, k);
+                if (p != kInvalid) atomicOr(ws.error, p >= I || step >= N ? 1u : 2u);
                 break;
-            } else if (const uint32_t h = phase_slot(P, p); h != kInvalid) {
-                const int side = am_left ? 0 : 1;
-#pragma unroll
-                for (int q = 0; q < 7; ++q)
-                    P.kd[h][side][q] = make_float4(k.mn[q], __uint_as_float(k.imn[q]), k.mx[q], __uint_as_float(k.imx[q]));
-                P.span[h][side] = span;
-                P.cnt[h][side] = count;
-                const uint32_t a = __hip_atomic_fetch_add(&P.arrive[h], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (a == 0u) break;  // first arrival: the sibling continues (or the end fold defers p)
-                if (a != 1u) { atomicOr(ws.error, 2u); break; }
-#pragma unroll
-                for (int q = 0; q < 7; ++q) {
-                    const float4 x = P.kd[h][side ^ 1][q];
-                    o.mn[q] = x.x; o.imn[q] = __float_as_uint(x.y);
-                    o.mx[q] = x.z; o.imx[q] = __float_as_uint(x.w);
-                }
-                so = P.span[h][side ^ 1];
-                co = P.cnt[h][side ^ 1];
-                ws.visit[p] = ((uint64_t)tag << 33) | 2ull;
-            } else {  // no LDS slot: the global arrival word (cur's k-DOP is already stored)
-                const uint64_t old = __hip_atomic_fetch_add(&ws.visit[p], ((uint64_t)tag << 32) | 1ull,
-                                                            __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const uint32_t cnt = (uint32_t)old, t1 = (uint32_t)(old >> 32);
-                if (cnt == 0) break;
-                if (cnt != 1) { atomicOr(ws.error, 2u); break; }
-                if (t1 != tag && (t1 >> 24) >= phase) {  // the other child finished in another workgroup
-                    if (last) atomicOr(ws.error, 2u);
-                    else defer(ws, phase, p, I);
-                    break;
-                }
-                kdop_load(ws.kdop, sib, o);
-                so = span_load(ws, sib, I, co);
             }
-            Kdop m;
-            if (am_left) merge_left_first(k, o, m); else merge_left_first(o, k, m);
-            k = m;
-            span = span_join(span, count, so, co, count);
-            kdop_store(ws.kdop, p, k);
-            span_store(ws, p, span, count);
+            const Topo C = topo_load(nodes, parents, ws, B.parent, I);
+            if (have) {
+                path_store<false>(ws, cur, q, k);
+                if (q == 0) ws.visit[p] = A.v + mine;
+            } else {
+                path_store<true>(ws, cur, q, k);
+                drain();
+                uint64_t old = 0;
+                if (q == 0)
+                    old = __hip_atomic_fetch_add(&ws.visit[p], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t c = (uint32_t)__shfl((int)(uint32_t)old, lead);
+                if (c == 0) break;  // first arrival: the sibling's path goes on
+                if (c != 1) { atomicOr(ws.error, 2u); break; }
+                asm volatile("" ::: "memory");
+                o = path_load<true>(ws, sib, I, q);
+            }
+            k = am_left ? path_merge(k, o, q) : path_merge(o, k, q);
+            fetch(B, p);
             completed(p);
-            sib_load(ws, B, p, phase, I, total, SA);  // the next level's sibling
             cur = p;
             p = A.parent;
             A = B;
@@ -926,50 +872,11 @@ __device__ __forceinline__ void phase_pass(PhaseTile& P, const kr_bvh_node* __re
         }
     }
     __syncthreads();
-    // pairs split between workgroups: fold the single arrival into the
-    // global word; the second fold defers the node
-    for (uint32_t h = t; h < (uint32_t)kPSlots; h += blockDim.x) {
-        const uint32_t p = P.key[h];
-        if (p == kInvalid || P.arrive[h] != 1u) continue;
-        const uint64_t old = __hip_atomic_fetch_add(&ws.visit[p], ((uint64_t)tag << 32) | 1ull, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
-        if ((uint32_t)old == 1u && !last) defer(ws, phase, p, I);
-        else if ((uint32_t)old != 0u) atomicOr(ws.error, 2u);
-    }
-    // the completed nodes go to the upper list in one block
-    if (t == 0) P.dbase = atomicAdd(&ws.nlist[kUpperList], min(P.ndone, (uint32_t)kPQueue));
-    __syncthreads();
-    const uint32_t nd = min(P.ndone, (uint32_t)kPQueue);
-    for (uint32_t i = t; i < nd; i += blockDim.x)
-        if (P.dbase + i < I) ws.list[(size_t)kUpperList * (I + 1) + P.dbase + i] = P.done[i];
-}
-
-// Phase 1 on `gridDim.x` workgroups; the last workgroup to finish (one
-// agent-scope release per workgroup, an acquire in the last) then runs the
-// last phase over the whole tree on the CU it holds, so that the last phase
-// does not wait for a CU to drain while the side stream fills the chip.  A
-// launch with one workgroup runs its phase as the last.
-__global__ __launch_bounds__(kPhaseThreads) void climb_phase(const kr_bvh_node* __restrict__ nodes,
-                                                    const uint32_t* __restrict__ parents, TreeWs ws, uint32_t N,
-                                                    uint32_t phase, uint32_t chunk) {
-    __shared__ PhaseTile P;
-    __shared__ uint32_t finished_last;
-    uint32_t wg = blockIdx.x, nwg = gridDim.x;
-    for (;;) {
-        phase_pass(P, nodes, parents, ws, N, phase, chunk, wg, nwg);
-        if (nwg == 1) return;
-        __syncthreads();
-        if (threadIdx.x == 0)
-            finished_last =
-                __hip_atomic_fetch_add(ws.phase_done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nwg - 1;
-        __syncthreads();
-        if (!finished_last) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        ++phase;
-        chunk = N;
-        wg = 0;
-        nwg = 1;
-    }
+    const uint32_t nd = min(ndone, kUpperDone);
+    uint32_t base = 0;
+    if (threadIdx.x == 0 && nd) base = atomicAdd(&ws.nlist[kUpperList], nd);
+    base = (uint32_t)__shfl((int)base, 0);
+    for (uint32_t s = threadIdx.x; s < nd; s += kUpperThreads) append(base + s, done[s]);
 }
 
 // ------------------------------------------------------- candidates --
@@ -1351,7 +1258,7 @@ __device__ void tile_chain(const uint32_t* __restrict__ parents, TreeWs& ws, uin
 }
 
 // Arrival word of a node completed by the tile climb: both tags are phase 0
-// (tag = owner + 1 < 2^23), so their sum stays below 2^24; later phases add
+// (tag = owner + 1 < 2^23), so their sum stays below 2^24; climb_upper adds
 // a tag of at least 2^24, a deferred node carries bit 63 (kDeferred) and a
 // hole's word is all ones.
 __device__ __forceinline__ bool tile_complete(uint64_t v) { return complete(v) && (uint32_t)(v >> 32) < (1u << 24); }
@@ -1431,19 +1338,20 @@ __device__ __forceinline__ void cand_block(const kr_vec3* __restrict__ V, TreeWs
     __syncthreads();  // T is reused by the workgroup's next round
 }
 
-// The candidate search, in two launches.  kUpper = false: the nodes the
-// tile climb completed (index order, one round per workgroup), launched
-// on the side stream beside the top-of-tree climb phases, which leave most
-// of the chip idle; holes get an AABB record.  kUpper = true: the nodes the
-// later phases completed (their list), and workgroups below `cblocks` find
-// the refit tiles' ancestor chains.
-template <bool kUpper>
+// The candidate search.  Large trees take two launches.  kTileNodes: the nodes
+// the tile climb completed (index order, one round per workgroup), beside
+// climb_upper, which leaves most of the chip idle; holes get an AABB record.
+// kUpperNodes: the nodes climb_upper completed (their list).  Small trees take
+// one, kAllNodes, after climb_upper.  In the last two workgroups below
+// `cblocks` find the refit tiles' ancestor chains.
+enum CandNodes { kTileNodes, kUpperNodes, kAllNodes };
+template <int kNodes>
 __global__ __launch_bounds__(kCandBlock, 4) void candidates(const kr_vec3* __restrict__ V,
                                                             const uint32_t* __restrict__ parents, TreeWs ws,
                                                             uint32_t N, uint32_t cblocks) {
     __shared__ CandTile T;
     const uint32_t t = threadIdx.x, I = N - 1;
-    if (kUpper && blockIdx.x < cblocks) {
+    if (kNodes != kTileNodes && blockIdx.x < cblocks) {
         const uint32_t tile = blockIdx.x * kCandBlock + t;
         if (tile < (N + kRTile - 1) / kRTile) {
             if (*ws.error != 0) ws.tmeta[tile] = make_uint2(0u, kInvalid);
@@ -1452,12 +1360,12 @@ __global__ __launch_bounds__(kCandBlock, 4) void candidates(const kr_vec3* __res
         return;
     }
     const bool bad = *ws.error != 0;
-    if (!kUpper) {
-        const uint32_t node = blockIdx.x * kCandBlock + t;
+    if (kNodes != kUpperNodes) {
+        const uint32_t node = (blockIdx.x - cblocks) * kCandBlock + t;
         bool mine = false;
         if (node < I) {
             const uint64_t vw = ws.visit[node];
-            mine = hole(vw) || tile_complete(vw);
+            mine = hole(vw) || (kNodes == kAllNodes ? complete(vw) : tile_complete(vw));
         }
         cand_block(V, ws, I, T, mine ? node : kInvalid, bad);
         return;
@@ -1957,9 +1865,8 @@ size_t tree_carve(TreeWs* ws, void* base, size_t cap, uint32_t N) {
     const size_t I = N ? N - 1 : 0, total = N ? 2 * (size_t)N - 1 : 0;
     ws->visit = c.take<uint64_t>(I + 1);
     ws->error = c.take<uint32_t>(8);
-    ws->nlist = ws->error ? ws->error + 2 : nullptr;  // error[2 .. 2 + kMaxPhases)
-    ws->phase_done = ws->error ? ws->error + 6 : nullptr;
-    ws->list = c.take<uint32_t>((size_t)kMaxPhases * (I + 1));
+    ws->nlist = ws->error ? ws->error + 2 : nullptr;  // error[2 .. 2 + kNodeLists)
+    ws->list = c.take<uint32_t>((size_t)kNodeLists * (I + 1));
     ws->span = c.take<uint2>(total);
     ws->count = c.take<uint32_t>(I + 1);
     ws->kdop = c.take<float4>(total * 7);
@@ -1971,15 +1878,21 @@ size_t tree_carve(TreeWs* ws, void* base, size_t cap, uint32_t N) {
     return c.used;
 }
 
-// Per device: a second stream (default priority) and the events that fork
-// the first candidate launch onto it and join it back.  One lock covers a whole call's
-// enqueue sequence, so calls from several host threads cannot interleave
+// Per device: a second stream (default priority) and the events that fork the
+// first candidate launch onto it and join it back.  One lock covers a call's enqueue
+// sequence between them, so calls from several host threads cannot interleave
 // their record / wait pairs.
 namespace {
 struct SideStream {
     hipStream_t s = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
 };
+// Up to this many leaves all kernels run on the caller's stream: the hand-offs
+// between streams cost 10-15 us, more than the top of the tree takes from the
+// candidate search beside it.  Measured, one stream / two (icospheres, us):
+// 5120 leaves 110 / 124, 100820 144 / 162, 200000 183 / 187, 338000 235 / 231,
+// 499280 294 / 279.
+constexpr uint32_t kOneStream = 1u << 18;
 constexpr int kMaxDevices = 64;
 std::mutex g_side_mu;
 SideStream g_side[kMaxDevices];
@@ -2009,37 +1922,44 @@ kr_error tree_launch(const kr_bvh_node* nodes, const uint32_t* parents, const kr
     if (workspace == nullptr || ws_bytes < need) return "obvh_obb_tree: workspace too small";
     const uint32_t I = N - 1;
     auto blocks = [](uint32_t n, uint32_t b) { return dim3((n + b - 1) / b); };
-    std::lock_guard<std::mutex> lock(g_side_mu);
-    SideStream* side = nullptr;
-    if (kr_error e = side_stream(&side)) return e;
     hipLaunchKernelGGL(tree_clear, dim3(1024), dim3(256), 0, stream, ws.visit, I + 1, ws);
     if (bm.K > 1)
         hipLaunchKernelGGL(batch_holes, dim3(min((bm.K + 255) / 256, 1024u)), dim3(256), 0, stream, ws, bm);
-    // climb: 512-leaf tiles, then 32768-leaf workgroups, then one workgroup
-    // for the rest
     hipLaunchKernelGGL(climb_leaves, blocks(N, kTile), dim3(kTile), 0, stream, nodes, parents, V, F, ws, N, obbs, mats,
                        bm);
-    // The side stream takes the candidate search of the nodes the tile climb
-    // completed (nearly all of them; VALU-bound) beside the top-of-tree climb
-    // phases, which are latency-bound on a few dozen workgroups.  The launch
-    // stream joins it before the refit.
     if (I > 0) {
-        OBVH_HIP_TRY(hipEventRecord(side->fork, stream));
-        OBVH_HIP_TRY(hipStreamWaitEvent(side->s, side->fork, 0));
-        hipLaunchKernelGGL(candidates<false>, blocks(I, kCandBlock), dim3(kCandBlock), 0, side->s, V, parents, ws, N,
-                           0u);
-        OBVH_HIP_TRY(hipEventRecord(side->join, side->s));
-    }
-    if (N > kTile) {  // phase 1 (and its last workgroup phase 2), or one phase for a small tree
-        const uint32_t c = N > kChunk1 ? kChunk1 : N;
-        hipLaunchKernelGGL(climb_phase, blocks(N, c), dim3(kPhaseThreads), 0, stream, nodes, parents, ws, N, 1u, c);
-    }
-    if (I > 0) {
-        // the nodes the phases completed, and the refit tiles' chains
-        const uint32_t cb = (((N + kRTile - 1) / kRTile) + kCandBlock - 1) / kCandBlock;
-        const uint32_t ub = min((I + kCandBlock - 1) / kCandBlock, 1024u);
-        hipLaunchKernelGGL(candidates<true>, dim3(cb + ub), dim3(kCandBlock), 0, stream, V, parents, ws, N, cb);
-        OBVH_HIP_TRY(hipStreamWaitEvent(stream, side->join, 0));
+        // About one deferred node per tile, if the leaves lie in tree order;
+        // at most an eighth of the chip's waves, so that the candidate search
+        // beside it fills the rest (64 trees of 3.8M triangles: 1696 us with up
+        // to 1024, 1773 with up to 8192).
+        const dim3 upper_grid(min(N / kTile + 1, 1024u));
+        const uint32_t cb = (((N + kRTile - 1) / kRTile) + kCandBlock - 1) / kCandBlock;  // the refit tiles' chains
+        if (N <= kOneStream) {
+            if (N > kTile)
+                hipLaunchKernelGGL(climb_upper, upper_grid, dim3(kUpperThreads), 0, stream, nodes, parents, ws, N);
+            hipLaunchKernelGGL(candidates<kAllNodes>, dim3(cb + (I + kCandBlock - 1) / kCandBlock), dim3(kCandBlock), 0,
+                               stream, V, parents, ws, N, cb);
+        } else {
+            // The candidate search of the nodes the tile climb completed
+            // (nearly all of them; VALU-bound) runs on the side stream beside
+            // the top of the tree (latency-bound on a few waves) and its
+            // search on the caller's stream, joined before the refit.  The
+            // other way round the top's waves come last onto a full chip: 2M
+            // triangles 890 us against 876.
+            std::lock_guard<std::mutex> lock(g_side_mu);
+            SideStream* side = nullptr;
+            if (kr_error e = side_stream(&side)) return e;
+            const uint32_t ub = min((I + kCandBlock - 1) / kCandBlock, 1024u);
+            OBVH_HIP_TRY(hipEventRecord(side->fork, stream));
+            hipLaunchKernelGGL(climb_upper, upper_grid, dim3(kUpperThreads), 0, stream, nodes, parents, ws, N);
+            OBVH_HIP_TRY(hipStreamWaitEvent(side->s, side->fork, 0));
+            hipLaunchKernelGGL(candidates<kTileNodes>, blocks(I, kCandBlock), dim3(kCandBlock), 0, side->s, V, parents,
+                               ws, N, 0u);
+            hipLaunchKernelGGL(candidates<kUpperNodes>, dim3(cb + ub), dim3(kCandBlock), 0, stream, V, parents, ws, N,
+                               cb);
+            OBVH_HIP_TRY(hipEventRecord(side->join, side->s));
+            OBVH_HIP_TRY(hipStreamWaitEvent(stream, side->join, 0));
+        }
         hipLaunchKernelGGL(cand_redo, dim3(kRedoBlocks), dim3(1024), 0, stream, V, ws, I);
         hipLaunchKernelGGL(refit, blocks(N, kRTile), dim3(kRTile), 0, stream, nodes, parents, V, F, ws, N);
         hipLaunchKernelGGL(finalize, blocks(I, kStage), dim3(kStage), 0, stream, ws, obbs, mats, I, bm);

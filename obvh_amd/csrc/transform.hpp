@@ -14,16 +14,15 @@ struct Cand {
     int32_t pad;
 };
 
-constexpr int kMaxPhases = 4;
+constexpr int kNodeLists = 3;
 
 struct TreeWs {
     uint64_t* visit;   // per internal node: arrivals (low word) + sum of arrival tags (high word)
     uint32_t* nlist;   // per node list: number of entries
-    uint32_t* phase_done;  // workgroups of climb phase 1 that finished
-    uint32_t* list;    // per climb phase: nodes deferred to the next phase
+    uint32_t* list;    // the node lists, I + 1 entries each
     uint2* span;       // per node: first and last leaf position below it (bit 31 of .y: the
                        // leaves below are not every position from first to last)
-    uint32_t* count;   // per internal node with bit 31 of its span set: leaves below it
+    uint32_t* count;   // per internal node with bit 31 of its span set (others: unused): leaves below it
     uint32_t* error;   // 1: parent index out of range / too deep, 2: parent/child mismatch,
                        // 4: face id out of range, 8: a node did not complete
     float4* kdop;      // 7 per node: {min, min vertex id, max, max vertex id}
@@ -39,7 +38,7 @@ struct TreeWs {
 };
 constexpr uint32_t kRTile = 512;  // leaves per refit workgroup (tiles aligned to multiples of it)
 constexpr uint32_t kTChain = 64;
-static_assert(2 + kMaxPhases <= 8, "error words 2 .. 2 + kMaxPhases hold the phase list counts");
+static_assert(2 + kNodeLists <= 8, "error words 2 .. 2 + kNodeLists hold the list counts");
 
 size_t tree_carve(TreeWs* ws, void* base, size_t cap, uint32_t N);
 struct BatchMap;

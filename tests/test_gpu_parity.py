@@ -298,6 +298,34 @@ def test_obb_tree_contiguous_topology(torch, oracle_lib, n, spine):
     assert np.array_equal(mats.cpu().numpy(), em)
 
 
+# edges of the climb's forms: one 512-leaf tile (nothing above it), the first sizes with a top of the tree, more paths
+# than one wave takes at once, and both sides of the size from which the search runs on two streams; eager and captured
+@pytest.mark.parametrize("kind,n", [("random", 512), ("random", 513), ("contiguous", 1025), ("random", 9000),
+                                    ("contiguous", 262144), ("contiguous", 262145)])
+def test_obb_tree_climb_edges(torch, oracle_lib, kind, n):
+    say(f"[obb_tree] climb edges {kind} n={n}")
+    V, F = synth.hairball(tubes=n // 40 + 1, seed=11)
+    F = F[:n]
+    nodes, parents = random_tree(n, seed=n) if kind == "random" else contiguous_tree(n, seed=n)
+    a = (torch.from_numpy(nodes.view(np.uint8)).cuda(), torch.from_numpy(parents.view(np.int32)).cuda(),
+         torch.from_numpy(V).cuda(), torch.from_numpy(np.ascontiguousarray(F).view(np.int32)).cuda())
+    obbs, mats, ids = ops.obb_tree(*a, with_ids=True)
+    torch.cuda.synchronize()
+    eo, em, ei = oracle_lib.obb_tree(nodes, parents, V, F, with_ids=True)
+    assert np.array_equal(ids.cpu().numpy().view(np.uint32), ei)
+    assert np.array_equal(obbs.cpu().numpy(), eo)
+    assert np.array_equal(mats.cpu().numpy(), em)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = ops.obb_tree(*a, with_ids=True)
+    for _ in range(3):
+        for x in captured:
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x.view(torch.int32), y.view(torch.int32)) for x, y in zip(captured, (obbs, mats, ids)))
+
+
 def renumber(nodes, parents, perm, lperm):
     """The same tree with internal node i stored at perm[i] (perm[0] = 0) and
     the leaf at position j stored at position lperm[j]."""
