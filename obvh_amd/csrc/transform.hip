@@ -1395,8 +1395,9 @@ __global__ __launch_bounds__(1024) void cand_redo(const kr_vec3* __restrict__ V,
 // takes a tile of 512 consecutive leaves and splits each leaf's ancestors
 // in three tiers:
 //   A  below the lowest ancestor holding all 64 leaves of the lane's wave:
-//      each lane folds its triangle's keys into LDS (a slot per internal
-//      node of the tile's index range, a small hash for other nodes);
+//      each group of four lanes folds its triangles' keys into LDS (a slot
+//      per internal node of the tile's index range, a small hash for other
+//      nodes);
 //   B  from that node up to the lowest ancestor holding the whole tile: the
 //      wave walks together, reduces the 64 lanes' keys with DPP and one lane
 //      folds them into LDS;
@@ -1417,17 +1418,41 @@ __global__ __launch_bounds__(1024) void cand_redo(const kr_vec3* __restrict__ V,
 // per tile by the candidate kernel's leading workgroups, so no workgroup
 // walks the ~10-30 dependent parent loads itself; ancestors beyond the list
 // (very deep trees) are walked by every wave with its lanes' triangles.
+//
+// Bound by latency and LDS throughput at three workgroups of 52 KB per CU: of a
+// workgroup's 67 us on a 1M-leaf tree the loads and the vertex set take 18,
+// tier A 20, tier B 8, tier C 10, the write-back 7.  1M leaves 118 us, 129
+// before the leaf's loads started ahead of the set-up, the vertices' positions
+// came from their lanes' registers instead of a second gather, an axis read
+// became three 16-byte words read a level ahead, and the keys of a node inside
+// the tile replaced its range instead of being merged into it; 3.8M leaves 331,
+// from 374.
 
 constexpr int kRHash = 256;      // LDS hash for ancestors outside the tile's index range
 constexpr int kVSet = 2048;      // distinct vertex ids per tile (hash set)
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr int32_t kKeyHi = 0x7FFFFFFF, kKeyLo = (int32_t)0x80000000;
 
-struct RefitNodes {              // internal nodes lo .. lo + 511 (tiers A and B)
-    float b[9][kRTile];          // candidate axes
-    uint2 span[kRTile];
-    uint32_t parent[kRTile];
-    uint8_t degen[kRTile];
+// An internal node for tiers A and B: three 16-byte words, the candidate axes
+// (9 floats), the parent and the span; bit 31 of the span's first leaf marks a
+// degenerate node.
+struct RefitNode {
+    float4 w[3];
+
+    __device__ __forceinline__ void set(const float b[9], uint32_t parent, uint2 span, bool degen) {
+        w[0] = make_float4(b[0], b[1], b[2], b[3]);
+        w[1] = make_float4(b[4], b[5], b[6], b[7]);
+        w[2] = make_float4(b[8], __uint_as_float(parent), __uint_as_float(span.x | (degen ? kGap : 0u)),
+                           __uint_as_float(span.y));
+    }
+    __device__ __forceinline__ f3 axis(int a) const {
+        return a == 0 ? f3{w[0].x, w[0].y, w[0].z} : a == 1 ? f3{w[0].w, w[1].x, w[1].y} : f3{w[1].z, w[1].w, w[2].x};
+    }
+    __device__ __forceinline__ uint32_t parent() const { return __float_as_uint(w[2].y); }
+    __device__ __forceinline__ uint2 span() const {
+        return make_uint2(__float_as_uint(w[2].z) & ~kGap, __float_as_uint(w[2].w));
+    }
+    __device__ __forceinline__ bool degen() const { return (__float_as_uint(w[2].z) & kGap) != 0; }
 };
 
 struct RefitTile {
@@ -1436,34 +1461,31 @@ struct RefitTile {
     int32_t hval[kRHash][6];
     uint32_t vkey[kVSet];        // distinct vertex ids of the tile's triangles
     union {
-        RefitNodes nd;           // until tiers A and B end
-        float upos[kVSet][3];    // then: the distinct vertices' positions, compacted
+        RefitNode nd[kRTile];    // internal nodes lo .. lo + 511, until tiers A and B end
+        float upos[3 * kRTile][3];  // then: the distinct vertices' positions, compacted
     };
     uint32_t chain[kTChain];     // tile-common node and its ancestors
-    uint32_t nchain, nuniq, overflow, rest;
+    uint32_t nchain, nuniq, overflow, rest, unsafe;
 };
 
-// Parent, span and candidate axes of internal node p for tiers A and B.
-__device__ __forceinline__ void refit_node(const RefitTile& R, const TreeWs& ws, const uint32_t* parents,
-                                           uint32_t lo, uint32_t p, uint32_t& parent, uint2& span, Cand& c) {
-    const uint32_t s = p - lo;
-    if (s < kRTile) {
-        parent = R.nd.parent[s];
-        span = R.nd.span[s];
-#pragma unroll
-        for (int j = 0; j < 9; ++j) c.b[j] = R.nd.b[j][s];
-        c.degen = R.nd.degen[s];
-    } else {
-        parent = parents[p];
-        span = ws.span[p];
-        c = ws.cand[p];
-    }
+// Lanes below this one in a ballot.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+__device__ __forceinline__ RefitNode refit_node(const RefitTile& R, const TreeWs& ws, const uint32_t* parents,
+                                                uint32_t lo, uint32_t p) {
+    if (p - lo < kRTile) return R.nd[p - lo];
+    RefitNode n;
+    const Cand c = ws.cand[p];
+    n.set(c.b, parents[p], ws.span[p], c.degen != 0);
+    return n;
 }
 
 // Order-preserving key of a float (same map as f2ord, without a branch).
 __device__ __forceinline__ int32_t okey(float f) {
     const int32_t i = __float_as_int(f);
-    return i ^ (int32_t)((uint32_t)(i >> 31) >> 1);
+    return i ^ ((i >> 31) & 0x7FFFFFFF);
 }
 
 // Unconditional: reading the current keys first to skip atomics made every
@@ -1480,9 +1502,37 @@ __device__ __forceinline__ void fold_global(int32_t* rk, const int32_t v[6]) {
 __device__ __forceinline__ void fold_lds(int32_t* slot, const int32_t v[6]) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        if (v[a] < slot[a]) atomicMin(&slot[a], v[a]);
-        if (v[3 + a] > slot[3 + a]) atomicMax(&slot[3 + a], v[3 + a]);
+        atomicMin(&slot[a], v[a]);
+        atomicMax(&slot[3 + a], v[3 + a]);
     }
+}
+
+// One step of fold_quads: lanes i and i ^ kBit with the same tag combine their
+// keys, and the upper one drops out (a tag of its own).
+template <int kBit, int kPerm>
+__device__ __forceinline__ void fold_quad_step(uint32_t& tag, int32_t k[6]) {
+    const bool same = (uint32_t)dpp_mov<kPerm>((int32_t)tag) == tag;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int32_t mn = min(k[a], dpp_mov<kPerm>(k[a])), mx = max(k[3 + a], dpp_mov<kPerm>(k[3 + a]));
+        k[a] = same ? mn : k[a];
+        k[3 + a] = same ? mx : k[3 + a];
+    }
+    if (same && (lane_id() & kBit)) tag = 0x80000000u | (uint32_t)lane_id();
+}
+// Keys of the lanes that hold the same node p, combined within each group of
+// four lanes.  Called by the whole wave, lanes without keys with on = false.
+// True for the lanes left to fold: where a node's leaves are consecutive lanes,
+// one or two of a group.  The LDS atomics of one wave on one node are made one
+// lane after the other and bound the tier; a lane's key reads before them, to
+// skip some, took as long (both on 1M triangles, with the reads 437 us the
+// transform, all lanes' atomics 434, groups of four 429, of sixteen 433).
+__device__ __forceinline__ bool fold_quads(bool on, uint32_t p, int32_t k[6]) {
+    const uint32_t mine = on ? p : 0x80000000u | (uint32_t)lane_id();
+    uint32_t tag = mine;
+    fold_quad_step<1, 0xB1>(tag, k);  // quad_perm [1,0,3,2]
+    fold_quad_step<2, 0x4E>(tag, k);  // quad_perm [2,3,0,1]
+    return on && tag == mine;
 }
 
 __device__ __forceinline__ void fold_tile(RefitTile& R, int32_t* range, uint32_t lo, uint32_t p, const int32_t k[6]) {
@@ -1510,10 +1560,10 @@ __device__ __forceinline__ void fold_tile(RefitTile& R, int32_t* range, uint32_t
 // never NaN and that is the integer min / max of the keys (up to the sign of
 // a zero).  Otherwise the compare-and-select chain is evaluated as written,
 // and a NaN result gives the neutral key, i.e. never enters the range.
-__device__ __forceinline__ void tri_keys(const Cand& c, f3 v0, f3 v1, f3 v2, bool fin, int32_t k[6]) {
+__device__ __forceinline__ void tri_keys(const f3 axes[3], f3 v0, f3 v1, f3 v2, bool fin, int32_t k[6]) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const f3 b = f3{c.b[3 * a], c.b[3 * a + 1], c.b[3 * a + 2]};
+        const f3 b = axes[a];
         const float d0 = dot3(v0, b), d1 = dot3(v1, b), d2 = dot3(v2, b);
         if (fin) {
             const int32_t k0 = okey(d0), k1 = okey(d1), k2 = okey(d2);
@@ -1550,6 +1600,11 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
     const uint32_t I = N - 1, t = threadIdx.x;
     const uint32_t lo = blockIdx.x * kRTile;
     const uint32_t thi = min(lo + kRTile, N) - 1;  // last leaf position of the tile
+    const uint32_t pos = lo + t;
+    const bool valid = pos < N;
+    // the chain leaf -> face -> vertices starts first: the tile's set-up runs under its latency
+    const uint32_t f = valid ? nodes[I + pos].u.primitivesOffset : kInvalid;
+    const uint32_t leaf_parent = valid ? parents[I + pos] : kInvalid;
 #pragma unroll
     for (int a = 0; a < 3; ++a) { R.tk[t][a] = kKeyHi; R.tk[t][3 + a] = kKeyLo; }
     if (t < kRHash) {
@@ -1558,14 +1613,9 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
         for (int a = 0; a < 3; ++a) { R.hval[t][a] = kKeyHi; R.hval[t][3 + a] = kKeyLo; }
     }
     for (uint32_t h = t; h < kVSet; h += kRTile) R.vkey[h] = kEmpty;
-    if (lo + t < I) {  // the tile's own index range, for tiers A and B
-        const uint32_t node = lo + t;
-        const Cand c = ws.cand[node];
-#pragma unroll
-        for (int j = 0; j < 9; ++j) R.nd.b[j][t] = c.b[j];
-        R.nd.degen[t] = (uint8_t)(c.degen != 0);
-        R.nd.span[t] = ws.span[node];
-        R.nd.parent[t] = parents[node];
+    if (pos < I) {  // the tile's own index range, for tiers A and B
+        const Cand c = ws.cand[pos];
+        R.nd[t].set(c.b, parents[pos], ws.span[pos], c.degen != 0);
     }
     if (t == 0) {
         bad = *ws.error;  // one read per workgroup: the exit is uniform
@@ -1574,81 +1624,101 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
         R.rest = m.y;
         R.nuniq = 0;
         R.overflow = 0;
+        R.unsafe = 0;
     }
     if (t < kTChain) R.chain[t] = ws.tchain[(size_t)blockIdx.x * kTChain + t];  // entries past the count unused
+    kr_uvec4 face = {};
+    if (f < N) face = F[f];  // (a face id out of range set the error, and the workgroup ends below)
     __syncthreads();
     if (bad != 0) return;
 
-    const uint32_t pos = lo + t;
     const uint32_t wlo = pos - (uint32_t)lane_id();
     const uint32_t whi = min(wlo + kWave - 1, N - 1);
-    const bool valid = pos < N;
-    f3 v0 = f3{0, 0, 0}, v1 = v0, v2 = v0;
+    f3 v[3] = {f3{0, 0, 0}, f3{0, 0, 0}, f3{0, 0, 0}};
     bool fin = true;
+    uint32_t own = 0;  // bit j: the tile's distinct vertices list vertex j from this lane
     if (valid) {
-        const kr_uvec4 face = F[nodes[I + pos].u.primitivesOffset];
-        v0 = ldv(V, face.x);
-        v1 = ldv(V, face.y);
-        v2 = ldv(V, face.z);
-        fin = finite3(v0) && finite3(v1) && finite3(v2);
-        // the tile-wide pass projects vertices, not triangles: a tile with a
-        // non-finite vertex keeps the per-triangle rule up to the root
-        if (!fin) R.overflow = 1;
         const uint32_t vid[3] = {face.x, face.y, face.z};
 #pragma unroll
+        for (int j = 0; j < 3; ++j) v[j] = ldv(V, vid[j]);
+        uint32_t h[3], key[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            h[j] = (vid[j] * 2654435761u) >> 21;
+            key[j] = R.vkey[h[j]];
+        }
+#pragma unroll
         for (int j = 0; j < 3; ++j) {  // distinct vertex ids of the tile
-            uint32_t h = (vid[j] * 2654435761u) >> 21;
             bool placed = false;
             for (int probe = 0; probe < 32 && !placed; ++probe) {
-                uint32_t key = R.vkey[h];
-                if (key == kEmpty) key = atomicCAS(&R.vkey[h], kEmpty, vid[j]);
-                placed = key == kEmpty || key == vid[j];
-                h = (h + 1) & (kVSet - 1);
+                if (probe != 0) {
+                    h[j] = (h[j] + 1) & (kVSet - 1);
+                    key[j] = R.vkey[h[j]];
+                }
+                if (key[j] == kEmpty) {
+                    key[j] = atomicCAS(&R.vkey[h[j]], kEmpty, vid[j]);
+                    if (key[j] == kEmpty) own |= 1u << j;
+                }
+                placed = key[j] == kEmpty || key[j] == vid[j];
             }
             if (!placed) R.overflow = 1;
         }
+        fin = finite3(v[0]) && finite3(v[1]) && finite3(v[2]);
+        // the tile-wide pass projects vertices, not triangles: a tile with a
+        // non-finite vertex keeps the per-triangle rule up to the root
+        if (!fin) R.overflow = 1;
+        if (!sane_points(v, 3)) R.unsafe = 1;
     }
+    // places of the lane's own vertices in the list: one count per wave
+    const uint64_t o0 = __ballot(own & 1u), o1 = __ballot(own & 2u), o2 = __ballot(own & 4u);
+    uint32_t u0 = 0;
+    if (lane_id() == 0) u0 = atomicAdd(&R.nuniq, (uint32_t)(__popcll(o0) + __popcll(o1) + __popcll(o2)));
+    u0 = __builtin_amdgcn_readfirstlane(u0) + lanes_below(o0) + lanes_below(o1) + lanes_below(o2);
     __syncthreads();
     // tier C needs the tile-common node (chain[0]) and a vertex set that fit
     const bool tile_pass = R.overflow == 0 && R.nchain != 0;
     const uint32_t q0 = tile_pass ? R.chain[0] : kInvalid;
 
     if (wlo < N) {  // wave-uniform
-        // tier A
-        uint32_t common = kInvalid;
-        if (valid) {
-            uint32_t p = parents[I + pos];
-            for (uint32_t step = 0; p != kInvalid && p < I && step < N; ++step) {
-                uint32_t pp;
-                uint2 sp;
-                Cand c;
-                refit_node(R, ws, parents, lo, p, pp, sp, c);
-                if (holds(sp, wlo, whi)) { common = p; break; }
-                if (!c.degen) {
-                    int32_t k[6];
-                    tri_keys(c, v0, v1, v2, fin, k);
-                    fold_tile(R, ws.range, lo, p, k);
-                }
-                p = pp;
+        // tier A: the next node is read while this one's keys are made
+        uint32_t common = kInvalid, p = leaf_parent;
+        bool on = valid && p < I;
+        RefitNode c = {};
+        if (on) c = refit_node(R, ws, parents, lo, p);
+        for (uint32_t step = 0; step < N && __ballot(on) != 0; ++step) {  // uniform
+            if (on && holds(c.span(), wlo, whi)) {
+                common = p;
+                on = false;
             }
+            const uint32_t pp = on ? c.parent() : kInvalid;
+            RefitNode n = c;
+            if (pp < I) n = refit_node(R, ws, parents, lo, pp);
+            const f3 axes[3] = {c.axis(0), c.axis(1), c.axis(2)};
+            int32_t k[6];
+            tri_keys(axes, v[0], v[1], v[2], fin, k);
+            if (fold_quads(on && !c.degen(), p, k)) fold_tile(R, ws.range, lo, p, k);
+            on = pp < I;
+            c = n;
+            p = pp;
         }
         // tier B; lane 0 is valid (wlo < N) and a well-formed tree gives
         // every valid lane the same node
         const uint32_t c0 = __builtin_amdgcn_readfirstlane(common);
         if (__ballot(valid && common != c0) != 0) {
             if (lane_id() == 0) atomicOr(ws.error, 2u);
-        } else {
+        } else if (c0 < I && c0 != q0) {  // tier C takes q0 and above
             uint32_t q = c0;
-            for (uint32_t step = 0; q != kInvalid && q < I && step < N; ++step) {  // uniform
-                uint32_t qp;
-                uint2 sp;
-                Cand c;
-                if (q == q0) break;  // tier C takes q and above
-                refit_node(R, ws, parents, lo, q, qp, sp, c);
-                if (!c.degen) {
+            RefitNode c = refit_node(R, ws, parents, lo, q);
+            for (uint32_t step = 0; step < N; ++step) {  // uniform
+                const uint32_t qp = __builtin_amdgcn_readfirstlane(c.parent());
+                const bool last = qp >= I || qp == q0;
+                RefitNode n = c;
+                if (!last) n = refit_node(R, ws, parents, lo, qp);
+                if (!c.degen()) {
+                    const f3 axes[3] = {c.axis(0), c.axis(1), c.axis(2)};
                     int32_t k[6];
                     if (valid) {
-                        tri_keys(c, v0, v1, v2, fin, k);
+                        tri_keys(axes, v[0], v[1], v[2], fin, k);
                     } else {
 #pragma unroll
                         for (int a = 0; a < 3; ++a) { k[a] = kKeyHi; k[3 + a] = kKeyLo; }
@@ -1656,22 +1726,23 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
                     wave_keys(k);
                     if (lane_id() == 0) fold_tile(R, ws.range, lo, q, k);
                 }
-                q = __builtin_amdgcn_readfirstlane(qp);
+                if (last) break;
+                q = qp;
+                c = n;
             }
         }
     }
     __syncthreads();
 
     if (tile_pass) {
-        for (uint32_t h = t; h < kVSet; h += kRTile) {
-            const uint32_t id = R.vkey[h];
-            if (id == kEmpty) continue;
-            const uint32_t u = atomicAdd(&R.nuniq, 1u);
-            const f3 p = ldv(V, id);
-            R.upos[u][0] = p.x;
-            R.upos[u][1] = p.y;
-            R.upos[u][2] = p.z;
-        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (own & (1u << j)) {
+                R.upos[u0][0] = v[j].x;
+                R.upos[u0][1] = v[j].y;
+                R.upos[u0][2] = v[j].z;
+                ++u0;
+            }
         __syncthreads();
         // tier C over the distinct vertices; each wave reads the axes and
         // current keys of its next ancestor while it works on this one (the
@@ -1736,7 +1807,9 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
                 if (!c.degen) {
                     int32_t k[6];
                     if (valid) {
-                        tri_keys(c, v0, v1, v2, fin, k);
+                        const f3 axes[3] = {f3{c.b[0], c.b[1], c.b[2]}, f3{c.b[3], c.b[4], c.b[5]},
+                                            f3{c.b[6], c.b[7], c.b[8]}};
+                        tri_keys(axes, v[0], v[1], v[2], fin, k);
                     } else {
 #pragma unroll
                         for (int a = 0; a < 3; ++a) { k[a] = kKeyHi; k[3 + a] = kKeyLo; }
@@ -1749,23 +1822,29 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
         }
     }
     __syncthreads();
-    // fold the tile's LDS keys into global memory.  A node whose leaves all
-    // lie in this tile has no contributor outside this workgroup, and within
-    // it only the LDS slot (tier C, which folds with atomics, never takes
-    // such a node except the tile-common node, whose span is the tile): its
-    // keys are merged with a plain read-modify-write.  The others are merged
-    // with atomics.
+    // Write the tile's LDS keys to global memory.  A node whose leaves all lie
+    // in this tile has no contributor outside this workgroup, and within it
+    // only the LDS slot (tier C, which folds with atomics, never takes such a
+    // node except the tile-common node, whose span is the tile): its keys
+    // replace the candidate search's range, which came from some of the same
+    // vertices by the same dot products.  Where the tile has a non-finite or
+    // huge vertex that range may hold more (the search's reference mode), and
+    // the keys are merged into it; the other nodes' are merged with atomics.
     if (lo + t < I && (R.tk[t][0] != kKeyHi || R.tk[t][3] != kKeyLo)) {
         const uint32_t node = lo + t;
         const uint2 sp = ws.span[node];
         int32_t* rk = &ws.range[(size_t)node * 6];
         const bool chain_node = node == q0;
         if (sp.x >= lo && span_hi(sp) <= thi && !chain_node) {
+            int32_t k[6];
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                rk[a] = min(rk[a], R.tk[t][a]);
-                rk[3 + a] = max(rk[3 + a], R.tk[t][3 + a]);
+            for (int a = 0; a < 6; ++a) k[a] = R.tk[t][a];
+            if (R.unsafe) {
+#pragma unroll
+                for (int a = 0; a < 3; ++a) { k[a] = min(rk[a], k[a]); k[3 + a] = max(rk[3 + a], k[3 + a]); }
             }
+#pragma unroll
+            for (int a = 0; a < 6; ++a) rk[a] = k[a];
         } else {
             fold_global(rk, R.tk[t]);
         }
