@@ -64,26 +64,52 @@ __global__ void lbvh_init(const kr_vec3* V, uint32_t nf, LbvhWs ws) {
 }
 
 constexpr int kBoxThreads = 1024;
+constexpr int kBoxGroups = 2 * kBoxThreads / 256, kBoxGroupWaves = 256 / kWave;
 
 __global__ __launch_bounds__(kBoxThreads) void lbvh_centroid_box(const kr_vec3* V, const kr_uvec4* F, uint32_t nf,
                                                          LbvhWs ws) {
-    __shared__ float sh[6][kBoxThreads / kWave];
+    __shared__ float sh[6][2 * kBoxThreads / kWave], group[6][kBoxGroups];
     const float INF = FLT_MAX * 2.0f;
-    float mn[3] = {INF, INF, INF}, mx[3] = {-INF, -INF, -INF};
-    for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
-        f3 c = box_center(tri_box(V, F[f]));
-        mn[0] = fminf(mn[0], c.x); mn[1] = fminf(mn[1], c.y); mn[2] = fminf(mn[2], c.z);
-        mx[0] = fmaxf(mx[0], c.x); mx[1] = fmaxf(mx[1], c.y); mx[2] = fmaxf(mx[2], c.z);
+    float mn[2][3] = {{INF, INF, INF}, {INF, INF, INF}}, mx[2][3] = {{-INF, -INF, -INF}, {-INF, -INF, -INF}};
+    const uint32_t stride = gridDim.x * kBoxThreads;
+    for (uint32_t f0 = blockIdx.x * kBoxThreads + threadIdx.x; f0 < nf; f0 += 2 * stride) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t f = f0 + h * stride;
+            if (f >= nf) continue;
+            const f3 c = box_center(tri_box(V, F[f]));
+            mn[h][0] = fminf(mn[h][0], c.x); mn[h][1] = fminf(mn[h][1], c.y); mn[h][2] = fminf(mn[h][2], c.z);
+            mx[h][0] = fmaxf(mx[h][0], c.x); mx[h][1] = fmaxf(mx[h][1], c.y); mx[h][2] = fmaxf(mx[h][2], c.z);
+        }
     }
-    for (int k = 0; k < 3; ++k) { mn[k] = wave_min(mn[k]); mx[k] = wave_max(mx[k]); }
-    if (lane_id() == 0)
-        for (int k = 0; k < 3; ++k) { sh[k][wave_id()] = mn[k]; sh[3 + k][wave_id()] = mx[k]; }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        for (int k = 0; k < 3; ++k) {
+            const float a = wave_min(mn[h][k]), b = wave_max(mx[h][k]);
+            if (lane_id() == 0) {
+                sh[k][h * (kBoxThreads / kWave) + wave_id()] = a;
+                sh[3 + k][h * (kBoxThreads / kWave) + wave_id()] = b;
+            }
+        }
+    __syncthreads();
+    // The bounds of each 256 threads, of a thread's first, third, ... and of its
+    // second, fourth, ... face: a bound that is not finite is left out (no
+    // faces, or one of infinite extent among them, whose fellows' bound is then
+    // left out too).  Up to 2^19 faces these are 256 consecutive faces.
+    if (threadIdx.x < 6 * kBoxGroups) {
+        const int k = threadIdx.x % 6, g = threadIdx.x / 6;
+        const float* w = &sh[k][g * kBoxGroupWaves];
+        float a = w[0];
+        for (int i = 1; i < kBoxGroupWaves; ++i) a = k < 3 ? fminf(a, w[i]) : fmaxf(a, w[i]);
+        if (!(a != INF && a != -INF)) a = k < 3 ? INF : -INF;
+        group[k][g] = a;
+    }
     __syncthreads();
     if (threadIdx.x < 6) {
         const int k = threadIdx.x;
-        float a = sh[k][0];
-        for (int w = 1; w < kBoxThreads / kWave; ++w) a = k < 3 ? fminf(a, sh[k][w]) : fmaxf(a, sh[k][w]);
-        if (a == a && a != INF && a != -INF) {
+        float a = group[k][0];
+        for (int g = 1; g < kBoxGroups; ++g) a = k < 3 ? fminf(a, group[k][g]) : fmaxf(a, group[k][g]);
+        if (a != INF && a != -INF) {
             // filtered: only a workgroup that improves the current bound
             // issues the atomic (thousands of same-address atomics serialise:
             // 2048 workgroups took 27 us, 256 take 10)

@@ -210,3 +210,31 @@ def test_obb_tree_huge_coordinates(torch, oracle_lib, kind):
     go, gm = obbs.cpu().numpy(), mats.cpu().numpy()
     bad = [v for v in range(len(go)) if not (same(go[v], eo[v]) and same(gm[v], em[v]))]
     assert not bad, (bad[:10], go[bad[0]], eo[bad[0]])
+
+
+# A face of infinite extent leaves the bound of its 256 faces out of the centroid box (and only theirs): leaf order
+# against Morton codes made here.
+@pytest.mark.parametrize("nf", [1024, 1600, 5120])
+def test_lbvh_infinite_face_drops_its_group(torch, nf):
+    rng = np.random.default_rng(nf)
+    V = (rng.uniform(-1, 1, (nf, 1, 3)) + rng.uniform(-0.02, 0.02, (nf, 3, 3))).reshape(-1, 3).astype(np.float32)
+    V[256 * 3 * 2:256 * 3 * 3, 1] += 3  # the third group's faces lie above the others
+    F = np.zeros((nf, 4), dtype=np.uint32)
+    F[:, :3] = np.arange(3 * nf).reshape(nf, 3)
+    V[3 * (256 * 2 + 5), 1] = np.inf
+    got = ops.lbvh_build(torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda())
+    torch.cuda.synchronize()
+    half = np.float32(0.5)
+    bmin, bmax = V.reshape(nf, 3, 3).min(1), V.reshape(nf, 3, 3).max(1)
+    c = (bmin + bmax) * half
+    lo, hi = np.full(3, np.inf, np.float32), np.full(3, -np.inf, np.float32)
+    for g in range(0, nf, 256):
+        a, b = c[g:g + 256].min(0), c[g:g + 256].max(0)
+        lo = np.where(np.isfinite(a), np.minimum(lo, a), lo)
+        hi = np.where(np.isfinite(b), np.maximum(hi, b), hi)
+    if nf % 256:
+        lo, hi = np.minimum(lo, V[0]), np.maximum(hi, V[0])
+    u = ((bmin - lo) + (bmax - lo)) * half / (hi - lo)
+    q = np.minimum(np.maximum(u * np.float32(1024), 0), 1023).astype(np.int64)
+    code = sum(((q[:, a] >> b) & 1) << (3 * b + 2 - a) for a in range(3) for b in range(10))
+    assert np.array_equal(ops.nodes_to_numpy(got["nodes"])["a"][nf - 1:], np.argsort(code, kind="stable"))
