@@ -425,22 +425,29 @@ __device__ __forceinline__ bool leaf_kdop_global(const kr_bvh_node* nodes, const
 // [w*kTile, (w+1)*kTile) and the internal nodes with the same indices (for a
 // Karras-ordered tree these are the internal nodes whose leaves lie in the
 // range).  The workgroup first loads the tile's topology into LDS (children
-// and parents of its internal nodes, parents and vertex ids of its leaves)
-// and checks that every child of its internal nodes points back to it.
+// and parents of its internal nodes, vertex ids of its leaves) and checks that every child of its internal nodes points back to it.
 // Then one lane per leaf climbs: at a parent in the tile the arrival is
 // counted in LDS, the first child stops and the second merges, reading the
 // sibling's k-DOP from LDS (internal node of the tile, or a leaf's k-DOP
 // left in the parent's slot), recomputing it (a leaf that left none) or
 // loading it (node completed outside the tile's index range).  At the
 // first level two leaf siblings in one wave merge without an arrival count:
-// the left one takes the right one's k-DOP by lane shuffles.  Parents outside the tile use the global arrival word with
-// the workgroup's tag; such a parent is deferred to climb_upper when its
+// the left one takes the right one's k-DOP by lane shuffles.  Parents outside
+// the tile use the global arrival word with the workgroup's tag; such a parent is deferred to climb_upper when its
 // children finished in different workgroups.  Finally tile nodes reached by
 // one child only are folded into the global arrival words, and the k-DOPs,
 // spans and arrival words of tile nodes completed here are written back
 // contiguously.  The merge keeps the left child's extreme on ties.  Last,
 // the tile's leaf boxes (transforms.cu:803-834) from the triangles each lane
 // loaded, staged in the same LDS and written back contiguously.
+//
+// Bound by latency at two workgroups of 78 KB per CU: of a workgroup's 46 us on
+// a 1M-leaf tree the loads take 7, the climb 16 (about 13 levels), the k-DOPs'
+// write-back 8, the leaf boxes 13.  1M leaves 130 us (2.6 TB/s written), 2M 255.
+// A half-reached node's count is looked at after the write-back and its leaf
+// child's k-DOP comes from LDS (before, from the vertices again): transforms of
+// 2M leaves 853 -> 839 us, 3.8M 1625 -> 1611.  Eight lanes per node above the
+// first level, as in climb_upper, took 186 us for 1M.
 constexpr uint32_t kTile = 512;  // leaves per workgroup
 
 struct ClimbTile {
@@ -451,7 +458,6 @@ struct ClimbTile {
     uint32_t arrive[kTile];     // arrivals at internal node lo + s from this workgroup
     uint2 kids[kTile];          // children of internal node lo + s
     uint32_t par_int[kTile];    // parent of internal node lo + s
-    uint32_t par_leaf[kTile];   // parent of the leaf at position lo + s
 };
 union ClimbLds {
     ClimbTile L;
@@ -480,12 +486,30 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
     Kdop k = {};
     bool climbing = false;
     f3 v0 = f3{0, 0, 0}, v1 = v0, v2 = v0;  // the lane's triangle, for its leaf box
+    // the tile's internal nodes' loads go out before the chain leaf -> face ->
+    // vertices waits
+    uint32_t l = 0, r = 0, par = kInvalid, f = kInvalid, leaf_parent = kInvalid;
+    uint64_t slot = 0;
+    if (pos < I) {
+        l = nodes[pos].u.children.left;
+        r = nodes[pos].u.children.right;
+        par = parents[pos];
+        slot = ws.visit[pos];
+    }
     if (pos < N) {
-        const uint32_t leaf = I + pos;
-        L.par_leaf[t] = parents[leaf];
-        const uint32_t f = nodes[leaf].u.primitivesOffset;
+        leaf_parent = parents[I + pos];
+        f = nodes[I + pos].u.primitivesOffset;
+    }
+    kr_uvec4 face = {};
+    if (f < N) face = F[f];
+    if (pos < I) {
+        L.kids[t] = make_uint2(l, r);
+        L.par_int[t] = par;
+        // (an unused slot of a batch has no children: no check)
+        if ((l >= total || r >= total || parents[l] != pos || parents[r] != pos) && !hole(slot)) atomicOr(ws.error, 2u);
+    }
+    if (pos < N) {
         if (f < N) {
-            const kr_uvec4 face = F[f];
             const uint32_t vid[3] = {face.x, face.y, face.z};
             L.lid[t][0] = vid[0];
             L.lid[t][1] = vid[1];
@@ -500,27 +524,19 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
             atomicOr(ws.error, 4u);  // faces has one entry per leaf
         }
     }
-    if (pos < I) {
-        const uint32_t l = nodes[pos].u.children.left, r = nodes[pos].u.children.right;
-        L.kids[t] = make_uint2(l, r);
-        L.par_int[t] = parents[pos];
-        // (an unused slot of a batch has no children: no check)
-        if ((l >= total || r >= total || parents[l] != pos || parents[r] != pos) && !hole(ws.visit[pos]))
-            atomicOr(ws.error, 2u);
-    }
     L.arrive[t] = 0;
     __syncthreads();
 
     // First level, all lanes together: two leaf siblings in one wave are
     // merged by the left one (the right one's k-DOP comes by a lane shuffle)
     // without an arrival count.  Any other leaf with a parent in the tile
-    // leaves its k-DOP in the parent's LDS slot before it arrives (when its
-    // sibling is internal, or it is the left one of two leaves), so that a
-    // sibling arriving second reads it from LDS instead of recomputing it.
+    // leaves its k-DOP in the parent's LDS slot before it arrives (unless it is
+    // the right one of two leaves of the tile), so that a sibling arriving
+    // second reads it from LDS instead of recomputing it.
     uint32_t cur = I + pos;
     uint2 span = leaf_span(pos);
     uint32_t count = 1;
-    uint32_t p = L.par_leaf[t];
+    uint32_t p = leaf_parent;
     bool climb = climbing;  // the lane climbs on past the first level
     {
         const uint64_t climbers = __ballot(climbing);
@@ -537,7 +553,7 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
                     pair_right = !am_left;
                     src = sl;
                 } else {
-                    stash = sib < I || am_left;
+                    stash = sib < I || am_left || sib - I - lo >= kTile;
                 }
             }
         }
@@ -658,25 +674,26 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
     }
     __syncthreads();
 
-    // tile nodes reached by one child: publish a tile-leaf child, then the
-    // global arrival (the other child finishes in another workgroup)
-    if (pos < I && L.arrive[t] == 1u) {
+    // Tile nodes reached by one child: publish a tile-leaf child (its k-DOP
+    // is in the node's slot), then the global arrival: the other child
+    // finishes in another workgroup.  What the count held is looked at last.
+    uint64_t old = 0;
+    const bool half = pos < I && L.arrive[t] == 1u;
+    if (half) {
         const uint2 kc = L.kids[t];
         const uint32_t c2[2] = {kc.x, kc.y};
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const uint32_t ss = c2[j] - I - lo;
             if (c2[j] >= I && c2[j] < total && ss < kTile && L.lid[ss][0] != kInvalid) {
-                Kdop o;
-                tile_leaf_kdop(L, V, ss, o);
-                kdop_store(ws.kdop, c2[j], o);
+                float4* d = ws.kdop + (size_t)c2[j] * 7;
+#pragma unroll
+                for (int q = 0; q < 7; ++q) d[q] = L.kd[t][q];
                 ws.span[c2[j]] = leaf_span(c2[j] - I);
             }
         }
-        const uint64_t old = __hip_atomic_fetch_add(&ws.visit[pos], ((uint64_t)tag << 32) | 1ull,
-                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if ((uint32_t)old == 1u) defer(ws, pos, I);
-        else if ((uint32_t)old != 0u) atomicOr(ws.error, 2u);
+        old = __hip_atomic_fetch_add(&ws.visit[pos], ((uint64_t)tag << 32) | 1ull, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     // write back the tile nodes completed here
     const uint32_t nin = lo < I ? min(kTile, I - lo) : 0u;
@@ -697,6 +714,10 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
     }
     __syncthreads();
     stage_flush(U.st, obbs, mats, (size_t)I + lo, min(kTile, N - lo), bm);
+    if (half) {
+        if ((uint32_t)old == 1u) defer(ws, pos, I);
+        else if ((uint32_t)old != 0u) atomicOr(ws.error, 2u);
+    }
 }
 
 // The rest of the bottom-up k-DOP pass: the nodes the tile climb deferred (both
