@@ -37,6 +37,13 @@
 //
 // Data per internal node visit: metadata 8 B + two 48 B matrices; per
 // triangle: face 16 B + three 12 B vertices.
+//
+// Bound by VALU issue (373 instructions an iteration at 5 waves per SIMD) and
+// the long rays: on 1M rays (60 steps on average, 600 the longest) a wave has
+// 56 lanes busy until no ray is left to take, 14 in its last iterations.
+// Merging a workgroup's waves then (rays handed over through LDS) and an exact
+// entry test for flat boxes by axis pairs gained nothing: the first lengthens
+// the longest rays' iterations, the second costs registers.
 #include "common.hpp"
 #include "traverse.hpp"
 
@@ -343,7 +350,8 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
     // a leaf whose primitives [k, end) remain to be tested.
     uint32_t ray = 0, hit = 0, steps = 0;
     int32_t hit_slot = 0;
-    bool busy = false, exhausted = false, aborted = false;
+    bool busy = false, done = false, aborted = false;
+    bool exhausted = false;  // wave-uniform
     f3 org{0.0f, 0.0f, 0.0f}, dir{0.0f, 0.0f, 0.0f};
     float hitT = 0.0f, bx = 0.0f, by = 0.0f;
     int sp = 0;
@@ -357,11 +365,35 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
                                   : deep[(size_t)(s - kTravLdsSlots - 1) * stride];
     };
 
+    // A finished ray's record.  The lanes that wait for a refill write theirs
+    // together: at each ray's end it ran for one or two lanes at a time, in a
+    // third of all iterations, with two dependent loads (1M camera rays 1740 us
+    // then, 1670 now, random rays 1563 and 1500).
+    auto finish = [&]() {
+        kr_intersection o;
+        o.instance = aborted ? kTravAborted : 0u;
+        o.primitive = hit;
+        if (hit == 0xFFFFFFFFu) {
+            o.geom_normal = kr_vec3{dir.x, dir.y, dir.z};
+            o.barys = kr_vec2{0.5f, 0.5f};
+        } else {
+            f3 va, vb, vc;
+            tree.hit_vertices(hit, hit_slot, va, vb, vc);
+            const f3 nrm = vm::normalize(vm::cross(sub3(vb, va), sub3(vc, va)));
+            o.geom_normal = kr_vec3{nrm.x, nrm.y, nrm.z};
+            o.barys = kr_vec2{bx, by};
+        }
+        a.out[ray] = o;
+        done = false;
+    };
+
     for (;;) {
-        const bool wants = !busy && !exhausted;
+        const bool wants = !busy;
         const uint64_t idle = __ballot(wants);
         const int nidle = __popcll(idle);
-        if (nidle >= kTravRefill || (nidle > 0 && __ballot(busy) == 0)) {  // wave-uniform
+        if (nidle == kWave || (nidle >= kTravRefill && !exhausted)) {  // wave-uniform
+            if (done) finish();
+            if (exhausted) break;
             uint32_t base = 0;
             if (lane == 0) base = atomicAdd(a.counter, (uint32_t)nidle);
             base = (uint32_t)__shfl((int)base, 0, kWave);
@@ -380,12 +412,11 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
                     aborted = false;
                     sp = 0;
                     cur = 0;
-                } else {
-                    exhausted = true;
                 }
             }
+            exhausted = a.n - min(base, a.n) <= (uint32_t)nidle;  // the last rays are taken
+            if (__ballot(busy) == 0) break;
         }
-        if (__ballot(busy) == 0) break;  // every lane exhausted
 
         // One step per lane: an internal node or one primitive of a leaf.
         // (Holding triangle steps back until more lanes want one, or
@@ -477,22 +508,9 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
             }
         }
 
-        if (busy && cur == kTravSentinel) {  // ray finished: write its record, free the lane
-            kr_intersection o;
-            o.instance = aborted ? kTravAborted : 0u;
-            o.primitive = hit;
-            if (hit == 0xFFFFFFFFu) {
-                o.geom_normal = kr_vec3{dir.x, dir.y, dir.z};
-                o.barys = kr_vec2{0.5f, 0.5f};
-            } else {
-                f3 va, vb, vc;
-                tree.hit_vertices(hit, hit_slot, va, vb, vc);
-                const f3 nrm = vm::normalize(vm::cross(sub3(vb, va), sub3(vc, va)));
-                o.geom_normal = kr_vec3{nrm.x, nrm.y, nrm.z};
-                o.barys = kr_vec2{bx, by};
-            }
-            a.out[ray] = o;
+        if (busy && cur == kTravSentinel) {  // ray finished: free the lane
             busy = false;
+            done = true;
         }
     }
 }

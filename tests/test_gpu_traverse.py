@@ -208,3 +208,21 @@ def test_empty_and_all_miss(torch, oracle_lib):
     got = ops.isects_to_numpy(out)
     assert (got["primitive"] == MISS).all()
     assert np.array_equal(got["normal"], rays["direction"])
+
+
+# ray counts around a wave, its refill (16 idle lanes) and the lanes of the whole grid (524288): records are written when
+# lanes wait for a refill and at a wave's end
+@pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 1000, 600001])
+def test_ray_count_edges(torch, oracle_lib, n):
+    say(f"[traverse] {n} rays")
+    V, F = synth.icosphere(6, seed=4)
+    Vd, Fd, t, mats = device_tree(torch, V, F, "lbvh")
+    packed = ops.soa_pack(t["nodes"], mats)
+    rays = synth.random_rays(V, n, seed=n)
+    out = ops.soa_intersect(packed, Vd, Fd, rays)
+    out_r = ops.records_intersect(ops.records_pack(t["nodes"], mats, Vd, Fd), rays)
+    torch.cuda.synchronize()
+    eL, eR, em = oracle_lib.obvh_pack(ops.nodes_to_numpy(t["nodes"]), mats.cpu().numpy())
+    exp = oracle_lib.obvh_intersect(eL, eR, em, V, F, None, rays, threads=8)
+    same_isects(ops.isects_to_numpy(out), exp)
+    assert np.array_equal(out_r.cpu().numpy(), out.cpu().numpy())
