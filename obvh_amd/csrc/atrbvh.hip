@@ -77,8 +77,12 @@ __device__ __forceinline__ uint64_t discretize21(float x) {
 
 // ----------------------------------------------------------- build --
 
-__global__ void atr_init(AtrWs ws, uint32_t nf) {
+__device__ __forceinline__ void pass_clear(const AtrWs& ws, uint32_t nf) {
     phase_clear(ws.ph, nf);
+    if (blockIdx.x == 0 && threadIdx.x < 64) ws.top[threadIdx.x] = 0;
+}
+__global__ void atr_init(AtrWs ws, uint32_t nf) {
+    pass_clear(ws, nf);
     if (blockIdx.x == 0 && threadIdx.x < 6) ws.sbox[threadIdx.x] = threadIdx.x < 3 ? 0x7FFFFFFF : (int32_t)0x80000000;
 }
 
@@ -243,14 +247,14 @@ __global__ __launch_bounds__(kTreeThreads) void atr_tree(const kr_vec3* V, const
     AtrRec(ws, ri).set_parent((uint32_t)i);
 }
 
-__global__ void atr_clear(AtrWs ws, uint32_t nf) { phase_clear(ws.ph, nf); }
+__global__ void atr_clear(AtrWs ws, uint32_t nf) { pass_clear(ws, nf); }
 
 // ------------------------------------------------------- optimiser --
 //
 // A treelet is a chain of dependent steps (find the largest leaf, read its
 // children, again; find the closest pair, merge, again), so a pass is bound
 // by latency: tree levels x time per treelet (a 200 K-triangle hairball has
-// 24 levels of treelet roots; the phases' longest paths add up to 47).  Hence
+// 24 levels of treelet roots).  Hence
 //  - one half-wave (32 lanes, as the reference's warps) per treelet and per
 //    path to the root: the lanes climb alone below the first treelet roots,
 //    which go to a ready list; the half-waves of the workgroup then take
@@ -264,8 +268,29 @@ __global__ void atr_clear(AtrWs ws, uint32_t nf) { phase_clear(ws.ph, nf); }
 //    expansion;
 //  - tournaments as integer DPP minima and a ballot instead of shuffle
 //    rounds, boxes in LDS, distances in registers.
-// 200 K-triangle hairball, treelet size 9, 2 passes: 5529 -> 930 us; a treelet
+// 200 K-triangle hairball, treelet size 9, 2 passes: 5529 -> 790 us (930 with
+// the top in two launches of 8192-leaf workgroups and one workgroup); a treelet
 // takes about 20 K cycles (5 K reading, 4 K forming, 10 K merging).
+
+// The top pass (everything above the chunks) runs on one XCD, whose L2 all its
+// CUs share: a half-wave that completes a node waits until its records are in
+// the L2, counts its arrival, and the one that arrives second drops its CU's L1
+// and goes on with the parent.  So the passes' paths join into one (24 treelets
+// of a 200 K hairball, where 512-, 8192- and all-leaf workgroups had 47 in a
+// row), and reads stay L2 hits (past the L2, for all XCDs, a trip takes twice as
+// long, four of them a treelet).  The grid covers every CU of the chip; the
+// first workgroup to arrive names the XCD, those of the others end.  Any one
+// workgroup would do all the work.
+constexpr int kXccId = 20 | (4 - 1) << 11;  // s_getreg: XCC_ID, 4 bits
+constexpr int kTopNext = 32;  // of ws.top: entries taken ([0]: the XCD, plus one); a cache line of its own
+constexpr int kTopThreads = 512;      // 16 half-waves per CU (8 take the same time)
+constexpr uint32_t kTopBlocks = 256;  // a workgroup per CU of every XCD
+// From this many leaves on, 8192-leaf workgroups on all XCDs come between: the
+// roots are then more than one XCD's 512 half-waves are quick with.  Builds
+// with treelet size 7, 2 passes, without / with: 338 K triangles 1308 / 1155 us,
+// 400 K hairball 1442 / 1255, 1 M 2848 / 1850, 2 M 5290 / 2950 (with 4096 leaves
+// 2 M 3295 and 338 K 1125, with 16384 2922 and 1194).
+constexpr uint32_t kTopLeaves = 1u << 18;
 
 constexpr int kDistStride = kMaxTreelet + 1;  // odd: the lanes of a row update touch different banks
 
@@ -439,14 +464,25 @@ __device__ __forceinline__ float treelet_merge(TreeletLds& S, int ts, float ci, 
 }
 
 // One optimiser pass, one phase of the bottom-up protocol (phased.hpp).
-// kFirst: the pass also makes the internal nodes' working boxes.
-template <bool kFirst, int kThreads>
+// kFirst: the pass also makes the internal nodes' working boxes.  kTop: the top
+// pass (chunk is nf), with small nodes on the same paths as the treelet roots.
+template <bool kFirst, int kThreads, bool kTop>
 __global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, int ts, int gamma, float ci,
                                                      uint32_t phase, uint32_t chunk) {
     __shared__ TreeletLds lds[kThreads / kHalf];
     __shared__ uint32_t nready, nextready;
     const uint32_t I = nf - 1;
-    const uint32_t tag = (phase << 24) | (blockIdx.x + 1u);
+    if (kTop) {  // the first workgroup's XCD takes all; the others' end here
+        __shared__ bool join;
+        if (threadIdx.x == 0) {
+            const uint32_t xcd = __builtin_amdgcn_s_getreg(kXccId) + 1u;
+            const uint32_t old = atomicCAS(&ws.top[0], 0u, xcd);
+            join = old == 0u || old == xcd;
+        }
+        __syncthreads();
+        if (!join) return;
+    }
+    const uint32_t tag = (phase << 24) | (kTop ? 1u : blockIdx.x + 1u);
     const uint64_t lo = (uint64_t)blockIdx.x * chunk, hi = lo + chunk;
     const uint32_t nin = phase == 0 ? 0 : min(ws.ph.nlist[phase - 1], I);
     const uint2* in = phase == 0 ? nullptr : ws.ph.list + (size_t)(phase - 1) * (I + 1);
@@ -455,14 +491,14 @@ __global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, 
     // chunk, so there are at most `chunk` of them.
     uint32_t* ready = ws.ready + lo;
     if (threadIdx.x == 0) nready = nextready = 0;
-    __syncthreads();
+    if (!kTop) __syncthreads();
     auto defer = [&](uint32_t node, uint32_t key) {
         const uint32_t slot = atomicAdd(&ws.ph.nlist[phase], 1u);
         if (slot < I) out[slot] = make_uint2(node, key);
     };
 
     // Below the treelet roots: one lane per leaf (or deferred node).
-    const uint32_t nstart = phase == 0 ? chunk : nin;
+    const uint32_t nstart = kTop ? 0 : phase == 0 ? chunk : nin;
     for (uint32_t r0 = threadIdx.x; r0 < nstart; r0 += blockDim.x) {
         uint32_t p;          // the node to complete next
         bool both = false;   // its children are known to be complete
@@ -544,7 +580,7 @@ __global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, 
         const int e = min(logical + kHalf * k, kMaxTreelet * (kMaxTreelet - 1) / 2 - 1), r = trm_row(e);
         pair_rc[k] = (uint32_t)(r << 8 | (e - trm_index(r, 0)));
     }
-    const uint32_t nroots = (uint32_t)min((uint64_t)min(nready, chunk), (uint64_t)nf - lo);
+    const uint32_t nroots = kTop ? nin : (uint32_t)min((uint64_t)min(nready, chunk), (uint64_t)nf - lo);
     bool have = false;
     uint32_t root = 0, steps = 0;
     uint4 rt = make_uint4(0u, 0u, kNoNode, 0u);  // the root's left, right, parent
@@ -553,16 +589,20 @@ __global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, 
             const uint64_t idle = __ballot(!have && hl == 0);
             if (idle) {
                 uint32_t slot = 0;
-                if (!have && hl == 0) slot = atomicAdd(&nextready, 1u);
+                if (!have && hl == 0)
+                    slot = kTop ? __hip_atomic_fetch_add(&ws.top[kTopNext], 1u, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_WORKGROUP)
+                                : atomicAdd(&nextready, 1u);
                 slot = half_pick(slot, 0, 0, upper);
                 if (!have && slot < nroots) {
-                    have = true;
-                    root = ready[slot];
-                    rt = AtrRec(ws, root).topo();
+                    root = kTop ? in[slot].x : ready[slot];
+                    have = root < I;
+                    if (have) rt = AtrRec(ws, root).topo();
                     steps = 0;
                 }
             }
             if (__ballot(have) == 0) break;
+            if (kTop) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // what the XCD's other CUs wrote
         }
         const AtrRec X(ws, root);
         const uint32_t parent = rt.z;
@@ -618,102 +658,107 @@ __global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, 
         }
         xmx.w = ci * xmn.w + mx.w + dpp_xor1(mx.w);
 
-        // formTreelet (Treelet.cuh:55-127): expand the treelet leaf with the
-        // largest area ts - 2 times.  A single largest area among values that
-        // compare is the reference's winner whatever its tournament order.
-        // The loop stops early (for both halves) at a tie, an area that does
-        // not compare, or a node whose children are below the loaded levels.
-        int slot = hl < 2 ? hl : -1;  // treelet leaf index of this lane's node
-        int it = 0;
-        for (; it < ts - 2; ++it) {
-            const bool inner = have && slot >= 0 && id < I;
-            const int32_t key = inner && mn.w >= 0.0f ? __float_as_int(mn.w + 0.0f) + 1 : 0;
-            const int32_t best = half_reduce<false>(key, upper);
-            const uint64_t eq = __ballot(key == best && have);
-            const uint32_t ea = (uint32_t)eq, eb = (uint32_t)(eq >> 32);
-            constexpr uint32_t kTop = (1u << (kHeapNodes / 2 - 1)) - 1;  // lanes whose children are loaded
-            if ((ea & (ea - 1)) != 0 || (eb & (eb - 1)) != 0 || ((ea | eb) & ~kTop) != 0 ||
-                __ballot(inner && !(mn.w >= 0.0f)) != 0)
-                break;  // wave-uniform
-            const int ia = ea ? __builtin_ctz(ea) : 0, ib = eb ? __builtin_ctz(eb) : 0;
-            const uint32_t rep = half_pick(id, ia, ib, upper);
-            const int from = (int)half_pick((uint32_t)slot, ia, ib, upper);
-            const int idx = upper ? ib : ia;
-            if (hl == it + 1) tin = rep;
-            if (hl == idx) slot = -1;
-            if (hl == 2 * idx + 2) slot = from;
-            if (hl == 2 * idx + 3) slot = it + 2;
-        }
-        // to leaf order: lane hl takes treelet leaf hl
-        if (have && slot >= 0) {
-            S.box[slot][0] = make_float4(mn.x, mn.y, mn.z, mx.w);
-            S.box[slot][1] = make_float4(mx.x, mx.y, mx.z, __uint_as_float(id));
-            S.kids[slot] = make_uint2(lkid, rkid);
-            S.area[slot] = mn.w;
-        }
-        wave_sync();
-        const int sl = min(hl, kMaxTreelet - 1);
-        {
-            const float4 b0 = S.box[sl][0], b1 = S.box[sl][1];
-            mn = make_float4(b0.x, b0.y, b0.z, S.area[sl]);
-            mx = make_float4(b1.x, b1.y, b1.z, b0.w);
-            id = __float_as_uint(b1.w);
-        }
-        // the remaining expansions, by the reference's tournament where the
-        // largest area is tied or does not compare
-        if (it < ts - 2) {
-            const uint2 kk = S.kids[sl];
-            lkid = kk.x;
-            rkid = kk.y;
+        // (the top pass also gets nodes below gamma: no treelet)
+        const bool work = have && (!kTop || (int32_t)half_pick(tri, 0, 0, upper) >= gamma);
+        bool keep = false;
+        if (!kTop || __ballot(work) != 0) {
+            // formTreelet (Treelet.cuh:55-127): expand the treelet leaf with the
+            // largest area ts - 2 times.  A single largest area among values that
+            // compare is the reference's winner whatever its tournament order.
+            // The loop stops early (for both halves) at a tie, an area that does
+            // not compare, or a node whose children are below the loaded levels.
+            int slot = hl < 2 ? hl : -1;  // treelet leaf index of this lane's node
+            int it = 0;
             for (; it < ts - 2; ++it) {
-                int idx = -1;
-                float w = -FLT_MAX;
-                if (have && hl < 2 + it) {
-                    idx = hl;
-                    w = id >= I ? -FLT_MAX : mn.w;
-                }
-                for (int n = 2 + it, amount = n / 2; n > 1; n = (n + 1) / 2, amount = n / 2) {
-                    const int oi = __shfl_down(idx, amount, kHalf);
-                    const float ow = __shfl_down(w, amount, kHalf);
-                    if (ow > w) { w = ow; idx = oi; }
-                }
-                const int ia = __builtin_amdgcn_readlane(idx, 0) & (kHalf - 1);
-                const int ib = __builtin_amdgcn_readlane(idx, kHalf) & (kHalf - 1);
+                const bool inner = work && slot >= 0 && id < I;
+                const int32_t key = inner && mn.w >= 0.0f ? __float_as_int(mn.w + 0.0f) + 1 : 0;
+                const int32_t best = half_reduce<false>(key, upper);
+                const uint64_t eq = __ballot(key == best && work);
+                const uint32_t ea = (uint32_t)eq, eb = (uint32_t)(eq >> 32);
+                constexpr uint32_t kLoaded = (1u << (kHeapNodes / 2 - 1)) - 1;  // lanes whose children are loaded
+                if ((ea & (ea - 1)) != 0 || (eb & (eb - 1)) != 0 || ((ea | eb) & ~kLoaded) != 0 ||
+                    __ballot(inner && !(mn.w >= 0.0f)) != 0)
+                    break;  // wave-uniform
+                const int ia = ea ? __builtin_ctz(ea) : 0, ib = eb ? __builtin_ctz(eb) : 0;
                 const uint32_t rep = half_pick(id, ia, ib, upper);
-                const uint32_t l2 = half_pick(lkid, ia, ib, upper), r2 = half_pick(rkid, ia, ib, upper);
-                idx = upper ? ib : ia;
+                const int from = (int)half_pick((uint32_t)slot, ia, ib, upper);
+                const int idx = upper ? ib : ia;
                 if (hl == it + 1) tin = rep;
-                if (have && (hl == idx || hl == it + 2)) {
-                    id = hl == idx ? l2 : r2;
-                    const AtrRec C(ws, id);
-                    mn = C.r[0];
-                    mx = C.r[1];
-                    const uint4 t = C.topo();
-                    lkid = t.x;
-                    rkid = t.y;
+                if (hl == idx) slot = -1;
+                if (hl == 2 * idx + 2) slot = from;
+                if (hl == 2 * idx + 3) slot = it + 2;
+            }
+            // to leaf order: lane hl takes treelet leaf hl
+            if (work && slot >= 0) {
+                S.box[slot][0] = make_float4(mn.x, mn.y, mn.z, mx.w);
+                S.box[slot][1] = make_float4(mx.x, mx.y, mx.z, __uint_as_float(id));
+                S.kids[slot] = make_uint2(lkid, rkid);
+                S.area[slot] = mn.w;
+            }
+            wave_sync();
+            const int sl = min(hl, kMaxTreelet - 1);
+            {
+                const float4 b0 = S.box[sl][0], b1 = S.box[sl][1];
+                mn = make_float4(b0.x, b0.y, b0.z, S.area[sl]);
+                mx = make_float4(b1.x, b1.y, b1.z, b0.w);
+                id = __float_as_uint(b1.w);
+            }
+            // the remaining expansions, by the reference's tournament where the
+            // largest area is tied or does not compare
+            if (it < ts - 2) {
+                const uint2 kk = S.kids[sl];
+                lkid = kk.x;
+                rkid = kk.y;
+                for (; it < ts - 2; ++it) {
+                    int idx = -1;
+                    float w = -FLT_MAX;
+                    if (work && hl < 2 + it) {
+                        idx = hl;
+                        w = id >= I ? -FLT_MAX : mn.w;
+                    }
+                    for (int n = 2 + it, amount = n / 2; n > 1; n = (n + 1) / 2, amount = n / 2) {
+                        const int oi = __shfl_down(idx, amount, kHalf);
+                        const float ow = __shfl_down(w, amount, kHalf);
+                        if (ow > w) { w = ow; idx = oi; }
+                    }
+                    const int ia = __builtin_amdgcn_readlane(idx, 0) & (kHalf - 1);
+                    const int ib = __builtin_amdgcn_readlane(idx, kHalf) & (kHalf - 1);
+                    const uint32_t rep = half_pick(id, ia, ib, upper);
+                    const uint32_t l2 = half_pick(lkid, ia, ib, upper), r2 = half_pick(rkid, ia, ib, upper);
+                    idx = upper ? ib : ia;
+                    if (hl == it + 1) tin = rep;
+                    if (work && (hl == idx || hl == it + 2)) {
+                        id = hl == idx ? l2 : r2;
+                        const AtrRec C(ws, id);
+                        mn = C.r[0];
+                        mx = C.r[1];
+                        const uint4 t = C.topo();
+                        lkid = t.x;
+                        rkid = t.y;
+                    }
                 }
+                wave_sync();
+                if (hl < ts) {
+                    S.box[hl][0] = make_float4(mn.x, mn.y, mn.z, mx.w);
+                    S.box[hl][1] = make_float4(mx.x, mx.y, mx.z, __uint_as_float(id));
+                }
+                wave_sync();
             }
-            wave_sync();
-            if (hl < ts) {
-                S.box[hl][0] = make_float4(mn.x, mn.y, mn.z, mx.w);
-                S.box[hl][1] = make_float4(mx.x, mx.y, mx.z, __uint_as_float(id));
-            }
-            wave_sync();
+
+            const float big = fmaxf(fmaxf(fmaxf(fabsf(mn.x), fabsf(mn.y)), fmaxf(fabsf(mn.z), fabsf(mx.x))),
+                                    fmaxf(fabsf(mx.y), fabsf(mx.z)));
+            const bool sane = big < 0x1p61f && mn.x == mn.x && mn.y == mn.y && mn.z == mn.z && mx.x == mx.x &&
+                              mx.y == mx.y && mx.z == mx.z;
+            float total;
+            if (__ballot(work && hl < ts && !sane) == 0)
+                total = treelet_merge<true>(S, ts, ci, hl, logical, upper, tin, pair_rc);
+            else
+                total = treelet_merge<false>(S, ts, ci, hl, logical, upper, tin, pair_rc);
+
+            // updateTreelet: keep the new topology when its SAH is lower
+            const uint64_t better = __ballot(work && hl == 0 && total < xmx.w);
+            keep = ((better >> (upper ? kHalf : 0)) & 1ull) != 0;
         }
-
-        const float big = fmaxf(fmaxf(fmaxf(fabsf(mn.x), fabsf(mn.y)), fmaxf(fabsf(mn.z), fabsf(mx.x))),
-                                fmaxf(fabsf(mx.y), fabsf(mx.z)));
-        const bool sane = big < 0x1p61f && mn.x == mn.x && mn.y == mn.y && mn.z == mn.z && mx.x == mx.x &&
-                          mx.y == mx.y && mx.z == mx.z;
-        float total;
-        if (__ballot(have && hl < ts && !sane) == 0)
-            total = treelet_merge<true>(S, ts, ci, hl, logical, upper, tin, pair_rc);
-        else
-            total = treelet_merge<false>(S, ts, ci, hl, logical, upper, tin, pair_rc);
-
-        // updateTreelet: keep the new topology when its SAH is lower
-        const uint64_t better = __ballot(have && hl == 0 && total < xmx.w);
-        const bool keep = ((better >> (upper ? kHalf : 0)) & 1ull) != 0;
         const uint32_t v = (uint32_t)__shfl_up((int)tin, 1, kHalf);  // tin[hl - 1]
         if (have && hl == 0) {
             X.set_span(slo, shi, tri);
@@ -737,6 +782,7 @@ __global__ __launch_bounds__(kThreads) void atr_treelets(AtrWs ws, uint32_t nf, 
         }
 
         // up to the parent
+        if (kTop) drain();  // this half's records are in the XCD's L2
         bool arrive = have && parent < I && ++steps <= nf;
         uint64_t old = 0;
         if (arrive && hl == 0)
@@ -801,6 +847,7 @@ size_t atr_carve(AtrWs* ws, void* base, size_t cap, uint32_t nf) {
     ws->vals_out = c.take<uint32_t>(nf);
     ws->rec = c.take<float4>(4 * total);
     ws->ready = c.take<uint32_t>(nf);
+    ws->top = c.take<uint32_t>(64);
     ws->sort_bytes = atr_sort_bytes(nf);
     ws->sort_tmp = c.take<char>(ws->sort_bytes);
     return c.used;
@@ -829,24 +876,22 @@ kr_error atr_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, int treele
     int gamma = treelet_size;
     for (int it = 0; it < iterations && nf > 1; ++it) {
         if (it > 0) hipLaunchKernelGGL(atr_clear, dim3(gb), dim3(256), 0, stream, ws, nf);
-        // Phases of 512, 8192, 131072 (large meshes) and all leaves.  A phase
-        // costs its own path of treelets, the last one runs on one CU.
-        // Measured with treelet size 7, 2 passes: 200 K triangles 1.04 ms with
-        // 16384, 1.01 with 8192, 1.14 with 4096, 1.16 with 8192 and 131072;
-        // 2 M triangles 4.09, 5.00, 6.78 and 3.46 ms.
-        uint32_t phase = 0;
-        for (uint32_t chunk : {512u, 8192u, nf > (1u << 19) ? 131072u : nf, nf}) {
-            const uint32_t c = min(chunk, nf);
-            const dim3 grid((nf + c - 1) / c);
-            if (phase == 0) {
-                auto k = it == 0 ? atr_treelets<true, 512> : atr_treelets<false, 512>;
-                hipLaunchKernelGGL(k, grid, dim3(512), 0, stream, ws, nf, treelet_size, gamma, ci, phase, c);
-            } else {
-                auto k = it == 0 ? atr_treelets<true, 1024> : atr_treelets<false, 1024>;
-                hipLaunchKernelGGL(k, grid, dim3(1024), 0, stream, ws, nf, treelet_size, gamma, ci, phase, c);
-            }
+        // Phases of 512 leaves, 8192 (large meshes) and all.  Each costs its own
+        // path of treelets.
+        auto tile = it == 0 ? atr_treelets<true, 512, false> : atr_treelets<false, 512, false>;
+        hipLaunchKernelGGL(tile, dim3((nf + 511) / 512), dim3(512), 0, stream, ws, nf, treelet_size, gamma, ci, 0u,
+                           min(512u, nf));
+        uint32_t phase = 1;
+        if (nf > kTopLeaves) {
+            auto mid = it == 0 ? atr_treelets<true, 1024, false> : atr_treelets<false, 1024, false>;
+            hipLaunchKernelGGL(mid, dim3((nf + 8191) / 8192), dim3(1024), 0, stream, ws, nf, treelet_size, gamma, ci,
+                               phase, 8192u);
             ++phase;
-            if (c == nf) break;
+        }
+        if (nf > 512) {
+            auto top = it == 0 ? atr_treelets<true, kTopThreads, true> : atr_treelets<false, kTopThreads, true>;
+            hipLaunchKernelGGL(top, dim3(kTopBlocks), dim3(kTopThreads), 0, stream, ws, nf, treelet_size, gamma, ci,
+                               phase, nf);
         }
         gamma *= 2;
     }

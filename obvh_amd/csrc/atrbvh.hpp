@@ -18,6 +18,7 @@ struct AtrWs {
     uint32_t* vals_out;  // face ids in code order
     float4* rec;         // per node: 64-byte working record, see AtrRec in atrbvh.hip
     uint32_t* ready;     // treelet roots ready to run, one segment per workgroup's chunk
+    uint32_t* top;       // top pass: its XCD, entries taken (64 words)
     char* sort_tmp;
     size_t sort_bytes;
 };

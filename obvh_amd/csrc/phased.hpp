@@ -1,22 +1,23 @@
 // phased.hpp -- state of the phased bottom-up protocol (the ATRBVH optimiser).
 //
 // A pass visits every internal node after both of its children.  Phase k runs
-// workgroups that own leaf positions [w*chunk_k, (w+1)*chunk_k), the last
-// phase one workgroup for everything.  Phase 0 starts one lane per leaf; later phases start from the nodes the previous phase
-// deferred.  Each deferred node is listed with a key, a leaf position of its
-// subtree known to the lane that deferred it, and is taken by the workgroup
-// whose chunk holds the key; that workgroup runs it when the node's whole
-// leaf span lies in its chunk and defers it again otherwise.  Other
-// workgroups decide from the key alone and never read the node: a pass that
-// restructures the tree (ATRBVH treelets) may rewire a deferred node's
-// children as soon as its owner has completed it and an ancestor.  A lane that
-// completes a child adds (tag << 32) | 1 to the parent's 64-bit arrival word
-// (tag = (phase << 24) | (workgroup + 1)); the first arrival stops, the
-// second continues if the first came from an earlier kernel (visible after
-// the kernel boundary) or from its own workgroup (workgroup-scope acq_rel
-// orders the data), and otherwise defers the parent to the next phase.  Only
-// workgroup-scope ordering is used inside a kernel; no device-scope fence is
-// issued.  The last phase owns every leaf and never defers.
+// workgroups that own leaf positions [w*chunk_k, (w+1)*chunk_k); the last one,
+// the top pass, is one group for everything.  Phase 0 starts one lane per leaf;
+// later phases start from the nodes the previous phase deferred.  Each deferred
+// node is listed with a key, a leaf position of its subtree known to the lane
+// that deferred it, and is taken by the workgroup whose chunk holds the key;
+// that workgroup runs it when the node's whole leaf span lies in its chunk and
+// defers it again otherwise.  Other workgroups decide from the key alone and
+// never read the node: a pass that restructures the tree (ATRBVH treelets) may
+// rewire a deferred node's children as soon as its owner has completed it and
+// an ancestor.  A lane that completes a child adds (tag << 32) | 1 to the
+// parent's 64-bit arrival word (tag = (phase << 24) | (workgroup + 1), one tag
+// for the whole top pass); the first arrival stops, the second continues if the
+// first came from an earlier kernel (visible after the kernel boundary) or from
+// its own group, and otherwise defers the parent to the next phase.  Inside a
+// kernel a group orders its data by workgroup-scope acq_rel, the top pass by
+// waiting for its stores and invalidating its L1; no device-scope release is
+// issued.  The top pass owns every leaf and never defers.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -25,7 +26,7 @@
 
 namespace obvh {
 
-constexpr int kPhases = 3;  // phases that defer, at most
+constexpr int kPhases = 2;  // phases that defer, at most
 
 struct PhaseWs {
     uint64_t* visit;   // per internal node: arrivals (low word) + sum of tags (high word)

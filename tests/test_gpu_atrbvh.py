@@ -104,7 +104,7 @@ def edge_mesh(nf, kind):
     return V.reshape(-1, 3).astype(np.float32), F
 
 
-# edges of the phases (512 and 8192 leaves; one workgroup up to 512), the smallest and largest treelets, distances
+# edges of the phases (512 leaves, one workgroup up to there; the top pass above), the smallest and largest treelets, distances
 # past one entry per lane (treelet size 9 and up), boxes that take the general merge
 @pytest.mark.parametrize("nf,ts,its,kind", [(1, 3, 1, "plain"), (2, 3, 1, "plain"), (3, 3, 2, "plain"),
                                             (20, 20, 1, "plain"), (512, 8, 2, "plain"), (513, 9, 2, "plain"),
@@ -120,3 +120,20 @@ def test_atrbvh_edges(torch, oracle_lib, nf, ts, its, kind):
     assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), en.view(np.uint8)), "nodes differ"
     assert np.array_equal(t["counts"].cpu().numpy().view(np.uint32), ec)
     assert np.array_equal(t["costs"].cpu().numpy(), eco, equal_nan=True)
+
+
+# the pass between the tiles and the top, from 2^18 leaves on: both sides, several builds alike (the top pass hands nodes
+# over between workgroups)
+@pytest.mark.parametrize("nf", [262144, 262145])
+def test_atrbvh_top_pass(torch, oracle_lib, nf):
+    say(f"[atrbvh] top pass, {nf} triangles")
+    V, F = edge_mesh(nf, "plain")
+    Vd, Fd = torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda()
+    en, ep, ec, eco = oracle_lib.atrbvh_build(V, F, 7, 2, CI, CT)
+    for _ in range(3):
+        t = ops.atrbvh_build(Vd, Fd, 7, 2, CI, CT)
+        torch.cuda.synchronize()
+        assert np.array_equal(t["parents"].cpu().numpy().view(np.uint32), ep), "parents differ"
+        assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), en.view(np.uint8)), "nodes differ"
+        assert np.array_equal(t["counts"].cpu().numpy().view(np.uint32), ec)
+        assert np.array_equal(t["costs"].cpu().numpy(), eco)
