@@ -71,9 +71,8 @@ def points_obb(points, return_time: bool = False):
     p = np.ascontiguousarray(points, dtype=np.float32).reshape(-1, 3)
     t = C.c_float(0.0)
     o = lib().kr_cuda_points_obb(p.ctypes.data_as(C.c_void_p), p.shape[0], C.byref(t))
-    out = np.array([o.mid.x, o.mid.y, o.mid.z, o.v0.x, o.v0.y, o.v0.z, o.v1.x, o.v1.y, o.v1.z,
-                    o.v2.x, o.v2.y, o.v2.z, o.ext.x, o.ext.y, o.ext.z], dtype=np.float32)
-    if np.isnan(out).all() and p.shape[0] > 0:
+    out = np.frombuffer(o, dtype=np.float32, count=15).copy()  # mid, v0, v1, v2, ext
+    if out[0] != out[0] and np.isnan(out).all() and p.shape[0] > 0:
         err = lib().obvh_last_error()
         raise ObvhError(err.decode() if err else "kr_cuda_points_obb failed")
     return (out, t.value) if return_time else out

@@ -388,6 +388,20 @@ def tied_points(n, seed):
     return p
 
 
+# host fits on both sides of the size up to which the points go through pinned memory (512 KB); repeated with other points
+# in the same buffers, and from device memory
+@pytest.mark.parametrize("n", [1, 43690, 43691])
+def test_points_obb_staging(torch, oracle_lib, n):
+    say(f"[points_obb] n={n}")
+    for seed in (1, 2):
+        p = synth.gaussian_points(n, seed=seed)
+        want = oracle_lib.points_obb(p)
+        assert np.array_equal(ops.points_obb(p), want, equal_nan=True)
+        d = torch.from_numpy(p).cuda()
+        o = ops.lib().kr_cuda_points_obb(ops.C.c_void_p(d.data_ptr()), n, None)
+        assert np.array_equal(np.frombuffer(o, np.float32), want, equal_nan=True)
+
+
 # edges of the single fit's forms: one workgroup (8192 points), tiles of 2048 that wait for each other (up to 128),
 # two launches above; of a tile's rows and steps
 @pytest.mark.parametrize("n", [1, 255, 1024, 1025, 2049, 8191, 8192, 8193, 10240, 10241, 262144, 262145, 300001])
