@@ -84,11 +84,18 @@ __device__ __forceinline__ obvh_dito_trace plain_trace(int degenerate) {
     return t;
 }
 
+// Batches up to this size get their tile table from the set-up's one workgroup
+// (four searches of a lane at a time, in LDS), which saves a launch: 8 sets of
+// 20 points 34.0 -> 31.0 us, 1000 of 10 36.3 -> 33.6, 290 of 30000 66.5 -> 65.9.
+// A wave writing set after set took 4 us more than the launch at 1000 sets.
+constexpr uint32_t kFillSets = 1024;
+constexpr size_t kFillTiles = 16384;
+
 __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_t single_count,
                                                    uint32_t nsets, uint32_t tile, uint64_t total,
-                                                   uint32_t cap_tiles, DitoWs ws,
+                                                   uint32_t cap_tiles, bool fill, DitoWs ws,
                                                    kr_obb3* out, obvh_dito_trace* trace) {
-    __shared__ uint32_t carry, limit;
+    __shared__ uint32_t carry, limit, firsts[kFillSets];
     __shared__ uint32_t wsum[1024 / kWave];
     if (threadIdx.x == 0) {
         carry = 0;
@@ -143,11 +150,27 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
             if (trace) trace[s] = plain_trace(4);
         }
         __syncthreads();
-        if (s < nsets) ws.first_tile[s] = min(incl - nt, limit);
+        const uint32_t first = min(incl - nt, limit);
+        if (s < nsets) ws.first_tile[s] = first;
+        if (fill && s < nsets) firsts[s] = first;
         if (threadIdx.x == blockDim.x - 1) carry = incl;
         __syncthreads();
     }
-    if (threadIdx.x == 0) ws.first_tile[nsets] = min(carry, limit);
+    const uint32_t T = min(carry, limit);
+    if (threadIdx.x == 0) ws.first_tile[nsets] = T;
+    if (!fill) return;
+    // the tile table, as dito_tile_table makes it: four searches of a lane at a time
+    for (uint32_t t0 = threadIdx.x; t0 < T; t0 += 4 * blockDim.x) {
+        uint32_t at[4] = {0, 0, 0, 0};
+        for (uint32_t step = kFillSets / 2; step != 0; step >>= 1) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (at[k] + step < nsets && firsts[at[k] + step] <= t0 + k * blockDim.x) at[k] += step;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (t0 + k * blockDim.x < T) ws.tile_set[t0 + k * blockDim.x] = at[k];
+    }
 }
 
 __global__ __launch_bounds__(256) void dito_tile_table(uint32_t nsets, DitoWs ws) {
@@ -1268,11 +1291,13 @@ kr_error dito_launch(const float* x, const float* y, const float* z,
     if (workers == 0) workers = (uint32_t)(T < 65536 ? T : 65536);
     if (workers > T) workers = (uint32_t)T;
     if (T > 0xFFFFFFF0ull) return "obvh_dito: too many tiles";
+    const bool fill = nsets <= kFillSets && T <= kFillTiles;
     hipLaunchKernelGGL(dito_setup, dim3(1), dim3(1024), 0, stream, offsets, single_count, nsets, tile, total,
-                       (uint32_t)T, ws, out, tr);
-    uint32_t tb = (uint32_t)((T + 255) / 256);
-    if (tb > 4096) tb = 4096;
-    hipLaunchKernelGGL(dito_tile_table, dim3(tb), dim3(256), 0, stream, nsets, ws);
+                       (uint32_t)T, fill, ws, out, tr);
+    if (!fill) {
+        const uint32_t tb = (uint32_t)min((T + 255) / 256, (size_t)4096);
+        hipLaunchKernelGGL(dito_tile_table, dim3(tb), dim3(256), 0, stream, nsets, ws);
+    }
     const PtsSoA p{x, y, z};
     const dim3 set_grid((nsets + kWaves - 1) / kWaves);
     hipLaunchKernelGGL(dito_pass1, dim3(workers), dim3(kBlock), 0, stream, p, offs, nsets, tile, ws);

@@ -388,6 +388,22 @@ def tied_points(n, seed):
     return p
 
 
+# both sides of the batch sizes whose tile table the set-up writes (1024 sets, 16384 tiles), empty sets at either end
+@pytest.mark.parametrize("nsets,tile,big", [(1, 0, 40), (64, 0, 40), (1024, 0, 40), (1025, 0, 40), (200, 512, 8340000),
+                                            (200, 512, 8350000)])
+def test_dito_batch_table_edges(torch, oracle_lib, nsets, tile, big):
+    say(f"[dito_batch] table edges {nsets} sets, tile={tile}, {big}")
+    rng = np.random.default_rng(nsets + big)
+    sizes = rng.integers(0, 60, nsets)
+    sizes[[0, -1]] = 0
+    sizes[nsets // 2] = big
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    p = rng.standard_normal((int(off[-1]), 3)).astype(np.float32)
+    out = ops.dito_batch(*soa(torch, p), torch.from_numpy(off).cuda(), tile_points=tile)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), oracle_lib.points_obb_batch(p, off, threads=8)[0], equal_nan=True)
+
+
 # host fits on both sides of the size up to which the points go through pinned memory (512 KB); repeated with other points
 # in the same buffers, and from device memory
 @pytest.mark.parametrize("n", [1, 43690, 43691])
