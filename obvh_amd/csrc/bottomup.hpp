@@ -10,15 +10,18 @@
 // child is completed elsewhere) goes on through global memory, in the same
 // launch: the payload is stored past the L2 caches, the arrival counted, and
 // the lane that arrives second loads its sibling's payload past the caches and
-// climbs on.  Nobody waits for anybody, and a payload is stored before its
+// climbs on.  Children, parents and arrival counts are loaded two nodes ahead;
+// a sibling seen to have arrived is loaded one ahead, and then nothing is
+// published.  Nobody waits for anybody, and a payload is stored before its
 // arrival is counted, so no order of the workgroups matters.
 //
 // Bound by latency: about 18 levels above the tiles of a 1 M-triangle LBVH,
-// each a store, an atomic and a load through memory (2.5 us), overlapped with
-// the tiles still running.  Against three phases in three launches, arrivals
-// and payloads through global memory from the leaves on: LBVH bounds of 1 M
-// triangles 173 -> 80 us, final bounds and collapse marks of a 200 K ATRBVH 96 -> 44
-// and 105 -> 39 us.
+// each a store, an atomic and a load through memory where the sibling was not
+// seen (2.5 us), overlapped with the tiles still running.  Against three phases
+// in three launches, arrivals and payloads through global memory from the
+// leaves on: LBVH bounds of 1 M triangles 173 -> 85 us (92 without the loads
+// ahead), final bounds and collapse marks of a 200 K ATRBVH 96 -> 42 and 105 ->
+// 38 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -38,6 +41,22 @@ struct UpTile {
     uint32_t parent[kUpTile];
     uint32_t arrive[kUpTile];
 };
+
+// A node's children, parent and arrivals (none past the internal nodes).
+struct UpTopo {
+    uint2 kids;
+    uint32_t parent, seen;
+};
+template <class Op>
+__device__ __forceinline__ UpTopo up_topo(uint32_t p, uint32_t I, uint32_t* visit, const Op& op) {
+    UpTopo T{make_uint2(0u, 0u), kUpNone, 0u};
+    if (p < I) {
+        T.kids = op.kids(p);
+        T.parent = op.parent(p);
+        T.seen = ld_agent(&visit[p]);
+    }
+    return T;
+}
 
 // Op provides
 //   uint2 kids(uint32_t p), uint32_t parent(uint32_t node)
@@ -107,22 +126,41 @@ __device__ __forceinline__ void bottom_up(uint32_t nf, uint32_t* visit, UpTile<P
                 }
             }
         }
-        for (uint32_t step = 0; go && step < nf; ++step) {
-            op.publish(cur, pay);
-            drain();
-            const uint32_t a = __hip_atomic_fetch_add(&visit[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint2 k = op.kids(p);
-            const uint32_t pp = op.parent(p);
-            const bool left = k.x == cur;
-            const uint32_t sib = left ? k.y : k.x;
-            if (a != 1 || sib >= total) break;  // first arrival: the sibling continues
+        if (!go) continue;
+        // children, parent and arrivals of the next two nodes
+        UpTopo A = up_topo(p, I, visit, op), B = up_topo(A.parent, I, visit, op);
+        Pay o{};  // the sibling's payload, if its arrival was seen
+        bool have = false;
+        auto look = [&](const UpTopo& T, uint32_t child) {
+            const uint32_t sib = T.kids.x == child ? T.kids.y : T.kids.x;
+            have = T.seen == 1 && sib < total;
             asm volatile("" ::: "memory");
-            const Pay o = op.fetch(sib);
-            pay = left ? op.merge(p, cur, sib, pay, o) : op.merge(p, sib, cur, o, pay);
-            cur = p;
-            p = pp;
-            if (p >= I) {  // the root
+            if (have) o = op.fetch(sib);
+        };
+        look(A, cur);
+        for (uint32_t step = 0; step < nf; ++step) {
+            const bool left = A.kids.x == cur;
+            const uint32_t sib = left ? A.kids.y : A.kids.x;
+            const UpTopo C = up_topo(B.parent, I, visit, op);
+            if (have) {
+                op.store(cur, pay);
+                __hip_atomic_fetch_add(&visit[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
                 op.publish(cur, pay);
+                drain();
+                const uint32_t a = __hip_atomic_fetch_add(&visit[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (a != 1 || sib >= total) break;  // first arrival: the sibling continues
+                asm volatile("" ::: "memory");
+                o = op.fetch(sib);
+            }
+            pay = left ? op.merge(p, cur, sib, pay, o) : op.merge(p, sib, cur, o, pay);
+            look(B, p);
+            cur = p;
+            p = A.parent;
+            A = B;
+            B = C;
+            if (p >= I) {  // the root
+                op.store(cur, pay);
                 break;
             }
         }
