@@ -237,6 +237,16 @@ __device__ __forceinline__ void stage_flush(StageT<R>& st, kr_obb3* obbs, kr_mat
                         [&](uint32_t j) { return st.mt[(j >> 4) * 17 + (j & 15)]; });
         return;
     }
+    // Rows of one tree (nearly always) are consecutive there too.  An index
+    // map's offset never decreases and a hole starts its tree, so the two ends
+    // tell.
+    const uint32_t o0 = batch_out_index(m, (uint32_t)first), o1 = batch_out_index(m, (uint32_t)first + cnt - 1);
+    if (o0 != kInvalid && o1 != kInvalid && o1 - o0 == cnt - 1) {
+        flush_dwords<R>(reinterpret_cast<float*>(obbs) + (size_t)o0 * 15, cnt * 15, [&](uint32_t j) { return st.ob[j]; });
+        flush_dwords<R>(reinterpret_cast<float*>(mats) + (size_t)o0 * 16, cnt * 16,
+                        [&](uint32_t j) { return st.mt[(j >> 4) * 17 + (j & 15)]; });
+        return;
+    }
     if (threadIdx.x < cnt) st.orow[threadIdx.x] = batch_out_index(m, (uint32_t)first + threadIdx.x);
     __syncthreads();
     float* go = reinterpret_cast<float*>(obbs);
@@ -252,6 +262,24 @@ __device__ __forceinline__ void stage_flush(StageT<R>& st, kr_obb3* obbs, kr_mat
 }
 
 // ------------------------------------------------------------ k-DOP --
+
+// The tree's topology: the children of an internal node, the face of a leaf,
+// read from the caller's nodes (36 bytes each) or from a batch's combined
+// ones (8 bytes each: no kernel reads a node's bounds).
+struct TreeNodes {
+    const uint32_t* w;  // of node 0
+    uint32_t stride;    // words per node
+
+    __device__ __forceinline__ uint2 kids(uint32_t i) const {
+        const uint32_t* p = w + (size_t)i * stride;
+        return make_uint2(p[0], p[1]);
+    }
+    __device__ __forceinline__ uint32_t face(uint32_t i) const { return w[(size_t)i * stride]; }
+};
+static TreeNodes tree_nodes(const kr_bvh_node* nodes) {
+    static_assert(sizeof(kr_bvh_node) == 36 && offsetof(kr_bvh_node, u) == 24, "children follow the bounds");
+    return TreeNodes{reinterpret_cast<const uint32_t*>(nodes) + 6, 9};
+}
 
 struct Kdop {
     float mn[7], mx[7];
@@ -469,7 +497,7 @@ __device__ __forceinline__ void tile_leaf_kdop(const ClimbTile& L, const kr_vec3
     leaf_kdop(ldv(V, vid[0]), ldv(V, vid[1]), ldv(V, vid[2]), vid, k);
 }
 
-__global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restrict__ nodes,
+__global__ __launch_bounds__(kTile) void climb_leaves(TreeNodes nodes,
                                                       const uint32_t* __restrict__ parents,
                                                       const kr_vec3* __restrict__ V,
                                                       const kr_uvec4* __restrict__ F, TreeWs ws, uint32_t N,
@@ -491,14 +519,15 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
     uint32_t l = 0, r = 0, par = kInvalid, f = kInvalid, leaf_parent = kInvalid;
     uint64_t slot = 0;
     if (pos < I) {
-        l = nodes[pos].u.children.left;
-        r = nodes[pos].u.children.right;
+        const uint2 lr = nodes.kids(pos);
+        l = lr.x;
+        r = lr.y;
         par = parents[pos];
         slot = ws.visit[pos];
     }
     if (pos < N) {
         leaf_parent = parents[I + pos];
-        f = nodes[I + pos].u.primitivesOffset;
+        f = nodes.face(I + pos);
     }
     kr_uvec4 face = {};
     if (f < N) face = F[f];
@@ -606,7 +635,8 @@ __global__ __launch_bounds__(kTile) void climb_leaves(const kr_bvh_node* __restr
             } else {  // parent outside the tile: publish, then global arrival
                 kdop_store(ws.kdop, cur, k);
                 span_store(ws, cur, span, count);
-                const uint32_t l = nodes[p].u.children.left, rr = nodes[p].u.children.right;
+                const uint2 lr = nodes.kids(p);
+                const uint32_t l = lr.x, rr = lr.y;
                 pp = parents[p];
                 const uint64_t old = __hip_atomic_fetch_add(&ws.visit[p], ((uint64_t)tag << 32) | 1ull,
                                                             __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -750,12 +780,13 @@ struct Topo {  // children, parent and arrival word of a node (zero / kInvalid p
     uint32_t l, r, parent;
     uint64_t v;
 };
-__device__ __forceinline__ Topo topo_load(const kr_bvh_node* __restrict__ nodes, const uint32_t* __restrict__ parents,
+__device__ __forceinline__ Topo topo_load(TreeNodes nodes, const uint32_t* __restrict__ parents,
                                           const TreeWs& ws, uint32_t p, uint32_t I) {
     Topo T = {0u, 0u, kInvalid, 0ull};
     if (p < I) {
-        T.l = nodes[p].u.children.left;
-        T.r = nodes[p].u.children.right;
+        const uint2 lr = nodes.kids(p);
+        T.l = lr.x;
+        T.r = lr.y;
         T.parent = parents[p];
         T.v = ld_agent(&ws.visit[p]);
     }
@@ -817,7 +848,7 @@ __device__ __forceinline__ uint4 path_merge(uint4 l, uint4 r, int q) {
     return make_uint4(sp.x, sp.y, c, 0u);
 }
 
-__global__ __launch_bounds__(kUpperThreads) void climb_upper(const kr_bvh_node* __restrict__ nodes,
+__global__ __launch_bounds__(kUpperThreads) void climb_upper(TreeNodes nodes,
                                                              const uint32_t* __restrict__ parents, TreeWs ws,
                                                              uint32_t N) {
     __builtin_amdgcn_s_setprio(3);  // wave priority
@@ -845,7 +876,8 @@ __global__ __launch_bounds__(kUpperThreads) void climb_upper(const kr_bvh_node* 
         if (cur >= I) { atomicOr(ws.error, 1u); continue; }
         uint32_t p = parents[cur];
         Topo A = topo_load(nodes, parents, ws, p, I);
-        const uint32_t l0 = nodes[cur].u.children.left, r0 = nodes[cur].u.children.right;
+        const uint2 lr = nodes.kids(cur);
+        const uint32_t l0 = lr.x, r0 = lr.y;
         if (l0 >= total || r0 >= total) { atomicOr(ws.error, 2u); continue; }
         uint4 k = path_merge(path_load<false>(ws, l0, I, q), path_load<false>(ws, r0, I, q), q);
         Topo B = topo_load(nodes, parents, ws, A.parent, I);
@@ -1612,7 +1644,7 @@ __device__ __forceinline__ void wave_keys(int32_t k[6]) {
     }
 }
 
-__global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ nodes,
+__global__ __launch_bounds__(kRTile) void refit(TreeNodes nodes,
                                                const uint32_t* __restrict__ parents,
                                                const kr_vec3* __restrict__ V,
                                                const kr_uvec4* __restrict__ F, TreeWs ws, uint32_t N) {
@@ -1624,7 +1656,7 @@ __global__ __launch_bounds__(kRTile) void refit(const kr_bvh_node* __restrict__ 
     const uint32_t pos = lo + t;
     const bool valid = pos < N;
     // the chain leaf -> face -> vertices starts first: the tile's set-up runs under its latency
-    const uint32_t f = valid ? nodes[I + pos].u.primitivesOffset : kInvalid;
+    const uint32_t f = valid ? nodes.face(I + pos) : kInvalid;
     const uint32_t leaf_parent = valid ? parents[I + pos] : kInvalid;
 #pragma unroll
     for (int a = 0; a < 3; ++a) { R.tk[t][a] = kKeyHi; R.tk[t][3 + a] = kKeyLo; }
@@ -2012,11 +2044,9 @@ kr_error side_stream(SideStream** out) {
 }
 }  // namespace
 
-kr_error tree_launch(const kr_bvh_node* nodes, const uint32_t* parents, const kr_vec3* V,
-                     const kr_uvec4* F, kr_obb3* obbs, kr_mat4* mats, uint32_t* ids, uint32_t N,
-                     void* workspace, size_t ws_bytes, hipStream_t stream, const BatchMap* batch) {
-    const BatchMap bm = batch ? *batch : BatchMap{nullptr, 0, 0};
-    if (N == 0) return nullptr;
+static kr_error tree_run(TreeNodes nodes, const uint32_t* parents, const kr_vec3* V, const kr_uvec4* F, kr_obb3* obbs,
+                         kr_mat4* mats, uint32_t N, void* workspace, size_t ws_bytes, hipStream_t stream,
+                         const BatchMap& bm) {
     TreeWs ws;
     size_t need = tree_carve(&ws, workspace, ws_bytes, N);
     if (workspace == nullptr || ws_bytes < need) return "obvh_obb_tree: workspace too small";
@@ -2064,9 +2094,24 @@ kr_error tree_launch(const kr_bvh_node* nodes, const uint32_t* parents, const kr
         hipLaunchKernelGGL(refit, blocks(N, kRTile), dim3(kRTile), 0, stream, nodes, parents, V, F, ws, N);
         hipLaunchKernelGGL(finalize, blocks(I, kStage), dim3(kStage), 0, stream, ws, obbs, mats, I, bm);
     }
-    if (ids)
-        hipLaunchKernelGGL(copy_ids, blocks(2 * N - 1, 256), dim3(256), 0, stream, nodes, V, F, ws, ids, 2 * N - 1);
     OBVH_HIP_TRY(hipGetLastError());
+    return nullptr;
+}
+
+kr_error tree_launch(const kr_bvh_node* nodes, const uint32_t* parents, const kr_vec3* V,
+                     const kr_uvec4* F, kr_obb3* obbs, kr_mat4* mats, uint32_t* ids, uint32_t N,
+                     void* workspace, size_t ws_bytes, hipStream_t stream) {
+    if (N == 0) return nullptr;
+    if (kr_error e = tree_run(tree_nodes(nodes), parents, V, F, obbs, mats, N, workspace, ws_bytes, stream,
+                              BatchMap{nullptr, 0, 0}))
+        return e;
+    if (ids) {
+        TreeWs ws;
+        tree_carve(&ws, workspace, ws_bytes, N);
+        const uint32_t total = 2 * N - 1;
+        hipLaunchKernelGGL(copy_ids, dim3((total + 255) / 256), dim3(256), 0, stream, nodes, V, F, ws, ids, total);
+        OBVH_HIP_TRY(hipGetLastError());
+    }
     return nullptr;
 }
 
@@ -2084,32 +2129,47 @@ kr_error tree_launch(const kr_bvh_node* nodes, const uint32_t* parents, const kr
 // internal slots L_k (k < K - 1) stay unused (holes: marked complete with
 // tag kHoleTag, skipped by the per-node kernels).  Every tree root has no
 // parent.  Tree t's nodes start at 2 L_t - t in the input layout.
+//
+// The combined nodes keep the children alone (8 bytes of 36), and boxes and
+// matrices of rows that lie in one tree go out as in a single transform: 64
+// trees of 3.8M triangles 1611 us with whole nodes and a row map, now 1554
+// (gathers 191 -> 151, leaf boxes and finalize 40 less; the nodes' gather moves
+// 395 MB in 110 us).
+
+// The tree of element i, found once for a workgroup whose 256 elements lie in one
+// tree (nearly all of them), per lane otherwise.
+template <class Of, class Begin>
+__device__ __forceinline__ uint32_t of_group(Of of, Begin begin, uint32_t i, uint32_t n) {
+    const uint32_t first = i - threadIdx.x;
+    const uint32_t t = of(__builtin_amdgcn_readfirstlane(first));
+    return first + 256u <= begin(t + 1) || n <= begin(t + 1) ? t : of(i);
+}
 
 // One lane per input node: write the combined node and parent.  Bad local
 // indices (children, parents, face ids outside the tree, an empty tree) set
 // the batch error word and are mapped out of range, where the transform's
 // own checks report them.
 __global__ void batch_gather_nodes(BatchMap m, const kr_bvh_node* __restrict__ nodes,
-                                   const uint32_t* __restrict__ parents, kr_bvh_node* cn, uint32_t* cp,
+                                   const uint32_t* __restrict__ parents, uint2* cn, uint32_t* cp,
                                    uint32_t* berr, uint32_t total_in) {
     const uint32_t I = m.Nsum - 1, total = 2 * m.Nsum - 1;
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total_in; g += gridDim.x * blockDim.x) {
-        const uint32_t t = batch_tree_of_node(m, g);
+        const uint32_t t = of_group([&](uint32_t i) { return batch_tree_of_node(m, i); },
+                                    [&](uint32_t k) { return 2u * m.prim_off[k] - k; }, g, total_in);
         const uint32_t Lt = m.prim_off[t], N = m.prim_off[t + 1] - Lt;
         if (N == 0) { atomicOr(berr, 1u); continue; }
         const uint32_t nb = 2 * Lt - t, j = g - nb, nn = 2 * N - 1;
         if (j >= nn) { atomicOr(berr, 1u); continue; }
         const uint32_t c = batch_map(m, t, Lt, N, j);
-        kr_bvh_node o = nodes[g];
+        uint2 o = make_uint2(nodes[g].u.children.left, nodes[g].u.children.right);
         if (j + 1 < N) {
-            const uint32_t l = o.u.children.left, r = o.u.children.right;
+            const uint32_t l = o.x, r = o.y;
             if (l >= nn || r >= nn) atomicOr(berr, 2u);
-            o.u.children.left = l < nn ? batch_map(m, t, Lt, N, l) : total;
-            o.u.children.right = r < nn ? batch_map(m, t, Lt, N, r) : total;
+            o.x = l < nn ? batch_map(m, t, Lt, N, l) : total;
+            o.y = r < nn ? batch_map(m, t, Lt, N, r) : total;
         } else {
-            const uint32_t f = o.u.primitivesOffset;
-            if (f >= N) atomicOr(berr, 4u);
-            o.u.primitivesOffset = f < N ? Lt + f : 0xFFFFFFFFu;
+            if (o.x >= N) atomicOr(berr, 4u);
+            o.x = o.x < N ? Lt + o.x : 0xFFFFFFFFu;  // its face
         }
         cn[c] = o;
         const uint32_t p = parents[g];
@@ -2122,7 +2182,7 @@ __global__ void batch_gather_nodes(BatchMap m, const kr_bvh_node* __restrict__ n
     // the unused internal slots L_k (k < K - 1) between the trees
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k + 1 < m.K; k += gridDim.x * blockDim.x) {
         const uint32_t idx = m.prim_off[k];
-        cn[idx] = kr_bvh_node{};
+        cn[idx] = make_uint2(0u, 0u);
         cp[idx] = kInvalid;
     }
     (void)I;
@@ -2132,7 +2192,8 @@ __global__ void batch_gather_nodes(BatchMap m, const kr_bvh_node* __restrict__ n
 __global__ void batch_gather_faces(BatchMap m, const uint32_t* __restrict__ vert_off,
                                    const kr_uvec4* __restrict__ faces, kr_uvec4* cf, uint32_t* berr) {
     for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < m.Nsum; f += gridDim.x * blockDim.x) {
-        const uint32_t t = batch_tree_of_leaf(m, f);
+        const uint32_t t = of_group([&](uint32_t i) { return batch_tree_of_leaf(m, i); },
+                                    [&](uint32_t k) { return m.prim_off[k]; }, f, m.Nsum);
         const uint32_t vb = vert_off[t], nv = vert_off[t + 1] - vb;
         kr_uvec4 a = faces[f];
         if (a.x >= nv || a.y >= nv || a.z >= nv) {
@@ -2150,7 +2211,7 @@ __global__ void batch_gather_faces(BatchMap m, const uint32_t* __restrict__ vert
 }
 
 struct BatchWs {
-    kr_bvh_node* nodes;
+    uint2* nodes;  // children, or a leaf's face and 0
     uint32_t* parents;
     kr_uvec4* faces;
     uint32_t* berr;
@@ -2162,7 +2223,7 @@ size_t batch_carve(BatchWs* w, void* base, size_t cap, uint32_t Nsum) {
     Carver c{(char*)base, 0, cap};
     const size_t total = 2 * (size_t)Nsum - 1;
     w->berr = c.take<uint32_t>(4);
-    w->nodes = c.take<kr_bvh_node>(total);
+    w->nodes = c.take<uint2>(total);
     w->parents = c.take<uint32_t>(total);
     w->faces = c.take<kr_uvec4>(Nsum);
     TreeWs tw;
@@ -2198,8 +2259,8 @@ kr_error tree_batch_launch(const kr_bvh_node* nodes, const uint32_t* parents, co
     OBVH_HIP_TRY(hipGetLastError());
     // climb_leaves and finalize write every node's box and matrix straight
     // to its place in the caller's per-tree layout
-    return tree_launch(w.nodes, w.parents, V, w.faces, obbs, mats, nullptr, Nsum, w.tree_ws, w.tree_ws_bytes, stream,
-                       &m);
+    return tree_run(TreeNodes{reinterpret_cast<const uint32_t*>(w.nodes), 2}, w.parents, V, w.faces, obbs, mats, Nsum,
+                    w.tree_ws, w.tree_ws_bytes, stream, m);
 }
 
 __global__ void copy_batch_status(const uint32_t* berr, const uint32_t* error, uint32_t* status) {

@@ -41,10 +41,9 @@ constexpr uint32_t kTChain = 64;
 static_assert(2 + kNodeLists <= 8, "error words 2 .. 2 + kNodeLists hold the list counts");
 
 size_t tree_carve(TreeWs* ws, void* base, size_t cap, uint32_t N);
-struct BatchMap;
 kr_error tree_launch(const kr_bvh_node* nodes, const uint32_t* parents, const kr_vec3* V,
                      const kr_uvec4* F, kr_obb3* obbs, kr_mat4* mats, uint32_t* ids, uint32_t N,
-                     void* workspace, size_t ws_bytes, hipStream_t stream, const BatchMap* batch = nullptr);
+                     void* workspace, size_t ws_bytes, hipStream_t stream);
 
 // Copy the call's device error word (0 = success) into `status` (device or
 // pinned host memory) on `stream`, and its meaning.
