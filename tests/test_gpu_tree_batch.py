@@ -101,6 +101,23 @@ def test_batch_equals_single_tree_calls_and_oracle(torch, oracle_lib, builder):
         assert np.array_equal(gm[s:s + 2 * n - 1], em), t
 
 
+# workgroups whose rows lie in one tree, in several, in runs of one-triangle trees (no internal node, consecutive rows),
+# at the batch's ends; trees of a workgroup's size and around
+@pytest.mark.parametrize("sizes", [[1] * 700, [1, 600, 1, 1, 513, 2, 512, 1], [256, 256, 255, 257, 1, 1, 1500], [3000, 1]])
+def test_batch_row_runs(torch, oracle_lib, sizes):
+    say(f"[tree batch] {len(sizes)} trees of {sizes[:8]}")
+    V, F = synth.hairball(tubes=80, seed=21)
+    trees = build_trees(oracle_lib, [(V, F[k % 50:k % 50 + n]) for k, n in enumerate(sizes)], "lbvh")
+    b = ops.pack_trees(to_dev(torch, trees))
+    status = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    obbs, mats = ops.obb_tree_batch(b, status=status)
+    torch.cuda.synchronize()
+    assert int(status.item()) == 0
+    want = [oracle_lib.obb_tree(*t) for t in trees]
+    assert np.array_equal(obbs.cpu().numpy(), np.concatenate([w[0] for w in want]))
+    assert np.array_equal(mats.cpu().numpy(), np.concatenate([w[1] for w in want]))
+
+
 def test_batch_replays_from_a_graph(torch, oracle_lib):
     say("[tree batch] graph capture, 3 replays")
     trees = build_trees(oracle_lib, meshes(9)[:12], "lbvh")
