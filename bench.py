@@ -57,8 +57,8 @@ def pmc_traffic(profile: str):
 
 # The kernels of one transform call; the roofline's device time is the call's,
 # on the launch stream.
-CALL_KERNELS = ("obb_tree call: tree_clear, climb_leaves, climb_phase, candidates x 2 (the first on a second "
-                "stream beside climb_phase), cand_redo, refit, finalize")
+CALL_KERNELS = ("obb_tree call: tree_clear, climb_leaves, climb_upper, candidates x 2 (the first on a second "
+                "stream beside climb_upper), cand_redo, refit, finalize")
 
 
 def pmc_value(profile: str, key: str):
@@ -211,7 +211,7 @@ def dito_legs(args) -> dict:
         r = ops.points_obb(p)
         legacy.append(time.perf_counter() - w0)
     out["single_131072"] = {"device_us": round(single * 1e6, 2), "Gpts_per_s": round(131072 / single / 1e9, 3),
-                            "entry": "obvh_dito_soa_noalloc (two launches)",
+                            "entry": "obvh_dito_soa_noalloc (one launch)",
                             "soa_device_us": round(fit_us["soa"], 2),
                             "legacy_wall_us": round(min(legacy) * 1e6, 1),
                             "equal_to_legacy": bool(np.array_equal(o1.cpu().numpy(),

@@ -4,9 +4,10 @@
 * ``Autotuner``     times (tile_points, workers) candidates on the real batch
                     with HIP events and caches the winner per shape bucket in a
                     JSON file (``$OBVH_CACHE_DIR`` or ``~/.cache/obvh_amd``).
-* ``BatchGraph``    captures one ``obvh_dito_batch`` call (setup, tile table,
-                    pass 1, candidates, pass 2, finalise: six kernels, no
-                    allocation, no memset) into a HIP graph and replays it.
+* ``BatchGraph``    captures one ``obvh_dito_batch`` call (setup with the
+                    tile table, pass 1, candidates, pass 2, finalise: five
+                    kernels, six past 1024 sets or 16384 tiles; no allocation,
+                    no memset) into a HIP graph and replays it.
 """
 from __future__ import annotations
 

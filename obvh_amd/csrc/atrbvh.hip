@@ -275,9 +275,9 @@ __global__ void atr_clear(AtrWs ws, uint32_t nf) { pass_clear(ws, nf); }
 // The top pass (everything above the chunks) runs on one XCD, whose L2 all its
 // CUs share: a half-wave that completes a node waits until its records are in
 // the L2, counts its arrival, and the one that arrives second drops its CU's L1
-// and goes on with the parent.  So the passes' paths join into one (24 treelets
-// of a 200 K hairball, where 512-, 8192- and all-leaf workgroups had 47 in a
-// row), and reads stay L2 hits (past the L2, for all XCDs, a trip takes twice as
+// and goes on with the parent.  So what were two launches' longest paths one
+// after the other is one path (300 and 340 us a pass of a 200 K hairball with
+// 8192-leaf workgroups and one for the rest, 255 and 260 now), and reads stay L2 hits (past the L2, for all XCDs, a trip takes twice as
 // long, four of them a treelet).  The grid covers every CU of the chip; the
 // first workgroup to arrive names the XCD, those of the others end.  Any one
 // workgroup would do all the work.

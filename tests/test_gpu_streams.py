@@ -131,3 +131,48 @@ def test_concurrent_calls_from_two_threads(torch, oracle_lib):
         eo, em = job["expect"]
         for i, (o, m) in enumerate(job["outs"]):
             assert torch.equal(bits(o), bits(eo)) and torch.equal(bits(m), bits(em)), (k, i)
+
+
+def test_side_stream_of_large_trees(torch, oracle_lib):
+    """Trees of more than 2^18 leaves run their candidate search on the library's second stream: a captured call
+    replayed while two host threads call on two other streams."""
+    say("[streams] trees above 2^18 leaves: two host threads and a graph")
+    jobs = []
+    for V, F in (synth.icosphere(116, seed=15), synth.hairball(tubes=7000, seed=16)):
+        Vd, Fd, t = device_tree(torch, V, F)
+        jobs.append({"args": (t["nodes"], t["parents"], Vd, Fd), "expect": checked_eager(torch, oracle_lib, V, F, Vd, Fd, t),
+                     "ws": workspace(torch, len(F)), "outs": [outputs(torch, len(F)) for _ in range(5)],
+                     "stream": torch.cuda.Stream()})
+    captured, ws = outputs(torch, jobs[0]["args"][3].shape[0]), workspace(torch, jobs[0]["args"][3].shape[0])
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ops.obb_tree(*jobs[0]["args"], workspace=ws, out=captured)
+    torch.cuda.synchronize()
+    start = threading.Barrier(len(jobs))
+    errors = []
+
+    def run(job):
+        try:
+            start.wait()
+            for out in job["outs"]:
+                ops.obb_tree(*job["args"], stream=job["stream"], workspace=job["ws"], out=out)
+        except Exception as e:  # reported from the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(j,)) for j in jobs]
+    for th in threads:
+        th.start()
+    for _ in range(3):
+        for x in captured:
+            x.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(bits(x), bits(e)) for x, e in zip(captured, jobs[0]["expect"]))
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for k, job in enumerate(jobs):
+        for i, out in enumerate(job["outs"]):
+            assert all(torch.equal(bits(x), bits(e)) for x, e in zip(out, job["expect"])), (k, i)
