@@ -486,6 +486,7 @@ struct ClimbTile {
     uint32_t arrive[kTile];     // arrivals at internal node lo + s from this workgroup
     uint2 kids[kTile];          // children of internal node lo + s
     uint32_t par_int[kTile];    // parent of internal node lo + s
+    uint32_t par_leaf[kTile];   // parent of the leaf at position lo + s
 };
 union ClimbLds {
     ClimbTile L;
@@ -534,9 +535,8 @@ __global__ __launch_bounds__(kTile) void climb_leaves(TreeNodes nodes,
     if (pos < I) {
         L.kids[t] = make_uint2(l, r);
         L.par_int[t] = par;
-        // (an unused slot of a batch has no children: no check)
-        if ((l >= total || r >= total || parents[l] != pos || parents[r] != pos) && !hole(slot)) atomicOr(ws.error, 2u);
     }
+    L.par_leaf[t] = leaf_parent;
     if (pos < N) {
         if (f < N) {
             const uint32_t vid[3] = {face.x, face.y, face.z};
@@ -555,6 +555,16 @@ __global__ __launch_bounds__(kTile) void climb_leaves(TreeNodes nodes,
     }
     L.arrive[t] = 0;
     __syncthreads();
+
+    // every child points back (an unused slot of a batch has none)
+    if (pos < I && !hole(slot)) {
+        const auto points_back = [&](uint32_t c) {
+            if (c >= total) return false;
+            const uint32_t s = (c < I ? c : c - I) - lo;
+            return (s < kTile ? (c < I ? L.par_int[s] : L.par_leaf[s]) : parents[c]) == pos;
+        };
+        if (!points_back(l) || !points_back(r)) atomicOr(ws.error, 2u);
+    }
 
     // First level, all lanes together: two leaf siblings in one wave are
     // merged by the left one (the right one's k-DOP comes by a lane shuffle)
