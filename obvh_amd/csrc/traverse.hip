@@ -11,7 +11,7 @@
 //
 // Traversal (soa_obvh_persistent_intersect, intersectors.cu:801-972).  One
 // ray per lane, a persistent grid; a lane whose ray is finished waits until
-// a quarter of its wave is idle, then those lanes take consecutive rays from
+// 24 lanes of its wave are idle, then those take consecutive rays from
 // a global counter (one atomic per refill), so long rays do not hold idle
 // lanes back.  Per ray: the reference's depth-first walk -- at an internal
 // node both children are tested against the unit cube in their own frames
@@ -392,11 +392,11 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
         const uint64_t idle = __ballot(wants);
         const int nidle = __popcll(idle);
         if (nidle == kWave || (nidle >= kTravRefill && !exhausted)) {  // wave-uniform
-            if (done) finish();
-            if (exhausted) break;
             uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(a.counter, (uint32_t)nidle);
-            base = (uint32_t)__shfl((int)base, 0, kWave);
+            if (!exhausted && lane == 0) base = atomicAdd(a.counter, (uint32_t)nidle);
+            if (done) finish();  // while the counter answers
+            if (exhausted) break;
+            base = __builtin_amdgcn_readfirstlane(base);
             if (wants) {
                 const uint32_t r = base + (uint32_t)__popcll(idle & below);
                 if (r < a.n) {
@@ -419,8 +419,8 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
         }
 
         // One step per lane: an internal node or one primitive of a leaf.
-        // (Holding triangle steps back until more lanes want one, or
-        // refilling at 8 idle lanes instead of 16, measured slower.)
+        // (Holding triangle steps back until more lanes want one measured
+        // slower.)
         bool enter_leaf = false;
         if (cur >= 0 && cur != kTravSentinel) {
             M43 L, R;
