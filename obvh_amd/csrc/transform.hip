@@ -2039,8 +2039,8 @@ struct SideStream {
 // Up to this many leaves all kernels run on the caller's stream: the hand-offs
 // between streams cost 10-15 us, more than the top of the tree takes from the
 // candidate search beside it.  Measured, one stream / two (icospheres, us):
-// 5120 leaves 110 / 124, 100820 144 / 162, 200000 183 / 187, 338000 235 / 231,
-// 499280 294 / 279.
+// 100820 leaves 127 / 142, 200000 165 / 170, 264500 202 / 201, 338000 221 / 213,
+// 499280 267 / 254, 1003520 454 / 424.
 constexpr uint32_t kOneStream = 1u << 18;
 constexpr int kMaxDevices = 64;
 std::mutex g_side_mu;
