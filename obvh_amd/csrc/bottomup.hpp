@@ -33,6 +33,8 @@ namespace obvh {
 constexpr uint32_t kUpTile = 512;
 constexpr uint32_t kUpNone = 0xFFFFFFFFu;
 
+// 40 KB with the 32-byte payload of bounds: exactly four workgroups per CU (one
+// word more and the LBVH build of 1 M triangles takes 229 us, 217 with four).
 template <class Pay>
 struct UpTile {
     Pay leaf[kUpTile];        // of the leaves
