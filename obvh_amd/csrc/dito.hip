@@ -142,9 +142,9 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
         for (int w = 0; w < wave_id(); ++w) wpre += wsum[w];
         const uint32_t incl = carry + wpre + v;
         // Offsets that never decrease need at most cap_tiles - 1 tiles.  Where
-        // others (sets that overlap) need more, the sets from the first that
-        // does not fit on are invalid: no tiles, a NaN box.
-        if (nt != 0 && incl >= cap_tiles) {
+        // others (sets that overlap) need more than the arrays hold, the sets
+        // from the first that does not fit on are invalid: no tiles, a NaN box.
+        if (nt != 0 && incl > cap_tiles) {
             atomicMin(&limit, incl - nt);
             out[s] = nan_box();
             if (trace) trace[s] = plain_trace(4);

@@ -494,3 +494,25 @@ def test_lbvh_sort_edges(torch, oracle_lib, nf, cells):
     assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), nodes.view(np.uint8))
     assert np.array_equal(t["counts"].cpu().numpy().view(np.uint32), counts)
     assert np.array_equal(t["costs"].cpu().numpy(), costs)
+
+
+def test_dito_batch_overlapping_sets_that_just_fit(torch, oracle_lib):
+    """Overlapping sets that need exactly as many tiles as the workspace holds (13) keep their boxes; one point more
+    needs a 14th and makes the last of them invalid."""
+    say("[dito_batch] overlapping sets, a full tile table")
+    n = 5 * 512
+    p = synth.gaussian_points(n, seed=3)
+    x, y, z = soa(torch, p)
+    exp = oracle_lib.points_obb(p)
+    for last, fits in ((1536, True), (1537, False)):
+        off = torch.tensor([0, n, 0, n, 0, last, 0, 0], dtype=torch.int64).cuda()  # 5 + 5 + 3 tiles, or + 4
+        out, tr = ops.dito_batch(x, y, z, off, tile_points=512, trace=True)
+        torch.cuda.synchronize()
+        got, g = out.cpu().numpy(), ops.trace_to_numpy(tr)
+        assert np.array_equal(got[0], exp) and np.array_equal(got[2], exp)
+        if fits:
+            assert np.array_equal(got[4], oracle_lib.points_obb(p[:last]))
+        else:
+            assert np.isnan(got[4]).all() and g[4]["degenerate"] == 4
+        for s in (1, 3, 5):
+            assert np.isnan(got[s]).all() and g[s]["degenerate"] == 4, s
