@@ -169,6 +169,17 @@ kr_error obvh_dito_soa(const float* x, const float* y, const float* z, kr_size c
     return nullptr;
 }
 
+// For tests: obvh_dito_soa with a poll limit of the caller's, and the
+// workspace's completion counters cleared first only if `clear`.
+kr_error obvh_dito_soa_polls(const float* x, const float* y, const float* z, kr_size count, kr_obb3* out_obb,
+                             obvh_dito_trace* trace, void* workspace, size_t workspace_bytes, u32 polls, u32 clear,
+                             void* stream) {
+    bool first = clear != 0;
+    TRY(obvh::dito_one_launch(x, y, z, nullptr, count, out_obb, trace, workspace, workspace_bytes, first,
+                              (hipStream_t)stream, polls));
+    return nullptr;
+}
+
 // The allocation-free single-set fit: obvh_dito_soa's kernels with the
 // workspace in the file-scope device array `scratch` (its address per device
 // from hipGetSymbolAddress, taken once per device on the first call).

@@ -243,7 +243,7 @@ struct FitLds {
     float wrng[kThreads / kWave][8];   // per wave: minima (0..2) and negated maxima (4..6) on the axes
     float rng[8];
     SetState st;
-    uint32_t last, fail;
+    uint32_t last, given;
 };
 __device__ __forceinline__ int side_slot(int side) { return side < 7 ? side : side + 1; }
 
@@ -915,12 +915,21 @@ __global__ __launch_bounds__(kBlock) void dito_one_b(P pts, uint64_t n, uint32_t
 // A single set in one launch: its tiles hand their partial results over inside
 // the launch with the agent-scope accesses above.
 //
-// Waiting ends: the tiles wait for each other, and there are at most `cap` of
-// them, an eighth of the workgroups the device holds (so up to eight such
-// launches may share it; larger sets take two launches).  The polls are
-// bounded all the same; a fit that exceeds the bound gets a NaN box.
+// No tile depends on another one being scheduled: a tile that has polled for the
+// set's state long enough gives up and ends, and the searching tile takes its
+// axis pass over.  At most `cap` tiles wait, an eighth of the workgroups the
+// device holds, so that this does not happen unless the chip is held by others
+// for milliseconds (larger sets take two launches).  A tile gives up by writing
+// kGaveUp to its axis partial and then counting itself in sync->flag; it still
+// does its own pass if the count shows that the state is there and the mark was
+// not taken yet.  The searching tile sees in the count, as it publishes the
+// state, whether to look for marks.  (A count that comes after the last tile's
+// reset only makes the next call look: every tile clears its mark before it
+// counts its slab pass.)
 
-constexpr uint32_t kPollLimit = 1u << 22;
+constexpr uint32_t kStateUp = 1u << 31;       // sync->flag: the state is there; below: tiles that gave up
+constexpr uint32_t kGaveUp = 0x7FC00001u;     // NaN, as no axis partial is
+constexpr uint32_t kTakenOver = 0x7FC00002u;
 
 constexpr int kStateWords = sizeof(SetState) / 4;
 constexpr int kTraceWords = sizeof(obvh_dito_trace) / 4;
@@ -975,34 +984,55 @@ __device__ __forceinline__ void find_side(const f3 (&p)[J], uint32_t cnt, float 
     if (lane_id() == 0 && first != 0x7FFFFFFF) atomicMin(&L.idx[side_slot(kSide)], (uint32_t)first);
 }
 
-// Wave 0: the set's state for the axis pass, from the flag's set-up.
-// False when the poll limit is exceeded.
-__device__ __forceinline__ bool wait_state(const FitSync* sync, const SetState* state, SetState* lds) {
+__device__ __forceinline__ uint32_t* axis_mark(const DitoWs& ws, uint32_t tile) {
+    return reinterpret_cast<uint32_t*>(&ws.part2[(size_t)tile * 6]);
+}
+// The mark of a tile that gave up goes to one side: back to the tile, or to the
+// searching tile.
+__device__ __forceinline__ bool claim_mark(uint32_t* mark, uint32_t to) {
+    uint32_t expected = kGaveUp;
+    return __hip_atomic_compare_exchange_strong(mark, &expected, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Wave 0: the set's state for the axis pass, after the flag shows it.  False
+// when it is not there after `polls` polls: the tile's axis pass is the
+// searching tile's.
+__device__ __forceinline__ bool wait_state(FitSync* sync, const SetState* state, uint32_t* mark, uint32_t polls,
+                                           SetState* lds) {
     uint32_t up = 0;
-    for (uint32_t i = 0; i < kPollLimit && up == 0; ++i) {
+    for (uint32_t i = 0; i < polls && up < kStateUp; ++i) {
         if (i > 0) __builtin_amdgcn_s_sleep(8);
         up = __builtin_amdgcn_readfirstlane((int)ld_agent(&sync->flag));
+    }
+    if (up < kStateUp) {
+        bool mine = false;
+        if (lane_id() == 0) {
+            st_agent(mark, kGaveUp);
+            drain();
+            up = __hip_atomic_fetch_add(&sync->flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            mine = up >= kStateUp && claim_mark(mark, 0u);
+        }
+        if (__ballot(mine) == 0) return false;
     }
     asm volatile("" ::: "memory");
     if (lane_id() < kStateWords)
         reinterpret_cast<uint32_t*>(lds)[lane_id()] = ld_agent(reinterpret_cast<const uint32_t*>(state) + lane_id());
-    return up != 0;
-}
-
-__device__ __forceinline__ void fit_fail(kr_obb3* out, obvh_dito_trace* trace) {
-    *out = nan_box();
-    if (trace) trace->degenerate = 4;
+    return true;
 }
 
 // After the slab pass of tile `part` of nt (partials from tile ft), L.ext and
 // L.idx (indices from the tile's first point, `first` of the set): publish
 // them; the last tile searches.  Returns whether this workgroup did (L.st then
-// holds the state).  Ends with a barrier.
+// holds the state, `gave` of thread 0 how many tiles had given up waiting for
+// it).  Ends with a barrier.
 template <class P, int kThreads>
 __device__ __forceinline__ bool tile_search(P pts, uint64_t sbeg, uint64_t n, uint32_t first, uint32_t part,
                                             uint32_t ft, uint32_t nt, const DitoWs& ws, SetState* state,
-                                            FitSync* sync, obvh_dito_trace* trace, FitLds<kThreads>& L) {
+                                            FitSync* sync, obvh_dito_trace* trace, FitLds<kThreads>& L,
+                                            uint32_t& gave) {
     const int lane = lane_id(), wave = wave_id();
+    gave = 0;
     if (nt > 1) {
         if (wave == 0) {
             if (lane < 14) {
@@ -1012,6 +1042,7 @@ __device__ __forceinline__ bool tile_search(P pts, uint64_t sbeg, uint64_t n, ui
                 st_agent(&ws.part1_v[at], lane < 7 ? L.ext[slot] : -L.ext[slot]);
                 st_agent(&ws.part1_i[at], i == kNoIdx ? kNoIdx : first + i);
             }
+            if (lane == 14) st_agent(axis_mark(ws, ft + part), 0u);
             drain();
             if (lane == 0)
                 L.last = __hip_atomic_fetch_add(&sync->done1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nt - 1;
@@ -1038,7 +1069,8 @@ __device__ __forceinline__ bool tile_search(P pts, uint64_t sbeg, uint64_t n, ui
             if (lane < kStateWords)
                 st_agent(reinterpret_cast<uint32_t*>(state) + lane, reinterpret_cast<const uint32_t*>(&L.st)[lane]);
             drain();
-            if (lane == 0) st_agent(&sync->flag, 1u);
+            if (lane == 0)
+                gave = __hip_atomic_fetch_or(&sync->flag, kStateUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (trace && lane == 0) {  // the box's workgroup writes result_aabb
 #pragma unroll
@@ -1120,8 +1152,8 @@ __device__ __forceinline__ void tile_box(P pts, uint64_t sbeg, float (&r)[6], ui
 // again instead: tiles that wait in registers for their set's search held
 // 75 MB for 68 us each, three times the time of two readings.
 template <class P, int J, int kThreads>
-__device__ __forceinline__ void one_tile(P pts, uint64_t n, uint32_t part, uint32_t nt, const DitoWs& ws, kr_obb3* out,
-                                         obvh_dito_trace* trace, FitLds<kThreads>& L) {
+__device__ __forceinline__ void one_tile(P pts, uint64_t n, uint32_t part, uint32_t nt, const DitoWs& ws,
+                                         uint32_t polls, kr_obb3* out, obvh_dito_trace* trace, FitLds<kThreads>& L) {
     constexpr uint32_t kTilePts = J * kThreads;
     const float INF = FLT_MAX * 2.0f;
     FitSync* sync = reinterpret_cast<FitSync*>(ws.done);
@@ -1143,33 +1175,48 @@ __device__ __forceinline__ void one_tile(P pts, uint64_t n, uint32_t part, uint3
     find_side<9>(p, cnt, e[9], L); find_side<10>(p, cnt, e[10], L); find_side<11>(p, cnt, e[11], L);
     find_side<12>(p, cnt, e[12], L); find_side<13>(p, cnt, e[13], L);
     __syncthreads();
-    if (tile_search(pts, 0, n, (uint32_t)first, part, 0, nt, ws, ws.state, sync, trace, L)) {
+    uint32_t gave;
+    const bool searched = tile_search(pts, 0, n, (uint32_t)first, part, 0, nt, ws, ws.state, sync, trace, L, gave);
+    if (searched) {
         load_tile<P, J, kThreads>(pts, first, cnt, p);  // the search used the registers
     } else {
         if (wave_id() == 0) {
-            const bool ok = wait_state(sync, ws.state, &L.st);
-            if (lane_id() == 0) L.fail = ok ? 0u : 1u;
+            const bool ok = wait_state(sync, ws.state, axis_mark(ws, part), polls, &L.st);
+            if (lane_id() == 0) L.given = ok ? 0u : 1u;
         }
         __syncthreads();
-        if (L.fail != 0) {
-            if (threadIdx.x == 0) fit_fail(out, trace);
-            return;
-        }
+        if (L.given != 0) return;
     }
     f3 b[3];
     state_axes(L.st, b);
-    float r[6] = {INF, INF, INF, -INF, -INF, -INF};
+    auto axis_pass = [&](uint32_t tile) {
+        float r[6] = {INF, INF, INF, -INF, -INF, -INF};
 #pragma unroll
-    for (int j = 0; j < J; j += 2) axes_step(p[j], p[j + 1], b, r);
-    tile_box(pts, 0, r, part, 0, nt, ws, sync, out, trace, L);
+        for (int j = 0; j < J; j += 2) axes_step(p[j], p[j + 1], b, r);
+        tile_box(pts, 0, r, tile, 0, nt, ws, sync, out, trace, L);
+    };
+    axis_pass(part);
+    if (!searched || nt == 1) return;
+    if (threadIdx.x == 0) L.given = gave & ~kStateUp;
+    __syncthreads();
+    if (L.given == 0) return;
+    for (uint32_t t = 0; t < nt; ++t) {  // the tiles that gave up
+        __syncthreads();
+        if (threadIdx.x == 0) L.last = t != part && claim_mark(axis_mark(ws, t), kTakenOver);
+        __syncthreads();
+        if (L.last == 0) continue;
+        const uint64_t at = (uint64_t)t * kTilePts;
+        load_tile<P, J, kThreads>(pts, at, (uint32_t)min((uint64_t)kTilePts, n - at), p);
+        axis_pass(t);
+    }
 }
 
 // A set of n > 0 points, gridDim.x tiles.
 template <class P, int J, int kThreads>
-__global__ __launch_bounds__(kThreads) void dito_one(P pts, uint64_t n, DitoWs ws, kr_obb3* out,
+__global__ __launch_bounds__(kThreads) void dito_one(P pts, uint64_t n, DitoWs ws, uint32_t polls, kr_obb3* out,
                                                      obvh_dito_trace* trace) {
     __shared__ FitLds<kThreads> L;
-    one_tile<P, J, kThreads>(pts, n, blockIdx.x, gridDim.x, ws, out, trace, L);
+    one_tile<P, J, kThreads>(pts, n, blockIdx.x, gridDim.x, ws, polls, out, trace, L);
 }
 
 // ----------------------------------------------------------------- host --
@@ -1227,10 +1274,11 @@ static kr_error one_cap(uint32_t* cap) {
 constexpr int kOneRows = 8;  // points per lane of the single fit's workgroups
 
 template <class P>
-static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, uint32_t cap, DitoWs ws, kr_obb3* out,
-                       obvh_dito_trace* trace, bool& clear, hipStream_t stream) {
+static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, uint32_t cap, DitoWs ws, uint32_t polls,
+                       kr_obb3* out, obvh_dito_trace* trace, bool& clear, hipStream_t stream) {
     if (n <= 1024 * kOneRows) {
-        hipLaunchKernelGGL((dito_one<P, kOneRows, 1024>), dim3(1), dim3(1024), 0, stream, p, n, ws, out, trace);
+        hipLaunchKernelGGL((dito_one<P, kOneRows, 1024>), dim3(1), dim3(1024), 0, stream, p, n, ws, polls, out,
+                           trace);
         return;
     }
     if (clear) hipLaunchKernelGGL(dito_one_clear, dim3(1), dim3(64), 0, stream, ws);
@@ -1238,8 +1286,8 @@ static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, uint32_t cap,
     constexpr uint32_t kOneTile = kBlock * kOneRows;
     const uint64_t F = (n + kOneTile - 1) / kOneTile;
     if (F <= cap) {
-        hipLaunchKernelGGL((dito_one<P, kOneRows, kBlock>), dim3((uint32_t)F), dim3(kBlock), 0, stream, p, n, ws, out,
-                           trace);
+        hipLaunchKernelGGL((dito_one<P, kOneRows, kBlock>), dim3((uint32_t)F), dim3(kBlock), 0, stream, p, n, ws,
+                           polls, out, trace);
         return;
     }
     obvh_dito_trace* tr = trace ? trace : ws.trace_tmp;
@@ -1249,7 +1297,7 @@ static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, uint32_t cap,
 
 kr_error dito_one_launch(const float* x, const float* y, const float* z, const float* xyz, uint64_t n,
                          kr_obb3* out, obvh_dito_trace* trace, void* workspace, size_t ws_bytes, bool& clear,
-                         hipStream_t stream) {
+                         hipStream_t stream, uint32_t polls) {
     if (n == 0) return "obvh_dito: the single-set fit needs at least one point";
     // The two-launch form's tiles: at most 1024, since each workgroup pays one
     // agent-scope release and the last one reduces every tile.  At least the
@@ -1266,8 +1314,8 @@ kr_error dito_one_launch(const float* x, const float* y, const float* z, const f
     uint32_t cap = 0;
     if (kr_error e = one_cap(&cap)) return e;
     cap = (uint32_t)min((uint64_t)cap, (uint64_t)dito_max_tiles(1, n, tile));
-    if (xyz) launch_one(PtsAoS{xyz}, n, tile, (uint32_t)T, cap, ws, out, trace, clear, stream);
-    else launch_one(PtsSoA{x, y, z}, n, tile, (uint32_t)T, cap, ws, out, trace, clear, stream);
+    if (xyz) launch_one(PtsAoS{xyz}, n, tile, (uint32_t)T, cap, ws, polls, out, trace, clear, stream);
+    else launch_one(PtsSoA{x, y, z}, n, tile, (uint32_t)T, cap, ws, polls, out, trace, clear, stream);
     OBVH_HIP_TRY(hipGetLastError());
     return nullptr;
 }

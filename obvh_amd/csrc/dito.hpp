@@ -19,7 +19,7 @@ struct SetState {
 // Hand-over between the tiles of one set in a one-launch fit.
 struct FitSync {
     uint32_t done1, done2;  // tiles that finished the slab / axis pass
-    uint32_t flag;          // the set's state is there
+    uint32_t flag;          // bit 31: the set's state is there; below: tiles that gave up waiting for it
     uint32_t pad;
 };
 
@@ -51,6 +51,10 @@ kr_error dito_launch(const float* x, const float* y, const float* z,
                      kr_obb3* out, obvh_dito_trace* trace, uint32_t tile, uint32_t workers,
                      void* workspace, size_t ws_bytes, hipStream_t stream);
 
+// Polls (about a microsecond each) before a tile of the one-launch fit leaves
+// its axis pass to the searching tile, which searches for some 10 us.
+constexpr uint32_t kDitoPolls = 1u << 12;
+
 // One set of n > 0 points: one launch, or two for a set of more tiles than
 // may wait for each other.  `clear` zeroes the workspace's completion counters
 // first (needed before the first call on a workspace that uses them; every
@@ -58,6 +62,6 @@ kr_error dito_launch(const float* x, const float* y, const float* z,
 // not use them and leaves it as it is.
 kr_error dito_one_launch(const float* x, const float* y, const float* z, const float* xyz, uint64_t n,
                          kr_obb3* out, obvh_dito_trace* trace, void* workspace, size_t ws_bytes, bool& clear,
-                         hipStream_t stream);
+                         hipStream_t stream, uint32_t polls = kDitoPolls);
 
 }  // namespace obvh
