@@ -492,6 +492,15 @@ kr_error obvh_lbvh_build(const kr_vec3* vertices, const kr_uvec4* faces, u32 fac
     return nullptr;
 }
 
+// For tests: obvh_lbvh_build with a poll limit of the caller's for the sort.
+kr_error obvh_lbvh_build_polls(const kr_vec3* vertices, const kr_uvec4* faces, u32 face_count, kr_bvh_node* nodes,
+                               u32* parents, u32* primitive_counts, kr_scalar* costs, u32* mortons_sorted,
+                               void* workspace, size_t workspace_bytes, u32 polls, void* stream) {
+    TRY(obvh::lbvh_launch(vertices, faces, face_count, nodes, parents, primitive_counts, costs, mortons_sorted,
+                          workspace, workspace_bytes, (hipStream_t)stream, polls));
+    return nullptr;
+}
+
 // -------------------------------------------------------- collapse --
 
 size_t obvh_collapse_workspace_size(u32 primitive_count) {

@@ -299,7 +299,7 @@ size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf) {
 
 kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_node* nodes, uint32_t* parents,
                      uint32_t* counts, float* costs, uint32_t* mortons, void* workspace, size_t ws_bytes,
-                     hipStream_t stream) {
+                     hipStream_t stream, uint32_t polls) {
     if (nf == 0) return "obvh_lbvh_build: no faces";
     LbvhWs ws;
     size_t need = lbvh_carve(&ws, workspace, ws_bytes, nf);
@@ -312,7 +312,7 @@ kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_no
                        stream, V, F, nf, ws);
     hipLaunchKernelGGL(lbvh_codes, dim3(min((nf + 1023) / 1024, 256u)), dim3(1024), 0, stream, V, F, nf, ws);
     if (nf <= kRadixMax) {
-        radix_sort<kPasses>(ws.keys, ws.vals, ws.keys_tmp, ws.vals_tmp, nf, ws.radix, stream);
+        radix_sort<kPasses>(ws.keys, ws.vals, ws.keys_tmp, ws.vals_tmp, nf, ws.radix, polls, stream);
     } else {  // rocPRIM; its buffers swap roles
         hipLaunchKernelGGL(lbvh_iota, dim3(gb), dim3(256), 0, stream, ws.vals_tmp, nf);
         OBVH_HIP_TRY(hipMemcpyAsync(ws.keys_tmp, ws.keys, sizeof(uint32_t) * nf, hipMemcpyDeviceToDevice, stream));

@@ -22,6 +22,6 @@ struct LbvhWs {
 size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf);
 kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_node* nodes, uint32_t* parents,
                      uint32_t* counts, float* costs, uint32_t* mortons, void* workspace, size_t ws_bytes,
-                     hipStream_t stream);
+                     hipStream_t stream, uint32_t polls = kRadixPolls);
 
 }  // namespace obvh

@@ -7,9 +7,11 @@
 // and looks back over the earlier tiles' for its place, 64 tiles a trip to
 // memory, then puts its pairs in digit order in LDS and writes them in runs.
 // Counts are handed over with agent-scope accesses: one word holds a count and
-// whether it is the tile's own or includes all before it.  A tile waits only
-// for tiles taken before it, which wait for none after; the polls are bounded
-// all the same.
+// whether it is the tile's own or includes all before it.  (Onesweep: Adinets
+// and Merrill, 2022; the look-back is Merrill and Garland's, 2016.)  A tile
+// waits only for tiles taken before it, which wait for none after, and only so
+// long: past the poll limit it counts the earlier tile's keys itself (the pass's
+// input does not change), so the result never depends on the wait.
 //
 // Bound by latency: a pass over 1 M pairs takes 17 us for 16 MB moved (written
 // without the LDS order 22 us; with 256 threads and one look-back thread per
@@ -30,6 +32,7 @@ constexpr int kRadixGroups = kRadixThreads / kRadixBins;  // threads per bin in 
 constexpr int kRadixBack = 16;                            // earlier tiles a thread reads at once
 constexpr uint32_t kRadixOwn = 1u << 30, kRadixAll = 2u << 30, kRadixMask = kRadixOwn - 1;
 constexpr uint32_t kRadixMax = kRadixMask;  // pairs, at most
+constexpr uint32_t kRadixPolls = 1u << 12;  // about a microsecond each
 
 // Per pass: bin counts, then per tile and bin the published word, and the next
 // tile; all zero before the sort.
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(kRadixThreads) void radix_pass(const uint32_t* __re
                                                             const uint32_t* __restrict__ vals_in,
                                                             uint32_t* __restrict__ keys_out,
                                                             uint32_t* __restrict__ vals_out, uint32_t n, int pass,
-                                                            RadixWs ws) {
+                                                            uint32_t polls, RadixWs ws) {
     __shared__ uint32_t wh[kRadixWaves][kRadixBins];
     __shared__ uint32_t base[kRadixBins];
     __shared__ uint32_t part[kRadixGroups][kRadixBins];  // look-back: sums, bit 31: includes everything before
@@ -178,7 +181,7 @@ __global__ __launch_bounds__(kRadixThreads) void radix_pass(const uint32_t* __re
         const uint32_t from = seen + group * kRadixBack;
         const uint32_t want = from < tile ? min((uint32_t)kRadixBack, tile - from) : 0u;
         uint32_t sum = 0, got = 0;
-        for (uint32_t poll = 0; got < want && poll < (1u << 20); ++poll) {
+        for (uint32_t poll = 0; got < want && poll < polls; ++poll) {
             uint32_t s[kRadixBack];
 #pragma unroll
             for (int u = 0; u < kRadixBack; ++u)
@@ -190,6 +193,12 @@ __global__ __launch_bounds__(kRadixThreads) void radix_pass(const uint32_t* __re
                 sum += s[u] & kRadixMask;
                 got = (s[u] & kRadixAll) ? want + 1 : got + 1;
             }
+        }
+#pragma unroll 1
+        for (; got < want; ++got) {
+            const uint32_t lo = (tile - 1 - (from + got)) * (kItems * kRadixThreads);
+#pragma unroll 1
+            for (uint32_t k = 0; k < kItems * kRadixThreads; ++k) sum += digit(keys_in[lo + k], pass) == bin ? 1u : 0u;
         }
         part[group][bin] = sum | (got > want ? 0x80000000u : 0u);
         __syncthreads();
@@ -214,7 +223,6 @@ __global__ __launch_bounds__(kRadixThreads) void radix_pass(const uint32_t* __re
         const uint32_t j = i * kRadixThreads + tid;
         if (j >= cnt) continue;
         const uint32_t k = skey[j], to = base[digit(k, pass)] + j;
-        if (to >= n) continue;  // only after the poll limit
         keys_out[to] = k;
         vals_out[to] = sval[j];
     }
@@ -288,7 +296,7 @@ __global__ __launch_bounds__(kRadixThreads) void radix_small(uint32_t* __restric
 // keys: the keys, then the result with vals; keys_tmp, vals_tmp: scratch.
 template <int kPasses>
 inline void radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t n,
-                       const RadixWs& ws, hipStream_t stream) {
+                       const RadixWs& ws, uint32_t polls, hipStream_t stream) {
     static_assert(kPasses % 2 == 0, "the result is in the first buffers");
     if (n <= 4 * kRadixThreads) {  // LBVH build of 2000 faces: 57.6 us, with the launches below 69.7; of 5120 no gain
         auto k = n <= kRadixThreads       ? radix_small<1, kPasses>
@@ -303,7 +311,7 @@ inline void radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint3
         auto k = items == 1 ? radix_pass<1> : items == 2 ? radix_pass<2> : items == 4 ? radix_pass<4> : radix_pass<8>;
         hipLaunchKernelGGL(k, dim3(radix_tiles(n)), dim3(kRadixThreads), 0, stream, odd ? keys_tmp : keys,
                            p == 0 ? nullptr : (odd ? vals_tmp : vals), odd ? keys : keys_tmp, odd ? vals : vals_tmp, n,
-                           p, ws);
+                           p, polls, ws);
     }
 }
 
