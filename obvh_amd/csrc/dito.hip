@@ -95,8 +95,9 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
                                                    uint32_t nsets, uint32_t tile, uint64_t total,
                                                    uint32_t cap_tiles, bool fill, DitoWs ws,
                                                    kr_obb3* out, obvh_dito_trace* trace) {
-    __shared__ uint32_t carry, limit, firsts[kFillSets];
-    __shared__ uint32_t wsum[1024 / kWave];
+    // (sums of tiles in 64 bits: sets that overlap may need any number of them)
+    __shared__ uint64_t carry, wsum[1024 / kWave];
+    __shared__ uint32_t limit, firsts[kFillSets];
     if (threadIdx.x == 0) {
         carry = 0;
         limit = 0xFFFFFFFFu;
@@ -129,34 +130,34 @@ __global__ __launch_bounds__(1024) void dito_setup(const uint64_t* offs, uint64_
                 if (trace) trace[s] = plain_trace(3);
             }
         }
-        uint32_t v = nt;
+        uint64_t v = nt;
         const int lane = lane_id();
 #pragma unroll
         for (int m = 1; m < kWave; m <<= 1) {
-            const uint32_t o = (uint32_t)__shfl_up((int)v, m, kWave);
+            const uint64_t o = __shfl_up((unsigned long long)v, m, kWave);
             if (lane >= m) v += o;
         }
         if (lane == kWave - 1) wsum[wave_id()] = v;
         __syncthreads();
-        uint32_t wpre = 0;
+        uint64_t wpre = 0;
         for (int w = 0; w < wave_id(); ++w) wpre += wsum[w];
-        const uint32_t incl = carry + wpre + v;
+        const uint64_t incl = carry + wpre + v;
         // Offsets that never decrease need at most cap_tiles - 1 tiles.  Where
         // others (sets that overlap) need more than the arrays hold, the sets
         // from the first that does not fit on are invalid: no tiles, a NaN box.
         if (nt != 0 && incl > cap_tiles) {
-            atomicMin(&limit, incl - nt);
+            if (incl - nt <= cap_tiles) atomicMin(&limit, (uint32_t)(incl - nt));  // the first of them
             out[s] = nan_box();
             if (trace) trace[s] = plain_trace(4);
         }
         __syncthreads();
-        const uint32_t first = min(incl - nt, limit);
+        const uint32_t first = (uint32_t)min(incl - nt, (uint64_t)limit);
         if (s < nsets) ws.first_tile[s] = first;
         if (fill && s < nsets) firsts[s] = first;
         if (threadIdx.x == blockDim.x - 1) carry = incl;
         __syncthreads();
     }
-    const uint32_t T = min(carry, limit);
+    const uint32_t T = (uint32_t)min(carry, (uint64_t)limit);
     if (threadIdx.x == 0) ws.first_tile[nsets] = T;
     if (!fill) return;
     // the tile table, as dito_tile_table makes it: four searches of a lane at a time

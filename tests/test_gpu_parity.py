@@ -516,3 +516,20 @@ def test_dito_batch_overlapping_sets_that_just_fit(torch, oracle_lib):
             assert np.isnan(got[4]).all() and g[4]["degenerate"] == 4
         for s in (1, 3, 5):
             assert np.isnan(got[s]).all() and g[s]["degenerate"] == 4, s
+
+
+def test_dito_batch_overlapping_sets_past_2_to_32_tiles(torch, oracle_lib):
+    """Overlapping sets that ask for more than 2^32 tiles in all: those the table holds keep their boxes, all others are
+    invalid (the sums of tiles do not wrap)."""
+    say("[dito_batch] overlapping sets, 2^32 tiles")
+    n = 1 << 22                      # 8192 tiles a set
+    pairs = (1 << 19) + 200          # 2^32 tiles and some more
+    nsets = 2 * pairs - 1
+    p = synth.gaussian_points(n, seed=4)
+    x, y, z = soa(torch, p)
+    off = torch.tensor([0, n], dtype=torch.int64).repeat(pairs).cuda()
+    out = ops.dito_batch(x, y, z, off, tile_points=512).cpu().numpy()
+    fit = (n // 512 + nsets + 1) // 8192  # sets that fit the table
+    exp = oracle_lib.points_obb(p)
+    assert (out[0:2 * fit:2] == exp).all()
+    assert np.isnan(out[1:2 * fit:2]).all() and np.isnan(out[2 * fit:]).all()
