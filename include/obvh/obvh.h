@@ -289,7 +289,7 @@ kr_error obvh_validate_tree_host(const kr_bvh_node* nodes, const u32* parents,
  * bottom-up AABBs/counts/costs), the input side of the transform.
  * Replaces the build in src/ads/lbvh_gpu/lbvh.cu:1547-1692.
  * All pointers are device pointers; nodes/parents/primitive_counts/costs
- * have 2*face_count-1 entries.                                            */
+ * have 2*face_count-1 entries.  At most 2^30 faces (an error above).      */
 size_t obvh_lbvh_workspace_size(u32 face_count);
 kr_error obvh_lbvh_build(const kr_vec3* vertices, const kr_uvec4* faces, u32 face_count,
                          kr_bvh_node* nodes, u32* parents, u32* primitive_counts,

@@ -486,7 +486,6 @@ kr_error obvh_lbvh_build(const kr_vec3* vertices, const kr_uvec4* faces, u32 fac
                          void* workspace, size_t workspace_bytes, void* stream) {
     if (!vertices || !faces || !nodes || !parents || !primitive_counts || !costs)
         return fail("obvh_lbvh_build: NULL array");
-    if (face_count > 0x7FFFFFFFu) return fail("obvh_lbvh_build: too many faces");
     TRY(obvh::lbvh_launch(vertices, faces, face_count, nodes, parents, primitive_counts, costs, mortons_sorted,
                           workspace, workspace_bytes, (hipStream_t)stream));
     return nullptr;

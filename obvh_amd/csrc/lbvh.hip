@@ -19,8 +19,6 @@
 //     lbvh.cu:399-457, in one launch (bottomup.hpp).
 #include <float.h>
 
-#include <rocprim/device/device_radix_sort.hpp>
-
 #include "bottomup.hpp"
 #include "common.hpp"
 #include "lbvh.hpp"
@@ -160,10 +158,6 @@ __global__ __launch_bounds__(1024) void lbvh_codes(const kr_vec3* V, const kr_uv
         if (h[i]) atomicAdd(&ws.radix.hist[i], h[i]);
 }
 
-__global__ __launch_bounds__(256) void lbvh_iota(uint32_t* vals, uint32_t nf) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) vals[i] = i;
-}
-
 // The sorted codes around a workgroup's nodes in LDS (most nodes span a few
 // leaves, so nearly every probe of their searches lands there).
 constexpr int kTreeThreads = 256;
@@ -268,13 +262,6 @@ __global__ __launch_bounds__(kUpTile) void lbvh_aabbs(LbvhUp op, uint32_t nf, ui
     bottom_up(nf, visit, L, op);
 }
 
-size_t lbvh_sort_bytes(uint32_t nf) {
-    size_t bytes = 0;
-    rocprim::radix_sort_pairs((void*)nullptr, bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                              (uint32_t*)nullptr, nf, 0, 30);
-    return bytes;
-}
-
 size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf) {
     Carver c{(char*)base, 0, cap};
     ws->cbox = c.take<int32_t>(8);
@@ -283,17 +270,7 @@ size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf) {
     ws->vals = c.take<uint32_t>(nf);
     ws->keys_tmp = c.take<uint32_t>(nf);
     ws->vals_tmp = c.take<uint32_t>(nf);
-    ws->radix = RadixWs{};
-    ws->sort_bytes = 0;
-    ws->sort_tmp = nullptr;
-    if (nf <= kRadixMax) {
-        radix_carve(&ws->radix, c, nf, kPasses);
-    } else {
-        ws->sort_bytes = lbvh_sort_bytes(nf);
-        ws->sort_tmp = c.take<char>(ws->sort_bytes);
-        ws->radix.hist = c.take<uint32_t>(kPasses * kRadixBins);
-        ws->radix.words = kPasses * kRadixBins;
-    }
+    radix_carve(&ws->radix, c, nf, kPasses);
     return c.used;
 }
 
@@ -301,6 +278,7 @@ kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_no
                      uint32_t* counts, float* costs, uint32_t* mortons, void* workspace, size_t ws_bytes,
                      hipStream_t stream, uint32_t polls) {
     if (nf == 0) return "obvh_lbvh_build: no faces";
+    if (nf > kLbvhMaxFaces) return "obvh_lbvh_build: too many faces";
     LbvhWs ws;
     size_t need = lbvh_carve(&ws, workspace, ws_bytes, nf);
     if (!workspace || ws_bytes < need) return "obvh_lbvh_build: workspace too small";
@@ -311,15 +289,7 @@ kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_no
     hipLaunchKernelGGL(lbvh_centroid_box, dim3(min((nf + kBoxThreads - 1) / kBoxThreads, 256u)), dim3(kBoxThreads), 0,
                        stream, V, F, nf, ws);
     hipLaunchKernelGGL(lbvh_codes, dim3(min((nf + 1023) / 1024, 256u)), dim3(1024), 0, stream, V, F, nf, ws);
-    if (nf <= kRadixMax) {
-        radix_sort<kPasses>(ws.keys, ws.vals, ws.keys_tmp, ws.vals_tmp, nf, ws.radix, polls, stream);
-    } else {  // rocPRIM; its buffers swap roles
-        hipLaunchKernelGGL(lbvh_iota, dim3(gb), dim3(256), 0, stream, ws.vals_tmp, nf);
-        OBVH_HIP_TRY(hipMemcpyAsync(ws.keys_tmp, ws.keys, sizeof(uint32_t) * nf, hipMemcpyDeviceToDevice, stream));
-        size_t sb = ws.sort_bytes;
-        OBVH_HIP_TRY(rocprim::radix_sort_pairs(ws.sort_tmp, sb, ws.keys_tmp, ws.keys, ws.vals_tmp, ws.vals, nf, 0, 30,
-                                               stream));
-    }
+    radix_sort<kPasses>(ws.keys, ws.vals, ws.keys_tmp, ws.vals_tmp, nf, ws.radix, polls, stream);
     hipLaunchKernelGGL(lbvh_tree, blocks(nf, kTreeThreads), dim3(kTreeThreads), 0, stream, nf, ws, nodes, parents,
                        mortons);
     hipLaunchKernelGGL(lbvh_aabbs, up_grid(nf), dim3(kUpTile), 0, stream,

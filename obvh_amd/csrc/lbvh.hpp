@@ -15,9 +15,12 @@ struct LbvhWs {
     uint32_t* keys_tmp;  // the sort's other buffers
     uint32_t* vals_tmp;
     RadixWs radix;
-    char* sort_tmp;      // rocPRIM's scratch (more than 2^30 faces)
-    size_t sort_bytes;
 };
+
+// The tree's search probes up to 2^30 positions past its node in an int (more
+// faces gave a wrong tree), and the sort holds as many pairs.
+constexpr uint32_t kLbvhMaxFaces = 1u << 30;
+static_assert(kLbvhMaxFaces <= kRadixMax, "the sort's limit");
 
 size_t lbvh_carve(LbvhWs* ws, void* base, size_t cap, uint32_t nf);
 kr_error lbvh_launch(const kr_vec3* V, const kr_uvec4* F, uint32_t nf, kr_bvh_node* nodes, uint32_t* parents,

@@ -31,7 +31,7 @@ constexpr int kRadixWaves = kRadixThreads / kWave;
 constexpr int kRadixGroups = kRadixThreads / kRadixBins;  // threads per bin in the look-back
 constexpr int kRadixBack = 16;                            // earlier tiles a thread reads at once
 constexpr uint32_t kRadixOwn = 1u << 30, kRadixAll = 2u << 30, kRadixMask = kRadixOwn - 1;
-constexpr uint32_t kRadixMax = kRadixMask;  // pairs, at most
+constexpr uint32_t kRadixMax = kRadixMask + 1;  // pairs, at most (nobody reads the last tile's word)
 constexpr uint32_t kRadixPolls = 1u << 12;  // about a microsecond each
 
 // Per pass: bin counts, then per tile and bin the published word, and the next

@@ -81,3 +81,13 @@ def test_noalloc_dito_scratch_covers_its_limit():
     one = C.c_void_p(16)
     err = L.obvh_dito_soa_noalloc(one, one, one, limit + 1, one, None, None)
     assert err and b"OBVH_DITO_NOALLOC_MAX_POINTS" in err
+
+
+@pytest.mark.parametrize("nf", [(1 << 30) + 1, 0x7FFFFFFF, 0xFFFFFFFF])
+def test_lbvh_refuses_counts_it_cannot_build(nf):
+    """More than 2^30 faces are an error of their own (the arrays are never touched)."""
+    L = _lib.lib()
+    p = C.c_void_p(256)
+    err = L.obvh_lbvh_build(p, p, nf, p, p, p, p, p, p, 0, None)
+    assert err == b"obvh_lbvh_build: too many faces"
+    assert L.obvh_lbvh_build(p, p, 1 << 30, p, p, p, p, p, p, 0, None) == b"obvh_lbvh_build: workspace too small"
