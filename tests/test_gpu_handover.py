@@ -1,8 +1,9 @@
-"""Hand-overs between the workgroups of one launch when a workgroup does not
-get what it waits for in time (the poll limit set from the host: every kernel
-exits normally), against the oracle."""
+"""Hand-overs between the workgroups of one launch, against the oracle: calls at
+the same time, calls captured in a graph, and launches in which a workgroup
+stops waiting (the poll limit set from the host; every kernel exits normally)."""
 import ctypes as C
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -86,3 +87,91 @@ def test_sort_tiles_that_give_up(torch, oracle_lib, nf):
     assert np.array_equal(t["mortons"].cpu().numpy().view(np.uint32), mortons)
     assert np.array_equal(t["parents"].cpu().numpy().view(np.uint32), parents)
     assert np.array_equal(ops.nodes_to_numpy(t["nodes"]).view(np.uint8), nodes.view(np.uint8))
+
+
+def bits(t):
+    import torch
+
+    return t.contiguous().view(torch.uint8)
+
+
+class Job:
+    """One call that hands over between workgroups, with its own inputs, workspace and expected outputs."""
+
+    def __init__(self, torch, oracle_lib, kind, seed):
+        self.kind, lib = kind, _lib.lib()
+        if kind == "fit":  # 64 tiles
+            p = synth.gaussian_points(131072, seed=seed)
+            self.xyz = [torch.from_numpy(np.ascontiguousarray(p[:, k])).cuda() for k in range(3)]
+            need = lib.obvh_dito_workspace_size(131072)
+        else:
+            V, F = synth.icosphere(80, seed=seed) if kind == "lbvh" else synth.hairball(tubes=1500, seed=seed)
+            self.mesh = torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda()
+            need = (lib.obvh_lbvh_workspace_size if kind == "lbvh" else lib.obvh_atrbvh_workspace_size)(len(F))
+        self.ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        self.expect = self.call()
+        torch.cuda.synchronize()
+        if kind == "fit":
+            assert np.array_equal(self.expect[0].cpu().numpy(), oracle_lib.points_obb(p))
+        else:
+            build = oracle_lib.lbvh_build if kind == "lbvh" else oracle_lib.atrbvh_build
+            assert np.array_equal(ops.nodes_to_numpy(self.expect[0]).view(np.uint8), build(V, F)[0].view(np.uint8))
+
+    def call(self, stream=None):
+        if self.kind == "fit":
+            return (ops.dito(*self.xyz, stream=stream, workspace=self.ws),)
+        build = ops.lbvh_build if self.kind == "lbvh" else ops.atrbvh_build
+        t = build(*self.mesh, stream=stream, workspace=self.ws)
+        return t["nodes"], t["parents"], t["counts"], t["costs"]
+
+    def check(self, got):
+        return all(bool((bits(a) == bits(b)).all()) for a, b in zip(got, self.expect))
+
+
+@pytest.mark.parametrize("kinds", [("fit", "fit"), ("lbvh", "lbvh"), ("atrbvh", "atrbvh"), ("fit", "lbvh", "atrbvh")],
+                         ids="-".join)
+def test_handovers_on_several_streams(torch, oracle_lib, kinds):
+    """Calls that hand over inside a launch, at the same time from a host thread and a stream each."""
+    say(f"[handover] {kinds} at the same time")
+    jobs = [Job(torch, oracle_lib, k, seed=20 + i) for i, k in enumerate(kinds)]
+    streams = [torch.cuda.Stream() for _ in jobs]
+    torch.cuda.synchronize()
+    start, got, errors = threading.Barrier(len(jobs)), [[] for _ in jobs], []
+
+    def run(i):
+        try:
+            start.wait()
+            for _ in range(8):
+                got[i].append(jobs[i].call(streams[i]))
+        except Exception as e:  # reported from the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(len(jobs))]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i, job in enumerate(jobs):
+        for k, out in enumerate(got[i]):
+            assert job.check(out), (i, k)
+
+
+@pytest.mark.parametrize("kind", ["fit", "lbvh", "atrbvh"])
+def test_handovers_captured(torch, oracle_lib, kind):
+    """The same calls captured in a HIP graph and replayed, with eager calls between the replays."""
+    say(f"[handover] {kind} captured, 4 replays")
+    job, other = Job(torch, oracle_lib, kind, seed=30), Job(torch, oracle_lib, kind, seed=31)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = job.call()
+    torch.cuda.synchronize()
+    for rep in range(4):
+        for t in out:
+            t.zero_()
+        eager = other.call()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert job.check(out) and other.check(eager), rep

@@ -533,3 +533,9 @@ def test_dito_batch_overlapping_sets_past_2_to_32_tiles(torch, oracle_lib):
     exp = oracle_lib.points_obb(p)
     assert (out[0:2 * fit:2] == exp).all()
     assert np.isnan(out[1:2 * fit:2]).all() and np.isnan(out[2 * fit:]).all()
+
+
+@pytest.mark.parametrize("nf", [1250000, 1250001])
+def test_lbvh_sort_eight_per_thread(torch, oracle_lib, nf):
+    """The largest count with four pairs per thread, and the smallest with eight."""
+    test_lbvh_sort_edges(torch, oracle_lib, nf, 1000)

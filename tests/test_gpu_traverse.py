@@ -226,3 +226,9 @@ def test_ray_count_edges(torch, oracle_lib, n):
     exp = oracle_lib.obvh_intersect(eL, eR, em, V, F, None, rays, threads=8)
     same_isects(ops.isects_to_numpy(out), exp)
     assert np.array_equal(out_r.cpu().numpy(), out.cpu().numpy())
+
+
+# a wave refills once 24 of its lanes wait: counts around it, and one whose last rays are taken by one refill
+@pytest.mark.parametrize("n", [23, 24, 25, 64 + 24, 64 + 25])
+def test_ray_count_refill(torch, oracle_lib, n):
+    test_ray_count_edges(torch, oracle_lib, n)
