@@ -40,14 +40,6 @@ __device__ __forceinline__ float wave_max(float v) {
     for (int m = 1; m < kWave; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, kWave));
     return v;
 }
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) {
-        uint32_t o = (uint32_t)__shfl_xor((int)v, m, kWave);
-        v = o < v ? o : v;
-    }
-    return v;
-}
 
 // Integer min / max over the 64 lanes, result uniform (in every lane).  Four
 // DPP steps leave each 16-lane row's result in all of its lanes (xor 1, xor 2,

@@ -2169,7 +2169,7 @@ __device__ __forceinline__ uint32_t of_group(Of of, Begin begin, uint32_t i, uin
 __global__ void batch_gather_nodes(BatchMap m, const kr_bvh_node* __restrict__ nodes,
                                    const uint32_t* __restrict__ parents, uint2* cn, uint32_t* cp,
                                    uint32_t* berr, uint32_t total_in) {
-    const uint32_t I = m.Nsum - 1, total = 2 * m.Nsum - 1;
+    const uint32_t total = 2 * m.Nsum - 1;
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total_in; g += gridDim.x * blockDim.x) {
         const uint32_t t = of_group([&](uint32_t i) { return batch_tree_of_node(m, i); },
                                     [&](uint32_t k) { return 2u * m.prim_off[k] - k; }, g, total_in);
@@ -2202,7 +2202,6 @@ __global__ void batch_gather_nodes(BatchMap m, const kr_bvh_node* __restrict__ n
         cn[idx] = make_uint2(0u, 0u);
         cp[idx] = kInvalid;
     }
-    (void)I;
 }
 
 // One lane per face: vertex ids rebased to the batch's vertex array.
