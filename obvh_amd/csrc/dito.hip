@@ -734,21 +734,29 @@ __global__ __launch_bounds__(kBlock) void dito_cand(PtsSoA pts, const uint64_t* 
 
 // --------------------------------------------------------------- pass 2 --
 
+// Each lane's ranges of a tile's cnt points on the set's three axes (min b0..b2,
+// max b0..b2).
+template <class T>
+__device__ __forceinline__ void tile_ranges(const T& pts, uint32_t cnt, const SetState* st, float (&r)[6]) {
+    const float INF = FLT_MAX * 2.0f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { r[k] = INF; r[3 + k] = -INF; }
+    if (st->mode == 1) return;
+    f3 b[3];
+    state_axes(*st, b);
+    stream_tile(pts, cnt, [&](uint32_t, const f3 (&p)[kRows]) {
+#pragma unroll
+        for (int j = 0; j < kRows; j += 2) axes_step(p[j], p[j + 1], b, r);
+    });
+}
+
 // Ranges of a tile's cnt points on the set's three axes: 6 floats (min b0..b2,
 // max b0..b2) written to out6 by threads 0..7.  Ends with a barrier.
 template <class T>
 __device__ __forceinline__ void tile_pass2(const T& pts, uint32_t cnt, const SetState* st, FitLds<kBlock>& L,
                                            float* out6) {
-    const float INF = FLT_MAX * 2.0f;
-    float r[6] = {INF, INF, INF, -INF, -INF, -INF};
-    if (st->mode != 1) {
-        f3 b[3];
-        state_axes(*st, b);
-        stream_tile(pts, cnt, [&](uint32_t, const f3 (&p)[kRows]) {
-#pragma unroll
-            for (int j = 0; j < kRows; j += 2) axes_step(p[j], p[j + 1], b, r);
-        });
-    }
+    float r[6];
+    tile_ranges(pts, cnt, st, r);
 #pragma unroll
     for (int k = 3; k < 6; ++k) r[k] = -r[k];
     const float y = wave_min6(r);
@@ -857,58 +865,6 @@ __global__ __launch_bounds__(kBlock) void dito_final(PtsSoA pts, const uint64_t*
     const uint32_t ft = ws.first_tile[s], nt = ws.first_tile[s + 1] - ft;
     if (nt == 0) return;
     set_final(pts, sbeg, ft, nt, ws.part2, &ws.state[s], &out[s], &trace[s]);
-}
-
-// ------------------------------------------------- one set, two launches --
-//
-// A single set of n > 0 points in tiles of `tile` points, one workgroup per
-// tile (grid = tile count).  Launch A: slab extremes per tile; the last
-// workgroup to finish (completion counter done[0]) reduces them and runs the
-// candidate search.  Launch B: axis ranges per tile; the last workgroup
-// (done[1]) reduces them and writes the box.  A workgroup publishes its tile
-// result with one agent-scope release (the atomic on the counter); the last
-// one acquires before reading the others'.  The counters must be zero before
-// the first call on a workspace (dito_one_clear, or a clear at allocation);
-// each last workgroup resets its counter, so later calls need no clear.
-
-__global__ void dito_one_clear(DitoWs ws) {
-    if (threadIdx.x < 4) ws.done[threadIdx.x] = 0;
-}
-
-template <class P>
-__global__ __launch_bounds__(kBlock) void dito_one_a(P pts, uint64_t n, uint32_t tile, DitoWs ws,
-                                                     obvh_dito_trace* trace) {
-    __shared__ FitLds<kBlock> L;
-    const uint32_t t = blockIdx.x, T = gridDim.x;
-    const uint64_t base = (uint64_t)t * tile;
-    tile_pass1(tile_of(pts, base), (uint32_t)min((uint64_t)tile, n - base), L);
-    // threads 0..13 (wave 0) write the tile's pairs; thread 0's release
-    // orders them before its count
-    store_pairs(L, (uint32_t)base, &ws.part1_v[(size_t)t * 14], &ws.part1_i[(size_t)t * 14]);
-    if (threadIdx.x == 0)
-        L.last = __hip_atomic_fetch_add(&ws.done[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
-    __syncthreads();
-    if (!L.last || wave_id() != 0) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    set_cand(pts, 0, n, 0, T, ws.part1_v, ws.part1_i, ws.state, trace);
-    if (lane_id() == 0) __hip_atomic_store(&ws.done[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <class P>
-__global__ __launch_bounds__(kBlock) void dito_one_b(P pts, uint64_t n, uint32_t tile, DitoWs ws, kr_obb3* out,
-                                                     obvh_dito_trace* trace) {
-    __shared__ FitLds<kBlock> L;
-    const uint32_t t = blockIdx.x, T = gridDim.x;
-    const uint64_t base = (uint64_t)t * tile;
-    tile_pass2(tile_of(pts, base), (uint32_t)min((uint64_t)tile, n - base), ws.state, L,
-               &ws.part2[(size_t)t * 6]);  // threads 0..7 write
-    if (threadIdx.x == 0)
-        L.last = __hip_atomic_fetch_add(&ws.done[1], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == T - 1;
-    __syncthreads();
-    if (!L.last || wave_id() != 0) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    set_final(pts, 0, 0, T, ws.part2, ws.state, out, trace);
-    if (lane_id() == 0) __hip_atomic_store(&ws.done[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ------------------------------------------------------- one-launch fits --
@@ -1119,12 +1075,17 @@ __device__ __forceinline__ void tile_box(P pts, uint64_t sbeg, float (&r)[6], ui
         if ((uint32_t)__builtin_amdgcn_readfirstlane((int)old) != nt - 1) return;
         asm volatile("" ::: "memory");
         float q[6] = {INF, INF, INF, -INF, -INF, -INF};
-        for (uint32_t j = lane; j < nt; j += kWave) {
-            float o[6];
+        for (uint32_t j0 = lane; j0 < nt; j0 += 4 * kWave) {  // four tiles of a lane a trip to memory
+            float o[4][6];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) o[k] = ld_agent(&ws.part2[(size_t)(ft + j) * 6 + k]);
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int k = 0; k < 3; ++k) { q[k] = fminf(q[k], o[k]); q[3 + k] = fmaxf(q[3 + k], o[3 + k]); }
+                for (int k = 0; k < 6; ++k)
+                    o[u][k] = ld_agent(&ws.part2[(size_t)(ft + min(j0 + u * kWave, nt - 1)) * 6 + k]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) { q[k] = fminf(q[k], o[u][k]); q[3 + k] = fmaxf(q[3 + k], o[u][3 + k]); }
         }
 #pragma unroll
         for (int k = 3; k < 6; ++k) q[k] = -q[k];
@@ -1220,6 +1181,37 @@ __global__ __launch_bounds__(kThreads) void dito_one(P pts, uint64_t n, DitoWs w
     one_tile<P, J, kThreads>(pts, n, blockIdx.x, gridDim.x, ws, polls, out, trace, L);
 }
 
+__global__ void dito_one_clear(DitoWs ws) {
+    if (threadIdx.x < 4) ws.done[threadIdx.x] = 0;
+}
+
+// ------------------------------------------------------- two-launch fits --
+//
+// Sets of more tiles than may wait: the same hand-overs, the slab pass with the
+// search and the axis pass with the box in a launch each.
+
+template <class P>
+__global__ __launch_bounds__(kBlock) void dito_one_a(P pts, uint64_t n, uint32_t tile, DitoWs ws,
+                                                     obvh_dito_trace* trace) {
+    __shared__ FitLds<kBlock> L;
+    const uint64_t base = (uint64_t)blockIdx.x * tile;
+    tile_pass1(tile_of(pts, base), (uint32_t)min((uint64_t)tile, n - base), L);
+    uint32_t gave;
+    tile_search(pts, 0, n, (uint32_t)base, blockIdx.x, 0, gridDim.x, ws, ws.state, reinterpret_cast<FitSync*>(ws.done),
+                trace, L, gave);
+}
+
+template <class P>
+__global__ __launch_bounds__(kBlock) void dito_one_b(P pts, uint64_t n, uint32_t tile, DitoWs ws, kr_obb3* out,
+                                                     obvh_dito_trace* trace) {
+    __shared__ FitLds<kBlock> L;
+    if (threadIdx.x == 0) L.st = *ws.state;
+    const uint64_t base = (uint64_t)blockIdx.x * tile;
+    float r[6];
+    tile_ranges(tile_of(pts, base), (uint32_t)min((uint64_t)tile, n - base), ws.state, r);
+    tile_box(pts, 0, r, blockIdx.x, 0, gridDim.x, ws, reinterpret_cast<FitSync*>(ws.done), out, trace, L);
+}
+
 // ----------------------------------------------------------------- host --
 
 size_t dito_max_tiles(uint32_t nsets, uint64_t total, uint32_t tile) {
@@ -1291,9 +1283,8 @@ static void launch_one(P p, uint64_t n, uint32_t tile, uint32_t T, uint32_t cap,
                            polls, out, trace);
         return;
     }
-    obvh_dito_trace* tr = trace ? trace : ws.trace_tmp;
-    hipLaunchKernelGGL(dito_one_a<P>, dim3(T), dim3(kBlock), 0, stream, p, n, tile, ws, tr);
-    hipLaunchKernelGGL(dito_one_b<P>, dim3(T), dim3(kBlock), 0, stream, p, n, tile, ws, out, tr);
+    hipLaunchKernelGGL(dito_one_a<P>, dim3(T), dim3(kBlock), 0, stream, p, n, tile, ws, trace);
+    hipLaunchKernelGGL(dito_one_b<P>, dim3(T), dim3(kBlock), 0, stream, p, n, tile, ws, out, trace);
 }
 
 kr_error dito_one_launch(const float* x, const float* y, const float* z, const float* xyz, uint64_t n,
