@@ -116,7 +116,8 @@ kr_error noalloc_scratch(void** out, bool* first) {
     return nullptr;
 }
 
-// The two-launch fit ran on the current device's `scratch`: its counters are zero from now on.
+// A fit of several tiles ran on the current device's `scratch`: its counters are
+// zero from now on (a fit of one workgroup does not touch them).
 void noalloc_scratch_used() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return;

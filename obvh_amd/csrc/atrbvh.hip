@@ -280,16 +280,22 @@ __global__ void atr_clear(AtrWs ws, uint32_t nf) { pass_clear(ws, nf); }
 // 8192-leaf workgroups and one for the rest, 255 and 260 now), and reads stay L2 hits (past the L2, for all XCDs, a trip takes twice as
 // long, four of them a treelet).  The grid covers every CU of the chip; the
 // first workgroup to arrive names the XCD, those of the others end.  Any one
-// workgroup would do all the work.
+// workgroup would do all the work.  Builds at the same time tend to share an
+// XCD: one 200 K hairball takes 945 us, 2 and 4 on as many streams 1105 and 1458
+// (5674, 5765 and 6032 us in phases of single workgroups).
 constexpr int kXccId = 20 | (4 - 1) << 11;  // s_getreg: XCC_ID, 4 bits
 constexpr int kTopNext = 32;  // of ws.top: entries taken ([0]: the XCD, plus one); a cache line of its own
 constexpr int kTopThreads = 512;      // 16 half-waves per CU (8 take the same time)
 constexpr uint32_t kTopBlocks = 256;  // a workgroup per CU of every XCD
 // From this many leaves on, 8192-leaf workgroups on all XCDs come between: the
-// roots are then more than one XCD's 512 half-waves are quick with.  Builds
-// with treelet size 7, 2 passes, without / with: 338 K triangles 1308 / 1155 us,
-// 400 K hairball 1442 / 1255, 1 M 2848 / 1850, 2 M 5290 / 2950 (with 4096 leaves
-// 2 M 3295 and 338 K 1125, with 16384 2922 and 1194).
+// roots are then more than one XCD's 512 half-waves are quick with.  Builds of
+// icospheres and hairballs, 2 passes, without / with them, treelet size 7: 68 K
+// 611-637 / 780-803 us, 180 K 834-843 / 900-919, 220 K 923-930 / 945-978, 260 K
+// 991-997 / 974-996, 300 K 1231-1241 / 1119-1156, 340 K 1304 / 1152-1207; size 9:
+// 220 K 1019-1045 / 1089-1138, 260 K 1077 / 1104-1148, 300 K 1322-1345 /
+// 1259-1316, 340 K 1406-1417 / 1282-1357.  400 K hairball 1442 / 1255, 1 M 2848 /
+// 1850, 2 M 5290 / 2950 (with 4096 leaves 2 M 3295 and 338 K 1125, with 16384
+// 2922 and 1194).
 constexpr uint32_t kTopLeaves = 1u << 18;
 
 constexpr int kDistStride = kMaxTreelet + 1;  // odd: the lanes of a row update touch different banks

@@ -785,12 +785,13 @@ __global__ __launch_bounds__(kTile) void climb_leaves(TreeNodes nodes,
 // appended to a list for the candidate search.
 //
 // Bound by latency: a level takes 1.5 us on an idle chip (5120 triangles: 15
-// levels, 23 us) and 3 us beside the candidate search (1M triangles: 26 levels,
-// 77 us, 2M 117 us), which hides it.  Without the loads ahead 114 and 334 us;
-// with eight paths in a wave from the start 107, 226, and 31 us for 5120
-// triangles (a wave is as slow as its slowest path).  Before, 32768-leaf
-// workgroups with hand-overs in LDS and one last workgroup took 106, 190 and
-// 30 us.  Random topology (nearly every node is up here), whole transform:
+// levels, 23 us) and 3 us beside the candidate search, which hides it (26 levels
+// of a 1M icosphere 91 us, a 2M one 128, a 2M hairball's ATRBVH 215).  Timed
+// against each other on 1M and 2M triangles: 77 and 117 us; without the loads
+// ahead 114 and 334; with eight paths in a wave from the start 107, 226, and 31
+// for 5120 triangles (a wave is as slow as its slowest path); 32768-leaf
+// workgroups with hand-overs in LDS and one last workgroup, which it replaced,
+// 106, 190 and 30.  Random topology (nearly every node is up here), whole transform:
 // 100000 leaves 14.1 ms then, 8.6 now.  The waves run at raised priority: they
 // are few, and issue little between their waits.
 struct Topo {  // children, parent and arrival word of a node (zero / kInvalid past the internal nodes)

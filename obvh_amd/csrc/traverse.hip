@@ -38,9 +38,12 @@
 // Data per internal node visit: metadata 8 B + two 48 B matrices; per
 // triangle: face 16 B + three 12 B vertices.
 //
-// Bound by VALU issue (373 instructions an iteration at 5 waves per SIMD) and
-// the long rays: on 1M rays (60 steps on average, 600 the longest) a wave has
-// 56 lanes busy until no ray is left to take, 14 in its last iterations.
+// Bound by VALU issue (380 instructions an iteration at 5 waves per SIMD) with
+// 20 or 21 of 64 lanes active in an instruction, and by the long rays.  On 1M
+// rays into 1M triangles (camera / random; 61 / 66 steps a ray, 600 the longest)
+// a wave has 55 / 51 lanes busy until no ray is left to take, 13 / 12 after that,
+// in a third of its iterations; 33 / 31 lanes are in a node step (99 % of the
+// iterations), 11 / 10 in a triangle step (86 %).
 // Merging a workgroup's waves then (rays handed over through LDS) and an exact
 // entry test for flat boxes by axis pairs gained nothing: the first lengthens
 // the longest rays' iterations, the second costs registers.
@@ -367,8 +370,9 @@ __global__ __launch_bounds__(kTravThreads) void trace(Tree tree, TraceIO a) {
 
     // A finished ray's record.  The lanes that wait for a refill write theirs
     // together: at each ray's end it ran for one or two lanes at a time, in a
-    // third of all iterations, with two dependent loads (1M camera rays 1740 us
-    // then, 1670 now, random rays 1563 and 1500).
+    // third of all iterations, with two dependent loads.  (1M camera rays 1740 us
+    // then, 1670 with this, random rays 1563 and 1500; with the refill at 24 as
+    // well, side by side, 1717 -> 1628 and 1538 -> 1442.)
     auto finish = [&]() {
         kr_intersection o;
         o.instance = aborted ? kTravAborted : 0u;

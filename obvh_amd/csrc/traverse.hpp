@@ -15,8 +15,14 @@ constexpr int kTravDeepSlots = kTravSlots - kTravLdsSlots;  // 25..63 in global 
 constexpr uint32_t kTravMaxBlocks = 2048;      // persistent grid cap (256 CUs x 8)
 constexpr uint32_t kTravAborted = 0xFFFFFFFFu; // kr_intersection.instance of an aborted ray
 // Idle lanes that trigger a refill of the wave.  Rays taken together stay
-// together: 1M camera / random rays with 8 1920 / 1870 us, 12 1725 / 1590, 16 1635 /
-// 1430, 24 1604 / 1412, 32 1614 / 1437, 40 1632 / 1497.
+// together: 1M camera (SoA) / random (records) rays into 1M triangles with 8
+// 1920 / 1870 us, 12 1725 / 1590, 16 1635 / 1430, 24 1604 / 1412, 32 1614 / 1437,
+// 40 1632 / 1497.  16 against 24 in one run: 1M rays into icospheres of 2 K
+// triangles 544 / 719 and 472 / 576 us, 72 K 825 / 921 and 705 / 768, 1M 1628 /
+// 1467 and 1628 / 1442, into hairballs of 40 K 803 / 1086 and 767 / 1097, 400 K
+// 2554 / 3023 and 2543 / 3080.  Up to 100 K rays, few of which are ever refilled,
+// the two differ by up to 3 % either way (100 K random rays into 2 K triangles
+// 110 and 112).
 constexpr int kTravRefill = 24;
 // Every lane asks the counter for at most one ray past the end, so it never
 // exceeds ray_count + 64 x (waves of the grid); this bound keeps it in range.

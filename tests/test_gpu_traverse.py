@@ -212,6 +212,7 @@ def test_empty_and_all_miss(torch, oracle_lib):
 
 # ray counts around a wave, its refill (16 idle lanes) and the lanes of the whole grid (524288): records are written when
 # lanes wait for a refill and at a wave's end
+# (the refill is at 24 idle lanes: test_ray_count_refill has the counts around it)
 @pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 1000, 600001])
 def test_ray_count_edges(torch, oracle_lib, n):
     say(f"[traverse] {n} rays")
