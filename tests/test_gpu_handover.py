@@ -100,10 +100,11 @@ class Job:
 
     def __init__(self, torch, oracle_lib, kind, seed):
         self.kind, lib = kind, _lib.lib()
-        if kind == "fit":  # 64 tiles
-            p = synth.gaussian_points(131072, seed=seed)
+        if kind in ("fit", "large"):  # 64 tiles in one launch, 196 in two
+            n = 131072 if kind == "fit" else 400001
+            p = synth.gaussian_points(n, seed=seed)
             self.xyz = [torch.from_numpy(np.ascontiguousarray(p[:, k])).cuda() for k in range(3)]
-            need = lib.obvh_dito_workspace_size(131072)
+            need = lib.obvh_dito_workspace_size(n)
         else:
             V, F = synth.icosphere(80, seed=seed) if kind == "lbvh" else synth.hairball(tubes=1500, seed=seed)
             self.mesh = torch.from_numpy(V).cuda(), torch.from_numpy(F.view(np.int32)).cuda()
@@ -111,14 +112,14 @@ class Job:
         self.ws = torch.empty(need, dtype=torch.uint8, device="cuda")
         self.expect = self.call()
         torch.cuda.synchronize()
-        if kind == "fit":
+        if kind in ("fit", "large"):
             assert np.array_equal(self.expect[0].cpu().numpy(), oracle_lib.points_obb(p))
         else:
             build = oracle_lib.lbvh_build if kind == "lbvh" else oracle_lib.atrbvh_build
             assert np.array_equal(ops.nodes_to_numpy(self.expect[0]).view(np.uint8), build(V, F)[0].view(np.uint8))
 
     def call(self, stream=None):
-        if self.kind == "fit":
+        if self.kind in ("fit", "large"):
             return (ops.dito(*self.xyz, stream=stream, workspace=self.ws),)
         build = ops.lbvh_build if self.kind == "lbvh" else ops.atrbvh_build
         t = build(*self.mesh, stream=stream, workspace=self.ws)
@@ -128,7 +129,8 @@ class Job:
         return all(bool((bits(a) == bits(b)).all()) for a, b in zip(got, self.expect))
 
 
-@pytest.mark.parametrize("kinds", [("fit", "fit"), ("lbvh", "lbvh"), ("atrbvh", "atrbvh"), ("fit", "lbvh", "atrbvh")],
+@pytest.mark.parametrize("kinds", [("fit", "fit"), ("large", "large"), ("lbvh", "lbvh"), ("atrbvh", "atrbvh"),
+                                   ("fit", "large", "lbvh", "atrbvh")],
                          ids="-".join)
 def test_handovers_on_several_streams(torch, oracle_lib, kinds):
     """Calls that hand over inside a launch, at the same time from a host thread and a stream each."""
@@ -158,7 +160,7 @@ def test_handovers_on_several_streams(torch, oracle_lib, kinds):
             assert job.check(out), (i, k)
 
 
-@pytest.mark.parametrize("kind", ["fit", "lbvh", "atrbvh"])
+@pytest.mark.parametrize("kind", ["fit", "large", "lbvh", "atrbvh"])
 def test_handovers_captured(torch, oracle_lib, kind):
     """The same calls captured in a HIP graph and replayed, with eager calls between the replays."""
     say(f"[handover] {kind} captured, 4 replays")
